@@ -375,6 +375,31 @@ int mpsa_attn_fwd_routed(const uint8_t* q4, const uint8_t* qs4, const uint8_t* q
                          int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal,
                          const int32_t* order, const int32_t* counts, mpsa_stream_t stream);
 
+/*
+ * A whole attention call -- smooth-K mean, operand preparation, routing or tile skipping, attention -- on one block of
+ * caller-owned memory: the body of the reference's wrapper (ours/mxfp_attn_kernel.py:19-100) behind one entry point, for
+ * callers whose short calls are bound by the host.  The same kernels with the same results as the separate entry points.
+ * A description holds no pointers and can be kept and shared between threads; one that is not valid gives the error of
+ * the entry point that refuses it.
+ */
+typedef struct mpsa_attn_desc {
+    int64_t B, Hq, Hkv, nq, nk, D;
+    int64_t q_strides[4], k_strides[4], v_strides[4], o_strides[4];   /* elements, in [B,H,N,D] order */
+    int32_t dtype;          /* of q, k, v: MPSA_BF16 | MPSA_F16 (P follows it) */
+    int32_t o_dtype;
+    int32_t tile, causal, mode, fmt8;
+    int32_t smooth_k;       /* subtract K's mean over the sequence */
+    int32_t skip;           /* skip_thresh is given: the tile-skipping rule, or the router's skip class in MPSA_MODE_ROUTED */
+    float pre_scale_q;      /* sm_scale * log2(e) */
+    float skip_thresh, route_thresh;
+} mpsa_attn_desc;
+
+/* bytes of workspace a call of this description needs (16-byte aligned), or a negative MPSA_E* code */
+int64_t mpsa_attn_call_workspace(const mpsa_attn_desc* desc);
+/* skipped_share: NULL, or one float that receives the share of the visited tile pairs that a skipping or routed run left out */
+int mpsa_attn_call(const mpsa_attn_desc* desc, const void* q, const void* k, const void* v, void* o, void* workspace,
+                   float* skipped_share, mpsa_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -27,6 +27,11 @@ static inline bool mpsa_aligned16(const void* p) { return (reinterpret_cast<uint
 bool mpsa_register_lds_kernel(const void* kern, int bytes);      // api.hip; always returns true
 int mpsa_ensure_init();                                          // api.hip; MPSA_OK or the failure of mpsa_init()
 int mpsa_seq_mean_static_resolve();                              // quantize.hip; address of the built-in partial-sum array
+// prepare.hip: the operand preparation with the sets to make named apart for Q and K
+int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                          int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int64_t D, int tile, int fmt8, float pre_scale_q,
+                          const void* k_sub, bool q_do4, bool q_do8, bool k_do4, bool k_do8, uint8_t* q4, uint8_t* qs4, uint8_t* q8, uint8_t* qs8,
+                          uint8_t* k4, uint8_t* ks4, uint8_t* k8, uint8_t* ks8, void* v_tiles, hipStream_t st);
 
 #define MPSA_CHECK_LAUNCH(what)                                                        \
     do {                                                                               \

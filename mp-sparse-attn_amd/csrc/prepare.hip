@@ -53,9 +53,9 @@ void launch_td(const PrepArgs& p, int tile, int d, unsigned grid, hipStream_t st
 }
 
 template <int XDT>
-void launch_mode(const PrepArgs& p, int mode, int fmt8, int tile, int d, unsigned grid, hipStream_t st) {
-    if (mode == MPSA_MODE_MXFP4) launch_td<XDT, true, false, MPSA_FMT_E4M3>(p, tile, d, grid, st);
-    else if (mode == MPSA_MODE_MXFP8) {
+void launch_mode(const PrepArgs& p, bool do4, bool do8, int fmt8, int tile, int d, unsigned grid, hipStream_t st) {
+    if (!do8) launch_td<XDT, true, false, MPSA_FMT_E4M3>(p, tile, d, grid, st);
+    else if (!do4) {
         if (fmt8 == MPSA_FMT_E5M2) launch_td<XDT, false, true, MPSA_FMT_E5M2>(p, tile, d, grid, st);
         else                       launch_td<XDT, false, true, MPSA_FMT_E4M3>(p, tile, d, grid, st);
     } else {
@@ -65,6 +65,53 @@ void launch_mode(const PrepArgs& p, int mode, int fmt8, int tile, int d, unsigne
 }
 
 }  // namespace
+
+// Host side of the preparation: which of the operand sets are made is up to the caller (do4 / do8 of either side; the
+// mixed mode multiplies 8-bit Q with 4-bit K and needs one set of each).
+int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                          int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int64_t D, int tile, int fmt8, float pre_scale_q,
+                          const void* k_sub, bool q_do4, bool q_do8, bool k_do4, bool k_do8, uint8_t* q4, uint8_t* qs4, uint8_t* q8, uint8_t* qs8,
+                          uint8_t* k4, uint8_t* ks4, uint8_t* k8, uint8_t* ks8, void* v_tiles, hipStream_t st) {
+    const int64_t nq_pad = (Nq + tile - 1) / tile * tile, nk_pad = (Nk + tile - 1) / tile * tile;
+    constexpr int EMAX4 = 3, EMAX8 = 7;            // ours/quant_mxint8.py:303, :191
+    if (mpsa_quantize_sw_encoders() && q) {
+        // the cross-checking encoders exist only as stand-alone kernels
+        auto one = [&](const void* x, int64_t H, int64_t N, const int64_t* xs, const void* sub, float pre, bool do4, bool do8,
+                       uint8_t* c4, uint8_t* s4, uint8_t* c8, uint8_t* s8, int64_t rows) {
+            if (do4 && do8) return mpsa_quantize_mx_dual(x, dtype, B, H, N, D, xs, sub, pre, EMAX4, fmt8, EMAX8, c4, s4, c8, s8, rows, st);
+            return mpsa_quantize_mx(x, dtype, B, H, N, D, xs, sub, pre, do4 ? MPSA_FMT_E2M1 : fmt8, do4 ? EMAX4 : EMAX8, do4 ? c4 : c8, do4 ? s4 : s8, rows, st);
+        };
+        int rc = one(q, Hq, Nq, q_strides, nullptr, pre_scale_q, q_do4, q_do8, q4, qs4, q8, qs8, nq_pad);
+        if (rc != MPSA_OK) return rc;
+        rc = one(k, Hkv, Nk, k_strides, k_sub, 1.0f, k_do4, k_do8, k4, ks4, k8, ks8, nk_pad);
+        if (rc != MPSA_OK) return rc;
+        return mpsa_v_tiles(v, dtype, B, Hkv, Nk, D, v_strides, tile, v_tiles, st);
+    }
+    PrepArgs p;
+    unsigned bq = 0, bk = 0, bv = 0;
+    int rc = MPSA_OK;
+    if (q) {
+        rc = mpsa_quantize_setup(q, dtype, B, Hq, Nq, D, q_strides, nullptr, pre_scale_q, q_do4, EMAX4, q_do8, fmt8, EMAX8, q4, qs4, q8, qs8, nq_pad, &p.q, &bq);
+        if (rc != MPSA_OK) return rc;
+    } else {
+        p.q = QuantArgs{};                       // no Q job: the attention kernel quantizes Q itself (mpsa_attn_fwd_q16)
+        q_do4 = q_do8 = false;
+    }
+    rc = mpsa_quantize_setup(k, dtype, B, Hkv, Nk, D, k_strides, k_sub, 1.0f, k_do4, EMAX4, k_do8, fmt8, EMAX8, k4, ks4, k8, ks8, nk_pad, &p.k, &bk);
+    if (rc != MPSA_OK) return rc;
+    rc = mpsa_v_tiles_setup(v, dtype, B, Hkv, Nk, D, v_strides, tile, v_tiles, &p.v, &bv);
+    if (rc != MPSA_OK) return rc;
+    const int64_t total = (int64_t)bq * Hq * B + (int64_t)(bk + bv) * Hkv * B;
+    if (total >= (int64_t(1) << 31)) return mpsa_fail(MPSA_EUNSUPPORTED, "prepare: problem too large for one launch");
+    p.bq = bq; p.bk = bk; p.bv = bv; p.hq = (uint32_t)Hq; p.hkv = (uint32_t)Hkv;
+    p.q_total = (uint32_t)((int64_t)bq * Hq * B); p.k_total = (uint32_t)((int64_t)bk * Hkv * B);
+    p.v_total = (uint32_t)((int64_t)bv * Hkv * B);
+    const bool do4 = q_do4 || k_do4, do8 = q_do8 || k_do8;
+    if (dtype == MPSA_BF16) launch_mode<MPSA_BF16>(p, do4, do8, fmt8, tile, (int)D, (unsigned)((total + 1) / 2), st);
+    else                    launch_mode<MPSA_F16>(p, do4, do8, fmt8, tile, (int)D, (unsigned)((total + 1) / 2), st);
+    MPSA_CHECK_LAUNCH("prepare");
+    return MPSA_OK;
+}
 
 extern "C" int mpsa_attn_prepare(const void* q, const int64_t q_strides[4], const void* k, const int64_t k_strides[4],
                                  const void* v, const int64_t v_strides[4], int dtype,
@@ -77,39 +124,6 @@ extern "C" int mpsa_attn_prepare(const void* q, const int64_t q_strides[4], cons
     if (tile != 64 && tile != 128) return mpsa_fail(MPSA_EUNSUPPORTED, "prepare: tile must be 64 or 128 (got %d)", tile);
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || Nq <= 0 || Nk <= 0 || Hq % Hkv) return mpsa_fail(MPSA_EINVAL, "prepare: bad shape (B=%lld Hq=%lld Hkv=%lld Nq=%lld Nk=%lld)", (long long)B, (long long)Hq, (long long)Hkv, (long long)Nq, (long long)Nk);
     const bool do4 = mode != MPSA_MODE_MXFP8, do8 = mode != MPSA_MODE_MXFP4;
-    const int64_t nq_pad = (Nq + tile - 1) / tile * tile, nk_pad = (Nk + tile - 1) / tile * tile;
-    constexpr int EMAX4 = 3, EMAX8 = 7;            // ours/quant_mxint8.py:303, :191
-    if (mpsa_quantize_sw_encoders() && q) {
-        // the cross-checking encoders exist only as stand-alone kernels
-        int rc = do4 && do8 ? mpsa_quantize_mx_dual(q, dtype, B, Hq, Nq, D, q_strides, nullptr, pre_scale_q, EMAX4, fmt8, EMAX8, q4, qs4, q8, qs8, nq_pad, stream)
-                            : mpsa_quantize_mx(q, dtype, B, Hq, Nq, D, q_strides, nullptr, pre_scale_q, do4 ? MPSA_FMT_E2M1 : fmt8, do4 ? EMAX4 : EMAX8, do4 ? q4 : q8, do4 ? qs4 : qs8, nq_pad, stream);
-        if (rc != MPSA_OK) return rc;
-        rc = do4 && do8 ? mpsa_quantize_mx_dual(k, dtype, B, Hkv, Nk, D, k_strides, k_sub, 1.0f, EMAX4, fmt8, EMAX8, k4, ks4, k8, ks8, nk_pad, stream)
-                        : mpsa_quantize_mx(k, dtype, B, Hkv, Nk, D, k_strides, k_sub, 1.0f, do4 ? MPSA_FMT_E2M1 : fmt8, do4 ? EMAX4 : EMAX8, do4 ? k4 : k8, do4 ? ks4 : ks8, nk_pad, stream);
-        if (rc != MPSA_OK) return rc;
-        return mpsa_v_tiles(v, dtype, B, Hkv, Nk, D, v_strides, tile, v_tiles, stream);
-    }
-    PrepArgs p;
-    unsigned bq = 0, bk = 0, bv = 0;
-    int rc = MPSA_OK;
-    if (q) {
-        rc = mpsa_quantize_setup(q, dtype, B, Hq, Nq, D, q_strides, nullptr, pre_scale_q, do4, EMAX4, do8, fmt8, EMAX8, q4, qs4, q8, qs8, nq_pad, &p.q, &bq);
-        if (rc != MPSA_OK) return rc;
-    } else {
-        p.q = QuantArgs{};                       // no Q job: the attention kernel quantizes Q itself (mpsa_attn_fwd_q16)
-    }
-    rc = mpsa_quantize_setup(k, dtype, B, Hkv, Nk, D, k_strides, k_sub, 1.0f, do4, EMAX4, do8, fmt8, EMAX8, k4, ks4, k8, ks8, nk_pad, &p.k, &bk);
-    if (rc != MPSA_OK) return rc;
-    rc = mpsa_v_tiles_setup(v, dtype, B, Hkv, Nk, D, v_strides, tile, v_tiles, &p.v, &bv);
-    if (rc != MPSA_OK) return rc;
-    const int64_t total = (int64_t)bq * Hq * B + (int64_t)(bk + bv) * Hkv * B;
-    if (total >= (int64_t(1) << 31)) return mpsa_fail(MPSA_EUNSUPPORTED, "prepare: problem too large for one launch");
-    p.bq = bq; p.bk = bk; p.bv = bv; p.hq = (uint32_t)Hq; p.hkv = (uint32_t)Hkv;
-    p.q_total = (uint32_t)((int64_t)bq * Hq * B); p.k_total = (uint32_t)((int64_t)bk * Hkv * B);
-    p.v_total = (uint32_t)((int64_t)bv * Hkv * B);
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype == MPSA_BF16) launch_mode<MPSA_BF16>(p, mode, fmt8, tile, (int)D, (unsigned)((total + 1) / 2), st);
-    else                    launch_mode<MPSA_F16>(p, mode, fmt8, tile, (int)D, (unsigned)((total + 1) / 2), st);
-    MPSA_CHECK_LAUNCH("prepare");
-    return MPSA_OK;
+    return mpsa_prepare_operands(q, q_strides, k, k_strides, v, v_strides, dtype, B, Hq, Hkv, Nq, Nk, D, tile, fmt8, pre_scale_q, k_sub,
+                                 do4, do8, do4, do8, q4, qs4, q8, qs8, k4, ks4, k8, ks8, v_tiles, (hipStream_t)stream);
 }

@@ -167,14 +167,15 @@ __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, 
     const int64_t oc = head * chunks + c;                                 // flat output chunk
     const bool quad_leader = (threadIdx.x & 3u) == 0u;
 
-    if constexpr (DO4) {
+    // an output set that is not wanted has no pointer (one side of a mixed preparation: 8-bit Q, 4-bit K)
+    if (DO4 && a.codes4) {
         const int se = e - a.emax4;
         const uint32_t word = zero ? 0u : e2m1_pack8<!SW8>(x, se, a.exact16 != 0);
         reinterpret_cast<uint32_t*>(a.codes4)[oc] = word;
         const int sbyte = zero ? 0 : min(max(se + 127, 0), 254);
         if (quad_leader) a.scales4[oc >> 2] = (uint8_t)sbyte;
     }
-    if constexpr (DO8) {
+    if (DO8 && a.codes8) {
         const int se = e - a.emax8;
         const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
         uint2 w = make_uint2(0u, 0u);

@@ -18,6 +18,16 @@ LIB_PATH = os.environ.get("MPSA_LIB_PATH") or os.path.join(os.path.dirname(_HERE
 
 _i64, _int, _vp, _f32 = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_float
 _p64 = ctypes.POINTER(ctypes.c_int64)
+_four = ctypes.c_int64 * 4
+
+
+class AttnDesc(ctypes.Structure):
+    """``mpsa_attn_desc`` of include/mpsa.h."""
+    _fields_ = ([(n, _i64) for n in ("B", "Hq", "Hkv", "nq", "nk", "D")]
+                + [(n, _i64 * 4) for n in ("q_strides", "k_strides", "v_strides", "o_strides")]
+                + [(n, ctypes.c_int32) for n in ("dtype", "o_dtype", "tile", "causal", "mode", "fmt8", "smooth_k", "skip")]
+                + [(n, _f32) for n in ("pre_scale_q", "skip_thresh", "route_thresh")])
+
 
 # name -> (restype, argtypes); must list every symbol include/mpsa.h declares
 SIGNATURES = {
@@ -58,6 +68,8 @@ SIGNATURES = {
     "mpsa_skip_route_supported": (_int, [_i64, _i64, _i64, _int, _int, _int]),
     "mpsa_skip_route_workspace": (_i64, [_i64, _i64, _i64, _i64, _int]),
     "mpsa_skip_route": (_int, [_vp] * 8 + [_int, _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _f32, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "mpsa_attn_call_workspace": (_i64, [ctypes.POINTER(AttnDesc)]),
+    "mpsa_attn_call": (_int, [ctypes.POINTER(AttnDesc)] + [_vp] * 7),
     "mpsa_attn_fwd_routed": (_int, [_vp] * 8 + [_int, _vp, _int, _vp, _int, _p64,
                                     _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp, _vp]),
 }
@@ -103,16 +115,14 @@ def check(status):
         raise MpsaError(status, lib().mpsa_last_error().decode("utf-8", "replace"))
 
 
+_DTYPE_IDS = {torch.bfloat16: BF16, torch.float16: F16, torch.float32: F32, torch.float8_e5m2: F8E5M2}
+
+
 def dtype_id(dtype):
-    if dtype == torch.bfloat16:
-        return BF16
-    if dtype == torch.float16:
-        return F16
-    if dtype == torch.float32:
-        return F32
-    if dtype == torch.float8_e5m2:
-        return F8E5M2
-    raise ValueError(f"unsupported dtype {dtype}")
+    try:
+        return _DTYPE_IDS[dtype]
+    except KeyError:
+        raise ValueError(f"unsupported dtype {dtype}") from None
 
 
 def require_device(*tensors):
@@ -123,13 +133,35 @@ def require_device(*tensors):
 
 
 def stream_ptr(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """Handle of torch's current stream on a device (an int; 0 is the default stream).  The raw query takes a tenth of a
+    microsecond, building a ``torch.cuda.Stream`` to read its handle two."""
+    index = getattr(device, "index", None)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
+
+
+class on_device:
+    """``torch.cuda.device`` for the entry points: nothing but one query where the device is current already."""
+
+    __slots__ = ("want", "before")
+
+    def __init__(self, device):
+        self.want = device.index
+
+    def __enter__(self):
+        self.before = torch._C._cuda_getDevice()
+        if self.before != self.want:
+            torch.cuda.set_device(self.want)
+
+    def __exit__(self, *exc):
+        if self.before != self.want:
+            torch.cuda.set_device(self.before)
+        return False
 
 
 def strides4(t):
     assert t.dim() == 4
-    return (ctypes.c_int64 * 4)(*t.stride())
+    return _four(*t.stride())

@@ -12,7 +12,7 @@ in the reference's packed form ``[B,H,rows/128,K/128,32,4,4]``.
 import torch
 
 from . import _lib
-from .block_scaled_matmul import VEC_SIZE, _fmts_of, unpack_scale_5d
+from .block_scaled_matmul import VEC_SIZE, _bytes, _fmts_of, unpack_scale_5d
 # the reference defines the batched packaging here (ours/batched_block_scaled_matmul.py:239) and again, identically, next
 # to its attention kernel (ours/mxfp_attn_kernel.py:426); both names are one function in this package
 from .mxfp_attn_kernel import initialize_block_scaled_batched_from_tensor  # noqa: F401
@@ -32,8 +32,7 @@ def block_scaled_batched_matmul(a, a_scale, b, b_scale, dtype_dst, B, H, M, N, K
             b_scale = unpack_scale_5d(b_scale)
     width_a = K // 2 if fmt_a == _lib.FMT_E2M1 else K
     width_b = K // 2 if fmt_b == _lib.FMT_E2M1 else K
-    a = a.view(torch.uint8).contiguous()
-    b = b.view(torch.uint8).contiguous()
+    a, b = _bytes(a), _bytes(b)
     a_scale = a_scale.contiguous()
     b_scale = b_scale.contiguous()
     Hb = b.shape[1]
@@ -46,7 +45,7 @@ def block_scaled_batched_matmul(a, a_scale, b, b_scale, dtype_dst, B, H, M, N, K
         assert a_scale.shape == (B, H, M, K // VEC_SIZE) and b_scale.shape == (B, Hb, N, K // VEC_SIZE), "scales must be [B, H, rows, K/32]"
     out = torch.empty((B, H, M, N), dtype=dtype_dst, device=a.device)
     entry = _lib.lib().mpsa_gemm_mx_batched_packed if packed else _lib.lib().mpsa_gemm_mx_batched
-    with torch.cuda.device(a.device):
+    with _lib.on_device(a.device):
         _lib.check(entry(_lib.ptr(a), _lib.ptr(a_scale), fmt_a, _lib.ptr(b), _lib.ptr(b_scale), fmt_b,
                          B, H, Hb, M, N, K, _lib.ptr(out), _lib.dtype_id(dtype_dst), N, _lib.stream_ptr(a.device)))
     return out

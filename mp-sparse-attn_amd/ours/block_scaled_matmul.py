@@ -56,7 +56,7 @@ def pack_scale_5d(scale):
     rows, kb = scale.shape[-2], scale.shape[-1]
     batch = scale.numel() // max(rows * kb, 1)
     out = torch.empty((*scale.shape[:-2], rows // 128, kb // 4, 32, 4, 4), dtype=torch.uint8, device=scale.device)
-    with torch.cuda.device(scale.device):
+    with _lib.on_device(scale.device):
         _lib.check(_lib.lib().mpsa_scales_to_5d(_lib.ptr(scale), batch, rows, kb, _lib.ptr(out), _lib.stream_ptr(scale.device)))
     return out
 
@@ -70,9 +70,14 @@ def unpack_scale_5d(packed):
     rows, kb = packed.shape[-5] * 128, packed.shape[-4] * 4
     batch = packed.numel() // max(rows * kb, 1)
     out = torch.empty((*packed.shape[:-5], rows, kb), dtype=torch.uint8, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _lib.on_device(packed.device):
         _lib.check(_lib.lib().mpsa_scales_from_5d(_lib.ptr(packed), batch, rows, kb, _lib.ptr(out), _lib.stream_ptr(packed.device)))
     return out
+
+
+def _bytes(t):
+    """Codes as contiguous bytes."""
+    return (t if t.dtype is torch.uint8 else t.view(torch.uint8)).contiguous()
 
 
 def block_scaled_matmul(a, a_scale, b, b_scale, dtype_dst, M, N, K, configs):
@@ -92,8 +97,7 @@ def block_scaled_matmul(a, a_scale, b, b_scale, dtype_dst, M, N, K, configs):
             b_scale = unpack_scale_5d(b_scale)
     width_a = K // 2 if fmt_a == _lib.FMT_E2M1 else K
     width_b = K // 2 if fmt_b == _lib.FMT_E2M1 else K
-    a = a.view(torch.uint8).contiguous()
-    b = b.view(torch.uint8).contiguous()
+    a, b = _bytes(a), _bytes(b)
     a_scale = a_scale.contiguous()
     b_scale = b_scale.contiguous()
     assert a.shape == (M, width_a) and b.shape == (N, width_b), "operand shapes do not match M, N, K"
@@ -102,11 +106,15 @@ def block_scaled_matmul(a, a_scale, b, b_scale, dtype_dst, M, N, K, configs):
             "packed scales must be [rows/128, K/128, 32, 4, 4]"
     else:
         assert a_scale.shape == (M, K // VEC_SIZE) and b_scale.shape == (N, K // VEC_SIZE), "scales must be [rows, K/32]"
-    out = torch.empty((M, N), dtype=dtype_dst, device=a.device)
-    entry = _lib.lib().mpsa_gemm_mx_packed if packed else _lib.lib().mpsa_gemm_mx
-    with torch.cuda.device(a.device):
-        _lib.check(entry(_lib.ptr(a), _lib.ptr(a_scale), fmt_a, _lib.ptr(b), _lib.ptr(b_scale), fmt_b,
-                         M, N, K, _lib.ptr(out), _lib.dtype_id(dtype_dst), N, _lib.stream_ptr(a.device)))
+    device = a.device
+    out = torch.empty((M, N), dtype=dtype_dst, device=device)
+    lib = _lib.lib()
+    entry = lib.mpsa_gemm_mx_packed if packed else lib.mpsa_gemm_mx
+    with _lib.on_device(device):
+        status = entry(a.data_ptr(), a_scale.data_ptr(), fmt_a, b.data_ptr(), b_scale.data_ptr(), fmt_b,
+                       M, N, K, out.data_ptr(), _lib.dtype_id(dtype_dst), N, _lib.stream_ptr(device))
+    if status:
+        _lib.check(status)
     return out
 
 
@@ -115,7 +123,7 @@ def fp8_cast(x, fmt8):
     _lib.require_device(x)
     x = x.to(torch.float32).contiguous()
     out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         _lib.check(_lib.lib().mpsa_fp8_encode(_lib.ptr(x), x.numel(), fmt8, _lib.ptr(out), _lib.stream_ptr(x.device)))
     return out
 

@@ -16,7 +16,7 @@ from . import _lib
 
 def _flat_call(fn, src, out):
     src = src.contiguous()
-    with torch.cuda.device(src.device):
+    with _lib.on_device(src.device):
         _lib.check(fn(_lib.ptr(src), src.numel(), _lib.ptr(out), _lib.stream_ptr(src.device)))
     return out
 
@@ -78,7 +78,7 @@ class MXFP4Tensor:
         shape = list(data.shape)
         shape[dim] = (n + 1) // 2
         out = torch.empty(shape, dtype=torch.uint8, device=data.device)
-        with torch.cuda.device(data.device):
+        with _lib.on_device(data.device):
             _lib.check(_lib.lib().mpsa_e2m1_pack(_lib.ptr(data), outer, n, inner, _lib.ptr(out), _lib.stream_ptr(data.device)))
         return out
 
@@ -92,7 +92,7 @@ class MXFP4Tensor:
         outer = math.prod(original_shape[:dim])
         inner = math.prod(original_shape[dim + 1:])
         out = torch.empty(original_shape, dtype=torch.uint8, device=packed.device)
-        with torch.cuda.device(packed.device):
+        with _lib.on_device(packed.device):
             _lib.check(_lib.lib().mpsa_e2m1_unpack(_lib.ptr(packed), outer, n, inner, _lib.ptr(out), _lib.stream_ptr(packed.device)))
         return out
 

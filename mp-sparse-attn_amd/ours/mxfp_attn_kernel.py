@@ -1,11 +1,15 @@
 """Fused MXFP attention -- the reference's ``ours/mxfp_attn_kernel.py::mxfp_attn_kernel`` on HIP kernels.
 
-Pipeline per call (all on torch's current stream, no host synchronisation):
+Pipeline per call (all on torch's current stream, no host synchronisation), launched by one native call
+(``mpsa_attn_call``) on one block of workspace; the functions below run its stages one by one:
   1. MX-quantize Q (with ``scale*log2e`` folded in) and K, repack V into matrix-core operand order -- one launch,
      ``mpsa_attn_prepare`` (preceded by ``mpsa_seq_mean`` when ``smooth_k``);
   2. fused attention -- ``mpsa_attn_fwd`` / ``mpsa_attn_fwd_skip``; for ``block_scale_type="routed"`` the tile router
      (``mpsa_route_tiles``, integer work on the scale bytes) followed by ``mpsa_attn_fwd_routed``.
 """
+
+import ctypes
+import functools
 
 import torch
 
@@ -67,7 +71,7 @@ def prepare_operands(q, k, v, tile, block_scale_type, scale=None, smooth_k=False
                 ops["q8"], ops["qs8"] = u8(B, Hq, nq_pad, D), u8(B, Hq, nq_pad, D // 32)
             ops["k8"], ops["ks8"] = u8(B, Hkv, n_pad, D), u8(B, Hkv, n_pad, D // 32)
         v_tiles = torch.empty((B, Hkv, nt, tile * D), dtype=v.dtype, device=v.device)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(_lib.lib().mpsa_attn_prepare(
             _lib.ptr(None if fuse_q else q), _lib.strides4(q), _lib.ptr(k), _lib.strides4(k), _lib.ptr(v), _lib.strides4(v),
             _lib.dtype_id(q.dtype), B, Hq, Hkv, Nq, N, D, tile, mode, fmt8, pre, _lib.ptr(kmean),
@@ -90,7 +94,7 @@ def route_tiles(ops, is_causal, route_thresh=None, skip_thresh=None):
     tile = ops["tile"]
     dev = ops["qs4"].device
     ntq, ntk = (Nq + tile - 1) // tile, (N + tile - 1) // tile
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         work = torch.empty(_lib.lib().mpsa_route_workspace(B, Hq, Hkv, Nq, N, D, tile), dtype=torch.uint8, device=dev)
         cls = torch.empty((B, Hq, ntq, ntk), dtype=torch.uint8, device=dev)
         order = torch.empty((B, Hq, ntq, ntk), dtype=torch.int32, device=dev)
@@ -111,7 +115,7 @@ def skip_route(ops, is_causal, skip_thresh, skipped=None, want_cls=False):
     tile = ops["tile"]
     dev = ops["v_tiles"].device
     ntq, ntk = (Nq + tile - 1) // tile, (N + tile - 1) // tile
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         work = torch.empty(_lib.lib().mpsa_skip_route_workspace(B, Hq, Nq, N, tile), dtype=torch.uint8, device=dev)
         cls = torch.empty((B, Hq, ntq, ntk), dtype=torch.uint8, device=dev) if want_cls else None
         order = torch.empty((B, Hq, ntq, ntk), dtype=torch.int32, device=dev)
@@ -142,7 +146,7 @@ def attention_from_operands(ops, out, is_causal, skip_thresh=None, skipped=None,
     dev = out.device
     if skip_thresh is not None and not skip_in_kernel and ops["mode"] != _lib.MODE_ROUTED and skip_routable(ops, is_causal):
         _, order, counts = skip_route(ops, is_causal, skip_thresh, skipped)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             _lib.check(_lib.lib().mpsa_attn_fwd_routed(
                 _lib.ptr(ops["q4"]), _lib.ptr(ops["qs4"]), _lib.ptr(ops["q8"]), _lib.ptr(ops["qs8"]),
                 _lib.ptr(ops["k4"]), _lib.ptr(ops["ks4"]), _lib.ptr(ops["k8"]), _lib.ptr(ops["ks8"]), ops["fmt8"],
@@ -154,7 +158,7 @@ def attention_from_operands(ops, out, is_causal, skip_thresh=None, skipped=None,
         if route is None:
             raise ValueError("routed operands need route=(cls, order, counts) from route_tiles()")
         _, order, counts = route
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             _lib.check(_lib.lib().mpsa_attn_fwd_routed(
                 _lib.ptr(ops["q4"]), _lib.ptr(ops["qs4"]), _lib.ptr(ops["q8"]), _lib.ptr(ops["qs8"]),
                 _lib.ptr(ops["k4"]), _lib.ptr(ops["ks4"]), _lib.ptr(ops["k8"]), _lib.ptr(ops["ks8"]), ops["fmt8"],
@@ -166,7 +170,7 @@ def attention_from_operands(ops, out, is_causal, skip_thresh=None, skipped=None,
         if skip_thresh is not None:
             raise ValueError("tile skipping needs quantized Q operands (prepare_operands without fuse_q)")
         q = ops["q_raw"]
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             _lib.check(_lib.lib().mpsa_attn_fwd_q16(
                 _lib.ptr(q), _lib.strides4(q), _lib.dtype_id(q.dtype), ops["pre"],
                 _lib.ptr(ops["k4"]), _lib.ptr(ops["ks4"]), _lib.ptr(ops["k8"]), _lib.ptr(ops["ks8"]), ops["fmt8"],
@@ -174,7 +178,7 @@ def attention_from_operands(ops, out, is_causal, skip_thresh=None, skipped=None,
                 _lib.strides4(out), B, Hq, Hkv, N, D, ops["tile"], 1 if is_causal else 0, ops["mode"], _lib.stream_ptr(dev)))
         return out
     if skip_thresh is not None:
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             _lib.check(_lib.lib().mpsa_attn_fwd_skip(
                 _lib.ptr(ops["q4"]), _lib.ptr(ops["qs4"]), _lib.ptr(ops["q8"]), _lib.ptr(ops["qs8"]),
                 _lib.ptr(ops["k4"]), _lib.ptr(ops["ks4"]), _lib.ptr(ops["k8"]), _lib.ptr(ops["ks8"]), ops["fmt8"],
@@ -182,7 +186,7 @@ def attention_from_operands(ops, out, is_causal, skip_thresh=None, skipped=None,
                 _lib.strides4(out), B, Hq, Hkv, Nq, N, D, ops["tile"], 1 if is_causal else 0, ops["mode"],
                 float(skip_thresh), _lib.ptr(skipped), _lib.stream_ptr(dev)))
         return out
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(_lib.lib().mpsa_attn_fwd(
             _lib.ptr(ops["q4"]), _lib.ptr(ops["qs4"]), _lib.ptr(ops["q8"]), _lib.ptr(ops["qs8"]),
             _lib.ptr(ops["k4"]), _lib.ptr(ops["ks4"]), _lib.ptr(ops["k8"]), _lib.ptr(ops["ks8"]), ops["fmt8"],
@@ -280,7 +284,7 @@ def block_scaled_batched_attn(a_desc, a_scale, b_desc, b_scale, v_ori, dtype_dst
               _lib.ptr(k4), _lib.ptr(b_scale if k4 is not None else None), _lib.ptr(k8), _lib.ptr(b_scale if k8 is not None else None), fmt8,
               _lib.ptr(v_tiles), _lib.dtype_id(v_ori.dtype), _lib.ptr(out), _lib.dtype_id(dtype_dst), _lib.strides4(out),
               B, H, Hkv, M, N, K, tile, 1 if STAGE == 3 else 0, mode)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(_lib.lib().mpsa_v_tiles(_lib.ptr(v_ori), _lib.dtype_id(v_ori.dtype), B, Hkv, N, K, _lib.strides4(v_ori), tile,
                                            _lib.ptr(v_tiles), _lib.stream_ptr(dev)))
         if skip_thresh is not None:
@@ -294,7 +298,59 @@ def _normalise(q, k, v):
     """Reference prologue (ours/mxfp_attn_kernel.py:27-31): fp32/fp16 inputs run in fp16, everything else in
     bf16.  V follows Q/K's 16-bit dtype here (the reference always used fp16 for V)."""
     lp = torch.float16 if q.dtype in (torch.float32, torch.float16) else torch.bfloat16
-    return q.to(lp), k.to(lp), v.to(lp)
+    return tuple(t if t.dtype is lp else t.to(lp) for t in (q, k, v))
+
+
+def _aligned(t):
+    """The tensor, or a copy of it, with contiguous 16-byte aligned rows."""
+    if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]) or t.data_ptr() % 16:
+        return t.clone(memory_format=torch.contiguous_format)
+    return t
+
+
+@functools.lru_cache(maxsize=512)
+def _plan(q_shape, q_stride, k_shape, k_stride, v_shape, v_stride, dtype, is_causal, scale, smooth_k, tensor_layout, output_dtype,
+          block_scale_type, skip_thresh, tile, route_thresh):
+    """Checks the arguments of a call and describes it for ``mpsa_attn_call``: ``(description, workspace bytes, output shape,
+    whether tiles can be left out)``, or None if a row is not contiguous or not 16-byte aligned.  A pure function of shapes,
+    strides and options, kept for the last few hundred different ones: of a short call's host time it would be the largest
+    part."""
+    if tensor_layout not in ("HND", "NHD"):
+        raise ValueError(f"Unknown tensor layout: {tensor_layout}")
+    if any(len(s) != 4 for s in (q_shape, k_shape, v_shape)):
+        raise ValueError("expected a 4-D tensor")
+    bhnd = (lambda s: s) if tensor_layout == "HND" else (lambda s: (s[0], s[2], s[1], s[3]))
+    B, Hq, N, D = bhnd(q_shape)
+    _, Hkv, Nk, _ = bhnd(k_shape)
+    assert D in [64, 128], "headdim should be in [64, 128]."
+    assert k_shape[0] == v_shape[0] == B and k_shape[3] == v_shape[3] == D, "q, k and v must have the same batch size and head dim"
+    assert bhnd(v_shape)[2] == Nk, "k and v must have the same sequence length"
+    if Nk != N:                      # cross attention: the reference's kernel takes M and N apart as well
+        assert not is_causal, "causal masking needs q and k of the same sequence length"
+        assert _MODES.get(block_scale_type) != _lib.MODE_DIAG, "the diag types need q and k of the same sequence length"
+    assert Hkv == bhnd(v_shape)[1] and Hq % Hkv == 0, "query heads must be a multiple of key/value heads"
+    assert tile in (64, 128), "tile must be 64 or 128"
+    if output_dtype not in (torch.float16, torch.bfloat16, torch.float32):
+        raise ValueError(f"Unsupported dtype: {output_dtype}")       # ours/mxfp_attn_kernel.py:389
+    if block_scale_type not in _MODES:
+        raise ValueError(f"Invalid block scale type: {block_scale_type}")
+    mode = _MODES[block_scale_type]
+    if route_thresh is not None and mode != _lib.MODE_ROUTED:
+        raise ValueError("route_thresh needs block_scale_type=\"routed\"")
+    if any(s[-1] != 1 or any(x % 8 for x in s[:-1]) for s in (q_stride, k_stride, v_stride)):
+        return None
+    out_shape = (B, Hq, N, D) if tensor_layout == "HND" else (B, N, Hq, D)
+    out_stride = (Hq * N * D, N * D, D, 1) if tensor_layout == "HND" else (N * Hq * D, D, Hq * D, 1)
+    four = ctypes.c_int64 * 4
+    desc = _lib.AttnDesc(
+        B, Hq, Hkv, N, Nk, D, four(*bhnd(q_stride)), four(*bhnd(k_stride)), four(*bhnd(v_stride)), four(*out_stride),
+        _lib.dtype_id(dtype), _lib.dtype_id(output_dtype), tile, is_causal, mode,
+        _lib.FMT_E5M2 if block_scale_type.endswith("e5") else _lib.FMT_E4M3, smooth_k, skip_thresh is not None,
+        pre_scale_q(D, scale), skip_thresh or 0.0, route_thresh or 0.0)
+    nbytes = _lib.lib().mpsa_attn_call_workspace(desc)
+    if nbytes < 0:
+        _lib.check(nbytes)
+    return desc, nbytes, out_shape, mode == _lib.MODE_ROUTED or skip_thresh is not None
 
 
 def _reject_unsupported(attn_mask, dropout_p, attention_sink):
@@ -322,47 +378,27 @@ def mxfp_attn_kernel(q, k, v, attn_mask=None, dropout_p=0.0,
     MXFP8, one below ``skip_thresh`` times it is skipped, the rest runs in MXFP4."""
     _lib.require_device(q, k, v)
     _reject_unsupported(attn_mask, dropout_p, attention_sink)
-    torch.cuda.set_device(v.device)
+    device = v.device
+    if torch._C._cuda_getDevice() != device.index:
+        torch.cuda.set_device(device)
     q, k, v = _normalise(q, k, v)
-    q, k, v = _as_bhnd(q, tensor_layout), _as_bhnd(k, tensor_layout), _as_bhnd(v, tensor_layout)
-    B, Hq, N, D = q.shape
-    assert D in [64, 128], "headdim should be in [64, 128]."
-    Nk = k.shape[2]
-    assert v.shape[2] == Nk, "k and v must have the same sequence length"
-    if Nk != N:                      # cross attention: the reference's kernel takes M and N apart as well
-        assert not is_causal, "causal masking needs q and k of the same sequence length"
-        assert _MODES.get(block_scale_type) != _lib.MODE_DIAG, "the diag types need q and k of the same sequence length"
-    assert k.shape[1] == v.shape[1] and Hq % k.shape[1] == 0, "query heads must be a multiple of key/value heads"
-    assert tile in (64, 128), "tile must be 64 or 128"
-    if output_dtype not in (torch.float16, torch.bfloat16, torch.float32):
-        raise ValueError(f"Unsupported dtype: {output_dtype}")       # ours/mxfp_attn_kernel.py:389
-    if v.stride(-1) != 1:
-        v = v.contiguous()
-    # shapes of the paired-tile kernel: Q stays unquantized in HBM and the attention kernel quantizes it in registers
-    fuse_q = skip_thresh is None and q.stride(-1) == 1 and q.dtype == v.dtype and q_fusable(q, k, tile, block_scale_type, is_causal)
-    ops = prepare_operands(q, k, v, tile, block_scale_type, scale, smooth_k=smooth_k, fuse_q=fuse_q)
-    nt, ntk = (N + tile - 1) // tile, (Nk + tile - 1) // tile       # query tiles, key tiles
-    skipped = None
-    routed = ops["mode"] == _lib.MODE_ROUTED
-    route = route_tiles(ops, is_causal, route_thresh, skip_thresh) if routed else None
-    if routed:
-        skip_thresh = None
-    elif route_thresh is not None:
-        raise ValueError("route_thresh needs block_scale_type=\"routed\"")
-    if skip_thresh is not None and return_sparsity:
-        skipped = torch.zeros((B, Hq, nt), dtype=torch.int32, device=q.device)
-    if tensor_layout == "HND":
-        out = torch.empty((B, Hq, N, D), dtype=output_dtype, device=q.device)
-        attention_from_operands(ops, out, is_causal, skip_thresh, skipped, route)
-    else:
-        out = torch.empty((B, N, Hq, D), dtype=output_dtype, device=q.device)
-        attention_from_operands(ops, out.transpose(1, 2), is_causal, skip_thresh, skipped, route)
-    if not return_sparsity:
-        return out
+    if (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16:
+        q, k, v = (_aligned(t) for t in (q, k, v))
+    plan = _plan(q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), q.dtype, bool(is_causal),
+                 None if scale is None else float(scale), bool(smooth_k), tensor_layout, output_dtype, block_scale_type,
+                 None if skip_thresh is None else float(skip_thresh), tile, None if route_thresh is None else float(route_thresh))
+    if plan is None:                     # some row is not contiguous or not 16-byte aligned
+        return mxfp_attn_kernel(_aligned(q), _aligned(k), _aligned(v), None, 0.0, is_causal, scale, smooth_k, False, tensor_layout,
+                                output_dtype, return_sparsity, block_scale_type, skip_thresh, tile, route_thresh)
+    desc, nbytes, out_shape, leaves_out = plan
+    out = torch.empty(out_shape, dtype=output_dtype, device=device)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    share = None
+    if return_sparsity:
+        share = torch.empty((), dtype=torch.float32, device=device) if leaves_out else torch.zeros((), dtype=torch.float32, device=device)
+    status = _lib.lib().mpsa_attn_call(desc, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), work.data_ptr(),
+                                       share.data_ptr() if share is not None and leaves_out else None, _lib.stream_ptr(device))
+    if status:
+        _lib.check(status)
     # share of the visited (query tile, key tile) pairs that were skipped
-    visited = B * Hq * (nt * (nt + 1) // 2 if is_causal else nt * ntk)
-    if routed:
-        return out, (route[0] == 0).sum().to(torch.float32) / visited
-    if skipped is None:
-        return out, torch.zeros((), dtype=torch.float32, device=q.device)
-    return out, skipped.sum().to(torch.float32) / visited
+    return (out, share) if return_sparsity else out

@@ -13,6 +13,8 @@ reference, all deliberate:
 Scales are linear ``[B, H, L, D/32]`` uint8 (E8M0), as in the reference.
 """
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -38,7 +40,8 @@ def _check_input(x):
         raise ValueError("expected a 4-D tensor")
     if x.dtype not in (torch.bfloat16, torch.float16):
         raise ValueError(f"the quantizer takes bf16 or fp16, got {x.dtype}")
-    if x.stride(-1) != 1 or any(s % 8 for s in x.stride()[:3]) or x.data_ptr() % 16:
+    sb, sh, sn, sd = x.stride()
+    if sd != 1 or (sb | sh | sn) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
     return x
 
@@ -47,7 +50,7 @@ def pre_scale_q(head_dim, sm_scale=None):
     """``sm_scale * 1.44269504`` as float32 (ours/quant_mxint8.py:479-480, :494)."""
     if sm_scale is None:
         sm_scale = head_dim ** -0.5
-    return float(torch.tensor(sm_scale * LOG2E, dtype=torch.float32).item())
+    return ctypes.c_float(sm_scale * LOG2E).value
 
 
 def seq_mean(x):
@@ -59,7 +62,7 @@ def seq_mean(x):
     mean = torch.empty((B, H, D), dtype=x.dtype, device=x.device)
     nbytes = _lib.lib().mpsa_seq_mean_workspace(B, H, L, D)
     work = torch.empty((max(nbytes // 4, 1),), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         _lib.check(_lib.lib().mpsa_seq_mean(_lib.ptr(x), _lib.dtype_id(x.dtype), B, H, L, D, _lib.strides4(x),
                                             _lib.ptr(work), _lib.ptr(mean), _lib.stream_ptr(x.device)))
     return mean
@@ -84,12 +87,15 @@ def quantize_mx(x, pre_scale, fmt, emax_elem=None, out_rows=None, sub=None):
     if emax_elem is None:
         emax_elem = EMAX_E2M1 if fmt == _lib.FMT_E2M1 else EMAX_8BIT
     width = D // 2 if fmt == _lib.FMT_E2M1 else D
-    codes = torch.empty((B, H, rows, width), dtype=torch.uint8, device=x.device)
-    scales = torch.empty((B, H, rows, D // 32), dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.lib().mpsa_quantize_mx(
-            _lib.ptr(x), _lib.dtype_id(x.dtype), B, H, L, D, _lib.strides4(x), _sub_ptr(sub, x), pre_scale, fmt, emax_elem,
-            _lib.ptr(codes), _lib.ptr(scales), rows, _lib.stream_ptr(x.device)))
+    device = x.device
+    codes = torch.empty((B, H, rows, width), dtype=torch.uint8, device=device)
+    scales = torch.empty((B, H, rows, D // 32), dtype=torch.uint8, device=device)
+    with _lib.on_device(device):
+        status = _lib.lib().mpsa_quantize_mx(
+            x.data_ptr(), _lib.dtype_id(x.dtype), B, H, L, D, _lib.strides4(x), _sub_ptr(sub, x), pre_scale, fmt, emax_elem,
+            codes.data_ptr(), scales.data_ptr(), rows, _lib.stream_ptr(device))
+    if status:
+        _lib.check(status)
     return codes, scales
 
 
@@ -104,7 +110,7 @@ def quantize_mx_dual(x, pre_scale, fmt8=_lib.FMT_E4M3, out_rows=None, sub=None):
     s4 = torch.empty((B, H, rows, D // 32), dtype=torch.uint8, device=dev)
     c8 = torch.empty((B, H, rows, D), dtype=torch.uint8, device=dev)
     s8 = torch.empty((B, H, rows, D // 32), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(_lib.lib().mpsa_quantize_mx_dual(
             _lib.ptr(x), _lib.dtype_id(x.dtype), B, H, L, D, _lib.strides4(x), _sub_ptr(sub, x), pre_scale,
             EMAX_E2M1, fmt8, EMAX_8BIT, _lib.ptr(c4), _lib.ptr(s4), _lib.ptr(c8), _lib.ptr(s8), rows,

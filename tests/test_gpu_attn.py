@@ -814,3 +814,29 @@ def test_q16_entry_point_rejects_other_shapes():
                              _lib.ptr(ops["ks8"]), 0, _lib.ptr(ops["v_tiles"]), _lib.BF16, _lib.ptr(out), _lib.BF16, _lib.strides4(out),
                              1, 2, 2, 512, 128, 128, 1, _lib.MODE_DIAG, _lib.stream_ptr())
     assert rc == -1 and b"dtype" in L.mpsa_last_error()
+
+
+@pytest.mark.parametrize("bst,N,D,tile,causal,skip,route", [
+    ("diag", 160, 128, 128, True, None, None), ("mixed", 200, 64, 64, False, None, None), ("mixed", 700, 128, 128, False, None, None),
+    ("mxfp8", 300, 64, 128, True, None, None), ("mxfp4", 1100, 128, 128, False, 1.0, None), ("mixed_e5", 500, 128, 128, True, 1.0, None),
+    ("routed", 1100, 128, 128, False, 0.6, 0.95)])
+def test_one_native_call_equals_its_stages(bst, N, D, tile, causal, skip, route):
+    """mpsa_attn_call (one workspace, one foreign call) against the separate stages, smooth-K and the skipped share included."""
+    from ours.mxfp_attn_kernel import attention_from_operands, mxfp_attn_kernel, prepare_operands, route_tiles
+    q, k, v = (t.to(DEV) for t in make_qkv(2, 4, 2, N, D, 91, outliers=True))
+    out, share = mxfp_attn_kernel(q, k, v, is_causal=causal, smooth_k=True, output_dtype=torch.bfloat16, return_sparsity=True,
+                                  block_scale_type=bst, skip_thresh=skip, tile=tile, route_thresh=route)
+    ops = prepare_operands(q, k, v, tile, bst, smooth_k=True)
+    nt = (N + tile - 1) // tile
+    visited = 2 * 4 * (nt * (nt + 1) // 2 if causal else nt * nt)
+    want, left_out = torch.empty_like(q), 0
+    if bst == "routed":
+        lists = route_tiles(ops, causal, route, skip)
+        attention_from_operands(ops, want, causal, route=lists)
+        left_out = int((lists[0] == 0).sum())
+    else:
+        skipped = torch.zeros((2, 4, nt), dtype=torch.int32, device=DEV)
+        attention_from_operands(ops, want, causal, skip, skipped)
+        left_out = int(skipped.sum())
+    assert torch.equal(out, want)
+    assert share.shape == () and float(share) == float(torch.tensor(left_out, dtype=torch.float32) / visited)
