@@ -501,3 +501,25 @@ def test_8bit_against_4bit_products_are_cut_the_same_way(fmt, M, N):
     exact = (ad.double() @ bd.double().T).float()
     assert (out.cpu() != exact).any()
 
+
+
+# a row count per tile height of the kernels behind mpsa_gemm_mx (16-row blocks with K split between the waves, 128 x 128,
+# 256 x 256 with ragged edges), its remainders, and K with and without half a unit of 256
+@pytest.mark.parametrize("fmt_a,fmt_b", [(4, 4), (0, 4), (0, 0), (4, 1), (1, 4)])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 128), (16, 4095, 384), (17, 1025, 2176), (33, 4100, 1152), (65, 130, 4096), (129, 4096, 256),
+                                   (300, 1000, 1408), (700, 2500, 1152), (900, 3200, 640), (1000, 14336, 256), (2303, 2817, 512),
+                                   (2304, 2816, 128)])
+def test_every_kernel_at_its_edges(fmt_a, fmt_b, M, N, K):
+    g = torch.Generator().manual_seed(M * 7 + N)
+    a = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    b = torch.randn(N, K, generator=g).to(torch.bfloat16)
+    (ac, sa), (bc, sb) = O.quantize_mx(a, 1.0, fmt_a), O.quantize_mx(b, 1.0, fmt_b)
+    out = torch.full((M + 1, N), 7.0, device=DEV)        # one row more than the product has
+    ad, sad, bd, sbd = (t.to(DEV) for t in (ac, sa, bc, sb))
+    _lib.check(_lib.lib().mpsa_gemm_mx(_lib.ptr(ad), _lib.ptr(sad), fmt_a, _lib.ptr(bd), _lib.ptr(sbd), fmt_b, M, N, K,
+                                       _lib.ptr(out), _lib.F32, N, _lib.stream_ptr()))
+    da = O.dequantize_mx(ac, sa, fmt_a, torch.float32).to(DEV).double()
+    db = O.dequantize_mx(bc, sb, fmt_b, torch.float32).to(DEV).double()
+    err, size = (out[:M].double() - da @ db.t()).abs(), da.abs() @ db.abs().t()
+    assert bool((err <= (1e-7 if fmt_a == fmt_b == 4 else 1e-4) * size).all())
+    assert bool((out[M] == 7.0).all())
