@@ -18,7 +18,7 @@ LIB = os.path.join(LIBDIR, "libmpsa.so")
 BENCH_LIB = os.path.join(LIBDIR, "libmpsa_bench.so")
 BENCH_SOURCES = ["bench/mfma_stream.hip"]
 
-SOURCES = ["api.hip", "formats.hip", "quantize.hip", "v_tiles.hip", "prepare.hip", "gemm_mx.hip", "gemm_mx_split.hip", "gemm_mx_tile.hip", "gemm_mx_edge.hip", "attn_fwd.hip", "attn_fwd_skip.hip", "attn_fwd_routed.hip", "attn_fwd_pp.hip", "attn_call.hip", "route.hip", "skip_route.hip"]
+SOURCES = ["api.hip", "formats.hip", "quantize.hip", "v_tiles.hip", "prepare.hip", "gemm_mx.hip", "gemm_mx_split.hip", "gemm_mx_tile.hip", "gemm_mx_edge.hip", "attn_fwd.hip", "attn_fwd_skip.hip", "attn_fwd_routed.hip", "attn_fwd_pp.hip", "attn_call.hip", "attn_fwd_short.hip", "route.hip", "skip_route.hip"]
 
 # packed-fp32 instructions are switched off on purpose (the flag is for the device pass; the host
 # pass warns that it does not know the feature, which is harmless)

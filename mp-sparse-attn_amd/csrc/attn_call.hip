@@ -12,7 +12,8 @@ namespace {
 // Byte offsets into the workspace, -1 where a call does not need the buffer.
 struct Layout {
     int64_t q4, qs4, q8, qs8, k4, ks4, k8, ks8, v, mean, mean_work, work, cls, order, counts, skipped, total;
-    bool fuse_q, routed, ahead;       // Q quantized inside the attention kernel; tile router; skipping decided ahead
+    bool fuse_q, short_kernel;        // Q quantized inside the attention kernel; the short-sequence one
+    bool routed, ahead;               // tile router; skipping decided ahead
     int64_t ntq, ntk;
 };
 
@@ -27,7 +28,9 @@ int plan(const mpsa_attn_desc* d, Layout* l) {
     l->routed = d->mode == MPSA_MODE_ROUTED;
     const bool skip = d->skip && !l->routed;
     l->ahead = skip && mpsa_skip_route_supported(d->nq, d->nk, d->D, d->tile, d->causal, d->mode);
-    l->fuse_q = !skip && d->nq == d->nk && mpsa_attn_fwd_q16_supported(d->B, d->Hq, d->Hkv, d->nk, d->D, d->tile, d->causal, d->mode);
+    const bool paired = d->nq == d->nk && mpsa_attn_fwd_q16_supported(d->B, d->Hq, d->Hkv, d->nk, d->D, d->tile, d->causal, d->mode);
+    l->short_kernel = !skip && !l->routed && attn_short_wanted(d->B, d->Hq, d->Hkv, d->nq, d->nk, d->D, d->tile, d->causal, d->mode);
+    l->fuse_q = !skip && (l->short_kernel || paired);
     l->ntq = tiles(d->nq, d->tile);
     l->ntk = tiles(d->nk, d->tile);
     int64_t at = 0;
@@ -104,7 +107,10 @@ extern "C" int mpsa_attn_call(const mpsa_attn_desc* d, const void* q, const void
     rc = mpsa_prepare_operands(l.fuse_q ? nullptr : q, d->q_strides, k, d->k_strides, v, d->v_strides, d->dtype, d->B, d->Hq, d->Hkv, d->nq, d->nk,
                                d->D, d->tile, d->fmt8, d->pre_scale_q, at(l.mean), l.q4 >= 0, l.q8 >= 0, l.k4 >= 0, l.k8 >= 0, q4, qs4, q8, qs8, k4, ks4, k8, ks8, at(l.v), (hipStream_t)stream);
     if (rc != MPSA_OK) return rc;
-    if (l.fuse_q) {
+    if (l.short_kernel) {
+        rc = mpsa_attn_fwd_short(q, d->q_strides, d->dtype, d->pre_scale_q, k4, ks4, k8, ks8, d->fmt8, at(l.v), o, d->o_dtype, d->o_strides,
+                                 d->B, d->Hq, d->Hkv, d->nq, d->nk, d->D, d->tile, d->causal, d->mode, stream);
+    } else if (l.fuse_q) {
         rc = mpsa_attn_fwd_q16(q, d->q_strides, d->dtype, d->pre_scale_q, k4, ks4, k8, ks8, d->fmt8, at(l.v), d->dtype, o, d->o_dtype, d->o_strides,
                                d->B, d->Hq, d->Hkv, d->nk, d->D, d->tile, d->causal, d->mode, stream);
     } else if (l.routed || l.ahead) {

@@ -21,6 +21,7 @@ struct AttnArgs {
     const void* q_raw;
     int64_t q_sb, q_sh, q_sn;
     float q_pre;
+    int q_exact16;             // q_pre is a power of two: scaled values keep their 16-bit significands (short-sequence kernel)
 };
 
 template <int PVT> struct PV;
@@ -109,6 +110,46 @@ __device__ __forceinline__ int scalar_load(const int32_t* uniform_ptr) {
     asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(x) : "s"(uniform_bits(uniform_ptr)) : "memory");
     return x;
 }
+
+// Stores 16 dims of a query's output: lane (h, r) holds dims dim0 + 4 h .. + 3 (x) and dim0 + 8 + 4 h .. + 3 (y) of query
+// `query` (both lanes of a query must call it: 16-bit outputs trade register groups for 16-byte stores).
+__device__ __forceinline__ void store_16_dims(const AttnArgs& a, int b, int hq, int query, int dim0, int h, v4f x, v4f y, float inv) {
+    uint8_t* const base = static_cast<uint8_t*>(a.o);
+    const int64_t off = (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)query * a.o_sn + dim0;
+    x *= inv;
+    y *= inv;
+    if (a.o_dtype == MPSA_F32) {
+        if (query >= a.nq) return;
+        *reinterpret_cast<v4f*>(base + (off + 4 * h) * 4) = x;
+        *reinterpret_cast<v4f*>(base + (off + 8 + 4 * h) * 4) = y;
+        return;
+    }
+    int px[2], py[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        px[c] = a.o_dtype == MPSA_BF16 ? __builtin_bit_cast(int, PV<MPSA_BF16>::pack(x[2 * c], x[2 * c + 1])) : __builtin_bit_cast(int, PV<MPSA_F16>::pack(x[2 * c], x[2 * c + 1]));
+        py[c] = a.o_dtype == MPSA_BF16 ? __builtin_bit_cast(int, PV<MPSA_BF16>::pack(y[2 * c], y[2 * c + 1])) : __builtin_bit_cast(int, PV<MPSA_F16>::pack(y[2 * c], y[2 * c + 1]));
+    }
+    if (((a.o_sn | a.o_sh | a.o_sb) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.o) & 15) == 0) {
+        // lane half 0 hands over dims 8..11 and receives dims 4..7: each lane owns eight consecutive dims
+#pragma unroll
+        for (int c = 0; c < 2; ++c) asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(px[c]), "+v"(py[c]));
+        if (query < a.nq) *reinterpret_cast<v4i*>(base + (off + 8 * h) * 2) = (v4i){px[0], px[1], py[0], py[1]};
+        return;
+    }
+    if (query >= a.nq) return;
+    *reinterpret_cast<int2*>(base + (off + 4 * h) * 2) = make_int2(px[0], px[1]);
+    *reinterpret_cast<int2*>(base + (off + 8 + 4 * h) * 2) = make_int2(py[0], py[1]);
+}
+
+// Short-sequence kernel (attn_fwd_short.hip): every mode but routed, any shape; a.q_raw != nullptr: unquantized Q
+int attn_short_launch(const AttnArgs& a, int pv_dtype, hipStream_t st);
+// attn_fwd.hip: whether it is taken for a shape
+bool attn_short_wanted(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode);
+// attn_fwd.hip: mpsa_attn_fwd_q16 on the short-sequence kernel
+int mpsa_attn_fwd_short(const void* q, const int64_t q_strides[4], int q_dtype, float pre_scale_q, const uint8_t* k4, const uint8_t* ks4,
+                        const uint8_t* k8, const uint8_t* ks8, int fmt8, const void* v_tiles, void* o, int o_dtype, const int64_t o_strides[4],
+                        int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode, mpsa_stream_t stream);
 
 // Tile-skipping variants of the general kernel (modes mxfp4 / mxfp8): attn_fwd_skip.hip
 int attn_skip_launch(const AttnArgs& a, int pv_dtype, hipStream_t st);

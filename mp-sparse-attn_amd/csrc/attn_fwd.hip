@@ -31,6 +31,7 @@
 // registers (see attn_fwd_kernel.h).  K scales are read from global memory one step ahead.  80 KiB of LDS and at most 256 registers per workgroup let two workgroups share a CU, so one's matrix
 // instructions overlap the other's softmax VALU work.
 #include "attn_fwd_kernel.h"
+#include <cstring>
 
 namespace {
 
@@ -55,7 +56,7 @@ int launch_dt(const AttnArgs& a, int pv_dtype, hipStream_t st) {
 
 }  // namespace
 
-struct RawQ { const void* q; const int64_t* strides; int dtype; float pre; };
+struct RawQ { const void* q; const int64_t* strides; int dtype; float pre; bool short_kernel; };
 
 static int attn_entry(const RawQ* rq, const uint8_t* q4, const uint8_t* qs4, const uint8_t* q8, const uint8_t* qs8,
                       const uint8_t* k4, const uint8_t* ks4, const uint8_t* k8, const uint8_t* ks8, int fmt8,
@@ -112,14 +113,18 @@ static int attn_entry(const RawQ* rq, const uint8_t* q4, const uint8_t* qs4, con
     a.d = (int)D; a.tile = tile;
     a.skip_thresh = skip_thresh; a.skipped = skipped;
     a.order = order; a.counts = counts;
-    a.q_raw = nullptr; a.q_sb = a.q_sh = a.q_sn = 0; a.q_pre = 1.0f;
+    a.q_raw = nullptr; a.q_sb = a.q_sh = a.q_sn = 0; a.q_pre = 1.0f; a.q_exact16 = 0;
     hipStream_t st = (hipStream_t)stream;
     if (rq) {
         a.q_raw = rq->q; a.q_sb = rq->strides[0]; a.q_sh = rq->strides[1]; a.q_sn = rq->strides[2]; a.q_pre = rq->pre;
+        uint32_t bits;
+        memcpy(&bits, &a.q_pre, 4);
+        a.q_exact16 = (bits & 0x007FFFFFu) == 0u && (bits & 0x7F800000u) != 0u && (bits & 0x7F800000u) != 0x7F800000u;
+        if (rq->short_kernel) return attn_short_launch(a, pv_dtype, st);
         if (!attn_pp_supported(a, pv_dtype))
             return mpsa_fail(MPSA_EUNSUPPORTED, "attn: unquantized q needs the paired-tile kernel's shape (D = 128, tile = 128; "
                                                 "causal: at least two tiles, unmasked: at least six); quantize q with mpsa_attn_prepare and call mpsa_attn_fwd");
-        return attn_pp_launch(a, pv_dtype, st);
+        return attn_short_wanted(B, Hq, Hkv, nq, n, D, tile, causal, mode) ? attn_short_launch(a, pv_dtype, st) : attn_pp_launch(a, pv_dtype, st);
     }
     if (routed) return attn_routed_launch(a, pv_dtype, st);
     if (skip) {
@@ -127,6 +132,7 @@ static int attn_entry(const RawQ* rq, const uint8_t* q4, const uint8_t* qs4, con
         if (skipped && (reinterpret_cast<uintptr_t>(skipped) & 3)) return mpsa_fail(MPSA_EALIGN, "attn: skipped must be 4-byte aligned");
         return attn_skip_launch(a, pv_dtype, st);
     }
+    if (attn_short_wanted(B, Hq, Hkv, nq, n, D, tile, causal, mode)) return attn_short_launch(a, pv_dtype, st);
     if (attn_pp_supported(a, pv_dtype)) return attn_pp_launch(a, pv_dtype, st);
     if (D == 128 && tile == 128) return launch_dt<128, 128>(a, pv_dtype, st);
     if (D == 64 && tile == 64)   return launch_dt<64, 64>(a, pv_dtype, st);
@@ -166,9 +172,17 @@ extern "C" int mpsa_attn_fwd_q16(const void* q, const int64_t q_strides[4], int 
                                  const void* v_tiles, int pv_dtype, void* o, int o_dtype, const int64_t o_strides[4],
                                  int64_t B, int64_t Hq, int64_t Hkv, int64_t n, int64_t D, int tile, int causal, int mode,
                                  mpsa_stream_t stream) {
-    const RawQ rq = {q, q_strides, q_dtype, pre_scale_q};
+    const RawQ rq = {q, q_strides, q_dtype, pre_scale_q, false};
     return attn_entry(&rq, nullptr, nullptr, nullptr, nullptr, k4, ks4, k8, ks8, fmt8, v_tiles, pv_dtype, o, o_dtype, o_strides,
                       B, Hq, Hkv, n, n, D, tile, causal, mode, false, 0.0f, nullptr, nullptr, nullptr, stream);
+}
+
+int mpsa_attn_fwd_short(const void* q, const int64_t q_strides[4], int q_dtype, float pre_scale_q, const uint8_t* k4, const uint8_t* ks4,
+                        const uint8_t* k8, const uint8_t* ks8, int fmt8, const void* v_tiles, void* o, int o_dtype, const int64_t o_strides[4],
+                        int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode, mpsa_stream_t stream) {
+    const RawQ rq = {q, q_strides, q_dtype, pre_scale_q, true};
+    return attn_entry(&rq, nullptr, nullptr, nullptr, nullptr, k4, ks4, k8, ks8, fmt8, v_tiles, q_dtype, o, o_dtype, o_strides,
+                      B, Hq, Hkv, nq, nk, D, tile, causal, mode, false, 0.0f, nullptr, nullptr, nullptr, stream);
 }
 
 extern "C" int mpsa_attn_fwd_q16_supported(int64_t B, int64_t Hq, int64_t Hkv, int64_t n, int64_t D, int tile, int causal, int mode) {
@@ -179,4 +193,38 @@ extern "C" int mpsa_attn_fwd_q16_supported(int64_t B, int64_t Hq, int64_t Hkv, i
     a.nt = (int)((n + tile - 1) / (tile > 0 ? tile : 1)); a.n_pad = a.nt * tile;
     a.nq = a.n; a.ntq = a.nt; a.nq_pad = a.n_pad;
     return (tile == 64 || tile == 128) && attn_pp_supported(a, MPSA_BF16) ? 1 : 0;
+}
+
+// Whether the short-sequence kernel (attn_fwd_short.hip) is estimated to finish first: microseconds of either side, fitted
+// to measurements at 20 shapes (head counts 4 - 128, 77 - 8192 keys, D = 64 and 128, masked and not).  Its cost is workgroups
+// (32 queries each) and 32 x 32 blocks spread over the chip; a tile kernel's is its longest workgroup while there are no
+// more of them than CUs.  With 32 heads and D = 128 the line falls near 1500 tokens.
+bool attn_short_wanted(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode) {
+    const bool d128 = D == 128, paired = nq == nk && mpsa_attn_fwd_q16_supported(B, Hq, Hkv, nk, D, tile, causal, mode);
+    // unmasked self-attention of D = 128 below the paired-tile kernel's range stays on the general kernel: there a routed run
+    // whose lists name one precision returns the bits of the fixed-precision run
+    if (d128 && !causal && nq == nk && !paired && tile == 128) return false;
+    auto tiles = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
+    const double heads = (double)(B * Hq), qb = (double)tiles(nq, 32), kb = (double)tiles(nk, 32);
+    if (heads * qb >= 32768.0) return false;                  // the kernel's index arithmetic; far beyond its use
+    const double blocks = heads * (causal ? qb * (qb + 1.0) / 2.0 : qb * kb) / 1024.0;
+    const double spread = d128 ? 8.6 * heads * qb / 768.0 + 0.377 * blocks : 5.0 * heads * qb / 1024.0 + 0.28 * blocks;
+    const double longest = d128 ? 4.0 + 0.75 * kb / 4.0 : 3.0 + 0.5 * kb / 4.0;
+    const double mine = spread > longest ? spread : longest;
+
+    const double ntq = (double)tiles(nq, tile), ntk = (double)tiles(nk, tile);
+    double other;
+    if (paired) {                                             // attn_fwd_pp.hip: two query tiles a workgroup, one workgroup a CU
+        const double pairs = heads * (double)((int64_t)(ntq + 1.0) / 2), one = 10.4 + 1.61 * ntk;
+        if (!causal)           other = (double)tiles((int64_t)pairs, 256) * one;
+        else if (pairs <= 256.0)  other = one;
+        else                      other = 24.0 + 2.1 * pairs * (ntk + 2.0) / 2.0 / 256.0;
+    } else {                                                  // attn_fwd_kernel.h, and Q's quantization in front of it
+        const bool t128 = tile == 128;
+        const double wgs = heads * ntq, steps = wgs * (causal ? (ntk + 1.0) / 2.0 : ntk);
+        const double step = t128 ? (d128 ? 1.5 : 1.2) : (d128 ? 0.6 : 0.45), slots = d128 && t128 ? 512.0 : 1024.0;
+        const double full = 8.0 * wgs / slots + step * steps / 256.0, one = 8.0 + (t128 ? 1.0 : 0.75) * ntk;
+        other = (full > one ? full : one) + 1.0 + heads * (double)nq * (double)D * 3.5 / 4.5e6;
+    }
+    return mine < other;
 }

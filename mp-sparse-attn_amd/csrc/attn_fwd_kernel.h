@@ -56,11 +56,18 @@ __global__ __launch_bounds__(TILE * 2, 2) void attn_fwd_kernel(AttnArgs a) {
     // ---- which (batch, kv head, query head, query tile) -- XCD-aware, heavy causal tiles first ----
     const int group = a.Hq / a.Hkv;
     const int total = a.B * a.Hq * a.ntq;
-    int L = blockIdx.x;
-    if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);      // XCD x gets one contiguous logical range
-    const int per_unit = group * a.ntq;
-    const int unit = L / per_unit;
-    const int rem = L - unit * per_unit;
+    const int units = a.B * a.Hkv;
+    int unit, rem;
+    if (a.causal && (units & 7)) {          // fewer KV heads than XCDs, or an uneven number: every XCD gets long and short rows
+        rem = blockIdx.x / units;
+        unit = blockIdx.x - rem * units;
+    } else {
+        int L = blockIdx.x;
+        if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);      // XCD x gets one contiguous logical range
+        const int per_unit = group * a.ntq;
+        unit = L / per_unit;
+        rem = L - unit * per_unit;
+    }
     const int rank = rem / group;
     const int hq = (unit % a.Hkv) * group + (rem - rank * group);
     const int b = unit / a.Hkv;

@@ -79,11 +79,20 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
     const int npairs = (a.nt + 1) >> 1;          // an odd tile count leaves the last pair with its lower tile only
     const int group = a.Hq / a.Hkv;
     const int total = a.B * a.Hq * npairs;
-    int L = blockIdx.x;
-    if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);
-    const int per_unit = group * npairs;
-    const int unit = L / per_unit;
-    const int rem = L - unit * per_unit;
+    const int units = a.B * a.Hkv;
+    int unit, rem;
+    if (CAUSAL && (units & 7)) {
+        // fewer KV heads than XCDs, or an uneven number: contiguous ranges would give one XCD a head's long rows and
+        // another its short ones (one KV head, N = 8192: 134 us, this way 85); the rows are dealt out instead
+        rem = blockIdx.x / units;
+        unit = blockIdx.x - rem * units;
+    } else {
+        int L = blockIdx.x;
+        if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);
+        const int per_unit = group * npairs;
+        unit = L / per_unit;
+        rem = L - unit * per_unit;
+    }
     const int rank = rem / group;
     const int hq = (unit % a.Hkv) * group + (rem - rank * group);
     const int b = unit / a.Hkv;

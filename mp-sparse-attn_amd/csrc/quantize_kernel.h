@@ -124,6 +124,44 @@ __device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool
     return word;
 }
 
+// One lane's eight elements (a quarter of an MX block; the quad's other lanes hold the rest): codes and the block's scale
+// bytes in the formats asked for.  x comes back multiplied by `pre`.
+template <bool DO4, bool DO8, int FMT8, bool SW8>
+__device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8) {
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        x[i] = x[i] * pre;
+        amax = __builtin_fmaxf(amax, __builtin_fabsf(x[i]));
+    }
+    amax = __builtin_fmaxf(amax, dpp_f32<0xB1>(amax));   // quad_perm [1,0,3,2]
+    amax = __builtin_fmaxf(amax, dpp_f32<0x4E>(amax));   // quad_perm [2,3,0,1]
+
+    const uint32_t ab = mpsa_f2u(amax);
+    const bool zero = (ab == 0u);
+    const uint32_t ef = ab >> 23;
+    const int e = ef ? (int)ef - 127 : (31 - __builtin_clz(ab | 1u)) - 149;   // floor(log2(amax)), subnormals included
+    w4 = 0u; s4 = 0;
+    w8 = make_uint2(0u, 0u); s8 = 0;
+    if constexpr (DO4) {
+        const int se = e - emax4;
+        w4 = zero ? 0u : e2m1_pack8<!SW8>(x, se, exact16);
+        s4 = zero ? 0 : min(max(se + 127, 0), 254);
+    }
+    if constexpr (DO8) {
+        const int se = e - emax8;
+        const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
+        if (!zero) {
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = __builtin_fminf(__builtin_fmaxf(ldexpf(x[i], -se), -lim), lim);
+            w8.x = fp8_pack4<FMT8, SW8>(y[0], y[1], y[2], y[3]);
+            w8.y = fp8_pack4<FMT8, SW8>(y[4], y[5], y[6], y[7]);
+        }
+        s8 = zero ? 0 : min(max(se + 127, 0), 254);
+    }
+}
+
 // One workgroup's share: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb (nh heads).
 template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8>
 __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh) {
@@ -150,45 +188,20 @@ __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, 
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = 0.0f;
     }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        x[i] = x[i] * a.pre;
-        amax = __builtin_fmaxf(amax, __builtin_fabsf(x[i]));
-    }
-    amax = __builtin_fmaxf(amax, dpp_f32<0xB1>(amax));   // quad_perm [1,0,3,2]
-    amax = __builtin_fmaxf(amax, dpp_f32<0x4E>(amax));   // quad_perm [2,3,0,1]
-
-    const uint32_t ab = mpsa_f2u(amax);
-    const bool zero = (ab == 0u);
-    const uint32_t ef = ab >> 23;
-    const int e = ef ? (int)ef - 127 : (31 - __builtin_clz(ab | 1u)) - 149;   // floor(log2(amax)), subnormals included
-
+    uint32_t w4;
+    uint2 w8;
+    int s4, s8;
+    quantize_chunk<DO4, DO8, FMT8, SW8>(x, a.pre, a.exact16 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
     const int64_t oc = head * chunks + c;                                 // flat output chunk
     const bool quad_leader = (threadIdx.x & 3u) == 0u;
-
     // an output set that is not wanted has no pointer (one side of a mixed preparation: 8-bit Q, 4-bit K)
     if (DO4 && a.codes4) {
-        const int se = e - a.emax4;
-        const uint32_t word = zero ? 0u : e2m1_pack8<!SW8>(x, se, a.exact16 != 0);
-        reinterpret_cast<uint32_t*>(a.codes4)[oc] = word;
-        const int sbyte = zero ? 0 : min(max(se + 127, 0), 254);
-        if (quad_leader) a.scales4[oc >> 2] = (uint8_t)sbyte;
+        reinterpret_cast<uint32_t*>(a.codes4)[oc] = w4;
+        if (quad_leader) a.scales4[oc >> 2] = (uint8_t)s4;
     }
     if (DO8 && a.codes8) {
-        const int se = e - a.emax8;
-        const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
-        uint2 w = make_uint2(0u, 0u);
-        if (!zero) {
-            float y[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = __builtin_fminf(__builtin_fmaxf(ldexpf(x[i], -se), -lim), lim);
-            w.x = fp8_pack4<FMT8, SW8>(y[0], y[1], y[2], y[3]);
-            w.y = fp8_pack4<FMT8, SW8>(y[4], y[5], y[6], y[7]);
-        }
-        reinterpret_cast<uint2*>(a.codes8)[oc] = w;
-        const int sbyte = zero ? 0 : min(max(se + 127, 0), 254);
-        if (quad_leader) a.scales8[oc >> 2] = (uint8_t)sbyte;
+        reinterpret_cast<uint2*>(a.codes8)[oc] = w8;
+        if (quad_leader) a.scales8[oc >> 2] = (uint8_t)s8;
     }
 }
 

@@ -840,3 +840,20 @@ def test_one_native_call_equals_its_stages(bst, N, D, tile, causal, skip, route)
         left_out = int(skipped.sum())
     assert torch.equal(out, want)
     assert share.shape == () and float(share) == float(torch.tensor(left_out, dtype=torch.float32) / visited)
+
+
+@pytest.mark.parametrize("mode", ["diag", "mxfp4", "mxfp8", "mixed"])
+@pytest.mark.parametrize("N,Nk,D,tile,causal", [(1, 1, 128, 128, True), (31, 31, 64, 64, True), (33, 33, 128, 64, True), (130, 130, 128, 128, True),
+                                                (161, 161, 64, 64, False), (97, 97, 64, 128, False), (200, 200, 128, 64, False),
+                                                (64, 45, 64, 64, False), (300, 129, 64, 128, False), (900, 900, 128, 128, False)])
+def test_short_sequence_kernel_at_its_edges(mode, N, Nk, D, tile, causal):
+    """Key blocks dealt out to four waves: waves without a block, ragged last blocks, the own tile of a diag run alone and
+    next to a tail, both tile edges."""
+    from ours.mxfp_attn_kernel import mxfp_attn_kernel
+    if mode == "diag" and N != Nk:
+        pytest.skip("diag needs as many queries as keys")
+    q, _, _ = make_qkv(1, 4, 2, N, D, 500 + N, outliers=True)
+    _, k, v = make_qkv(1, 4, 2, Nk, D, 501 + N, outliers=False)
+    want = O.attn_mx(q, k, v, tile=tile, causal=causal, mode=mode, out_dtype=torch.float32)
+    run = lambda dt: mxfp_attn_kernel(q.to(DEV), k.to(DEV), v.to(DEV), is_causal=causal, block_scale_type=mode, tile=tile, output_dtype=dt)
+    check_attention(run, want, f"short {mode} {N}x{Nk} D{D}", torch.bfloat16)
