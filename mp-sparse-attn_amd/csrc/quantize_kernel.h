@@ -53,8 +53,7 @@ __device__ __forceinline__ uint32_t fp8_pack4(float y0, float y1, float y2, floa
 }
 
 template <int XDT>
-__device__ __forceinline__ void load8(const void* p, float (&x)[8]) {
-    const uint4 raw = *reinterpret_cast<const uint4*>(p);
+__device__ __forceinline__ void unpack8(const uint4& raw, float (&x)[8]) {
     const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -67,6 +66,9 @@ __device__ __forceinline__ void load8(const void* p, float (&x)[8]) {
         }
     }
 }
+
+template <int XDT>
+__device__ __forceinline__ void load8(const void* p, float (&x)[8]) { unpack8<XDT>(*reinterpret_cast<const uint4*>(p), x); }
 
 // round a float32 to the 16-bit dtype XDT (nearest even) and back
 template <int XDT>
