@@ -29,7 +29,7 @@ int plan(const mpsa_attn_desc* d, Layout* l) {
     const bool skip = d->skip && !l->routed;
     l->ahead = skip && mpsa_skip_route_supported(d->nq, d->nk, d->D, d->tile, d->causal, d->mode);
     const bool paired = d->nq == d->nk && mpsa_attn_fwd_q16_supported(d->B, d->Hq, d->Hkv, d->nk, d->D, d->tile, d->causal, d->mode);
-    l->short_kernel = !skip && !l->routed && attn_short_wanted(d->B, d->Hq, d->Hkv, d->nq, d->nk, d->D, d->tile, d->causal, d->mode);
+    l->short_kernel = !skip && !l->routed && attn_short_splits(d->B, d->Hq, d->Hkv, d->nq, d->nk, d->D, d->tile, d->causal, d->mode) != 0;
     l->fuse_q = !skip && (l->short_kernel || paired);
     l->ntq = tiles(d->nq, d->tile);
     l->ntk = tiles(d->nk, d->tile);

@@ -21,7 +21,6 @@ struct AttnArgs {
     const void* q_raw;
     int64_t q_sb, q_sh, q_sn;
     float q_pre;
-    int q_exact16;             // q_pre is a power of two: scaled values keep their 16-bit significands (short-sequence kernel)
 };
 
 template <int PVT> struct PV;
@@ -101,6 +100,25 @@ __device__ __forceinline__ void load16_to_lds_sv(uint32_t lane_off, const uint8_
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(base), "v"(lane_off), "s"(gb) : "memory", "m0");
 }
 
+// N such loads of 1024 bytes each, one behind the other in memory and in LDS: the instruction's offset goes to both addresses
+template <int N>
+__device__ __forceinline__ void load16n_to_lds_sv(uint32_t lane_off, const uint8_t* wave_base, uint8_t* lds_wave_base) {
+    static_assert(N >= 1 && N <= 4, "the offset has twelve bits");
+    const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds_wave_base);
+    const uint64_t gb = uniform_bits(wave_base);
+    if constexpr (N == 1) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(base), "v"(lane_off), "s"(gb) : "memory", "m0");
+    if constexpr (N == 2) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" ::"s"(base), "v"(lane_off), "s"(gb) : "memory", "m0");
+    if constexpr (N == 3) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024\n\tglobal_load_lds_dwordx4 %1, %2 offset:2048" ::"s"(base), "v"(lane_off), "s"(gb) : "memory", "m0");
+    if constexpr (N == 4) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024\n\tglobal_load_lds_dwordx4 %1, %2 offset:2048\n\tglobal_load_lds_dwordx4 %1, %2 offset:3072" ::"s"(base), "v"(lane_off), "s"(gb) : "memory", "m0");
+}
+
+// four bytes a lane: 256 in all
+__device__ __forceinline__ void load4_to_lds_sv(uint32_t lane_off, const uint8_t* wave_base, uint8_t* lds_wave_base) {
+    const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds_wave_base);
+    const uint64_t gb = uniform_bits(wave_base);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(base), "v"(lane_off), "s"(gb) : "memory", "m0");
+}
+
 // A scalar load of one list entry.  The compiler turns a plain load that follows a workgroup barrier into a vector
 // load plus a broadcast; as assembly it stays a scalar load.  The wait is part of the same statement (a register
 // that is still being loaded must not be visible to the compiler as holding a value), so callers place it where
@@ -111,41 +129,53 @@ __device__ __forceinline__ int scalar_load(const int32_t* uniform_ptr) {
     return x;
 }
 
-// Stores 16 dims of a query's output: lane (h, r) holds dims dim0 + 4 h .. + 3 (x) and dim0 + 8 + 4 h .. + 3 (y) of query
-// `query` (both lanes of a query must call it: 16-bit outputs trade register groups for 16-byte stores).
-__device__ __forceinline__ void store_16_dims(const AttnArgs& a, int b, int hq, int query, int dim0, int h, v4f x, v4f y, float inv) {
-    uint8_t* const base = static_cast<uint8_t*>(a.o);
+// Stores UNITS x 16 dims of a query's output, from dim0 on, times inv: piece(2 u) of lane (h, r) holds dims 16 u + 4 h .. + 3
+// of query r's unit u, piece(2 u + 1) dims 16 u + 8 + 4 h .. + 3.  Both lanes of a query must call it: for 16-bit outputs they
+// trade register groups (lane half 0 hands over dims 8..11 of a unit and receives dims 4..7), so that each owns eight
+// consecutive dims and stores 16 bytes (8-byte aligned at least) at a time.  The output type is looked at once, outside the
+// units: a look per register pair was a hundred scalar branches, 4300 clocks of every workgroup where this takes 1100.
+template <int UNITS, typename F>
+__device__ __forceinline__ void store_output(const AttnArgs& a, int b, int hq, int query, int dim0, int h, F&& piece, float inv) {
     const int64_t off = (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)query * a.o_sn + dim0;
-    x *= inv;
-    y *= inv;
+    const bool valid = query < a.nq;
     if (a.o_dtype == MPSA_F32) {
-        if (query >= a.nq) return;
-        *reinterpret_cast<v4f*>(base + (off + 4 * h) * 4) = x;
-        *reinterpret_cast<v4f*>(base + (off + 8 + 4 * h) * 4) = y;
+        v4f* const to = reinterpret_cast<v4f*>(static_cast<float*>(a.o) + off + 4 * h);
+        if (valid) {
+#pragma unroll
+            for (int x = 0; x < 2 * UNITS; ++x) to[2 * x] = piece(x) * inv;
+        }
         return;
     }
-    int px[2], py[2];
+    auto half = [&](auto type_c) __attribute__((always_inline)) {
+        typedef PV<decltype(type_c)::value> T;
+        v4i out[UNITS];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        px[c] = a.o_dtype == MPSA_BF16 ? __builtin_bit_cast(int, PV<MPSA_BF16>::pack(x[2 * c], x[2 * c + 1])) : __builtin_bit_cast(int, PV<MPSA_F16>::pack(x[2 * c], x[2 * c + 1]));
-        py[c] = a.o_dtype == MPSA_BF16 ? __builtin_bit_cast(int, PV<MPSA_BF16>::pack(y[2 * c], y[2 * c + 1])) : __builtin_bit_cast(int, PV<MPSA_F16>::pack(y[2 * c], y[2 * c + 1]));
-    }
-    if (((a.o_sn | a.o_sh | a.o_sb) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.o) & 15) == 0) {
-        // lane half 0 hands over dims 8..11 and receives dims 4..7: each lane owns eight consecutive dims
+        for (int u = 0; u < UNITS; ++u) {
+            const v4f x = piece(2 * u) * inv, y = piece(2 * u + 1) * inv;
+            int px[2], py[2];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(px[c]), "+v"(py[c]));
-        if (query < a.nq) *reinterpret_cast<v4i*>(base + (off + 8 * h) * 2) = (v4i){px[0], px[1], py[0], py[1]};
-        return;
-    }
-    if (query >= a.nq) return;
-    *reinterpret_cast<int2*>(base + (off + 4 * h) * 2) = make_int2(px[0], px[1]);
-    *reinterpret_cast<int2*>(base + (off + 8 + 4 * h) * 2) = make_int2(py[0], py[1]);
+            for (int c = 0; c < 2; ++c) {
+                px[c] = __builtin_bit_cast(int, T::pack(x[2 * c], x[2 * c + 1]));
+                py[c] = __builtin_bit_cast(int, T::pack(y[2 * c], y[2 * c + 1]));
+            }
+            asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3\n\ts_nop 1" : "+v"(px[0]), "+v"(py[0]), "+v"(px[1]), "+v"(py[1]));
+            out[u] = (v4i){px[0], px[1], py[0], py[1]};
+        }
+        typedef v4i v4i_8 __attribute__((aligned(8)));
+        v4i_8* const to = reinterpret_cast<v4i_8*>(static_cast<uint16_t*>(a.o) + off + 8 * h);
+        if (valid) {
+#pragma unroll
+            for (int u = 0; u < UNITS; ++u) to[2 * u] = out[u];
+        }
+    };
+    if (a.o_dtype == MPSA_BF16) half(std::integral_constant<int, MPSA_BF16>{});
+    else                        half(std::integral_constant<int, MPSA_F16>{});
 }
 
 // Short-sequence kernel (attn_fwd_short.hip): every mode but routed, any shape; a.q_raw != nullptr: unquantized Q
-int attn_short_launch(const AttnArgs& a, int pv_dtype, hipStream_t st);
-// attn_fwd.hip: whether it is taken for a shape
-bool attn_short_wanted(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode);
+int attn_short_launch(const AttnArgs& a, int pv_dtype, int splits, hipStream_t st);
+// attn_fwd.hip: its key splits for a shape (1, 2, 4), or 0 where another kernel is taken
+int attn_short_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode);
 // attn_fwd.hip: mpsa_attn_fwd_q16 on the short-sequence kernel
 int mpsa_attn_fwd_short(const void* q, const int64_t q_strides[4], int q_dtype, float pre_scale_q, const uint8_t* k4, const uint8_t* ks4,
                         const uint8_t* k8, const uint8_t* ks8, int fmt8, const void* v_tiles, void* o, int o_dtype, const int64_t o_strides[4],

@@ -31,7 +31,6 @@
 // registers (see attn_fwd_kernel.h).  K scales are read from global memory one step ahead.  80 KiB of LDS and at most 256 registers per workgroup let two workgroups share a CU, so one's matrix
 // instructions overlap the other's softmax VALU work.
 #include "attn_fwd_kernel.h"
-#include <cstring>
 
 namespace {
 
@@ -113,18 +112,16 @@ static int attn_entry(const RawQ* rq, const uint8_t* q4, const uint8_t* qs4, con
     a.d = (int)D; a.tile = tile;
     a.skip_thresh = skip_thresh; a.skipped = skipped;
     a.order = order; a.counts = counts;
-    a.q_raw = nullptr; a.q_sb = a.q_sh = a.q_sn = 0; a.q_pre = 1.0f; a.q_exact16 = 0;
+    a.q_raw = nullptr; a.q_sb = a.q_sh = a.q_sn = 0; a.q_pre = 1.0f;
     hipStream_t st = (hipStream_t)stream;
     if (rq) {
         a.q_raw = rq->q; a.q_sb = rq->strides[0]; a.q_sh = rq->strides[1]; a.q_sn = rq->strides[2]; a.q_pre = rq->pre;
-        uint32_t bits;
-        memcpy(&bits, &a.q_pre, 4);
-        a.q_exact16 = (bits & 0x007FFFFFu) == 0u && (bits & 0x7F800000u) != 0u && (bits & 0x7F800000u) != 0x7F800000u;
-        if (rq->short_kernel) return attn_short_launch(a, pv_dtype, st);
+        const int splits = attn_short_splits(B, Hq, Hkv, nq, n, D, tile, causal, mode);
+        if (rq->short_kernel) return attn_short_launch(a, pv_dtype, splits, st);
         if (!attn_pp_supported(a, pv_dtype))
             return mpsa_fail(MPSA_EUNSUPPORTED, "attn: unquantized q needs the paired-tile kernel's shape (D = 128, tile = 128; "
                                                 "causal: at least two tiles, unmasked: at least six); quantize q with mpsa_attn_prepare and call mpsa_attn_fwd");
-        return attn_short_wanted(B, Hq, Hkv, nq, n, D, tile, causal, mode) ? attn_short_launch(a, pv_dtype, st) : attn_pp_launch(a, pv_dtype, st);
+        return splits ? attn_short_launch(a, pv_dtype, splits, st) : attn_pp_launch(a, pv_dtype, st);
     }
     if (routed) return attn_routed_launch(a, pv_dtype, st);
     if (skip) {
@@ -132,7 +129,8 @@ static int attn_entry(const RawQ* rq, const uint8_t* q4, const uint8_t* qs4, con
         if (skipped && (reinterpret_cast<uintptr_t>(skipped) & 3)) return mpsa_fail(MPSA_EALIGN, "attn: skipped must be 4-byte aligned");
         return attn_skip_launch(a, pv_dtype, st);
     }
-    if (attn_short_wanted(B, Hq, Hkv, nq, n, D, tile, causal, mode)) return attn_short_launch(a, pv_dtype, st);
+    const int splits = attn_short_splits(B, Hq, Hkv, nq, n, D, tile, causal, mode);
+    if (splits) return attn_short_launch(a, pv_dtype, splits, st);
     if (attn_pp_supported(a, pv_dtype)) return attn_pp_launch(a, pv_dtype, st);
     if (D == 128 && tile == 128) return launch_dt<128, 128>(a, pv_dtype, st);
     if (D == 64 && tile == 64)   return launch_dt<64, 64>(a, pv_dtype, st);
@@ -195,22 +193,38 @@ extern "C" int mpsa_attn_fwd_q16_supported(int64_t B, int64_t Hq, int64_t Hkv, i
     return (tile == 64 || tile == 128) && attn_pp_supported(a, MPSA_BF16) ? 1 : 0;
 }
 
-// Whether the short-sequence kernel (attn_fwd_short.hip) is estimated to finish first: microseconds of either side, fitted
-// to measurements at 20 shapes (head counts 4 - 128, 77 - 8192 keys, D = 64 and 128, masked and not).  Its cost is workgroups
-// (32 queries each) and 32 x 32 blocks spread over the chip; a tile kernel's is its longest workgroup while there are no
-// more of them than CUs.  With 32 heads and D = 128 the line falls near 1500 tokens.
-bool attn_short_wanted(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode) {
+// Whether the short-sequence kernel (attn_fwd_short.hip) is estimated to finish first, and with how many key splits (0: it is
+// not).  Microseconds of either side, fitted to measurements at 90 shapes (1 - 256 heads, 45 - 8192 keys, D = 64 and 128, masked
+// and not); the choice costs 0.4 % over always taking the fastest.  A workgroup of the short kernel takes a fixed time and so
+// much a stage, `full` with all of a CU's places filled, `alone` at the head of the longest chain; a tile kernel's time is its
+// longest workgroup while there are no more of them than CUs.  With 32 heads and D = 128 four splits go up to 250 tokens, two
+// to 1900, where the paired-tile kernel takes over; one split serves many queries over few keys.
+int attn_short_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode) {
     const bool d128 = D == 128, paired = nq == nk && mpsa_attn_fwd_q16_supported(B, Hq, Hkv, nk, D, tile, causal, mode);
     // unmasked self-attention of D = 128 below the paired-tile kernel's range stays on the general kernel: there a routed run
     // whose lists name one precision returns the bits of the fixed-precision run
-    if (d128 && !causal && nq == nk && !paired && tile == 128) return false;
+    if (d128 && !causal && nq == nk && !paired && tile == 128) return 0;
     auto tiles = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
-    const double heads = (double)(B * Hq), qb = (double)tiles(nq, 32), kb = (double)tiles(nk, 32);
-    if (heads * qb >= 32768.0) return false;                  // the kernel's index arithmetic; far beyond its use
-    const double blocks = heads * (causal ? qb * (qb + 1.0) / 2.0 : qb * kb) / 1024.0;
-    const double spread = d128 ? 8.6 * heads * qb / 768.0 + 0.377 * blocks : 5.0 * heads * qb / 1024.0 + 0.28 * blocks;
-    const double longest = d128 ? 4.0 + 0.75 * kb / 4.0 : 3.0 + 0.5 * kb / 4.0;
-    const double mine = spread > longest ? spread : longest;
+    const double heads = (double)(B * Hq);
+    const int64_t qb = tiles(nq, 32), kb = tiles(nk, 32);
+    if (heads * (double)qb >= 32768.0) return 0;              // the kernel's index arithmetic; far beyond its use
+    struct Cost { int splits; double fixed, full, alone, places; };
+    static const Cost costs[2][3] = {{{1, 3.6, 0.62, 0.41, 768.0}, {2, 3.6, 0.74, 0.44, 768.0}, {4, 3.4, 0.52, 0.44, 512.0}},
+                                     {{1, 5.6, 0.85, 0.49, 512.0}, {2, 5.4, 0.86, 0.42, 512.0}, {4, 4.3, 0.48, 0.51, 256.0}}};
+    double mine = 1e300;
+    int splits = 0;
+    for (const Cost& c : costs[d128]) {
+        const double wgs = heads * (double)tiles(qb, 4 / c.splits), stages = (double)tiles(kb, c.splits);
+        double load = wgs / c.places;
+        if (c.splits == 4)    load = (double)(int64_t)(load + 1.0 - 1e-9);        // one workgroup a CU: whole rounds
+        else if (load < 1.0)  load = 1.0;
+        const double spread = c.fixed * load + c.full * wgs * (causal ? 0.5 * ((double)kb / c.splits + 1.0) : stages) / c.places;
+        const double longest = c.fixed + c.alone * stages, us = spread > longest ? spread : longest;
+        if (us < mine) {
+            mine = us;
+            splits = c.splits;
+        }
+    }
 
     const double ntq = (double)tiles(nq, tile), ntk = (double)tiles(nk, tile);
     double other;
@@ -226,5 +240,5 @@ bool attn_short_wanted(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t n
         const double full = 8.0 * wgs / slots + step * steps / 256.0, one = 8.0 + (t128 ? 1.0 : 0.75) * ntk;
         other = (full > one ? full : one) + 1.0 + heads * (double)nq * (double)D * 3.5 / 4.5e6;
     }
-    return mine < other;
+    return mine < other ? splits : 0;
 }

@@ -140,12 +140,6 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
                                                  // those of the parked 8-bit fragments in bytes 1 and 3)
     v4i kf4[KB][SST];
     int ksc[KB];
-    // shared exponent of an MX block from its largest magnitude, as the quantizer takes it (quantize_kernel.h)
-    auto block_exponent = [&](float amax) __attribute__((always_inline)) {
-        const uint32_t ab = mpsa_f2u(amax);
-        const uint32_t ef = ab >> 23;
-        return ef ? (int)ef - 127 : (31 - __builtin_clz(ab | 1u)) - 149;
-    };
     // Both precisions from one pass over the lane's query row: lane half h owns MX blocks h and 2 + h of the row's four
     // (the 4-bit operand layout), so a block's maximum and shared exponent are lane-local and serve both formats (the
     // element exponent limits differ: 3 and 7).  The 8-bit operand wants 16 bytes of EVERY block in each lane half
@@ -180,7 +174,10 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
                 const int se = ex - 3;                                         // emax of E2M1: ours/quant_mxint8.py:303
                 int w[4];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) w[c] = zero ? 0 : (int)e2m1_pack8<true>(x[c], se, false);
+                for (int c = 0; c < 4; ++c) {
+                    w[c] = (int)e2m1_pack8<true>(x[c], se, false);
+                    w[c] = zero ? 0 : w[c];
+                }
                 qf[s] = (v8i){w[0], w[1], w[2], w[3], 0, 0, 0, 0};
                 sbytes |= (uint32_t)(zero ? 0 : min(max(se + 127, 0), 254)) << (16 * s);
             }
@@ -756,61 +753,11 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
     // ---- epilogue: O = acc / l ; register e of lane (h, r): dim 32*db + 8*(e/4) + 4*h + e%4 of query r ----
     const float l_tot = sum_lane_pair(l_run);
     const float inv = 1.0f / l_tot;
-    const int q_global = i * TILE + q_local;
-    if (q_global >= a.nq) return;                       // a row of the ragged last tile's padding (both lanes of a query leave together)
-    uint8_t* orow = static_cast<uint8_t*>(a.o);
-    const int64_t off = (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)q_global * a.o_sn;
-    if (a.o_dtype != MPSA_F32 && ((a.o_sn | a.o_sh | a.o_sb) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.o) & 15) == 0) {
-        // 16-bit output: the two lanes of a query trade register groups (lane half 0 hands over dims 8..11 of every
-        // 16 and receives dims 4..7), so that each lane owns 8 consecutive dims and stores 16 bytes at a time
-#pragma unroll
-        for (int d = 0; d < NDB; ++d)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                int x[2], y[2];                           // packed dims 16u+4h .. +3 (x) and 16u+8+4h .. +3 (y)
-#pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const float x0 = acc[d][8 * u + 2 * c] * inv, x1 = acc[d][8 * u + 2 * c + 1] * inv;
-                    const float y0 = acc[d][8 * u + 4 + 2 * c] * inv, y1 = acc[d][8 * u + 4 + 2 * c + 1] * inv;
-                    if (a.o_dtype == MPSA_BF16) {
-                        typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-                        x[c] = __builtin_bit_cast(int, (v2bf){(__bf16)x0, (__bf16)x1});
-                        y[c] = __builtin_bit_cast(int, (v2bf){(__bf16)y0, (__bf16)y1});
-                    } else {
-                        typedef _Float16 v2hh __attribute__((ext_vector_type(2)));
-                        x[c] = __builtin_bit_cast(int, (v2hh){(_Float16)x0, (_Float16)x1});
-                        y[c] = __builtin_bit_cast(int, (v2hh){(_Float16)y0, (_Float16)y1});
-                    }
-                    // swap x of lanes 32-63 with y of lanes 0-31: half 0 ends with dims 16u .. 16u+7 in (x, y),
-                    // half 1 with dims 16u+8 .. 16u+15
-                    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x[c]), "+v"(y[c]));
-                }
-                const int dim = 32 * d + 16 * u + 8 * h;
-                const v4i pk8 = {x[0], x[1], y[0], y[1]};
-                *reinterpret_cast<v4i*>(orow + (off + dim) * 2) = pk8;
-            }
-        return;
-    }
-#pragma unroll
-    for (int d = 0; d < NDB; ++d)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-            const int dim = 32 * d + 8 * g4 + 4 * h;
-            const float o0 = acc[d][4 * g4 + 0] * inv, o1 = acc[d][4 * g4 + 1] * inv;
-            const float o2 = acc[d][4 * g4 + 2] * inv, o3 = acc[d][4 * g4 + 3] * inv;
-            if (a.o_dtype == MPSA_BF16) {
-                typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
-                const v4bf pk4 = {(__bf16)o0, (__bf16)o1, (__bf16)o2, (__bf16)o3};
-                *reinterpret_cast<v4bf*>(orow + (off + dim) * 2) = pk4;
-            } else if (a.o_dtype == MPSA_F16) {
-                typedef _Float16 v4hh __attribute__((ext_vector_type(4)));
-                const v4hh pk4 = {(_Float16)o0, (_Float16)o1, (_Float16)o2, (_Float16)o3};
-                *reinterpret_cast<v4hh*>(orow + (off + dim) * 2) = pk4;
-            } else {
-                const v4f pk4 = {o0, o1, o2, o3};
-                *reinterpret_cast<v4f*>(orow + (off + dim) * 4) = pk4;
-            }
-        }
+    store_output<2 * NDB>(a, b, hq, i * TILE + q_local, 0, h, [&](int x) __attribute__((always_inline)) {
+        const v16f& v = acc[x >> 2];
+        const int e = 4 * (x & 3);
+        return (v4f){v[e], v[e + 1], v[e + 2], v[e + 3]};
+    }, inv);
 }
 
 template <int PVT, int FMT8, int MODE, bool QRAW, bool CAUSAL>

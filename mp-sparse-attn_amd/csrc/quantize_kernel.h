@@ -28,8 +28,8 @@ namespace {
 
 
 template <int DPP_CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), DPP_CTRL, 0xf, 0xf, false));
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, DPP_CTRL, 0xf, 0xf, true);
 }
 
 template <int FMT8, bool SW8>
@@ -93,75 +93,107 @@ __device__ __forceinline__ float round16(float v) {
 // significant bits: such a value is either exactly a midpoint - where the two rules agree (both take the even
 // mantissa) - or at least 2^-12 away from one, so the check is skipped (`exact16`); it would otherwise fire on every
 // exact tie, which 16-bit data hits all the time.
-template <bool HW4>
-__device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool exact16) {
-    if constexpr (HW4) {
-        if (se >= -126) {
-            const float sc = mpsa_u2f((uint32_t)(se + 127) << 23);
-            const float dn = 1.0f - 0x1p-17f, up = 1.0f + 0x1p-17f;
-            if (exact16) {
-                uint32_t w = 0;
-                w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[0], x[1], sc, 0);
-                w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[2], x[3], sc, 1);
-                w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[4], x[5], sc, 2);
-                w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[6], x[7], sc, 3);
-                return w;
-            }
-            // no boundary between the two nudged values: the value itself converts to the same codes
-            uint32_t wd = 0, wu = 0;
-            wd = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wd, x[0] * dn, x[1] * dn, sc, 0);
-            wd = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wd, x[2] * dn, x[3] * dn, sc, 1);
-            wd = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wd, x[4] * dn, x[5] * dn, sc, 2);
-            wd = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wd, x[6] * dn, x[7] * dn, sc, 3);
-            wu = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wu, x[0] * up, x[1] * up, sc, 0);
-            wu = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wu, x[2] * up, x[3] * up, sc, 1);
-            wu = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wu, x[4] * up, x[5] * up, sc, 2);
-            wu = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(wu, x[6] * up, x[7] * up, sc, 3);
-            if (wd == wu) return wd;
-        }
-    }
-    uint32_t word = 0;
+// The explicit rule is rolled up (a hundred instructions, not seven hundred) and stands behind ONE branch: written as early
+// returns and conditional blocks, the quantizer took 800 clocks per eight elements of a lane, half of them in branches.
+__device__ __forceinline__ uint32_t e2m1_pack8_rule(const float (&x)[8], int se) {
+    float y[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) word |= e2m1_encode(ldexpf(x[i], -se)) << (4 * i);
+    for (int i = 0; i < 8; ++i) y[i] = x[i];
+    uint32_t word = 0;
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+        word = (word >> 4) | (e2m1_encode(ldexpf(y[0], -se)) << 28);
+#pragma unroll
+        for (int j = 0; j + 1 < 8; ++j) y[j] = y[j + 1];
+    }
     return word;
 }
 
+// the conversion, and whether the rule has to decide instead
+__device__ __forceinline__ uint32_t e2m1_try8(const float (&x)[8], int se, bool exact16, bool& rule) {
+    const float sc = mpsa_u2f((uint32_t)(se + 127) << 23);
+    auto convert = [&](float f) __attribute__((always_inline)) {
+        uint32_t w = 0;
+        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[0] * f, x[1] * f, sc, 0);
+        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[2] * f, x[3] * f, sc, 1);
+        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[4] * f, x[5] * f, sc, 2);
+        return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[6] * f, x[7] * f, sc, 3);
+    };
+    rule = se < -126;
+    if (exact16) return convert(1.0f);
+    // no boundary between the two nudged values: the value itself converts to the same codes
+    const uint32_t w = convert(1.0f - 0x1p-17f);
+    rule |= w != convert(1.0f + 0x1p-17f);
+    return w;
+}
+
+template <bool HW4>
+__device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool exact16) {
+    if constexpr (!HW4) return e2m1_pack8_rule(x, se);
+    bool rule;
+    uint32_t w = e2m1_try8(x, se, exact16, rule);
+    if (rule) w = e2m1_pack8_rule(x, se);
+    return w;
+}
+
+// floor(log2(amax)) of a block's largest magnitude, subnormals included; -1 for a block of zeros (whose codes and scale are
+// zero whatever it says)
+__device__ __forceinline__ int block_exponent(float amax) {
+    const int biased = (int)(mpsa_f2u(amax) >> 23), tiny = __builtin_amdgcn_frexp_expf(amax) - 1;
+    return biased ? biased - 127 : tiny;
+}
+
 // One lane's eight elements (a quarter of an MX block; the quad's other lanes hold the rest): codes and the block's scale
-// bytes in the formats asked for.  x comes back multiplied by `pre`.
+// bytes in the formats asked for.  x comes back multiplied by `pre`.  Where `rule` comes back true, the caller replaces w4 by
+// e2m1_pack8_rule(x, s): several chunks in a row share one branch that way, and run interleaved.
 template <bool DO4, bool DO8, int FMT8, bool SW8>
-__device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8) {
+__device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8, bool& rule, int& se4) {
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         x[i] = x[i] * pre;
         amax = __builtin_fmaxf(amax, __builtin_fabsf(x[i]));
     }
-    amax = __builtin_fmaxf(amax, dpp_f32<0xB1>(amax));   // quad_perm [1,0,3,2]
-    amax = __builtin_fmaxf(amax, dpp_f32<0x4E>(amax));   // quad_perm [2,3,0,1]
-
-    const uint32_t ab = mpsa_f2u(amax);
-    const bool zero = (ab == 0u);
-    const uint32_t ef = ab >> 23;
-    const int e = ef ? (int)ef - 127 : (31 - __builtin_clz(ab | 1u)) - 149;   // floor(log2(amax)), subnormals included
+    // magnitudes order like their bits
+    uint32_t ab = mpsa_f2u(amax);
+    ab = max(ab, dpp_u32<0xB1>(ab));                      // quad_perm [1,0,3,2]
+    ab = max(ab, dpp_u32<0x4E>(ab));                      // quad_perm [2,3,0,1]
+    const bool zero = ab == 0u;
+    const int e = block_exponent(mpsa_u2f(ab));
     w4 = 0u; s4 = 0;
     w8 = make_uint2(0u, 0u); s8 = 0;
+    rule = false;
+    se4 = e - emax4;
     if constexpr (DO4) {
-        const int se = e - emax4;
-        w4 = zero ? 0u : e2m1_pack8<!SW8>(x, se, exact16);
-        s4 = zero ? 0 : min(max(se + 127, 0), 254);
+        if constexpr (SW8) {
+            rule = !zero;
+        } else {
+            w4 = e2m1_try8(x, se4, exact16, rule);
+            rule &= !zero;
+        }
+        w4 = zero ? 0u : w4;
+        s4 = zero ? 0 : min(max(se4 + 127, 0), 254);
     }
     if constexpr (DO8) {
         const int se = e - emax8;
         const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
-        if (!zero) {
-            float y[8];
+        float y[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = __builtin_fminf(__builtin_fmaxf(ldexpf(x[i], -se), -lim), lim);
-            w8.x = fp8_pack4<FMT8, SW8>(y[0], y[1], y[2], y[3]);
-            w8.y = fp8_pack4<FMT8, SW8>(y[4], y[5], y[6], y[7]);
-        }
+        for (int i = 0; i < 8; ++i) y[i] = __builtin_fminf(__builtin_fmaxf(ldexpf(x[i], -se), -lim), lim);
+        w8.x = fp8_pack4<FMT8, SW8>(y[0], y[1], y[2], y[3]);
+        w8.y = fp8_pack4<FMT8, SW8>(y[4], y[5], y[6], y[7]);
+        w8.x = zero ? 0u : w8.x;
+        w8.y = zero ? 0u : w8.y;
         s8 = zero ? 0 : min(max(se + 127, 0), 254);
     }
+}
+
+template <bool DO4, bool DO8, int FMT8, bool SW8>
+__device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8) {
+    bool rule;
+    int se4;
+    quantize_most<DO4, DO8, FMT8, SW8>(x, pre, exact16, emax4, emax8, w4, s4, w8, s8, rule, se4);
+    if (DO4 && rule) w4 = e2m1_pack8_rule(x, se4);
 }
 
 // One workgroup's share: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb (nh heads).

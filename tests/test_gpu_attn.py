@@ -857,3 +857,18 @@ def test_short_sequence_kernel_at_its_edges(mode, N, Nk, D, tile, causal):
     want = O.attn_mx(q, k, v, tile=tile, causal=causal, mode=mode, out_dtype=torch.float32)
     run = lambda dt: mxfp_attn_kernel(q.to(DEV), k.to(DEV), v.to(DEV), is_causal=causal, block_scale_type=mode, tile=tile, output_dtype=dt)
     check_attention(run, want, f"short {mode} {N}x{Nk} D{D}", torch.bfloat16)
+
+
+@pytest.mark.parametrize("mode", ["diag", "mxfp4", "mxfp8", "mixed"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,Nk,D,tile,causal", [(2, 32, 8, 300, 300, 128, 128, True), (3, 32, 8, 161, 161, 64, 64, True), (4, 32, 8, 225, 225, 64, 128, False),
+                                                         (8, 32, 4, 200, 200, 128, 64, True), (8, 32, 8, 130, 77, 128, 128, False), (8, 32, 8, 260, 33, 64, 64, False)])
+def test_short_sequence_kernel_with_fewer_splits(mode, B, Hq, Hkv, N, Nk, D, tile, causal):
+    """Many heads, where two splits or none are taken: workgroups whose last 32 queries are missing, a diag workgroup over two tiles."""
+    from ours.mxfp_attn_kernel import mxfp_attn_kernel
+    if mode == "diag" and N != Nk:
+        pytest.skip("diag needs as many queries as keys")
+    q, _, _ = make_qkv(B, Hq, Hkv, N, D, 600 + N, outliers=True)
+    _, k, v = make_qkv(B, Hq, Hkv, Nk, D, 601 + N, outliers=False)
+    want = O.attn_mx(q, k, v, tile=tile, causal=causal, mode=mode, out_dtype=torch.float32)
+    run = lambda dt: mxfp_attn_kernel(q.to(DEV), k.to(DEV), v.to(DEV), is_causal=causal, block_scale_type=mode, tile=tile, output_dtype=dt)
+    check_attention(run, want, f"short {mode} {B}x{Hq}x{N}x{Nk} D{D}", torch.bfloat16)
