@@ -289,32 +289,42 @@ static int gemm_entry(const uint8_t* a, const uint8_t* sa, int fmt_a, const uint
     hipStream_t st = (hipStream_t)stream;
     const int rc = mpsa_ensure_init();
     if (rc != MPSA_OK) return rc;
-    // Which kernel: the one with the least estimated time (microseconds, fitted to measurements at 34 shapes and three types
-    // from 1 x 1024 x 4096 to 8192^3; within 15 % of them).  A tile costs a fixed part -- pipeline fill, epilogue -- and one
-    // per 1024 of K; a started round of 256 tiles counts whole, at a clock that falls as the chip fills.  The lines fall near
-    // M = 256 (4096-wide layer, K = 4096), where a 128-wide tile takes over from the 16-row blocks, and near 2000 rows,
-    // where 256-wide tiles fill the chip.
+    // Which kernel: the one with the least estimated time (microseconds, fitted to measurements at 130 shapes and three types
+    // from 1 x 1024 x 4096 to 8192^3; the choice costs 1 % over always taking the fastest).  A ring tile costs a fixed part --
+    // pipeline fill, epilogue -- and one per 1024 of K; a started round of 256 tiles counts whole, at a clock that falls as the
+    // chip fills, and every million outputs some.  The general kernel shares a CU between up to three tiles and has no rounds:
+    // it is the fastest a few tiles past a whole number of them, and where K is short.  The lines fall near M = 256 (4096-wide
+    // layer, K = 4096), where a 128-wide tile takes over from the 16-row blocks, and near 2000 rows, where 256-wide tiles fill
+    // the chip.
     const int64_t batches = batch * heads_a;
     const bool mixed = fmt_a != MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1;
     const int kind = fmt_a == MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1 ? 0 : mixed ? 1 : 2;
-    if (K % 128 || force_general()) {
+    struct Ring { double start, round, per_1024, empty, out; };              // empty: share of per_1024 at an empty chip
+    static const Ring RING[2][3] = {{{1.5, 3.8, 3.26, 0.72, 0.26}, {2.5, 3.0, 3.85, 0.79, 0.32}, {1.8, 3.2, 4.65, 0.70, 0.41}},
+                                    {{6.3, 0.0, 4.38, 1.40, 1.44}, {4.0, 6.4, 15.3, 0.59, 0.0}, {2.5, 9.0, 14.9, 0.59, 0.05}}};
+    struct Shared { double start, tile, least, base, per_1024; };            // tile, per_1024: for 256 tiles
+    static const Shared SHARED[3] = {{2.7, 1.6, 7.2, 3.8, 4.2}, {2.2, 2.75, 9.1, 6.7, 3.3}, {2.4, 1.8, 10.0, 4.8, 6.7}};
+    auto tiles = [&](int64_t edge) { return (double)((M + edge - 1) / edge) * (double)((N + edge - 1) / edge) * (double)batches; };
+    auto ring = [&](int which, int64_t edge) {
+        const Ring& r = RING[which][kind];
+        const double rounds = ceil(tiles(edge) / 256.0), clock = r.empty + (1.0 - r.empty) * tiles(edge) / (256.0 * rounds);
+        return r.start + rounds * (r.round + r.per_1024 * clock * (double)K / 1024.0) + r.out * 1e-6 * (double)M * (double)N * (double)batches;
+    };
+    const bool whole = M % BM == 0 && N % BN == 0;
+    const bool staged = (fmt_a == fmt_b || mixed) && (whole || kind != 0 || K % 256 == 0);
+    const Shared& sh = SHARED[kind];
+    const double load = tiles(128) / 256.0, slope = sh.base + sh.per_1024 * load;
+    const double general = sh.start + sh.tile * load + (double)K / 1024.0 * (slope > sh.least ? slope : sh.least);
+    int tile = 0;
+    const double cost16 = gemm_split_cost(g, batches, fmt_a, fmt_b, &tile), cost128 = ring(0, 128), cost256 = staged ? ring(1, 256) : 1e300;
+    const double least = fmin(fmin(cost16, cost128), cost256);
+    if (K % 128 || force_general() || general < least) {
         dim3 grid((unsigned)(((M + 127) / 128) * ((N + 127) / 128)), (unsigned)batches);
         launch_general(g, fmt_a, fmt_b, c_dtype, grid, st);
     } else {
-        static const double FIXED[2][3] = {{4.9, 4.6, 5.2}, {7.7, 7.5, 8.5}}, PER_1024[2][3] = {{3.1, 4.45, 4.75}, {6.5, 10.4, 11.2}};
-        auto tiled = [&](int which, int64_t edge) {
-            const double tiles = (double)((M + edge - 1) / edge) * (double)((N + edge - 1) / edge) * (double)batches, rounds = ceil(tiles / 256.0);
-            const double clock = which == 0 ? 0.65 + 0.35 * tiles / (256.0 * rounds) : 1.0;
-            return rounds * (FIXED[which][kind] + PER_1024[which][kind] * clock * (double)K / 1024.0);
-        };
-        const bool whole = M % BM == 0 && N % BN == 0;
-        const bool staged = (fmt_a == fmt_b || mixed) && (whole || kind != 0 || K % 256 == 0);
-        int tile = 0;
-        const double cost16 = gemm_split_cost(g, batches, fmt_a, fmt_b, &tile);
-        const double cost128 = tiled(0, 128), cost256 = staged ? tiled(1, 256) : cost128 + 1.0;
-        if (cost16 <= cost128 && cost16 <= cost256) {
+        if (cost16 == least) {
             gemm_split_launch(g, batches, tile, fmt_a, fmt_b, c_dtype, st);
-        } else if (cost128 < cost256) {
+        } else if (cost128 == least) {
             gemm_tile_launch(g, batches, fmt_a, fmt_b, c_dtype, st);
         } else if (!whole) {
             gemm_edge_launch(g, batches, fmt_a, fmt_b, c_dtype, st);

@@ -19,6 +19,7 @@
 // elements: registers 0-3 hold bytes 16g.. of the step's first 64 and registers 4-7 the same of its second 64.  The
 // result has row 4g + e of A and row r of B in register e.
 #include "gemm_mx_args.h"
+#include <cmath>
 #include <type_traits>
 
 namespace {
@@ -293,15 +294,20 @@ void launch_b(const GemmArgs& g, int64_t batches, int tile, int fmt_b, int c_dty
 // tile; beyond that the total falls as tiles grow.
 double gemm_split_cost(const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b, int* tile) {
     const int tiles[] = {11, 12, 14, 22, 24, 44};
-    double best = 0.0;
+    double best = 0.0, cost = 0.0;
     for (int t : tiles) {
         const int mb = t / 10, nb = t % 10;
         const double wgs = (double)((g.M + 16 * mb - 1) / (16 * mb)) * ((g.N + 16 * nb - 1) / (16 * nb)) * (double)batches;
         const double row = mb * (fmt_a == MPSA_FMT_E2M1 ? 0.5 : 1.0) + nb * (fmt_b == MPSA_FMT_E2M1 ? 0.5 : 1.0);
-        const double cost = (0.4 + 0.2 * mb * nb + 0.0145 * 16.0 * row * g.K / 1024.0) * (wgs > 256.0 ? wgs / 256.0 : 1.0);
-        if (best == 0.0 || cost < best) { best = cost; *tile = t; }
+        const double rank = (0.4 + 0.2 * mb * nb + 0.0145 * 16.0 * row * g.K / 1024.0) * (wgs > 256.0 ? wgs / 256.0 : 1.0);
+        if (best == 0.0 || rank < best) {
+            best = rank;
+            *tile = t;
+            // against the other kernels: what it takes with the chip's load (within 14 %)
+            cost = 2.0 + (0.05 * mb * nb + 0.06 * row * g.K / 1024.0) * pow(wgs > 256.0 ? wgs / 256.0 : 1.0, 0.95) * (1.0 + 5.3 * (wgs < 256.0 ? wgs / 256.0 : 1.0));
+        }
     }
-    return best;
+    return cost;
 }
 
 void gemm_split_launch(const GemmArgs& g, int64_t batches, int tile, int fmt_a, int fmt_b, int c_dtype, hipStream_t st) {
