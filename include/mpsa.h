@@ -126,6 +126,12 @@ int mpsa_quantize_mx(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N
                      const int64_t x_strides[4], const void* sub, float pre_scale, int fmt, int emax_elem,
                      uint8_t* codes, uint8_t* scales, int64_t out_rows, mpsa_stream_t stream);
 
+/* mpsa_quantize_mx with a choice of layouts: code_per_byte != 0 leaves E2M1 codes one per byte ([B,H,out_rows,D], low nibble;
+ * 8-bit formats: ignored); scales_5d != 0 leaves the scales as mpsa_scales_to_5d does (out_rows and D in multiples of 128). */
+int mpsa_quantize_mx_as(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,
+                        const int64_t x_strides[4], const void* sub, float pre_scale, int fmt, int emax_elem,
+                        uint8_t* codes, uint8_t* scales, int64_t out_rows, int code_per_byte, int scales_5d, mpsa_stream_t stream);
+
 /*
  * Both precisions in one pass over x (the diagonal-tiled attention needs Q and K in E2M1 and in
  * an 8-bit format).  Same contract as two mpsa_quantize_mx calls with (E2M1, emax4) and

@@ -144,12 +144,35 @@ __global__ __launch_bounds__(256) void nibble_kernel(const uint8_t* src, uint8_t
     }
 }
 
+// The same along the innermost dimension (even n): sixteen codes and eight packed bytes per thread.  Copying memory with a
+// byte per thread and three 64-bit divisions each took 7.6 us for 4 MiB of codes; this way 3.
+template <bool PACK>
+__global__ __launch_bounds__(256) void nibble_flat_kernel(const uint8_t* src, uint8_t* dst, int64_t groups) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= groups) return;
+    if (PACK) {
+        const uint4 x = reinterpret_cast<const uint4*>(src)[i];
+        reinterpret_cast<uint2*>(dst)[i] = make_uint2(gather_nibbles(x.x) | (gather_nibbles(x.y) << 16), gather_nibbles(x.z) | (gather_nibbles(x.w) << 16));
+    } else {
+        const uint2 x = reinterpret_cast<const uint2*>(src)[i];
+        reinterpret_cast<uint4*>(dst)[i] = make_uint4(spread_nibbles(x.x & 0xFFFFu), spread_nibbles(x.x >> 16), spread_nibbles(x.y & 0xFFFFu), spread_nibbles(x.y >> 16));
+    }
+}
+
 int nibble_run(const char* what, const uint8_t* src, int64_t outer, int64_t n, int64_t inner, uint8_t* dst, bool pack, hipStream_t st) {
     if (outer < 0 || n < 0 || inner < 0) return mpsa_fail(MPSA_EINVAL, "%s: bad shape", what);
     const int64_t total = outer * ((n + 1) / 2) * inner;
     if (total == 0) return MPSA_OK;
     if (!src || !dst) return mpsa_fail(MPSA_EINVAL, "%s: null pointer", what);
     if (total >= (int64_t(1) << 39)) return mpsa_fail(MPSA_EUNSUPPORTED, "%s: tensor too large", what);
+    const uintptr_t wide = reinterpret_cast<uintptr_t>(pack ? src : dst), narrow = reinterpret_cast<uintptr_t>(pack ? dst : src);
+    if (inner == 1 && n % 2 == 0 && total % 8 == 0 && wide % 16 == 0 && narrow % 8 == 0) {
+        const dim3 flat((unsigned)((total / 8 + 255) / 256));
+        if (pack) hipLaunchKernelGGL(nibble_flat_kernel<true>, flat, dim3(256), 0, st, src, dst, total / 8);
+        else      hipLaunchKernelGGL(nibble_flat_kernel<false>, flat, dim3(256), 0, st, src, dst, total / 8);
+        MPSA_CHECK_LAUNCH(what);
+        return MPSA_OK;
+    }
     const dim3 grid((unsigned)((total + 255) / 256));
     if (pack) hipLaunchKernelGGL(nibble_kernel<true>, grid, dim3(256), 0, st, src, dst, outer, n, inner);
     else      hipLaunchKernelGGL(nibble_kernel<false>, grid, dim3(256), 0, st, src, dst, outer, n, inner);

@@ -74,3 +74,14 @@ __device__ __forceinline__ float e2m1_decode(uint32_t code) {
     const float mag = idx < 2u ? 0.5f * (float)idx : mpsa_u2f(((126u + (idx >> 1)) << 23) | ((idx & 1u) << 22));
     return (code & 8u) ? -mag : mag;
 }
+
+// four nibbles -> four bytes, and back (a byte's high nibble is dropped)
+__device__ __forceinline__ uint32_t spread_nibbles(uint32_t x) {
+    x = (x | (x << 8)) & 0x00FF00FFu;
+    return (x | (x << 4)) & 0x0F0F0F0Fu;
+}
+__device__ __forceinline__ uint32_t gather_nibbles(uint32_t x) {
+    x &= 0x0F0F0F0Fu;
+    x |= x >> 4;
+    return (x & 0xFFu) | ((x >> 8) & 0xFF00u);
+}

@@ -131,11 +131,14 @@ void launch(const QuantArgs& a, int fmt8, dim3 grid, hipStream_t st) {
 
 int quantize_common(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D, const int64_t* xs,
                     const void* sub, float pre, bool do4, int emax4, bool do8, int fmt8, int emax8,
-                    uint8_t* c4, uint8_t* s4, uint8_t* c8, uint8_t* s8, int64_t out_rows, hipStream_t st) {
+                    uint8_t* c4, uint8_t* s4, uint8_t* c8, uint8_t* s8, int64_t out_rows, hipStream_t st, bool spread = false, bool scales5d = false) {
     QuantArgs a;
     unsigned blocks = 0;
     const int rc = mpsa_quantize_setup(x, x_dtype, B, H, N, D, xs, sub, pre, do4, emax4, do8, fmt8, emax8, c4, s4, c8, s8, out_rows, &a, &blocks);
     if (rc != MPSA_OK || blocks == 0) return rc;
+    if (scales5d && (D % 128 || out_rows % 128)) return mpsa_fail(MPSA_EUNSUPPORTED, "quantize: packed scales need rows and D in multiples of 128 (got %lld, %lld)", (long long)out_rows, (long long)D);
+    a.spread = spread ? 1 : 0;
+    a.scales5d = scales5d ? 1 : 0;
     dim3 grid((blocks + 1) / 2, (unsigned)H, (unsigned)B);     // the kernel takes two blocks of chunks per workgroup
     if (x_dtype == MPSA_BF16) {
         if (do4 && do8) launch<MPSA_BF16, true, true>(a, fmt8, grid, st);
@@ -181,22 +184,29 @@ int mpsa_quantize_setup(const void* x, int x_dtype, int64_t B, int64_t H, int64_
     }
     a.emax4 = emax4; a.emax8 = emax8;
     a.codes4 = c4; a.scales4 = s4; a.codes8 = c8; a.scales8 = s8;
+    a.spread = a.scales5d = 0;
     *blocks = (unsigned)((chunks + 255) / 256);
     return MPSA_OK;
 }
 
 bool mpsa_quantize_sw_encoders() { return use_sw_fp8(); }
 
+extern "C" int mpsa_quantize_mx_as(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,
+                                   const int64_t x_strides[4], const void* sub, float pre_scale, int fmt, int emax_elem,
+                                   uint8_t* codes, uint8_t* scales, int64_t out_rows, int code_per_byte, int scales_5d, mpsa_stream_t stream) {
+    if (fmt == MPSA_FMT_E2M1)
+        return quantize_common(x, x_dtype, B, H, N, D, x_strides, sub, pre_scale, true, emax_elem, false, 0, 0,
+                               codes, scales, nullptr, nullptr, out_rows, (hipStream_t)stream, code_per_byte != 0, scales_5d != 0);
+    if (fmt == MPSA_FMT_E4M3 || fmt == MPSA_FMT_E5M2)
+        return quantize_common(x, x_dtype, B, H, N, D, x_strides, sub, pre_scale, false, 0, true, fmt, emax_elem,
+                               nullptr, nullptr, codes, scales, out_rows, (hipStream_t)stream, false, scales_5d != 0);
+    return mpsa_fail(MPSA_EINVAL, "quantize: unknown format %d", fmt);
+}
+
 extern "C" int mpsa_quantize_mx(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,
                                 const int64_t x_strides[4], const void* sub, float pre_scale, int fmt, int emax_elem,
                                 uint8_t* codes, uint8_t* scales, int64_t out_rows, mpsa_stream_t stream) {
-    if (fmt == MPSA_FMT_E2M1)
-        return quantize_common(x, x_dtype, B, H, N, D, x_strides, sub, pre_scale, true, emax_elem, false, 0, 0,
-                               codes, scales, nullptr, nullptr, out_rows, (hipStream_t)stream);
-    if (fmt == MPSA_FMT_E4M3 || fmt == MPSA_FMT_E5M2)
-        return quantize_common(x, x_dtype, B, H, N, D, x_strides, sub, pre_scale, false, 0, true, fmt, emax_elem,
-                               nullptr, nullptr, codes, scales, out_rows, (hipStream_t)stream);
-    return mpsa_fail(MPSA_EINVAL, "quantize: unknown format %d", fmt);
+    return mpsa_quantize_mx_as(x, x_dtype, B, H, N, D, x_strides, sub, pre_scale, fmt, emax_elem, codes, scales, out_rows, 0, 0, stream);
 }
 
 extern "C" int mpsa_quantize_mx_dual(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,

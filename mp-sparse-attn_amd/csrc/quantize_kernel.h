@@ -16,6 +16,8 @@ struct QuantArgs {
     int exact16;               // pre is a power of two: scaled values keep the inputs' 16-bit significands
     int emax4, emax8;
     uint8_t *codes4, *scales4, *codes8, *scales8;
+    int spread;                // 4-bit codes one per byte
+    int scales5d;              // scales as [rows/128, D/128, 32, 4, 4] (rows and D in multiples of 128)
 };
 
 // host side, defined in quantize.hip
@@ -227,15 +229,21 @@ __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, 
     int s4, s8;
     quantize_chunk<DO4, DO8, FMT8, SW8>(x, a.pre, a.exact16 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
     const int64_t oc = head * chunks + c;                                 // flat output chunk
+    int64_t os = oc >> 2;                                                 // and scale
+    if (a.scales5d) {
+        const uint32_t kc = cpr >> 4, block = col8 >> 2;
+        os = head * (chunks >> 2) + (((int64_t)(row >> 7) * kc + (block >> 2)) << 9) + ((row & 31) << 4) + ((row >> 5 & 3) << 2) + (block & 3);
+    }
     const bool quad_leader = (threadIdx.x & 3u) == 0u;
     // an output set that is not wanted has no pointer (one side of a mixed preparation: 8-bit Q, 4-bit K)
     if (DO4 && a.codes4) {
-        reinterpret_cast<uint32_t*>(a.codes4)[oc] = w4;
-        if (quad_leader) a.scales4[oc >> 2] = (uint8_t)s4;
+        if (a.spread) reinterpret_cast<uint2*>(a.codes4)[oc] = make_uint2(spread_nibbles(w4 & 0xFFFFu), spread_nibbles(w4 >> 16));
+        else          reinterpret_cast<uint32_t*>(a.codes4)[oc] = w4;
+        if (quad_leader) a.scales4[os] = (uint8_t)s4;
     }
     if (DO8 && a.codes8) {
         reinterpret_cast<uint2*>(a.codes8)[oc] = w8;
-        if (quad_leader) a.scales8[oc >> 2] = (uint8_t)s8;
+        if (quad_leader) a.scales8[os] = (uint8_t)s8;
     }
 }
 

@@ -43,6 +43,7 @@ SIGNATURES = {
     "mpsa_e2m1_unpack": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mpsa_scales_to_5d": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mpsa_scales_from_5d": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
+    "mpsa_quantize_mx_as": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _p64, _vp, _f32, _int, _int, _vp, _vp, _i64, _int, _int, _vp]),
     "mpsa_quantize_mx": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _p64, _vp, _f32, _int, _int, _vp, _vp, _i64, _vp]),
     "mpsa_seq_mean_workspace": (_i64, [_i64, _i64, _i64, _i64]),
     "mpsa_seq_mean": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _p64, _vp, _vp, _vp]),

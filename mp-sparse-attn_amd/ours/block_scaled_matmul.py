@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from .mxfp import MXFP4Tensor, MXScaleTensor
-from .quant_mxint8 import quantize_mx
+from .quant_mxint8 import _quantize_as
 
 VEC_SIZE = 32
 
@@ -237,8 +237,6 @@ def quantize_block_scaled_from_tensor(a_tensor, b_tensor, block_scale_type="mxfp
         raise ValueError(f"Invalid block scale type: {block_scale_type}")
     configs = make_configs(block_scale_type)
     fmt_a, fmt_b = _fmts_of(configs)
-    a, sa = quantize_mx(a_tensor[None, None], 1.0, fmt_a)
-    b, sb = quantize_mx(b_tensor[None, None], 1.0, fmt_b)
-    if packed_scales:
-        return a[0, 0], pack_scale_5d(sa[0, 0]), b[0, 0], pack_scale_5d(sb[0, 0]), configs
+    a, sa = _quantize_as(a_tensor[None, None], 1.0, fmt_a, scales_5d=packed_scales)
+    b, sb = _quantize_as(b_tensor[None, None], 1.0, fmt_b, scales_5d=packed_scales)
     return a[0, 0], sa[0, 0], b[0, 0], sb[0, 0], configs

@@ -18,7 +18,6 @@ import ctypes
 import torch
 
 from . import _lib
-from .mxfp import MXFP4Tensor
 
 LOG2E = 1.44269504          # ours/quant_mxint8.py:494
 EMAX_E2M1 = 3               # ours/quant_mxint8.py:303
@@ -81,19 +80,25 @@ def quantize_mx(x, pre_scale, fmt, emax_elem=None, out_rows=None, sub=None):
 
     ``out_rows`` >= L pads every head with zero rows (the attention kernel wants whole tiles).
     ``sub`` (``[B,H,D]``, x's dtype): quantize ``x - sub[:, :, None]`` (difference rounded to x's dtype)."""
+    return _quantize_as(x, pre_scale, fmt, emax_elem, out_rows, sub, False, False)
+
+
+def _quantize_as(x, pre_scale, fmt, emax_elem=None, out_rows=None, sub=None, code_per_byte=False, scales_5d=False):
+    """:func:`quantize_mx` with E2M1 codes one per byte, and with the scales in the packed ``[..., L/128, D/128, 32, 4, 4]``
+    layout (L and D multiples of 128), if asked for: ``mpsa_quantize_mx_as``."""
+    if emax_elem is None:
+        emax_elem = EMAX_E2M1 if fmt == _lib.FMT_E2M1 else EMAX_8BIT
     x = _check_input(x)
     B, H, L, D = x.shape
     rows = L if out_rows is None else int(out_rows)
-    if emax_elem is None:
-        emax_elem = EMAX_E2M1 if fmt == _lib.FMT_E2M1 else EMAX_8BIT
-    width = D // 2 if fmt == _lib.FMT_E2M1 else D
+    width = D // 2 if fmt == _lib.FMT_E2M1 and not code_per_byte else D
     device = x.device
     codes = torch.empty((B, H, rows, width), dtype=torch.uint8, device=device)
-    scales = torch.empty((B, H, rows, D // 32), dtype=torch.uint8, device=device)
+    scales = torch.empty((B, H, rows // 128, D // 128, 32, 4, 4) if scales_5d else (B, H, rows, D // 32), dtype=torch.uint8, device=device)
     with _lib.on_device(device):
-        status = _lib.lib().mpsa_quantize_mx(
+        status = _lib.lib().mpsa_quantize_mx_as(
             x.data_ptr(), _lib.dtype_id(x.dtype), B, H, L, D, _lib.strides4(x), _sub_ptr(sub, x), pre_scale, fmt, emax_elem,
-            codes.data_ptr(), scales.data_ptr(), rows, _lib.stream_ptr(device))
+            codes.data_ptr(), scales.data_ptr(), rows, code_per_byte, scales_5d, _lib.stream_ptr(device))
     if status:
         _lib.check(status)
     return codes, scales
@@ -118,12 +123,12 @@ def quantize_mx_dual(x, pre_scale, fmt8=_lib.FMT_E4M3, out_rows=None, sub=None):
     return c4, s4, c8, s8
 
 
-def _quant_pair(q, k, fmt, sm_scale, tensor_layout):
+def _quant_pair(q, k, fmt, sm_scale, tensor_layout, code_per_byte=False):
     q4 = _as_bhnd(q, tensor_layout)
     k4 = _as_bhnd(k, tensor_layout)
     head_dim = q4.shape[-1]
-    qc, qs = quantize_mx(q4, pre_scale_q(head_dim, sm_scale), fmt)
-    kc, ks = quantize_mx(k4, 1.0, fmt)
+    qc, qs = _quantize_as(q4, pre_scale_q(head_dim, sm_scale), fmt, code_per_byte=code_per_byte)
+    kc, ks = _quantize_as(k4, 1.0, fmt, code_per_byte=code_per_byte)
     return qc, qs, kc, ks
 
 
@@ -133,12 +138,7 @@ def quant_mxfp4(q, k, BLKQ=128, BLKK=64, sm_scale=None, tensor_layout="HND", pac
     Reference: ours/quant_mxint8.py:453-512.  ``BLKQ``/``BLKK`` were the reference's Triton tile
     heights and do not change the result; they are accepted and ignored.  Returns
     ``(q_codes, q_scale, k_codes, k_scale)`` in ``[B,H,L,*]`` order."""
-    qc, qs, kc, ks = _quant_pair(q, k, _lib.FMT_E2M1, sm_scale, tensor_layout)
-    if not packed:
-        unpack = MXFP4Tensor(size=(1,)).unpack_packed_tensor
-        qc = unpack(qc, 3, (*qc.shape[:3], qc.shape[3] * 2))
-        kc = unpack(kc, 3, (*kc.shape[:3], kc.shape[3] * 2))
-    return qc, qs, kc, ks
+    return _quant_pair(q, k, _lib.FMT_E2M1, sm_scale, tensor_layout, code_per_byte=not packed)
 
 
 def quant_mxfp8(q, k, BLKQ=128, BLKK=64, sm_scale=None, tensor_layout="HND"):

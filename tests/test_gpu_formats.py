@@ -87,3 +87,16 @@ def test_fp8_elementwise_cast_equals_torch(fmt, dt):
     nan = torch.isnan(want.view(dt).float())
     assert torch.equal(got[~nan], want[~nan])
     assert torch.isnan(got.view(dt).float()[nan]).all()          # NaN stays NaN (any payload)
+
+
+@pytest.mark.parametrize("shape,skew", [((1, 2), 0), ((3, 5), 0), ((4, 16), 0), ((257, 34), 0), ((1000, 128), 0), ((64, 64), 1), ((64, 64), 8)])
+def test_nibbles_along_the_last_dimension(shape, skew):
+    """Sixteen codes at a time, a code at a time where the length or the alignment does not allow it."""
+    from ours.mxfp import MXFP4Tensor
+    n = shape[0] * shape[1]
+    codes = torch.randint(0, 16, (n + skew,), dtype=torch.uint8, device="cuda")[skew:].view(shape)
+    tensor = MXFP4Tensor(data=codes, dtype=torch.uint8)
+    packed = tensor.to_packed_tensor(1)
+    padded = torch.nn.functional.pad(codes.cpu(), (0, shape[1] % 2))
+    assert torch.equal(packed.cpu(), padded[:, 0::2] | padded[:, 1::2] << 4)
+    assert torch.equal(tensor.unpack_packed_tensor(packed, 1, shape), codes)

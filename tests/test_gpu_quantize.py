@@ -199,3 +199,16 @@ def test_empty_and_single_row_inputs():
     x = torch.randn(1, 1, 1, 32).bfloat16()
     _check(x, 1.0, O.FMT_E2M1)
     _check(x, 1.0, O.FMT_E4M3, out_rows=5)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 4])
+@pytest.mark.parametrize("B,H,L,rows,D", [(1, 1, 128, 128, 128), (2, 3, 200, 256, 128), (1, 2, 128, 384, 640)])
+def test_layouts_written_directly_equal_the_separate_passes(fmt, B, H, L, rows, D):
+    from ours.block_scaled_matmul import pack_scale_5d
+    from ours.mxfp import MXFP4Tensor
+    from ours.quant_mxint8 import _quantize_as, quantize_mx
+    x = torch.randn(B, H, L, D, dtype=torch.bfloat16, device="cuda")
+    codes, scales = quantize_mx(x, 1.0, fmt, out_rows=rows)
+    wide, packed = _quantize_as(x, 1.0, fmt, out_rows=rows, code_per_byte=True, scales_5d=True)
+    want = MXFP4Tensor(size=(1,)).unpack_packed_tensor(codes, 3, (B, H, rows, D)) if fmt == 4 else codes
+    assert torch.equal(wide, want) and torch.equal(packed, pack_scale_5d(scales))
