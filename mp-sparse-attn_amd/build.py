@@ -17,6 +17,8 @@ LIB = os.path.join(LIBDIR, "libmpsa.so")
 # measurement kernels that bench.py loads by itself; not part of the library or its header
 BENCH_LIB = os.path.join(LIBDIR, "libmpsa_bench.so")
 BENCH_SOURCES = ["bench/mfma_stream.hip"]
+# the host side of short calls (csrc/host.cpp): a Python extension over torch's C++ API and libmpsa.so
+HOST_LIB = os.path.join(LIBDIR, "mpsa_host.so")
 
 SOURCES = ["api.hip", "formats.hip", "quantize.hip", "v_tiles.hip", "prepare.hip", "gemm_mx.hip", "gemm_mx_split.hip", "gemm_mx_tile.hip", "gemm_mx_edge.hip", "attn_fwd.hip", "attn_fwd_skip.hip", "attn_fwd_routed.hip", "attn_fwd_pp.hip", "attn_call.hip", "attn_fwd_short.hip", "route.hip", "skip_route.hip"]
 
@@ -46,6 +48,19 @@ def _run(cmd):
     return out
 
 
+def _build_host(obj):
+    """Compile host.cpp (no device code) with the host compiler."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))) if os.path.sep in _hipcc() else "/opt/rocm"
+    includes = cpp_extension.include_paths() + [sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DTORCH_EXTENSION_NAME=mpsa_host"]
+         + [x for i in includes for x in ("-isystem", i)] + ["-c", os.path.join(CSRC, "host.cpp"), "-o", obj])
+    return rocm
+
+
 def build_lib(verbose=False):
     os.makedirs(LIBDIR, exist_ok=True)
     objdir = os.path.join(HERE, "build")
@@ -59,10 +74,16 @@ def build_lib(verbose=False):
             print(out)
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + len(BENCH_SOURCES))) as ex:
+    host_obj = os.path.join(objdir, "host.o")
+    with ThreadPoolExecutor(max_workers=8) as ex:
+        host = ex.submit(_build_host, host_obj)
         objs = list(ex.map(compile_one, SOURCES + BENCH_SOURCES))
+        rocm = host.result()
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs[:len(SOURCES)])
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", BENCH_LIB] + objs[len(SOURCES):])
+    from torch.utils import cpp_extension
+    libs = [x for d in cpp_extension.library_paths() for x in ("-L", d)] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-L", os.path.join(rocm, "lib"), "-lamdhip64"]
+    _run([os.environ.get("CXX", "g++"), "-shared", "-o", HOST_LIB, host_obj, "-L", LIBDIR, "-lmpsa", "-Wl,-rpath,$ORIGIN"] + libs)
     return LIB
 
 

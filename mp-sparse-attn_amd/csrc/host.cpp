@@ -1,0 +1,113 @@
+// The host side of the calls that a decode step or a short prompt makes again and again, in native code.
+//
+// What bounds them is the host: allocating results, reading shapes and strides and marshalling fifteen arguments in Python took
+// 23 us for a 16-row linear layer (a quantization and a product) whose kernels take 7.  Here a call checks the usual case,
+// allocates and launches; it returns None for anything unusual -- another device current, a layout that needs a copy, a shape
+// or type that is an error -- and the caller goes on with its own code, which copies or says what is wrong.
+#include <torch/csrc/utils/pybind.h>
+#include <ATen/ATen.h>
+#include <hip/hip_runtime_api.h>
+#include "../../include/mpsa.h"
+
+namespace py = pybind11;
+using at::Tensor;
+
+namespace {
+
+// on the device that is current
+bool here(const Tensor& t) {
+    int device = -1;
+    return t.is_cuda() && hipGetDevice(&device) == hipSuccess && device == t.get_device();
+}
+
+bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0; }
+
+int dtype_id(at::ScalarType t) {
+    switch (t) {
+        case at::kBFloat16: return MPSA_BF16;
+        case at::kHalf: return MPSA_F16;
+        case at::kFloat: return MPSA_F32;
+        case at::kFloat8_e5m2: return MPSA_F8E5M2;
+        default: return -1;
+    }
+}
+
+mpsa_stream_t stream_of(int64_t s) { return reinterpret_cast<mpsa_stream_t>(s); }
+
+py::object quantize(const Tensor& x, double pre, int fmt, int emax, int64_t rows, bool code_per_byte, bool scales_5d, int64_t stream) {
+    if (x.dim() != 4 || !here(x) || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf)) return py::none();
+    const auto s = x.strides();
+    if (s[3] != 1 || ((s[0] | s[1] | s[2]) & 7) || !aligned16(x)) return py::none();
+    const int64_t B = x.size(0), H = x.size(1), L = x.size(2), D = x.size(3), n = rows < 0 ? L : rows;
+    if (D % 32 || D == 0 || n < L || (scales_5d && (D % 128 || n % 128))) return py::none();
+    const bool four = fmt == MPSA_FMT_E2M1;
+    const auto bytes = x.options().dtype(at::kByte);
+    Tensor codes = at::empty({B, H, n, four && !code_per_byte ? D / 2 : D}, bytes);
+    Tensor scales = scales_5d ? at::empty({B, H, n / 128, D / 128, 32, 4, 4}, bytes) : at::empty({B, H, n, D / 32}, bytes);
+    const int rc = mpsa_quantize_mx_as(x.const_data_ptr(), dtype_id(x.scalar_type()), B, H, L, D, s.data(), nullptr, (float)pre, fmt, emax,
+                                       codes.data_ptr<uint8_t>(), scales.data_ptr<uint8_t>(), n, code_per_byte, scales_5d, stream_of(stream));
+    if (rc != MPSA_OK) return py::none();
+    return py::make_tuple(std::move(codes), std::move(scales));
+}
+
+// codes of `rows` rows of K elements behind the leading dims, bytes, contiguous
+bool operand(const Tensor& t, const Tensor& scale, at::IntArrayRef lead, int64_t rows, int64_t K, int fmt, bool packed, int device) {
+    const size_t n = lead.size();
+    if (!t.is_cuda() || !scale.is_cuda() || t.get_device() != device || scale.get_device() != device) return false;
+    if (t.element_size() != 1 || scale.scalar_type() != at::kByte || !t.is_contiguous() || !scale.is_contiguous()) return false;
+    if (t.dim() != (int64_t)n + 2 || scale.dim() != (int64_t)n + (packed ? 5 : 2)) return false;
+    for (size_t i = 0; i < n; ++i)
+        if (t.size(i) != lead[i] || scale.size(i) != lead[i]) return false;
+    if (t.size(n) != rows || t.size(n + 1) != (fmt == MPSA_FMT_E2M1 ? K / 2 : K)) return false;
+    if (packed) return scale.size(n) == rows / 128 && scale.size(n + 1) == K / 128 && scale.size(n + 2) == 32 && scale.size(n + 3) == 4 && scale.size(n + 4) == 4;
+    return scale.size(n) == rows && scale.size(n + 1) == K / 32;
+}
+
+py::object matmul(const Tensor& a, const Tensor& sa, int fmt_a, const Tensor& b, const Tensor& sb, int fmt_b, at::ScalarType dtype,
+                  int64_t M, int64_t N, int64_t K, int64_t stream) {
+    const bool packed = sa.dim() == 5 && sb.dim() == 5;
+    if (!here(a) || dtype_id(dtype) < 0 || M <= 0 || N <= 0 || K <= 0 || !operand(a, sa, {}, M, K, fmt_a, packed, a.get_device()) ||
+        !operand(b, sb, {}, N, K, fmt_b, packed, a.get_device()))
+        return py::none();
+    Tensor c = at::empty({M, N}, a.options().dtype(dtype));
+    const auto entry = packed ? mpsa_gemm_mx_packed : mpsa_gemm_mx;
+    const int rc = entry(static_cast<const uint8_t*>(a.const_data_ptr()), sa.const_data_ptr<uint8_t>(), fmt_a, static_cast<const uint8_t*>(b.const_data_ptr()),
+                         sb.const_data_ptr<uint8_t>(), fmt_b, M, N, K, c.data_ptr(), dtype_id(dtype), N, stream_of(stream));
+    if (rc != MPSA_OK) return py::none();
+    return py::cast(std::move(c));
+}
+
+py::object matmul_batched(const Tensor& a, const Tensor& sa, int fmt_a, const Tensor& b, const Tensor& sb, int fmt_b, at::ScalarType dtype,
+                          int64_t B, int64_t H, int64_t M, int64_t N, int64_t K, int64_t stream) {
+    const bool packed = sa.dim() == 7 && sb.dim() == 7;
+    if (!here(a) || dtype_id(dtype) < 0 || b.dim() != 4 || B <= 0 || H <= 0 || M <= 0 || N <= 0 || K <= 0) return py::none();
+    const int64_t Hb = b.size(1);
+    if (Hb <= 0 || H % Hb || !operand(a, sa, {B, H}, M, K, fmt_a, packed, a.get_device()) || !operand(b, sb, {B, Hb}, N, K, fmt_b, packed, a.get_device()))
+        return py::none();
+    Tensor c = at::empty({B, H, M, N}, a.options().dtype(dtype));
+    const auto entry = packed ? mpsa_gemm_mx_batched_packed : mpsa_gemm_mx_batched;
+    const int rc = entry(static_cast<const uint8_t*>(a.const_data_ptr()), sa.const_data_ptr<uint8_t>(), fmt_a, static_cast<const uint8_t*>(b.const_data_ptr()),
+                         sb.const_data_ptr<uint8_t>(), fmt_b, B, H, Hb, M, N, K, c.data_ptr(), dtype_id(dtype), N, stream_of(stream));
+    if (rc != MPSA_OK) return py::none();
+    return py::cast(std::move(c));
+}
+
+// mpsa_attn_call with the output and the workspace allocated here; desc is the address of an mpsa_attn_desc
+py::object attention(int64_t desc, int64_t workspace, const std::vector<int64_t>& shape, at::ScalarType dtype, const Tensor& q, const Tensor& k,
+                     const Tensor& v, int64_t stream) {
+    if (!here(q)) return py::none();
+    Tensor out = at::empty(shape, q.options().dtype(dtype)), work = at::empty({workspace}, q.options().dtype(at::kByte));
+    const int rc = mpsa_attn_call(reinterpret_cast<const mpsa_attn_desc*>(desc), q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(),
+                                  out.data_ptr(), work.data_ptr(), nullptr, stream_of(stream));
+    if (rc != MPSA_OK) return py::none();
+    return py::cast(std::move(out));
+}
+
+}  // namespace
+
+PYBIND11_MODULE(mpsa_host, m) {
+    m.def("quantize", &quantize);
+    m.def("matmul", &matmul);
+    m.def("matmul_batched", &matmul_batched);
+    m.def("attention", &attention);
+}

@@ -5,6 +5,8 @@ pointers, sizes and element strides, and kernels are enqueued on torch's current
 """
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -111,6 +113,32 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+class _NoHost:
+    """Stands in for the extension where MPSA_LIB_PATH names another library than the one it is linked to."""
+    quantize = matmul = matmul_batched = attention = staticmethod(lambda *args: None)
+
+
+def host():
+    """The native host side of short calls (csrc/host.cpp).  Its functions return None for anything but the usual case."""
+    global _host
+    if _host is None:
+        lib()
+        if os.environ.get("MPSA_LIB_PATH"):
+            _host = _NoHost
+            return _host
+        path = os.path.join(os.path.dirname(LIB_PATH), "mpsa_host.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `python mp-sparse-attn_amd/build.py`")
+        loader = importlib.machinery.ExtensionFileLoader("mpsa_host", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("mpsa_host", path, loader=loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
+
+
 def check(status):
     if status != 0:
         raise MpsaError(status, lib().mpsa_last_error().decode("utf-8", "replace"))
@@ -131,6 +159,11 @@ def require_device(*tensors):
         if not isinstance(t, torch.Tensor) or not t.is_cuda:
             raise RuntimeError("the MXFP path runs on HIP device tensors only (got a %s tensor); "
                                "there is no CPU fallback" % (t.device if isinstance(t, torch.Tensor) else type(t)))
+
+
+def raw_stream(tensor):
+    """:func:`stream_ptr` of a device tensor's device."""
+    return torch._C._cuda_getCurrentRawStream(tensor.get_device())
 
 
 def stream_ptr(device=None):

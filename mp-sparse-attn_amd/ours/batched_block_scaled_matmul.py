@@ -24,6 +24,9 @@ def block_scaled_batched_matmul(a, a_scale, b, b_scale, dtype_dst, B, H, M, N, K
         raise ValueError(f"Unsupported dtype: {dtype_dst}")
     fmt_a, fmt_b = _fmts_of(configs)
     _lib.require_device(a, a_scale, b, b_scale)
+    done = _lib.host().matmul_batched(a, a_scale, fmt_a, b, b_scale, fmt_b, dtype_dst, B, H, M, N, K, _lib.raw_stream(a))
+    if done is not None:
+        return done
     packed = a_scale.dim() == 7 and b_scale.dim() == 7      # both packed: the kernel takes them as they are
     if not packed:
         if a_scale.dim() == 7:

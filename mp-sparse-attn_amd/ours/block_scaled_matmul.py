@@ -88,6 +88,9 @@ def block_scaled_matmul(a, a_scale, b, b_scale, dtype_dst, M, N, K, configs):
         raise ValueError(f"Unsupported dtype: {dtype_dst}")
     fmt_a, fmt_b = _fmts_of(configs)
     _lib.require_device(a, a_scale, b, b_scale)
+    done = _lib.host().matmul(a, a_scale, fmt_a, b, b_scale, fmt_b, dtype_dst, M, N, K, _lib.raw_stream(a))
+    if done is not None:
+        return done
     # the reference's packed scale layout goes to the kernel as it is when both operands come that way
     packed = a_scale.dim() == 5 and b_scale.dim() == 5
     if not packed:

@@ -312,7 +312,7 @@ def _aligned(t):
 def _plan(q_shape, q_stride, k_shape, k_stride, v_shape, v_stride, dtype, is_causal, scale, smooth_k, tensor_layout, output_dtype,
           block_scale_type, skip_thresh, tile, route_thresh):
     """Checks the arguments of a call and describes it for ``mpsa_attn_call``: ``(description, workspace bytes, output shape,
-    whether tiles can be left out)``, or None if a row is not contiguous or not 16-byte aligned.  A pure function of shapes,
+    whether tiles can be left out, the description's address)``, or None if a row is not contiguous or not 16-byte aligned.  A pure function of shapes,
     strides and options, kept for the last few hundred different ones: of a short call's host time it would be the largest
     part."""
     if tensor_layout not in ("HND", "NHD"):
@@ -350,7 +350,7 @@ def _plan(q_shape, q_stride, k_shape, k_stride, v_shape, v_stride, dtype, is_cau
     nbytes = _lib.lib().mpsa_attn_call_workspace(desc)
     if nbytes < 0:
         _lib.check(nbytes)
-    return desc, nbytes, out_shape, mode == _lib.MODE_ROUTED or skip_thresh is not None
+    return desc, nbytes, out_shape, mode == _lib.MODE_ROUTED or skip_thresh is not None, ctypes.addressof(desc)
 
 
 def _reject_unsupported(attn_mask, dropout_p, attention_sink):
@@ -390,7 +390,11 @@ def mxfp_attn_kernel(q, k, v, attn_mask=None, dropout_p=0.0,
     if plan is None:                     # some row is not contiguous or not 16-byte aligned
         return mxfp_attn_kernel(_aligned(q), _aligned(k), _aligned(v), None, 0.0, is_causal, scale, smooth_k, False, tensor_layout,
                                 output_dtype, return_sparsity, block_scale_type, skip_thresh, tile, route_thresh)
-    desc, nbytes, out_shape, leaves_out = plan
+    desc, nbytes, out_shape, leaves_out, address = plan
+    if not return_sparsity:
+        out = _lib.host().attention(address, nbytes, out_shape, output_dtype, q, k, v, _lib.raw_stream(q))
+        if out is not None:
+            return out
     out = torch.empty(out_shape, dtype=output_dtype, device=device)
     work = torch.empty(nbytes, dtype=torch.uint8, device=device)
     share = None
