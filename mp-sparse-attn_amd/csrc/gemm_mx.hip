@@ -50,6 +50,7 @@ __device__ __forceinline__ int load_scale(const uint8_t* s, int row, int kb, int
 
 template <int FA, int FB>
 constexpr int general_smem() { return 2 * (EdgeOp<FA>::BYTES + EdgeOp<FB>::BYTES); }
+static_assert(4 * rows16_bytes<2>() <= general_smem<MPSA_FMT_E2M1, MPSA_FMT_E2M1>(), "room for the results on their way out");
 
 template <int FA, int FB, typename OutT>
 __global__ __launch_bounds__(256, 2) void gemm_mx_general_kernel(GemmArgs g) {
@@ -180,6 +181,15 @@ __global__ __launch_bounds__(256, 2) void gemm_mx_general_kernel(GemmArgs g) {
 
     // accumulator register e of lane (h, r) is C[8*(e/4) + 4*h + e%4][r] of its 32 x 32 block
     OutT* c = static_cast<OutT*>(g.c) + (int64_t)bz * g.M * g.ldc;
+    if constexpr (sizeof(OutT) == 2) {
+        if (rows16_aligned(g)) {
+            __syncthreads();                             // everybody has read the last stage
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                store_rows16<2, OutT, true>(acc[i], smem + wave * rows16_bytes<2>(), c, g.ldc, m0 + i * 32, n0, g.M, g.N, lane);
+            return;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll

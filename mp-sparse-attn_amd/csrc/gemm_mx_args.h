@@ -48,4 +48,48 @@ template <> __device__ __forceinline__ OutE5M2 cvt_out<OutE5M2>(float v) {
     return OutE5M2{(uint8_t)(__builtin_amdgcn_cvt_pk_bf8_f32(v, v, 0, false) & 0xFF)};
 }
 
+// Whether 16-bit results may be stored in pieces of 16 bytes: every row starts on such a piece.
+__device__ __forceinline__ bool rows16_aligned(const GemmArgs& g) { return ((reinterpret_cast<uintptr_t>(g.c) | (uintptr_t)(2 * g.ldc)) & 15) == 0; }
+
+// LDS bytes a wave needs to store 32 rows of 32 * NJ 16-bit results
+template <int NJ> constexpr int rows16_bytes() { return 32 * (NJ * 64 + 64); }
+
+// A wave's NJ neighbouring 32 x 32 blocks (accumulator register e of lane (h, r) is element [8*(e/4) + 4*h + e%4][r]) as 16-bit
+// results, through LDS of the wave's own, in pieces of 16 bytes.  Straight from the registers a store moves 2 bytes a lane, half
+// of two rows' 128-byte lines, there are eight times as many, and ragged tiles check the edges for each element.  Measured
+// (bf16 results): 16 score products of 2048 x 2048 x 128, 4-bit, 29.4 -> 25.1 us (5.3 TB/s of results; a fill of that size
+// reaches 7.4), 8-bit 39.5 -> 31; 1000 x 14336 x 4096, 8-bit x 4-bit, 51.6 -> 47.5; 1000 x 4096 x 4096, 4-bit, 17.4 -> 16.4.
+// Two rows of two neighbouring lanes trade places first, so that LDS is written a word at a time; the row pitch (16 words past a
+// multiple of 32) puts the two rows of a write into different banks.
+template <int NJ, typename OutT, bool EDGE>
+__device__ __forceinline__ void store_rows16(const v16f (&acc)[NJ], uint8_t* lds, OutT* c, int64_t ldc, int row0, int col0, int M, int N, int lane) {
+    typedef OutT v2o __attribute__((ext_vector_type(2)));
+    constexpr int PITCH = NJ * 64 + 64, LPR = 4 * NJ;    // bytes from row to row; lanes per row on the way out
+    const int h = lane >> 5, r = lane & 31;
+    const uint32_t sel = (r & 1) ? 0x03020706u : 0x05040100u;
+    uint8_t* const to = lds + (4 * h + (r & 1)) * PITCH + (r >> 1) * 4;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; e += 2) {
+            const uint32_t own = __builtin_bit_cast(uint32_t, (v2o){cvt_out<OutT>(acc[j][e]), cvt_out<OutT>(acc[j][e + 1])});
+            const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)own, 0xB1, 0xf, 0xf, true);       // of lane ^ 1
+            *reinterpret_cast<uint32_t*>(to + (8 * (e >> 2) + (e & 3)) * PITCH + j * 64) = __builtin_amdgcn_perm(other, own, sel);
+        }
+    const int lrow = lane / LPR, col = col0 + 8 * (lane % LPR);
+    const uint8_t* const from = lds + lrow * PITCH + (lane % LPR) * 16;
+    OutT* out = c + (int64_t)(row0 + lrow) * ldc + col;
+#pragma unroll
+    for (int x = 0; x < 32; x += 64 / LPR) {
+        const v4i w = *reinterpret_cast<const v4i*>(from + x * PITCH);
+        if (!EDGE || (row0 + lrow + x < M && col + 8 <= N)) {
+            *reinterpret_cast<v4i*>(out + (int64_t)x * ldc) = w;
+        } else if (row0 + lrow + x < M) {
+#pragma unroll
+            for (int y = 0; y < 8; ++y)
+                if (col + y < N) out[(int64_t)x * ldc + y] = __builtin_bit_cast(OutT, (unsigned short)((uint32_t)w[y >> 1] >> (16 * (y & 1))));
+        }
+    }
+}
+
 }  // namespace

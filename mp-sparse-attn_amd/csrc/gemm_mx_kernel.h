@@ -36,7 +36,7 @@
 //
 // Ragged edges.  EDGE runs take any M and N: rows past the matrix are fetched from its last row (a lane's row offset is
 // capped with one comparison per load) and not stored.  Their own instantiations, so that whole tiles pay nothing: 1000 x
-// 14336 x 4096 takes 41 us 4-bit and 55 us 8-bit x 4-bit where 1024 rows take 38 and 52 (the general kernel: 102, 106).
+// 14336 x 4096 takes 37 us 4-bit and 47.5 us 8-bit x 4-bit where 1024 rows take 38 and 52 (the general kernel: 102, 106).
 #pragma once
 #include "gemm_mx_args.h"
 
@@ -512,6 +512,15 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
 
     // epilogue: accumulator register e of lane (h, r) is C[8*(e/4) + 4*h + e%4][r] of its 32x32 block
     OutT* c = static_cast<OutT*>(g.c) + (int64_t)bz * g.M * g.ldc;
+    if constexpr (EDGE && sizeof(OutT) == 2) {         // whole tiles gain nothing by it: 8192^3 0.98 to 1.014 of the time
+        if (rows16_aligned(g)) {
+            __syncthreads();                           // the ring is free: everybody has read it, and nothing is on its way into it
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                store_rows16<4, OutT, EDGE>(acc[i], smem + wave * rows16_bytes<4>(), c, g.ldc, m0 + wm * 128 + i * 32, n0 + wn * 128, g.M, g.N, lane);
+            return;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll

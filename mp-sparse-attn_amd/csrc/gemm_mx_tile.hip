@@ -55,6 +55,7 @@ struct TileGeom {
     static constexpr int SCALES = 256 * 16;              // one group: 128 rows of A, then 128 of B
     static constexpr int LOADS = OA::IPW + OB::IPW;      // code instructions per wave and unit
     static constexpr int SMEM = RING * UNIT + 4 * SCALES;
+    static_assert(4 * 16384 + TW * rows16_bytes<2>() <= SMEM, "the waves' sums, and behind them the results on their way out");
 };
 
 template <int FA, int FB, typename OutT>
@@ -224,15 +225,28 @@ __global__ __launch_bounds__(TW * 64, 1) void gemm_mx_tile_kernel(GemmArgs a) {
         for (int e = 0; e < 16; ++e) x[((half * 2 + j) * 16 + e) * 64 + lane] = half ? acc[0][j][e] : acc[1][j][e];
     __syncthreads();
     OutT* c = static_cast<OutT*>(a.c) + (int64_t)bz * a.M * a.ldc;
+    const int row0 = m0 + wm * 64 + half * 32;
+    v16f sum[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const float other = x[(((1 - half) * 2 + j) * 16 + e) * 64 + lane];
+            sum[j][e] = half ? other + acc[1][j][e] : acc[0][j][e] + other;          // first half of K first
+        }
+    if constexpr (sizeof(OutT) == 2) {
+        if (rows16_aligned(a)) {
+            store_rows16<2, OutT, true>(sum, smem + 4 * 16384 + wave * rows16_bytes<2>(), c, a.ldc, row0, n0 + wn * 64, a.M, a.N, lane);
+            return;
+        }
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int col = n0 + wn * 64 + j * 32 + r;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const float other = x[(((1 - half) * 2 + j) * 16 + e) * 64 + lane];
-            const float v = half ? other + acc[1][j][e] : acc[0][j][e] + other;      // first half of K first
-            const int row = m0 + wm * 64 + half * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-            if (row < a.M && col < a.N) c[(int64_t)row * a.ldc + col] = cvt_out<OutT>(v);
+            const int row = row0 + 8 * (e >> 2) + 4 * h + (e & 3);
+            if (row < a.M && col < a.N) c[(int64_t)row * a.ldc + col] = cvt_out<OutT>(sum[j][e]);
         }
     }
 }

@@ -607,3 +607,27 @@ def test_batched_slices_equal_the_2d_product_on_every_kernel(bst, packed):
             for h in range(H):
                 one = block_scaled_matmul(ac[i, h], sa[i, h], bc[i, h // 2], sb[i, h // 2], torch.float32, M, N, K, on)
                 assert torch.equal(got[i, h], one), (kernel, i, h)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kernel", ["general", "tile128", "tile256"])
+@pytest.mark.parametrize("M,N,ldc", [(1, 8, 8), (31, 250, 256), (129, 129, 136), (257, 263, 264), (300, 520, 520), (256, 512, 520),
+                                     (130, 77, 77), (257, 300, 303), (256, 256, 257)])
+def test_16bit_results_are_the_float32_ones_rounded_once(kernel, M, N, ldc, dtype):
+    """Rows in whole 16-byte pieces (row pitch a multiple of 8) and not, the last piece of a row cut, and nothing written
+    past a row's end: the same bits as float32 results rounded once, and the gap between rows as it was."""
+    K, L = 256, _lib.lib()
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randint(0, 256, (M, K // 2), dtype=torch.uint8, generator=g).to(DEV)
+    b = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=g).to(DEV)
+    sa = torch.randint(118, 130, (M, K // 32), dtype=torch.uint8, generator=g).to(DEV)
+    sb = torch.randint(118, 130, (N, K // 32), dtype=torch.uint8, generator=g).to(DEV)
+
+    def product(dt):
+        c = torch.full((M + 1, ldc), 7.0, dtype=dt, device=DEV)
+        _lib.check(L.mpsa_gemm_mx_on(_lib.GEMM_KERNELS[kernel], _lib.ptr(a), _lib.ptr(sa), 4, _lib.ptr(b), _lib.ptr(sb), 4, 0, 1, 1, 1, M, N, K,
+                                     _lib.ptr(c), _lib.dtype_id(dt), ldc, _lib.stream_ptr(a.device)))
+        return c
+
+    got, want = product(dtype), product(torch.float32).to(dtype)
+    assert torch.equal(got, want)
