@@ -107,12 +107,18 @@ extern "C" int mpsa_attn_call_on(int kernel, const mpsa_attn_desc* d, const void
     auto at = [&](int64_t off) { return off < 0 ? nullptr : w + off; };
     uint8_t *q4 = at(l.q4), *qs4 = at(l.qs4), *q8 = at(l.q8), *qs8 = at(l.qs8), *k4 = at(l.k4), *ks4 = at(l.ks4), *k8 = at(l.k8), *ks8 = at(l.ks8);
     int32_t *order = reinterpret_cast<int32_t*>(at(l.order)), *counts = reinterpret_cast<int32_t*>(at(l.counts)), *skipped = reinterpret_cast<int32_t*>(at(l.skipped));
+    MeanSource mean = MEAN_NONE;
+    const void* k_sub = nullptr;
     if (d->smooth_k) {
-        rc = mpsa_seq_mean(k, d->dtype, d->B, d->Hkv, d->nk, d->D, d->k_strides, reinterpret_cast<float*>(at(l.mean_work)), at(l.mean), stream);
+        mean = mpsa_mean_source(d->B, d->Hkv, d->nk, d->D);
+        float* const sums = reinterpret_cast<float*>(at(l.mean_work));
+        k_sub = mean == MEAN_SUMS ? static_cast<const void*>(sums) : at(l.mean);
+        if (mean == MEAN_GIVEN)     rc = mpsa_seq_mean(k, d->dtype, d->B, d->Hkv, d->nk, d->D, d->k_strides, sums, at(l.mean), stream);
+        else if (mean == MEAN_SUMS) rc = mpsa_seq_mean_partial(k, d->dtype, d->B, d->Hkv, d->nk, d->D, d->k_strides, sums, (hipStream_t)stream);
         if (rc != MPSA_OK) return rc;
     }
     rc = mpsa_prepare_operands(l.fuse_q ? nullptr : q, d->q_strides, k, d->k_strides, v, d->v_strides, d->dtype, d->B, d->Hq, d->Hkv, d->nq, d->nk,
-                               d->D, d->tile, d->fmt8, d->pre_scale_q, at(l.mean), l.q4 >= 0, l.q8 >= 0, l.k4 >= 0, l.k8 >= 0, q4, qs4, q8, qs8, k4, ks4, k8, ks8, at(l.v), (hipStream_t)stream);
+                               d->D, d->tile, d->fmt8, d->pre_scale_q, mean, k_sub, l.q4 >= 0, l.q8 >= 0, l.k4 >= 0, l.k8 >= 0, q4, qs4, q8, qs8, k4, ks4, k8, ks8, at(l.v), (hipStream_t)stream);
     if (rc != MPSA_OK) return rc;
     if (l.fuse_q) {
         rc = mpsa_attn_fwd_q16_on(l.kernel, q, d->q_strides, d->dtype, d->pre_scale_q, k4, ks4, k8, ks8, d->fmt8, at(l.v), d->dtype, o, d->o_dtype, d->o_strides,

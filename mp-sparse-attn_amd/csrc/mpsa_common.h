@@ -27,10 +27,15 @@ static inline bool mpsa_aligned16(const void* p) { return (reinterpret_cast<uint
 bool mpsa_register_lds_kernel(const void* kern, int bytes);      // api.hip; always returns true
 int mpsa_ensure_init();                                          // api.hip; MPSA_OK or the failure of mpsa_init()
 int mpsa_seq_mean_static_resolve();                              // quantize.hip; address of the built-in partial-sum array
+// quantize.hip: the float32 sums of chunks of 256 rows that mpsa_seq_mean starts with, without the mean
+int mpsa_seq_mean_partial(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D, const int64_t x_strides[4], float* workspace, hipStream_t st);
+// prepare.hip: how a preparation comes by the mean over K's sequence that it takes off K
+enum MeanSource { MEAN_NONE, MEAN_GIVEN, MEAN_SUMS, MEAN_ROWS_ITSELF };      // none; k_sub is the mean; k_sub is the chunks' sums; from K
+MeanSource mpsa_mean_source(int64_t B, int64_t Hkv, int64_t nk, int64_t D);
 // prepare.hip: the operand preparation with the sets to make named apart for Q and K
 int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides,
                           int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int64_t D, int tile, int fmt8, float pre_scale_q,
-                          const void* k_sub, bool q_do4, bool q_do8, bool k_do4, bool k_do8, uint8_t* q4, uint8_t* qs4, uint8_t* q8, uint8_t* qs8,
+                          MeanSource mean, const void* k_sub, bool q_do4, bool q_do8, bool k_do4, bool k_do8, uint8_t* q4, uint8_t* qs4, uint8_t* q8, uint8_t* qs8,
                           uint8_t* k4, uint8_t* ks4, uint8_t* k8, uint8_t* ks8, void* v_tiles, hipStream_t st);
 
 #define MPSA_CHECK_LAUNCH(what)                                                        \

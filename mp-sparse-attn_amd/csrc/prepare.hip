@@ -5,7 +5,7 @@
 // quantize_kernel / v_tiles_kernel (quantize_kernel.h, v_tiles_kernel.h); this file only routes workgroup ids.
 // Replaces the prologue of the reference's wrapper, ours/mxfp_attn_kernel.py:27-57 (dtype normalisation, quant_mxfp4 /
 // quant_mxfp8e5 calls, operand packaging).
-#include "quantize_kernel.h"
+#include "seq_mean_kernel.h"
 #include "v_tiles_kernel.h"
 
 namespace {
@@ -16,10 +16,43 @@ struct PrepArgs {
     uint32_t bq, bk, bv;          // workgroups per (batch, head) of each job
     uint32_t hq, hkv;
     uint32_t q_total, k_total, v_total;    // blocks of the Q job, of the K job, of the V job
+    const float* sums;            // [B,Hkv,nchunk,D]: sums of chunks of K's rows (MEAN_SUMS)
+    int nchunk;
+    float inv_n;
 };
 
-template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D>
-__device__ __forceinline__ void prepare_block(const PrepArgs& p, uint32_t blk) {
+// The mean over the sequence of one head of K, in the inputs' type, into LDS: from the chunks' sums, or from the rows
+// themselves (256 / D chunks at most, all asked for at once).  The additions of mpsa_seq_mean in their order, so its bits.
+template <int XDT, int SOURCE, int D>
+__device__ __forceinline__ void head_mean(const PrepArgs& p, uint32_t hh, uint32_t bb, uint16_t* mean) {
+    const int c = threadIdx.x;
+    float s = 0.0f;
+    if constexpr (SOURCE == MEAN_SUMS) {
+        if (c < D) s = seq_sum(p.sums + ((int64_t)bb * p.hkv + hh) * p.nchunk * D + c, p.nchunk, D);
+    } else {
+        constexpr int CHUNKS = 256 / D;
+        __shared__ float part[CHUNKS][256][9], sums[256];
+        const char* head = static_cast<const char*>(p.k.x) + 2 * ((int64_t)bb * p.k.sb + (int64_t)hh * p.k.sh);
+        MeanChunk<D> chunk[CHUNKS];
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k)
+            if (k < p.nchunk) chunk[k].request(head, p.k.sn, k * MEAN_ROWS, p.k.n);
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k)
+            if (k < p.nchunk) chunk[k].template add<XDT>(part[k], k * MEAN_ROWS, p.k.n);
+        __syncthreads();
+        if (c / D < p.nchunk) sums[c] = MeanChunk<D>::total(part[c / D], c % D);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < CHUNKS; ++k)
+            if (k < p.nchunk) s += sums[k * D + c % D];
+    }
+    if (c < D) mean[c] = mean_bits<XDT>(s * p.inv_n);
+    __syncthreads();
+}
+
+template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D, int SOURCE>
+__device__ __forceinline__ void prepare_block(const PrepArgs& p, uint32_t blk, bool again) {
     if (blk < p.q_total) {
         const uint32_t head = blk / p.bq;
         quantize_block<XDT, DO4, DO8, FMT8, false>(p.q, blk - head * p.bq, head % p.hq, head / p.hq, p.hq);
@@ -28,7 +61,20 @@ __device__ __forceinline__ void prepare_block(const PrepArgs& p, uint32_t blk) {
     blk -= p.q_total;
     if (blk < p.k_total) {
         const uint32_t head = blk / p.bk;
-        quantize_block<XDT, DO4, DO8, FMT8, false>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv);
+        if constexpr (SOURCE == MEAN_SUMS || SOURCE == MEAN_ROWS_ITSELF) {
+            __shared__ __attribute__((aligned(16))) uint16_t mean[D];
+            // (the second block of a workgroup is mostly of the first one's head)
+            if (!again || blk % p.bk == 0) {
+                if (again) __syncthreads();      // the other head's mean has been read
+                head_mean<XDT, SOURCE, D>(p, head % p.hkv, head / p.hkv, mean);
+            }
+            quantize_block_less<XDT, DO4, DO8, FMT8, false>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv,
+                                                            [&](int64_t, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
+                less_mean<XDT>(x, *reinterpret_cast<const uint4*>(mean + 8 * col8));
+            });
+        } else {
+            quantize_block<XDT, DO4, DO8, FMT8, false>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv);
+        }
         return;
     }
     blk -= p.k_total;
@@ -38,39 +84,61 @@ __device__ __forceinline__ void prepare_block(const PrepArgs& p, uint32_t blk) {
 }
 
 // two blocks of work per workgroup (measured on the stand-alone quantizer: 8-13 % more bandwidth than one)
-template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D>
+template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D, int SOURCE>
 __global__ __launch_bounds__(256) void prepare_kernel(PrepArgs p) {
-    prepare_block<XDT, DO4, DO8, FMT8, TILE, D>(p, 2 * blockIdx.x);
-    prepare_block<XDT, DO4, DO8, FMT8, TILE, D>(p, 2 * blockIdx.x + 1);
+    prepare_block<XDT, DO4, DO8, FMT8, TILE, D, SOURCE>(p, 2 * blockIdx.x, false);
+    prepare_block<XDT, DO4, DO8, FMT8, TILE, D, SOURCE>(p, 2 * blockIdx.x + 1, true);
+}
+
+template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D>
+void launch_source(const PrepArgs& p, MeanSource source, unsigned grid, hipStream_t st) {
+    if (source == MEAN_SUMS)             hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_SUMS>), dim3(grid), dim3(256), 0, st, p);
+    else if (source == MEAN_ROWS_ITSELF) hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_ROWS_ITSELF>), dim3(grid), dim3(256), 0, st, p);
+    else                                 hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_GIVEN>), dim3(grid), dim3(256), 0, st, p);
 }
 
 template <int XDT, bool DO4, bool DO8, int FMT8>
-void launch_td(const PrepArgs& p, int tile, int d, unsigned grid, hipStream_t st) {
-    if (tile == 128 && d == 128)      hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, 128, 128>), dim3(grid), dim3(256), 0, st, p);
-    else if (tile == 128 && d == 64)  hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, 128, 64>), dim3(grid), dim3(256), 0, st, p);
-    else if (tile == 64 && d == 128)  hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, 64, 128>), dim3(grid), dim3(256), 0, st, p);
-    else                              hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, 64, 64>), dim3(grid), dim3(256), 0, st, p);
+void launch_td(const PrepArgs& p, int tile, int d, MeanSource source, unsigned grid, hipStream_t st) {
+    if (tile == 128 && d == 128)      launch_source<XDT, DO4, DO8, FMT8, 128, 128>(p, source, grid, st);
+    else if (tile == 128 && d == 64)  launch_source<XDT, DO4, DO8, FMT8, 128, 64>(p, source, grid, st);
+    else if (tile == 64 && d == 128)  launch_source<XDT, DO4, DO8, FMT8, 64, 128>(p, source, grid, st);
+    else                              launch_source<XDT, DO4, DO8, FMT8, 64, 64>(p, source, grid, st);
 }
 
 template <int XDT>
-void launch_mode(const PrepArgs& p, bool do4, bool do8, int fmt8, int tile, int d, unsigned grid, hipStream_t st) {
-    if (!do8) launch_td<XDT, true, false, MPSA_FMT_E4M3>(p, tile, d, grid, st);
+void launch_mode(const PrepArgs& p, bool do4, bool do8, int fmt8, int tile, int d, MeanSource source, unsigned grid, hipStream_t st) {
+    if (!do8) launch_td<XDT, true, false, MPSA_FMT_E4M3>(p, tile, d, source, grid, st);
     else if (!do4) {
-        if (fmt8 == MPSA_FMT_E5M2) launch_td<XDT, false, true, MPSA_FMT_E5M2>(p, tile, d, grid, st);
-        else                       launch_td<XDT, false, true, MPSA_FMT_E4M3>(p, tile, d, grid, st);
+        if (fmt8 == MPSA_FMT_E5M2) launch_td<XDT, false, true, MPSA_FMT_E5M2>(p, tile, d, source, grid, st);
+        else                       launch_td<XDT, false, true, MPSA_FMT_E4M3>(p, tile, d, source, grid, st);
     } else {
-        if (fmt8 == MPSA_FMT_E5M2) launch_td<XDT, true, true, MPSA_FMT_E5M2>(p, tile, d, grid, st);
-        else                       launch_td<XDT, true, true, MPSA_FMT_E4M3>(p, tile, d, grid, st);
+        if (fmt8 == MPSA_FMT_E5M2) launch_td<XDT, true, true, MPSA_FMT_E5M2>(p, tile, d, source, grid, st);
+        else                       launch_td<XDT, true, true, MPSA_FMT_E4M3>(p, tile, d, source, grid, st);
     }
 }
 
 }  // namespace
 
+// Where the mean over K's sequence comes from.  On its own it takes two launches (sums of chunks of 256 rows; their sum), each
+// of which costs the host as much as the preparation does and the device a round trip to memory.  The preparation's workgroups
+// can add up the chunks' sums themselves, or, where a head is at most 128 KiB, its rows: every workgroup reads the whole head,
+// 512 of whose 16-byte pieces it quantizes, which pays until all of them together read some two million pieces.  Microseconds
+// of a call's kernels with the mean on its own, from sums, from rows (pieces in millions): 8 heads, 512 x 128, 16.6 15.4 12.9
+// (1.0); 8 of 1024 x 64 16.9 15.7 14.7 (1.0); 2 x 16 of 333 x 128, 4096 queries, 46.4 44.1 40.6 (1.8); 2 x 32 of 512 x 64 22.5
+// 21.0 20.8 (2.1); 4 x 32 of 512 x 64 27.4 25.2 30.0 (4.2); 2 x 24 of 512 x 128, 4096 queries, 61.4 59.7 61.3 (6.3).  Sums up to
+// 64 chunks (32 heads, 4096 x 64, 86.4 -> 84.8; 8 of 16384 x 64 249.4 -> 249.0), beyond that there is nothing to gain.
+MeanSource mpsa_mean_source(int64_t B, int64_t Hkv, int64_t nk, int64_t D) {
+    if (mpsa_quantize_sw_encoders()) return MEAN_GIVEN;      // stand-alone kernels
+    const double pieces = (double)nk * (double)D / 8.0;
+    if (pieces <= 8192.0 && (double)(B * Hkv) * pieces * pieces / 512.0 <= 2.2e6) return MEAN_ROWS_ITSELF;
+    return nk <= 64 * MEAN_ROWS ? MEAN_SUMS : MEAN_GIVEN;
+}
+
 // Host side of the preparation: which of the operand sets are made is up to the caller (do4 / do8 of either side; the
 // mixed mode multiplies 8-bit Q with 4-bit K and needs one set of each).
 int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides,
                           int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nk, int64_t D, int tile, int fmt8, float pre_scale_q,
-                          const void* k_sub, bool q_do4, bool q_do8, bool k_do4, bool k_do8, uint8_t* q4, uint8_t* qs4, uint8_t* q8, uint8_t* qs8,
+                          MeanSource mean, const void* k_sub, bool q_do4, bool q_do8, bool k_do4, bool k_do8, uint8_t* q4, uint8_t* qs4, uint8_t* q8, uint8_t* qs8,
                           uint8_t* k4, uint8_t* ks4, uint8_t* k8, uint8_t* ks8, void* v_tiles, hipStream_t st) {
     const int64_t nq_pad = (Nq + tile - 1) / tile * tile, nk_pad = (Nk + tile - 1) / tile * tile;
     constexpr int EMAX4 = 3, EMAX8 = 7;            // ours/quant_mxint8.py:303, :191
@@ -97,7 +165,7 @@ int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k
         p.q = QuantArgs{};                       // no Q job: the attention kernel quantizes Q itself (mpsa_attn_fwd_q16)
         q_do4 = q_do8 = false;
     }
-    rc = mpsa_quantize_setup(k, dtype, B, Hkv, Nk, D, k_strides, k_sub, 1.0f, k_do4, EMAX4, k_do8, fmt8, EMAX8, k4, ks4, k8, ks8, nk_pad, &p.k, &bk);
+    rc = mpsa_quantize_setup(k, dtype, B, Hkv, Nk, D, k_strides, mean == MEAN_GIVEN ? k_sub : nullptr, 1.0f, k_do4, EMAX4, k_do8, fmt8, EMAX8, k4, ks4, k8, ks8, nk_pad, &p.k, &bk);
     if (rc != MPSA_OK) return rc;
     rc = mpsa_v_tiles_setup(v, dtype, B, Hkv, Nk, D, v_strides, tile, v_tiles, &p.v, &bv);
     if (rc != MPSA_OK) return rc;
@@ -106,9 +174,12 @@ int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k
     p.bq = bq; p.bk = bk; p.bv = bv; p.hq = (uint32_t)Hq; p.hkv = (uint32_t)Hkv;
     p.q_total = (uint32_t)((int64_t)bq * Hq * B); p.k_total = (uint32_t)((int64_t)bk * Hkv * B);
     p.v_total = (uint32_t)((int64_t)bv * Hkv * B);
+    p.sums = mean == MEAN_SUMS ? static_cast<const float*>(k_sub) : nullptr;
+    p.nchunk = (int)((Nk + MEAN_ROWS - 1) / MEAN_ROWS);
+    p.inv_n = 1.0f / (float)Nk;
     const bool do4 = q_do4 || k_do4, do8 = q_do8 || k_do8;
-    if (dtype == MPSA_BF16) launch_mode<MPSA_BF16>(p, do4, do8, fmt8, tile, (int)D, (unsigned)((total + 1) / 2), st);
-    else                    launch_mode<MPSA_F16>(p, do4, do8, fmt8, tile, (int)D, (unsigned)((total + 1) / 2), st);
+    if (dtype == MPSA_BF16) launch_mode<MPSA_BF16>(p, do4, do8, fmt8, tile, (int)D, mean, (unsigned)((total + 1) / 2), st);
+    else                    launch_mode<MPSA_F16>(p, do4, do8, fmt8, tile, (int)D, mean, (unsigned)((total + 1) / 2), st);
     MPSA_CHECK_LAUNCH("prepare");
     return MPSA_OK;
 }
@@ -124,6 +195,6 @@ extern "C" int mpsa_attn_prepare(const void* q, const int64_t q_strides[4], cons
     if (tile != 64 && tile != 128) return mpsa_fail(MPSA_EUNSUPPORTED, "prepare: tile must be 64 or 128 (got %d)", tile);
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || Nq <= 0 || Nk <= 0 || Hq % Hkv) return mpsa_fail(MPSA_EINVAL, "prepare: bad shape (B=%lld Hq=%lld Hkv=%lld Nq=%lld Nk=%lld)", (long long)B, (long long)Hq, (long long)Hkv, (long long)Nq, (long long)Nk);
     const bool do4 = mode != MPSA_MODE_MXFP8, do8 = mode != MPSA_MODE_MXFP4;
-    return mpsa_prepare_operands(q, q_strides, k, k_strides, v, v_strides, dtype, B, Hq, Hkv, Nq, Nk, D, tile, fmt8, pre_scale_q, k_sub,
+    return mpsa_prepare_operands(q, q_strides, k, k_strides, v, v_strides, dtype, B, Hq, Hkv, Nq, Nk, D, tile, fmt8, pre_scale_q, k_sub ? MEAN_GIVEN : MEAN_NONE, k_sub,
                                  do4, do8, do4, do8, q4, qs4, q8, qs8, k4, ks4, k8, ks8, v_tiles, (hipStream_t)stream);
 }

@@ -15,15 +15,13 @@
 // Work mapping: one lane owns 8 consecutive elements (one 128-bit load), four neighbouring lanes
 // own one MX block, so the block maximum is two DPP quad exchanges.  The kernel is HBM-bound:
 // 2 B/element in, 0.5 (+1) B/element of codes and 1/32 (x2) B/element of scales out.
-#include "quantize_kernel.h"
+#include "seq_mean_kernel.h"
 #include <cstring>
 #include <mutex>
 
 namespace {
 
 // ---- mean over the sequence, per (batch, head, channel) ----
-constexpr int MEAN_ROWS = 256;     // rows per partial sum
-
 struct MeanArgs {
     const void* x;
     int64_t sb, sh, sn;
@@ -33,61 +31,18 @@ struct MeanArgs {
     float inv_n;
 };
 
-// partial sums x[0], x[stride], ... added in order; a batch of them is requested before its first is added (one at a time,
-// 128 of them took 31 us)
-__device__ __forceinline__ float seq_sum(const float* x, int count, int stride) {
-    constexpr int BATCH = 32;
-    float s = 0.0f;
-    for (int k = 0; k < count; k += BATCH) {
-        float v[BATCH];
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i) v[i] = x[(int64_t)min(k + i, count - 1) * stride];
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i)
-            if (k + i < count) s += v[i];
-    }
-    return s;
-}
-
-// One workgroup sums MEAN_ROWS rows of one head: a thread owns 8 channels of every (256*8/D)-th row; the row
-// groups are then added in a fixed order through LDS, so the result does not depend on timing.  A thread's rows are
-// requested before the first is added: with one load in flight a short sequence took a memory round trip per row
-// (2 x 16 heads, 333 rows: 8.3 us, this way 7.5).
+// one workgroup sums MEAN_ROWS rows of one head
 template <int XDT, int D>
 __global__ __launch_bounds__(256) void seq_mean_kernel(MeanArgs a) {
     __shared__ float part[256][9];
-    constexpr int cpr = D >> 3;                  // 8-channel groups per row (8 or 16)
-    constexpr int rthreads = 256 / cpr, each = MEAN_ROWS / rthreads;
-    const int cg = threadIdx.x % cpr, rt = threadIdx.x / cpr;
-    const int chunk = blockIdx.x;
-    const int row0 = chunk * MEAN_ROWS;
-    const int row1 = min(row0 + MEAN_ROWS, a.n);
-    const char* base = static_cast<const char*>(a.x) + 2 * ((int64_t)blockIdx.z * a.sb + (int64_t)blockIdx.y * a.sh + 8 * (int64_t)cg);
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint4 raw[each];
-#pragma unroll
-    for (int i = 0; i < each; ++i) {
-        const int row = min(row0 + rt + i * rthreads, a.n - 1);
-        raw[i] = *reinterpret_cast<const uint4*>(base + 2 * (int64_t)row * a.sn);
-    }
-#pragma unroll
-    for (int i = 0; i < each; ++i) {
-        if (row0 + rt + i * rthreads >= row1) break;
-        float x[8];
-        unpack8<XDT>(raw[i], x);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) acc[q] += x[q];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) part[threadIdx.x][i] = acc[i];
+    const int row0 = (int)blockIdx.x * MEAN_ROWS;
+    MeanChunk<D> chunk;
+    chunk.request(static_cast<const char*>(a.x) + 2 * ((int64_t)blockIdx.z * a.sb + (int64_t)blockIdx.y * a.sh), a.sn, row0, a.n);
+    chunk.template add<XDT>(part, row0, a.n);
     __syncthreads();
     if (threadIdx.x < D) {
-        const int c = threadIdx.x;               // channel
-        float s = 0.0f;
-#pragma unroll
-        for (int t = 0; t < rthreads; ++t) s += part[t * cpr + (c >> 3)][c & 7];
         const int64_t head = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
-        a.partial[(head * a.nchunk + chunk) * D + c] = s;
+        a.partial[(head * a.nchunk + blockIdx.x) * D + threadIdx.x] = MeanChunk<D>::total(part, threadIdx.x);
     }
 }
 
@@ -98,12 +53,7 @@ __global__ __launch_bounds__(128) void seq_mean_finish_kernel(MeanArgs a) {
     if (c >= a.d) return;
     const int64_t head = blockIdx.x;
     const float m = seq_sum(a.partial + head * a.nchunk * a.d + c, a.nchunk, a.d) * a.inv_n;
-    if constexpr (XDT == MPSA_BF16) {
-        const uint32_t u = mpsa_f2u(m);
-        static_cast<uint16_t*>(a.mean)[head * a.d + c] = (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-    } else {
-        static_cast<_Float16*>(a.mean)[head * a.d + c] = (_Float16)m;
-    }
+    static_cast<uint16_t*>(a.mean)[head * a.d + c] = mean_bits<XDT>(m);
 }
 
 // MPSA_FP8_ENCODE=sw or MPSA_FP4_ENCODE=sw in the environment selects the kernels that encode with explicit
@@ -224,9 +174,10 @@ extern "C" int64_t mpsa_seq_mean_workspace(int64_t B, int64_t H, int64_t N, int6
 
 namespace {
 
+// mean == nullptr: the partial sums only
 int seq_mean_common(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,
                     const int64_t x_strides[4], float* workspace, void* mean, hipStream_t st) {
-    if (!x || !x_strides || !workspace || !mean) return mpsa_fail(MPSA_EINVAL, "seq_mean: null pointer");
+    if (!x || !x_strides || !workspace) return mpsa_fail(MPSA_EINVAL, "seq_mean: null pointer");
     if (x_dtype != MPSA_BF16 && x_dtype != MPSA_F16) return mpsa_fail(MPSA_EINVAL, "seq_mean: x_dtype must be bf16 or f16");
     if (B <= 0 || H <= 0 || N <= 0) return mpsa_fail(MPSA_EINVAL, "seq_mean: bad shape");
     if (D != 64 && D != 128) return mpsa_fail(MPSA_EUNSUPPORTED, "seq_mean: D must be 64 or 128 (got %lld)", (long long)D);
@@ -242,11 +193,11 @@ int seq_mean_common(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N,
     if (x_dtype == MPSA_BF16) {
         if (d128) hipLaunchKernelGGL((seq_mean_kernel<MPSA_BF16, 128>), grid, dim3(256), 0, st, a);
         else      hipLaunchKernelGGL((seq_mean_kernel<MPSA_BF16, 64>), grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(seq_mean_finish_kernel<MPSA_BF16>, dim3((unsigned)(B * H)), dim3(128), 0, st, a);
+        if (mean) hipLaunchKernelGGL(seq_mean_finish_kernel<MPSA_BF16>, dim3((unsigned)(B * H)), dim3(128), 0, st, a);
     } else {
         if (d128) hipLaunchKernelGGL((seq_mean_kernel<MPSA_F16, 128>), grid, dim3(256), 0, st, a);
         else      hipLaunchKernelGGL((seq_mean_kernel<MPSA_F16, 64>), grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(seq_mean_finish_kernel<MPSA_F16>, dim3((unsigned)(B * H)), dim3(128), 0, st, a);
+        if (mean) hipLaunchKernelGGL(seq_mean_finish_kernel<MPSA_F16>, dim3((unsigned)(B * H)), dim3(128), 0, st, a);
     }
     MPSA_CHECK_LAUNCH("seq_mean");
     return MPSA_OK;
@@ -254,8 +205,13 @@ int seq_mean_common(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N,
 
 }  // namespace
 
+int mpsa_seq_mean_partial(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D, const int64_t x_strides[4], float* workspace, hipStream_t st) {
+    return seq_mean_common(x, x_dtype, B, H, N, D, x_strides, workspace, nullptr, st);
+}
+
 extern "C" int mpsa_seq_mean(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,
                              const int64_t x_strides[4], float* workspace, void* mean, mpsa_stream_t stream) {
+    if (!mean) return mpsa_fail(MPSA_EINVAL, "seq_mean: null pointer");
     return seq_mean_common(x, x_dtype, B, H, N, D, x_strides, workspace, mean, (hipStream_t)stream);
 }
 
@@ -294,6 +250,7 @@ int mpsa_seq_mean_static_resolve() {
 
 extern "C" int mpsa_seq_mean_static(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,
                                     const int64_t x_strides[4], void* mean, mpsa_stream_t stream) {
+    if (!mean) return mpsa_fail(MPSA_EINVAL, "seq_mean: null pointer");
     const int64_t need = mpsa_seq_mean_workspace(B, H, N, D);
     if (need > (int64_t)MPSA_SEQ_MEAN_STATIC_BYTES)
         return mpsa_fail(MPSA_EUNSUPPORTED, "seq_mean_static: B*H*ceil(N/256)*D*4 = %lld bytes of partial sums exceed the built-in %lld; use mpsa_seq_mean with a workspace",

@@ -199,8 +199,9 @@ __device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool ex
 }
 
 // One workgroup's share: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb (nh heads).
-template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8>
-__device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh) {
+// subtract(head, col8, x): what is taken off a row's chunk before anything else.
+template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8, typename Subtract>
+__device__ __forceinline__ void quantize_block_less(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh, Subtract subtract) {
     const uint32_t cpr = (uint32_t)a.d >> 3;                              // 16-byte chunks per row
     const uint32_t chunks = (uint32_t)a.out_rows * cpr;                   // per (b,h)
     const uint32_t c = bx * 256u + threadIdx.x;
@@ -214,12 +215,7 @@ __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, 
         const char* base = static_cast<const char*>(a.x) +
                            2 * ((int64_t)bb * a.sb + (int64_t)hh * a.sh + (int64_t)row * a.sn + 8 * (int64_t)col8);
         load8<XDT>(base, x);
-        if (a.sub) {
-            float m[8];
-            load8<XDT>(static_cast<const char*>(a.sub) + 2 * (head * a.d + 8 * (int64_t)col8), m);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] = round16<XDT>(x[i] - m[i]);
-        }
+        subtract(head, col8, x);
     } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = 0.0f;
@@ -245,6 +241,22 @@ __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, 
         reinterpret_cast<uint2*>(a.codes8)[oc] = w8;
         if (quad_leader) a.scales8[os] = (uint8_t)s8;
     }
+}
+
+// x - m in the inputs' 16-bit type
+template <int XDT>
+__device__ __forceinline__ void less_mean(float (&x)[8], const uint4& mean) {
+    float m[8];
+    unpack8<XDT>(mean, m);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = round16<XDT>(x[i] - m[i]);
+}
+
+template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8>
+__device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh) {
+    quantize_block_less<XDT, DO4, DO8, FMT8, SW8>(a, bx, hh, bb, nh, [&](int64_t head, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
+        if (a.sub) less_mean<XDT>(x, *reinterpret_cast<const uint4*>(static_cast<const char*>(a.sub) + 2 * (head * a.d + 8 * (int64_t)col8)));
+    });
 }
 
 template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8>

@@ -970,3 +970,23 @@ def test_skipping_and_lists_take_no_other_kernel():
         attention_from_operands(ops, out, False, route=route_tiles(ops, False, 0.9), kernel="paired")
     with pytest.raises(_lib.MpsaError, match="quantized q only"):
         attention_from_operands(prepare_operands(q, k, v, 128, "mxfp4", fuse_q=True), out, False, kernel="general")
+
+
+@pytest.mark.parametrize("layout", ["HND", "NHD"])
+@pytest.mark.parametrize("B,Hkv,N,D", [(1, 1, 1, 64), (1, 3, 31, 128), (2, 3, 255, 64), (1, 3, 256, 128), (1, 3, 257, 128), (1, 1, 512, 128), (1, 1, 513, 128),
+                                       (1, 3, 1000, 64), (1, 1, 1024, 64), (1, 1, 1025, 64), (2, 5, 333, 128), (4, 32, 511, 64), (1, 3, 2300, 128), (1, 1, 16384, 64),
+                                       (1, 1, 16385, 64)])
+@pytest.mark.parametrize("mode,dtype", [("mxfp8", torch.float16), ("diag", torch.bfloat16)])
+def test_mean_inside_the_preparation_gives_the_bits_of_the_mean_on_its_own(B, Hkv, N, D, layout, mode, dtype):
+    """A call takes the mean of K inside its preparation -- from K's rows or from sums of 256 of them, by size -- where the
+    stages one by one take it first: the same bits, for workgroups that cover two heads as well."""
+    from ours.mxfp_attn_kernel import attention_from_operands, mxfp_attn_kernel, prepare_operands
+    g = torch.Generator().manual_seed(N + D)
+    shape = (B, Hkv, N, D) if layout == "HND" else (B, N, Hkv, D)
+    q, k, v = ((torch.randn(*shape, generator=g) + off).to(dtype).to("cuda:0") for off in (0.0, 3.0, 0.0))
+    got = mxfp_attn_kernel(q, k, v, smooth_k=True, tensor_layout=layout, output_dtype=dtype, block_scale_type=mode, tile=64, kernel="short1")
+    bhnd = (lambda t: t) if layout == "HND" else (lambda t: t.transpose(1, 2))
+    ops = prepare_operands(bhnd(q), bhnd(k), bhnd(v), 64, mode, smooth_k=True)
+    want = torch.empty_like(got)
+    attention_from_operands(ops, bhnd(want), False, kernel="short1")
+    assert torch.equal(got, want)
