@@ -158,13 +158,18 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
         const char* row = static_cast<const char*>(a.q_raw) +
                           2 * ((int64_t)b * a.q_sb + (int64_t)hq * a.q_sh + row_idx * a.q_sn);
         uint32_t sbytes = 0, sbytes8 = 0;
+        uint4 raw[SST][4];
+#pragma unroll
+        for (int s = 0; s < SST; ++s)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) raw[s][c] = *reinterpret_cast<const uint4*>(row + 2 * (32 * (2 * s + h) + 8 * c));
 #pragma unroll
         for (int s = 0; s < SST; ++s) {
             float x[4][8];
             float amax = 0.0f;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                load8<PVT>(row + 2 * (32 * (2 * s + h) + 8 * c), x[c]);
+                unpack8<PVT>(raw[s][c], x[c]);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     x[c][e] = x[c][e] * a.q_pre;
@@ -173,31 +178,45 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
             }
             const bool zero = mpsa_f2u(amax) == 0u;
             const int ex = block_exponent(amax);
+            const int se = ex - 3, se8 = ex - 7;             // emax of E2M1: ours/quant_mxint8.py:303; of the 8-bit formats: :191
+            int w[4];
+            int w8[8];
+            bool rule[4], odd = false, again = false;        // chunks, and the block, that the conversions may not be right for
             if constexpr (WANT4) {
-                const int se = ex - 3;                                         // emax of E2M1: ours/quant_mxint8.py:303
-                int w[4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    w[c] = (int)e2m1_pack8<true>(x[c], se, false);
-                    w[c] = zero ? 0 : w[c];
+                    w[c] = (int)e2m1_try8(x[c], se, false, rule[c]);
+                    again |= rule[c];
                 }
-                qf[s] = (v8i){w[0], w[1], w[2], w[3], 0, 0, 0, 0};
+            }
+            if constexpr (WANT8) {
+                odd = fp8_odd(ex, se8);
+                again |= odd;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const uint2 y = fp8_convert8<FMT8>(x[c], se8);
+                    w8[2 * c] = (int)y.x;
+                    w8[2 * c + 1] = (int)y.y;
+                }
+            }
+            if (again && !zero) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if (WANT4 && rule[c]) w[c] = (int)e2m1_pack8_rule(x[c], se);
+                    if (WANT8 && odd) {
+                        const uint2 y = fp8_careful8<FMT8, false>(x[c], se8);
+                        w8[2 * c] = (int)y.x;
+                        w8[2 * c + 1] = (int)y.y;
+                    }
+                }
+            }
+            if constexpr (WANT4) {
+                qf[s] = (v8i){zero ? 0 : w[0], zero ? 0 : w[1], zero ? 0 : w[2], zero ? 0 : w[3], 0, 0, 0, 0};
                 sbytes |= (uint32_t)(zero ? 0 : min(max(se + 127, 0), 254)) << (16 * s);
             }
             if constexpr (WANT8) {
-                const int se8 = ex - 7;                                        // emax of the 8-bit formats: ours/quant_mxint8.py:191
-                // the quantizer's clamp to the format's maximum (quantize_kernel.h): finite blocks scale into
-                // [128, 256) and never meet it, a block with an infinity saturates there instead of giving NaN codes
-                const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
-                int w8[8];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    float y[8];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) y[e] = __builtin_fminf(__builtin_fmaxf(ldexpf(x[c][e], -se8), -lim), lim);
-                    w8[2 * c] = zero ? 0 : (int)fp8_pack4<FMT8, false>(y[0], y[1], y[2], y[3]);
-                    w8[2 * c + 1] = zero ? 0 : (int)fp8_pack4<FMT8, false>(y[4], y[5], y[6], y[7]);
-                }
+                for (int c = 0; c < 8; ++c) w8[c] = zero ? 0 : w8[c];
                 // w8[0..3] = bytes 0-15, w8[4..7] = bytes 16-31 of block 2s + h.  Lane half 0 keeps its low half in
                 // registers 0-3 and takes block 2s + 1's low half from its partner into 4-7; lane half 1 keeps its high
                 // half in 4-7 and takes block 2s's high half into 0-3: swap (lanes 32-63 of register i) with (lanes 0-31 of

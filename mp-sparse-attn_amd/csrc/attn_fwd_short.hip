@@ -169,19 +169,19 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 3) void attn_short_kernel(Short
             float x[BATCH][8];
             uint32_t w4[BATCH];
             uint2 w8[BATCH];
-            int s4[BATCH], s8[BATCH], se[BATCH];
-            bool rule[BATCH], any = false;
+            int s4[BATCH], s8[BATCH], e[BATCH];
+            bool again[BATCH], any = false;
 #pragma unroll
             for (int q = 0; q < BATCH; ++q) {
                 const int c = (q0 + q) * 256 + tid;
                 unpack8<PVT>(G::QR * p + c / (D / 8) < a.nq ? raw[q0 + q] : make_uint4(0, 0, 0, 0), x[q]);
-                quantize_most<Q4, Q8, FMT8, false>(x[q], a.q_pre, false, 3, 7, w4[q], s4[q], w8[q], s8[q], rule[q], se[q]);
-                any |= rule[q];
+                quantize_most<Q4, Q8, FMT8, false>(x[q], a.q_pre, false, 3, 7, w4[q], s4[q], w8[q], s8[q], again[q], e[q]);
+                any |= again[q];
             }
-            if (Q4 && any) {
+            if (any) {
 #pragma unroll
                 for (int q = 0; q < BATCH; ++q)
-                    if (rule[q]) w4[q] = e2m1_pack8_rule(x[q], se[q]);
+                    if (again[q]) quantize_again<Q4, Q8, FMT8, false>(x[q], e[q], 3, 7, false, w4[q], w8[q]);
             }
 #pragma unroll
             for (int q = 0; q < BATCH; ++q) put_q((q0 + q) * 256 + tid, w4[q], s4[q], w8[q], s8[q]);

@@ -86,18 +86,36 @@ __device__ __forceinline__ float round16(float v) {
 // Eight E2M1 codes (one packed word, element i in nibble i) of x[0..7] / 2^se.
 // Fast path: v_cvt_scalef32_pk_fp4_f32 divides by the power of two and rounds to nearest, ties to even.  The
 // reference's rule (argmin of float32 distances with 1e-6 taken off the even-mantissa candidate, e2m1_index in
-// mx_codec.h) differs from that only for a value within about 1e-6 of the midpoint between two E2M1 values.  Such
-// a value is found by converting the inputs nudged down and up by 2^-17 of themselves: if the two conversions
-// agree, no rounding boundary lies between them and that word is the result; if they differ anywhere in the word,
-// the lane falls back to the explicit rule.  (2^-17 of a value near a midpoint - the
-// smallest is 0.25 - is at least 1.9e-6.)  Scales too small for a normal float32 take the explicit rule as well.
+// mx_codec.h) differs from that only for a value within about 1e-6 of the midpoint between two E2M1 values.
+// The midpoints (0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5) have nothing but zeros below their first two mantissa bits, and dividing
+// by a power of two leaves the mantissa alone: a value close to one shows in the low 21 bits of x itself.  A value whose bits
+// are 128 units or more away from such a pattern is at least 1.9e-6 away from every midpoint (the smallest, 0.25, from below:
+// 128 * 2^-26), and the conversion is the result.  That is one shift-and-add an element and half a minimum; converting
+// the inputs twice, nudged down and up by 2^-17 of themselves, which this replaces, took two products and half a conversion.
+// With the scaled FP8 conversion below (a shift and a clamp an element less) and, in the paired-tile kernel, all of a lane's
+// loads in front: 32/8 heads, 8192 tokens, diag, 336.7 -> 334.5 us a call (kernels alone 359 -> 352); 8 heads of 1024 x 64
+// 15.3 -> 15.1; 2 x 24 heads, 8000 queries over 200 keys 68.4 -> 66.9.
+// The pattern is that of the E2M1 values and of zero as well; so a lane that finds it converts the nudged inputs, and if
+// they differ (a rounding boundary lies between) it takes the explicit rule.  (2^-17 of a value near a midpoint - the
+// smallest is 0.25 - is at least 1.9e-6.)  Small scales, where x may be subnormal, take the explicit rule as well.
 // When the pre-scale is a power of two the scaled values are 16-bit inputs times a power of two, at most 11
 // significant bits: such a value is either exactly a midpoint - where the two rules agree (both take the even
 // mantissa) - or at least 2^-12 away from one, so the check is skipped (`exact16`); it would otherwise fire on every
 // exact tie, which 16-bit data hits all the time.
-// The explicit rule is rolled up (a hundred instructions, not seven hundred) and stands behind ONE branch instead of early
-// returns and conditional blocks for every word.
-__device__ __forceinline__ uint32_t e2m1_pack8_rule(const float (&x)[8], int se) {
+constexpr int SMALLEST_SE = -100;      // x below 2^-126 is less than 2^-26 of a unit then: it rounds to zero in every format
+
+__device__ __forceinline__ uint32_t e2m1_convert8(const float (&x)[8], int se, float f) {
+    const float sc = mpsa_u2f((uint32_t)(se + 127) << 23);
+    uint32_t w = 0;
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[0] * f, x[1] * f, sc, 0);
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[2] * f, x[3] * f, sc, 1);
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[4] * f, x[5] * f, sc, 2);
+    return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[6] * f, x[7] * f, sc, 3);
+}
+
+// What a lane does whose conversion may not be the rule's result.  The explicit rule is rolled up (a hundred instructions, not
+// seven hundred) and stands behind ONE branch instead of early returns and conditional blocks for every word.
+__device__ __forceinline__ uint32_t e2m1_pack8_explicit(const float (&x)[8], int se) {
     float y[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) y[i] = x[i];
@@ -111,32 +129,67 @@ __device__ __forceinline__ uint32_t e2m1_pack8_rule(const float (&x)[8], int se)
     return word;
 }
 
-// the conversion, and whether the rule has to decide instead
-__device__ __forceinline__ uint32_t e2m1_try8(const float (&x)[8], int se, bool exact16, bool& rule) {
-    const float sc = mpsa_u2f((uint32_t)(se + 127) << 23);
-    auto convert = [&](float f) __attribute__((always_inline)) {
-        uint32_t w = 0;
-        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[0] * f, x[1] * f, sc, 0);
-        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[2] * f, x[3] * f, sc, 1);
-        w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[4] * f, x[5] * f, sc, 2);
-        return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, x[6] * f, x[7] * f, sc, 3);
-    };
-    rule = se < -126;
-    if (exact16) return convert(1.0f);
+__device__ __forceinline__ uint32_t e2m1_pack8_rule(const float (&x)[8], int se) {
     // no boundary between the two nudged values: the value itself converts to the same codes
-    const uint32_t w = convert(1.0f - 0x1p-17f);
-    rule |= w != convert(1.0f + 0x1p-17f);
-    return w;
+    const uint32_t w = e2m1_convert8(x, se, 1.0f - 0x1p-17f);
+    if (se >= SMALLEST_SE && w == e2m1_convert8(x, se, 1.0f + 0x1p-17f)) return w;
+    return e2m1_pack8_explicit(x, se);
+}
+
+// the conversion, and whether e2m1_pack8_rule has to look at it instead
+__device__ __forceinline__ uint32_t e2m1_try8(const float (&x)[8], int se, bool exact16, bool& rule) {
+    rule = se < SMALLEST_SE;
+    if (!exact16) {
+        uint32_t nearest = ~0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) nearest = min(nearest, (mpsa_f2u(x[i]) << 11) + (128u << 11));
+        rule |= nearest < (256u << 11);
+    }
+    return e2m1_convert8(x, se, 1.0f);
 }
 
 template <bool HW4>
 __device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool exact16) {
-    if constexpr (!HW4) return e2m1_pack8_rule(x, se);
+    if constexpr (!HW4) return e2m1_pack8_explicit(x, se);
     bool rule;
     uint32_t w = e2m1_try8(x, se, exact16, rule);
     if (rule) w = e2m1_pack8_rule(x, se);
     return w;
 }
+
+// Eight FP8 codes of x[0..7] / 2^se.  The scaled conversion divides and rounds in one instruction a pair; a finite block's
+// values lie below 256 then and never meet the format's maximum.
+template <int FMT8>
+__device__ __forceinline__ uint2 fp8_convert8(const float (&x)[8], int se) {
+    typedef short v2s __attribute__((ext_vector_type(2)));
+    const float sc = mpsa_u2f((uint32_t)(se + 127) << 23);
+    v2s lo = {0, 0}, hi = {0, 0};
+    if constexpr (FMT8 == MPSA_FMT_E4M3) {
+        lo = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(lo, x[0], x[1], sc, false);
+        lo = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(lo, x[2], x[3], sc, true);
+        hi = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(hi, x[4], x[5], sc, false);
+        hi = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(hi, x[6], x[7], sc, true);
+    } else {
+        lo = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(lo, x[0], x[1], sc, false);
+        lo = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(lo, x[2], x[3], sc, true);
+        hi = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(hi, x[4], x[5], sc, false);
+        hi = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(hi, x[6], x[7], sc, true);
+    }
+    return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+}
+
+// the same one step at a time, with the clamp to the format's maximum: a block with an infinity saturates there
+template <int FMT8, bool SW8>
+__device__ __forceinline__ uint2 fp8_careful8(const float (&x)[8], int se) {
+    const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = __builtin_fminf(__builtin_fmaxf(ldexpf(x[i], -se), -lim), lim);
+    return make_uint2(fp8_pack4<FMT8, SW8>(y[0], y[1], y[2], y[3]), fp8_pack4<FMT8, SW8>(y[4], y[5], y[6], y[7]));
+}
+
+// whether a block of largest magnitude 2^e or more wants fp8_careful8
+__device__ __forceinline__ bool fp8_odd(int e, int se) { return e >= 128 || se < SMALLEST_SE; }
 
 // floor(log2(amax)) of a block's largest magnitude, subnormals included; -1 for a block of zeros (whose codes and scale are
 // zero whatever it says)
@@ -146,10 +199,10 @@ __device__ __forceinline__ int block_exponent(float amax) {
 }
 
 // One lane's eight elements (a quarter of an MX block; the quad's other lanes hold the rest): codes and the block's scale
-// bytes in the formats asked for.  x comes back multiplied by `pre`.  Where `rule` comes back true, the caller replaces w4 by
-// e2m1_pack8_rule(x, s): several chunks in a row share one branch that way, and run interleaved.
+// bytes in the formats asked for.  x comes back multiplied by `pre`, e is the block's exponent.  Where `again` comes back
+// true, the caller has quantize_again finish the chunk: several chunks in a row share one branch that way, and run interleaved.
 template <bool DO4, bool DO8, int FMT8, bool SW8>
-__device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8, bool& rule, int& se4) {
+__device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8, bool& again, int& e) {
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -161,41 +214,49 @@ __device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exa
     ab = max(ab, dpp_u32<0xB1>(ab));                      // quad_perm [1,0,3,2]
     ab = max(ab, dpp_u32<0x4E>(ab));                      // quad_perm [2,3,0,1]
     const bool zero = ab == 0u;
-    const int e = block_exponent(mpsa_u2f(ab));
+    e = block_exponent(mpsa_u2f(ab));
     w4 = 0u; s4 = 0;
     w8 = make_uint2(0u, 0u); s8 = 0;
-    rule = false;
-    se4 = e - emax4;
+    again = SW8;
     if constexpr (DO4) {
-        if constexpr (SW8) {
-            rule = !zero;
-        } else {
-            w4 = e2m1_try8(x, se4, exact16, rule);
-            rule &= !zero;
+        const int se = e - emax4;
+        if constexpr (!SW8) {
+            w4 = e2m1_try8(x, se, exact16, again);
+            w4 = zero ? 0u : w4;
         }
-        w4 = zero ? 0u : w4;
-        s4 = zero ? 0 : min(max(se4 + 127, 0), 254);
+        s4 = zero ? 0 : min(max(se + 127, 0), 254);
     }
     if constexpr (DO8) {
         const int se = e - emax8;
-        const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
-        float y[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = __builtin_fminf(__builtin_fmaxf(ldexpf(x[i], -se), -lim), lim);
-        w8.x = fp8_pack4<FMT8, SW8>(y[0], y[1], y[2], y[3]);
-        w8.y = fp8_pack4<FMT8, SW8>(y[4], y[5], y[6], y[7]);
-        w8.x = zero ? 0u : w8.x;
-        w8.y = zero ? 0u : w8.y;
+        if constexpr (!SW8) {
+            w8 = fp8_convert8<FMT8>(x, se);
+            w8.x = zero ? 0u : w8.x;
+            w8.y = zero ? 0u : w8.y;
+            again |= fp8_odd(e, se);
+        }
         s8 = zero ? 0 : min(max(se + 127, 0), 254);
+    }
+    again &= !zero;
+}
+
+template <bool DO4, bool DO8, int FMT8, bool SW8>
+__device__ __forceinline__ void quantize_again(const float (&x)[8], int e, int emax4, int emax8, bool exact16, uint32_t& w4, uint2& w8) {
+    if constexpr (DO4) {
+        bool rule = true;
+        if constexpr (DO8 && !SW8) (void)e2m1_try8(x, e - emax4, exact16, rule);
+        if (rule) w4 = SW8 ? e2m1_pack8_explicit(x, e - emax4) : e2m1_pack8_rule(x, e - emax4);
+    }
+    if constexpr (DO8) {
+        if (SW8 || fp8_odd(e, e - emax8)) w8 = fp8_careful8<FMT8, SW8>(x, e - emax8);
     }
 }
 
 template <bool DO4, bool DO8, int FMT8, bool SW8>
 __device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8) {
-    bool rule;
-    int se4;
-    quantize_most<DO4, DO8, FMT8, SW8>(x, pre, exact16, emax4, emax8, w4, s4, w8, s8, rule, se4);
-    if (DO4 && rule) w4 = e2m1_pack8_rule(x, se4);
+    bool again;
+    int e;
+    quantize_most<DO4, DO8, FMT8, SW8>(x, pre, exact16, emax4, emax8, w4, s4, w8, s8, again, e);
+    if (again) quantize_again<DO4, DO8, FMT8, SW8>(x, e, emax4, emax8, exact16, w4, w8);
 }
 
 // One workgroup's share: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb (nh heads).

@@ -219,3 +219,17 @@ def test_fewer_output_rows_than_the_input_has_are_an_error(rows):
     x = torch.randn(1, 2, 100, 64, device=DEV).bfloat16()
     with pytest.raises(RuntimeError):
         quantize_mx(x, 1.0, O.FMT_E2M1, out_rows=rows)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("pre", [1.0, 0.1275174])
+def test_small_blocks_on_either_side_of_the_step_by_step_conversion(fmt, pre):
+    """Blocks whose scale is 2^-100 or less are converted step by step, the others by the scaled conversion: every exponent
+    around that line, with elements down to subnormal ones, zeros and exact ties."""
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(1, 1, 64, 64, generator=g)
+    x[..., ::7] = 0.0
+    x[..., 3::16] = torch.tensor([0.25, 0.75, 1.25, 2.5])
+    x[..., 5::16] *= 2.0 ** -24
+    x = (x * torch.exp2(torch.arange(-126, -62).float())[None, None, :, None]).bfloat16()
+    _check(x, pre, fmt)
