@@ -359,10 +359,16 @@ static int gemm_entry(int kernel, const uint8_t* a, const uint8_t* sa, int fmt_a
     g.packed = packed ? 1 : 0;
     hipStream_t st = (hipStream_t)stream;
     const int64_t batches = batch * heads_a;
+    const bool stage = kernel == MPSA_GEMM_AUTO && !force_general() && gemm_stage_takes(g, fmt_a, fmt_b, c_dtype);
     kernel = choose(kernel, g, batches, fmt_a, fmt_b);
     if (kernel < 0) return kernel;
     rc = mpsa_ensure_init();
     if (rc != MPSA_OK) return rc;
+    if (stage) {
+        gemm_stage_launch(g, batches, fmt_a, fmt_b, c_dtype, st);
+        MPSA_CHECK_LAUNCH("gemm");
+        return MPSA_OK;
+    }
     if (kernel == MPSA_GEMM_GENERAL) {
         dim3 grid((unsigned)(((M + 127) / 128) * ((N + 127) / 128)), (unsigned)batches);
         launch_general(g, fmt_a, fmt_b, c_dtype, grid, st);

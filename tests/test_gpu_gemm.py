@@ -631,3 +631,28 @@ def test_16bit_results_are_the_float32_ones_rounded_once(kernel, M, N, ldc, dtyp
 
     got, want = product(dtype), product(torch.float32).to(dtype)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("fmt_a,fmt_b", [(4, 4), (0, 0), (1, 1), (0, 4), (1, 4)])
+@pytest.mark.parametrize("batch,heads,heads_b,M,N", [(1, 1, 1, 128, 128), (1, 2, 1, 100, 130), (2, 4, 2, 1, 7), (1, 1, 1, 300, 4096), (2, 8, 4, 1024, 1024),
+                                                     (1, 4, 4, 2000, 2040), (1, 8, 2, 1408, 1536), (1, 16, 16, 1030, 1025)])
+def test_products_with_one_stage_of_k(batch, heads, heads_b, M, N, fmt_a, fmt_b):
+    """K == 128 has a kernel of its own, which walks several tiles a workgroup where there are many: the general kernel's bits,
+    whole and cut tiles, grouped heads, both scale layouts, and row pitches that it leaves to the general kernel."""
+    K, L = 128, _lib.lib()
+    packed_too = M % 128 == 0 and N % 128 == 0            # packed scales are whole chunks of 128 rows
+    g = torch.Generator().manual_seed(M * N + fmt_a)
+
+    def codes(rows, h, fmt):
+        # 8-bit codes without infinities and NaN: exponent field below the top one
+        c = torch.randint(0, 256, (batch, h, rows, K // 2 if fmt == 4 else K), generator=g, dtype=torch.uint8)
+        return (c if fmt == 4 else c & 0xBF).to(DEV)
+
+    a, b = codes(M, heads, fmt_a), codes(N, heads_b, fmt_b)
+    sa, sb = (torch.randint(118, 130, (batch, h, rows, K // 32), generator=g, dtype=torch.uint8).to(DEV) for h, rows in ((heads, M), (heads_b, N)))
+    for packed, dtype, ldc in [(p, d, l) for p in range(1 + packed_too) for d, l in ((torch.bfloat16, (N + 7) // 8 * 8), (torch.float16, N))]:
+        got, want = (torch.full((batch, heads, M, ldc), 3.0, dtype=dtype, device=DEV) for _ in range(2))
+        for out, kernel in ((got, "auto"), (want, "general")):
+            _lib.check(L.mpsa_gemm_mx_on(_lib.GEMM_KERNELS[kernel], _lib.ptr(a), _lib.ptr(sa), fmt_a, _lib.ptr(b), _lib.ptr(sb), fmt_b, packed, batch, heads, heads_b, M, N, K,
+                                         _lib.ptr(out), _lib.dtype_id(dtype), ldc, _lib.stream_ptr(a.device)))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
