@@ -92,6 +92,9 @@ int mpsa_fp8_encode(const float* x, int64_t n, int fmt, uint8_t* codes, mpsa_str
  * arrive one code per byte, as the reference's quantizer leaves them).
  */
 int mpsa_e2m1_pack(const uint8_t* codes, int64_t outer, int64_t n, int64_t inner, uint8_t* packed, mpsa_stream_t stream);
+/* mpsa_e2m1_pack along the last dimension (inner = 1) of two tensors in one launch. */
+int mpsa_e2m1_pack_pair(const uint8_t* a, int64_t outer_a, int64_t n_a, uint8_t* packed_a,
+                        const uint8_t* b, int64_t outer_b, int64_t n_b, uint8_t* packed_b, mpsa_stream_t stream);
 int mpsa_e2m1_unpack(const uint8_t* packed, int64_t outer, int64_t n, int64_t inner, uint8_t* codes, mpsa_stream_t stream);
 
 /*
@@ -131,6 +134,19 @@ int mpsa_quantize_mx(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N
 int mpsa_quantize_mx_as(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,
                         const int64_t x_strides[4], const void* sub, float pre_scale, int fmt, int emax_elem,
                         uint8_t* codes, uint8_t* scales, int64_t out_rows, int code_per_byte, int scales_5d, mpsa_stream_t stream);
+
+/* Two tensors of one 16-bit type in one launch -- the Q and K of a score product, the A and B of a matmul: two calls of
+ * mpsa_quantize_mx_as (without sub), same results.  A job names what those calls take for one tensor. */
+typedef struct mpsa_quantize_job {
+    const void* x;
+    int64_t B, H, N, D;
+    int64_t x_strides[4];
+    float pre_scale;
+    int32_t fmt, emax_elem;
+    uint8_t *codes, *scales;
+    int64_t out_rows;
+} mpsa_quantize_job;
+int mpsa_quantize_mx_pair(const mpsa_quantize_job* a, const mpsa_quantize_job* b, int x_dtype, int code_per_byte, int scales_5d, mpsa_stream_t stream);
 
 /*
  * Both precisions in one pass over x (the diagonal-tiled attention needs Q and K in E2M1 and in
@@ -228,7 +244,9 @@ int mpsa_gemm_mx_batched_packed(const uint8_t* a, const uint8_t* sa5, int fmt_a,
  * The kernels behind the four entry points above.  mpsa_gemm_mx_on is all four in one (packed != 0: scales in the packed form;
  * batch = heads_a = heads_b = 1: the 2-D product) with the kernel named by the caller, for comparisons and measurements;
  * MPSA_GEMM_AUTO is what the others take.  A kernel that does not take the shape gives MPSA_EUNSUPPORTED.
- * mpsa_gemm_kernel says which kernel a call takes (MPSA_GEMM_SPLIT resolved to its tile), or why it would be refused.
+ * mpsa_gemm_kernel says which kernel a call takes (MPSA_GEMM_SPLIT resolved to its tile), or why it would be refused.  (With
+ * MPSA_GEMM_AUTO a product with K == 128 and 16-bit results in rows that start on 16 bytes runs on a kernel of its own, which
+ * gives the bits of MPSA_GEMM_GENERAL.)
  */
 #define MPSA_GEMM_AUTO 0
 #define MPSA_GEMM_GENERAL 1                               /* 128 x 128 tiles, two-stage pipeline: every shape */

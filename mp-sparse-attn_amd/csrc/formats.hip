@@ -159,6 +159,16 @@ __global__ __launch_bounds__(256) void nibble_flat_kernel(const uint8_t* src, ui
     }
 }
 
+// two tensors' codes packed by one launch
+__global__ __launch_bounds__(256) void nibble_pair_kernel(const uint8_t* a, uint8_t* packed_a, int64_t groups_a, const uint8_t* b, uint8_t* packed_b, int64_t groups_b) {
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const bool first = i < groups_a;
+    if (!first) i -= groups_a;
+    if (!first && i >= groups_b) return;
+    const uint4 x = reinterpret_cast<const uint4*>(first ? a : b)[i];
+    reinterpret_cast<uint2*>(first ? packed_a : packed_b)[i] = make_uint2(gather_nibbles(x.x) | (gather_nibbles(x.y) << 16), gather_nibbles(x.z) | (gather_nibbles(x.w) << 16));
+}
+
 int nibble_run(const char* what, const uint8_t* src, int64_t outer, int64_t n, int64_t inner, uint8_t* dst, bool pack, hipStream_t st) {
     if (outer < 0 || n < 0 || inner < 0) return mpsa_fail(MPSA_EINVAL, "%s: bad shape", what);
     const int64_t total = outer * ((n + 1) / 2) * inner;
@@ -199,6 +209,20 @@ int scale_layout(const char* what, const uint8_t* src, int64_t batch, int64_t ro
 
 extern "C" int mpsa_e2m1_pack(const uint8_t* codes, int64_t outer, int64_t n, int64_t inner, uint8_t* packed, mpsa_stream_t stream) {
     return nibble_run("e2m1_pack", codes, outer, n, inner, packed, true, (hipStream_t)stream);
+}
+extern "C" int mpsa_e2m1_pack_pair(const uint8_t* a, int64_t outer_a, int64_t n_a, uint8_t* packed_a,
+                                   const uint8_t* b, int64_t outer_b, int64_t n_b, uint8_t* packed_b, mpsa_stream_t stream) {
+    auto flat = [](const uint8_t* src, int64_t outer, int64_t n, uint8_t* dst) {
+        return src && dst && outer > 0 && n > 0 && n % 2 == 0 && outer * n % 16 == 0 && outer * n < (int64_t(1) << 36) && reinterpret_cast<uintptr_t>(src) % 16 == 0 && reinterpret_cast<uintptr_t>(dst) % 8 == 0;
+    };
+    if (flat(a, outer_a, n_a, packed_a) && flat(b, outer_b, n_b, packed_b)) {
+        const int64_t ga = outer_a * n_a / 16, gb = outer_b * n_b / 16;
+        hipLaunchKernelGGL(nibble_pair_kernel, dim3((unsigned)((ga + gb + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a, packed_a, ga, b, packed_b, gb);
+        MPSA_CHECK_LAUNCH("e2m1_pack");
+        return MPSA_OK;
+    }
+    const int rc = nibble_run("e2m1_pack", a, outer_a, n_a, 1, packed_a, true, (hipStream_t)stream);
+    return rc == MPSA_OK ? nibble_run("e2m1_pack", b, outer_b, n_b, 1, packed_b, true, (hipStream_t)stream) : rc;
 }
 extern "C" int mpsa_e2m1_unpack(const uint8_t* packed, int64_t outer, int64_t n, int64_t inner, uint8_t* codes, mpsa_stream_t stream) {
     return nibble_run("e2m1_unpack", packed, outer, n, inner, codes, false, (hipStream_t)stream);

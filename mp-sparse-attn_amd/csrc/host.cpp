@@ -64,6 +64,64 @@ py::object quantize(const Tensor& x, double pre, int fmt, int emax, std::optiona
     return py::make_tuple(std::move(codes), std::move(scales));
 }
 
+// Two tensors of one type in one launch; two matrices count as [1, 1, rows, K] and their results come back as matrices.
+py::object quantize_pair(const Tensor& a, const Tensor& b, double pre_a, double pre_b, int fmt_a, int fmt_b, int emax_a, int emax_b, bool code_per_byte, bool scales_5d, int64_t stream) {
+    if (!here(a) || !b.is_cuda() || b.get_device() != a.get_device() || a.scalar_type() != b.scalar_type() || (a.scalar_type() != at::kBFloat16 && a.scalar_type() != at::kHalf)) return py::none();
+    mpsa_quantize_job jobs[2];
+    const Tensor* const x[2] = {&a, &b};
+    for (int i = 0; i < 2; ++i) {
+        const Tensor& t = *x[i];
+        mpsa_quantize_job& j = jobs[i];
+        if (t.dim() != a.dim() || (t.dim() != 4 && t.dim() != 2) || !aligned16(t) || t.numel() == 0) return py::none();
+        const bool matrix = t.dim() == 2;
+        j.B = matrix ? 1 : t.size(0); j.H = matrix ? 1 : t.size(1); j.N = t.size(-2); j.D = t.size(-1);
+        j.x_strides[0] = matrix ? 0 : t.stride(0); j.x_strides[1] = matrix ? 0 : t.stride(1); j.x_strides[2] = t.stride(-2); j.x_strides[3] = t.stride(-1);
+        if (j.x_strides[3] != 1 || ((j.x_strides[0] | j.x_strides[1] | j.x_strides[2]) & 7) || j.D % 32 || (scales_5d && (j.D % 128 || j.N % 128))) return py::none();
+        j.x = t.const_data_ptr();
+        j.out_rows = j.N;
+        j.pre_scale = (float)(i ? pre_b : pre_a); j.fmt = i ? fmt_b : fmt_a; j.emax_elem = i ? emax_b : emax_a;
+    }
+    Tensor codes[2], scales[2];
+    int rc;
+    {
+        Unlocked unlocked;
+        const auto bytes = a.options().dtype(at::kByte);
+        for (int i = 0; i < 2; ++i) {
+            mpsa_quantize_job& j = jobs[i];
+            const bool matrix = x[i]->dim() == 2;
+            const int64_t width = j.fmt == MPSA_FMT_E2M1 && !code_per_byte ? j.D / 2 : j.D;
+            codes[i] = matrix ? at::empty({j.N, width}, bytes) : at::empty({j.B, j.H, j.N, width}, bytes);
+            if (scales_5d) scales[i] = matrix ? at::empty({j.N / 128, j.D / 128, 32, 4, 4}, bytes) : at::empty({j.B, j.H, j.N / 128, j.D / 128, 32, 4, 4}, bytes);
+            else           scales[i] = matrix ? at::empty({j.N, j.D / 32}, bytes) : at::empty({j.B, j.H, j.N, j.D / 32}, bytes);
+            j.codes = codes[i].data_ptr<uint8_t>(); j.scales = scales[i].data_ptr<uint8_t>();
+        }
+        rc = mpsa_quantize_mx_pair(&jobs[0], &jobs[1], dtype_id(a.scalar_type()), code_per_byte, scales_5d, stream_of(stream));
+    }
+    if (rc != MPSA_OK) return py::none();
+    return py::make_tuple(std::move(codes[0]), std::move(scales[0]), std::move(codes[1]), std::move(scales[1]));
+}
+
+// E2M1 codes of two tensors, one per byte, packed along their last dim
+py::object pack_pair(const Tensor& a, const Tensor& b, int64_t stream) {
+    if (!here(a) || !b.is_cuda() || b.get_device() != a.get_device() || a.scalar_type() != at::kByte || b.scalar_type() != at::kByte || a.dim() == 0 || b.dim() == 0 ||
+        !a.is_contiguous() || !b.is_contiguous() || a.numel() == 0 || b.numel() == 0)
+        return py::none();
+    Tensor packed[2];
+    int rc;
+    {
+        Unlocked unlocked;
+        for (int i = 0; i < 2; ++i) {
+            auto shape = (i ? b : a).sizes().vec();
+            shape.back() = (shape.back() + 1) / 2;
+            packed[i] = at::empty(shape, a.options());
+        }
+        rc = mpsa_e2m1_pack_pair(a.const_data_ptr<uint8_t>(), a.numel() / a.size(-1), a.size(-1), packed[0].data_ptr<uint8_t>(),
+                                 b.const_data_ptr<uint8_t>(), b.numel() / b.size(-1), b.size(-1), packed[1].data_ptr<uint8_t>(), stream_of(stream));
+    }
+    if (rc != MPSA_OK) return py::none();
+    return py::make_tuple(std::move(packed[0]), std::move(packed[1]));
+}
+
 // codes of `rows` rows of K elements behind the leading dims, bytes, contiguous
 bool operand(const Tensor& t, const Tensor& scale, at::IntArrayRef lead, int64_t rows, int64_t K, int fmt, bool packed, int device) {
     const size_t n = lead.size();
@@ -137,6 +195,8 @@ py::object attention(int kernel, int64_t desc, int64_t workspace, const std::vec
 
 PYBIND11_MODULE(mpsa_host, m) {
     m.def("quantize", &quantize);
+    m.def("quantize_pair", &quantize_pair);
+    m.def("pack_pair", &pack_pair);
     m.def("matmul", &matmul);
     m.def("matmul_batched", &matmul_batched);
     m.def("attention", &attention);

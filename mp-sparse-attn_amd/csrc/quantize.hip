@@ -79,6 +79,42 @@ void launch(const QuantArgs& a, int fmt8, dim3 grid, hipStream_t st) {
     }
 }
 
+// Two tensors as two groups of workgroups of one launch.
+struct PairArgs {
+    QuantArgs a, b;
+    uint32_t blocks_a, blocks_b, heads_a, heads_b, total_a, total_b;       // blocks per (batch, head), heads, blocks of all heads
+};
+
+template <int XDT, int FA, int FB>
+__device__ __forceinline__ void quantize_pair_block(const PairArgs& p, uint32_t blk) {
+    if (blk < p.total_a) {
+        const uint32_t head = blk / p.blocks_a;
+        quantize_block<XDT, FA == MPSA_FMT_E2M1, FA != MPSA_FMT_E2M1, FA, false>(p.a, blk - head * p.blocks_a, head % p.heads_a, head / p.heads_a, p.heads_a);
+        return;
+    }
+    blk -= p.total_a;
+    if (blk >= p.total_b) return;
+    const uint32_t head = blk / p.blocks_b;
+    quantize_block<XDT, FB == MPSA_FMT_E2M1, FB != MPSA_FMT_E2M1, FB, false>(p.b, blk - head * p.blocks_b, head % p.heads_b, head / p.heads_b, p.heads_b);
+}
+
+template <int XDT, int FA, int FB>
+__global__ __launch_bounds__(256) void quantize_pair_kernel(PairArgs p) {
+    quantize_pair_block<XDT, FA, FB>(p, 2 * blockIdx.x);
+    quantize_pair_block<XDT, FA, FB>(p, 2 * blockIdx.x + 1);
+}
+
+template <int XDT>
+bool launch_pair(const PairArgs& p, int fa, int fb, unsigned grid, hipStream_t st) {
+    if (fa == MPSA_FMT_E2M1 && fb == MPSA_FMT_E2M1)      hipLaunchKernelGGL((quantize_pair_kernel<XDT, MPSA_FMT_E2M1, MPSA_FMT_E2M1>), dim3(grid), dim3(256), 0, st, p);
+    else if (fa == MPSA_FMT_E4M3 && fb == MPSA_FMT_E4M3) hipLaunchKernelGGL((quantize_pair_kernel<XDT, MPSA_FMT_E4M3, MPSA_FMT_E4M3>), dim3(grid), dim3(256), 0, st, p);
+    else if (fa == MPSA_FMT_E5M2 && fb == MPSA_FMT_E5M2) hipLaunchKernelGGL((quantize_pair_kernel<XDT, MPSA_FMT_E5M2, MPSA_FMT_E5M2>), dim3(grid), dim3(256), 0, st, p);
+    else if (fa == MPSA_FMT_E4M3 && fb == MPSA_FMT_E2M1) hipLaunchKernelGGL((quantize_pair_kernel<XDT, MPSA_FMT_E4M3, MPSA_FMT_E2M1>), dim3(grid), dim3(256), 0, st, p);
+    else if (fa == MPSA_FMT_E5M2 && fb == MPSA_FMT_E2M1) hipLaunchKernelGGL((quantize_pair_kernel<XDT, MPSA_FMT_E5M2, MPSA_FMT_E2M1>), dim3(grid), dim3(256), 0, st, p);
+    else return false;
+    return true;
+}
+
 int quantize_common(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D, const int64_t* xs,
                     const void* sub, float pre, bool do4, int emax4, bool do8, int fmt8, int emax8,
                     uint8_t* c4, uint8_t* s4, uint8_t* c8, uint8_t* s8, int64_t out_rows, hipStream_t st, bool spread = false, bool scales5d = false) {
@@ -151,6 +187,41 @@ extern "C" int mpsa_quantize_mx_as(const void* x, int x_dtype, int64_t B, int64_
         return quantize_common(x, x_dtype, B, H, N, D, x_strides, sub, pre_scale, false, 0, true, fmt, emax_elem,
                                nullptr, nullptr, codes, scales, out_rows, (hipStream_t)stream, false, scales_5d != 0);
     return mpsa_fail(MPSA_EINVAL, "quantize: unknown format %d", fmt);
+}
+
+extern "C" int mpsa_quantize_mx_pair(const mpsa_quantize_job* a, const mpsa_quantize_job* b, int x_dtype, int code_per_byte, int scales_5d, mpsa_stream_t stream) {
+    if (!a || !b) return mpsa_fail(MPSA_EINVAL, "quantize: null job");
+    auto alone = [&](const mpsa_quantize_job& j) {
+        return mpsa_quantize_mx_as(j.x, x_dtype, j.B, j.H, j.N, j.D, j.x_strides, nullptr, j.pre_scale, j.fmt, j.emax_elem, j.codes, j.scales, j.out_rows, code_per_byte, scales_5d, stream);
+    };
+    auto setup = [&](const mpsa_quantize_job& j, QuantArgs& q, unsigned& blocks) {
+        const bool four = j.fmt == MPSA_FMT_E2M1;
+        if (!four && j.fmt != MPSA_FMT_E4M3 && j.fmt != MPSA_FMT_E5M2) return mpsa_fail(MPSA_EINVAL, "quantize: unknown format %d", j.fmt);
+        const int rc = mpsa_quantize_setup(j.x, x_dtype, j.B, j.H, j.N, j.D, j.x_strides, nullptr, j.pre_scale, four, four ? j.emax_elem : 0, !four, four ? 0 : j.fmt, four ? 0 : j.emax_elem,
+                                           four ? j.codes : nullptr, four ? j.scales : nullptr, four ? nullptr : j.codes, four ? nullptr : j.scales, j.out_rows, &q, &blocks);
+        if (rc != MPSA_OK || blocks == 0) return rc;
+        if (scales_5d && (j.D % 128 || j.out_rows % 128)) return mpsa_fail(MPSA_EUNSUPPORTED, "quantize: packed scales need rows and D in multiples of 128 (got %lld, %lld)", (long long)j.out_rows, (long long)j.D);
+        q.spread = four && code_per_byte;
+        q.scales5d = scales_5d ? 1 : 0;
+        return (int)MPSA_OK;
+    };
+    PairArgs p;
+    unsigned blocks_a = 0, blocks_b = 0;
+    int rc = setup(*a, p.a, blocks_a);
+    if (rc == MPSA_OK) rc = setup(*b, p.b, blocks_b);
+    if (rc != MPSA_OK) return rc;
+    const int64_t total_a = (int64_t)blocks_a * a->H * a->B, total_b = (int64_t)blocks_b * b->H * b->B;
+    bool done = false;
+    if (total_a > 0 && total_b > 0 && total_a + total_b < (int64_t(1) << 31) && !use_sw_fp8()) {
+        p.blocks_a = blocks_a; p.heads_a = (uint32_t)a->H; p.total_a = (uint32_t)total_a;
+        p.blocks_b = blocks_b; p.heads_b = (uint32_t)b->H; p.total_b = (uint32_t)total_b;
+        const unsigned grid = (unsigned)((total_a + total_b + 1) / 2);
+        done = x_dtype == MPSA_BF16 ? launch_pair<MPSA_BF16>(p, a->fmt, b->fmt, grid, (hipStream_t)stream) : launch_pair<MPSA_F16>(p, a->fmt, b->fmt, grid, (hipStream_t)stream);
+        MPSA_CHECK_LAUNCH("quantize");
+    }
+    if (done) return MPSA_OK;
+    rc = alone(*a);
+    return rc == MPSA_OK ? alone(*b) : rc;
 }
 
 extern "C" int mpsa_quantize_mx(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D,

@@ -36,6 +36,12 @@ class AttnDesc(ctypes.Structure):
                 + [(n, _f32) for n in ("pre_scale_q", "skip_thresh", "route_thresh")])
 
 
+class QuantizeJob(ctypes.Structure):
+    """``mpsa_quantize_job`` of include/mpsa.h."""
+    _fields_ = ([("x", _vp)] + [(n, _i64) for n in ("B", "H", "N", "D")] + [("x_strides", _i64 * 4), ("pre_scale", _f32), ("fmt", ctypes.c_int32), ("emax_elem", ctypes.c_int32),
+                ("codes", _vp), ("scales", _vp), ("out_rows", _i64)])
+
+
 # name -> (restype, argtypes); must list every symbol include/mpsa.h declares
 SIGNATURES = {
     "mpsa_version": (_int, []),
@@ -47,10 +53,12 @@ SIGNATURES = {
     "mpsa_e8m0_decode": (_int, [_vp, _i64, _vp, _vp]),
     "mpsa_fp8_encode": (_int, [_vp, _i64, _int, _vp, _vp]),
     "mpsa_e2m1_pack": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
+    "mpsa_e2m1_pack_pair": (_int, [_vp, _i64, _i64, _vp] * 2 + [_vp]),
     "mpsa_e2m1_unpack": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mpsa_scales_to_5d": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mpsa_scales_from_5d": (_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "mpsa_quantize_mx_as": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _p64, _vp, _f32, _int, _int, _vp, _vp, _i64, _int, _int, _vp]),
+    "mpsa_quantize_mx_pair": (_int, [ctypes.POINTER(QuantizeJob)] * 2 + [_int, _int, _int, _vp]),
     "mpsa_quantize_mx": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _p64, _vp, _f32, _int, _int, _vp, _vp, _i64, _vp]),
     "mpsa_seq_mean_workspace": (_i64, [_i64, _i64, _i64, _i64]),
     "mpsa_seq_mean": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _p64, _vp, _vp, _vp]),
@@ -132,7 +140,7 @@ _host = None
 
 class _NoHost:
     """Stands in for the extension where MPSA_LIB_PATH names another library than the one it is linked to."""
-    quantize = matmul = matmul_batched = attention = staticmethod(lambda *args: None)
+    quantize = quantize_pair = pack_pair = matmul = matmul_batched = attention = staticmethod(lambda *args: None)
 
 
 def host():

@@ -16,7 +16,7 @@ import torch
 
 from . import _lib
 from .mxfp import MXFP4Tensor, MXScaleTensor
-from .quant_mxint8 import _quantize_as
+from .quant_mxint8 import _quantize_as, quantize_pair
 
 VEC_SIZE = 32
 
@@ -168,6 +168,16 @@ def _package_operand(t, four_bit, fmt8):
     return fp4.to_packed_tensor(dim=t.dim() - 1), lambda: fp4.to(torch.float32)
 
 
+def _package_operands(a, b, fmt_a, fmt_b):
+    """:func:`_package_operand` of A and B; two tensors of ready-made 4-bit codes are packed by one launch."""
+    fmt8 = fmt_a if fmt_a != _lib.FMT_E2M1 else _lib.FMT_E4M3
+    if fmt_a == fmt_b == _lib.FMT_E2M1 and a.dtype == b.dtype == torch.uint8 and a.is_cuda:
+        packed = _lib.host().pack_pair(a, b, _lib.raw_stream(a))
+        if packed is not None:
+            return tuple((p, lambda t=t: MXFP4Tensor(data=t, dtype=torch.uint8).to(torch.float32)) for p, t in zip(packed, (a, b)))
+    return _package_operand(a, fmt_a == _lib.FMT_E2M1, fmt8), _package_operand(b, fmt_b == _lib.FMT_E2M1, fmt8)
+
+
 def _package_scale(s):
     """Float scale factors -> E8M0 bytes through ``MXScaleTensor`` (ours/block_scaled_matmul.py:370-374); uint8 input
     is taken as ready-made E8M0 bytes (ours/mxfp_attn_kernel.py:505-506)."""
@@ -209,9 +219,7 @@ def initialize_block_scaled_from_tensor(a_tensor, b_tensor, a_scale, b_scale, bl
     assert tuple(b_scale.shape) == expected_b, f"b_scale shape mismatch: expected {expected_b}, got {tuple(b_scale.shape)}"
     configs = make_configs(block_scale_type)
     fmt_a, fmt_b = _fmts_of(configs)
-    f8 = fmt_a if fmt_a != _lib.FMT_E2M1 else _lib.FMT_E4M3
-    a, a_ref = _package_operand(a_tensor, fmt_a == _lib.FMT_E2M1, f8)
-    b, b_ref = _package_operand(b_tensor, fmt_b == _lib.FMT_E2M1, f8)
+    (a, a_ref), (b, b_ref) = _package_operands(a_tensor, b_tensor, fmt_a, fmt_b)
     a_scale, b_scale = _package_scale(a_scale), _package_scale(b_scale)
     reference = None
     if compute_reference:
@@ -248,6 +256,8 @@ def quantize_block_scaled_from_tensor(a_tensor, b_tensor, block_scale_type="mxfp
         raise ValueError(f"Invalid block scale type: {block_scale_type}")
     configs = make_configs(block_scale_type)
     fmt_a, fmt_b = _fmts_of(configs)
+    if a_tensor.dim() == b_tensor.dim() == 2:
+        return (*quantize_pair(a_tensor, b_tensor, 1.0, 1.0, fmt_a, fmt_b, scales_5d=packed_scales), configs)
     a, sa = _quantize_as(a_tensor[None, None], 1.0, fmt_a, scales_5d=packed_scales)
     b, sb = _quantize_as(b_tensor[None, None], 1.0, fmt_b, scales_5d=packed_scales)
     return a[0, 0], sa[0, 0], b[0, 0], sb[0, 0], configs

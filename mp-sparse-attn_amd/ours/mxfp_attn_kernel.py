@@ -217,7 +217,7 @@ def initialize_block_scaled_batched_from_tensor(a_tensor, b_tensor, a_scale, b_s
     ``compute_reference`` the reference's triple (:508-551): the float32 scores ``dq(A) @ dq(B)^T`` ``[B,H,M,N]`` (codes
     decoded, E8M0 bytes decoded and repeated over their 32 elements, ``torch.matmul``, all on the device) and the
     decoded codes of A and B without their scale factors, as the reference returns them."""
-    from .block_scaled_matmul import _TYPES, _fmts_of, _package_operand, _package_scale, _expanded_scales, make_configs, VEC_SIZE
+    from .block_scaled_matmul import _TYPES, _fmts_of, _package_operands, _package_scale, _expanded_scales, make_configs, VEC_SIZE
     if block_scale_type == "nvfp4":
         raise NotImplementedError("nvfp4 (16-element blocks, FP8 scale factors) is not available: the gfx950 scaled matrix "
                                   "instructions take one E8M0 scale per 32 elements")
@@ -234,9 +234,7 @@ def initialize_block_scaled_batched_from_tensor(a_tensor, b_tensor, a_scale, b_s
     configs = make_configs(block_scale_type)
     configs["BLOCK_SIZE_M"] = configs["BLOCK_SIZE_N"] = 128
     fmt_a, fmt_b = _fmts_of(configs)
-    f8 = fmt_a if fmt_a != _lib.FMT_E2M1 else _lib.FMT_E4M3
-    a, a_ref = _package_operand(a_tensor, fmt_a == _lib.FMT_E2M1, f8)
-    b, b_ref = _package_operand(b_tensor, fmt_b == _lib.FMT_E2M1, f8)
+    (a, a_ref), (b, b_ref) = _package_operands(a_tensor, b_tensor, fmt_a, fmt_b)
     a_scale, b_scale = _package_scale(a_scale), _package_scale(b_scale)
     reference = (None, None, None)
     if compute_reference:

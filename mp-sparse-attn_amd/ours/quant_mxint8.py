@@ -109,6 +109,22 @@ def _quantize_as(x, pre_scale, fmt, emax_elem=None, out_rows=None, sub=None, cod
     return codes, scales
 
 
+def quantize_pair(a, b, pre_a, pre_b, fmt_a, fmt_b, code_per_byte=False, scales_5d=False):
+    """Two tensors ``[B,H,L,D]``, or two matrices -> ``(codes, scales)`` of either, as two calls of :func:`_quantize_as` give them; in
+    one launch (``mpsa_quantize_mx_pair``) where both are of one 16-bit type and need no copy."""
+    _lib.require_device(a, b)
+    emax = [EMAX_E2M1 if fmt == _lib.FMT_E2M1 else EMAX_8BIT for fmt in (fmt_a, fmt_b)]
+    done = _lib.host().quantize_pair(a, b, pre_a, pre_b, fmt_a, fmt_b, emax[0], emax[1], code_per_byte, scales_5d, _lib.raw_stream(a))
+    if done is not None:
+        return done
+    out = []
+    for x, pre, fmt in ((a, pre_a, fmt_a), (b, pre_b, fmt_b)):
+        matrix = x.dim() == 2
+        codes, scales = _quantize_as(x[None, None] if matrix else x, pre, fmt, code_per_byte=code_per_byte, scales_5d=scales_5d)
+        out += [codes[0, 0], scales[0, 0]] if matrix else [codes, scales]
+    return tuple(out)
+
+
 def quantize_mx_dual(x, pre_scale, fmt8=_lib.FMT_E4M3, out_rows=None, sub=None):
     """E2M1 and an 8-bit format in one pass over x -> (codes4, scales4, codes8, scales8).  ``sub`` as in
     :func:`quantize_mx`."""
@@ -131,10 +147,10 @@ def quantize_mx_dual(x, pre_scale, fmt8=_lib.FMT_E4M3, out_rows=None, sub=None):
 def _quant_pair(q, k, fmt, sm_scale, tensor_layout, code_per_byte=False):
     q4 = _as_bhnd(q, tensor_layout)
     k4 = _as_bhnd(k, tensor_layout)
-    head_dim = q4.shape[-1]
-    qc, qs = _quantize_as(q4, pre_scale_q(head_dim, sm_scale), fmt, code_per_byte=code_per_byte)
-    kc, ks = _quantize_as(k4, 1.0, fmt, code_per_byte=code_per_byte)
-    return qc, qs, kc, ks
+    pre = pre_scale_q(q4.shape[-1], sm_scale)
+    if q4.dim() == k4.dim() == 4:
+        return quantize_pair(q4, k4, pre, 1.0, fmt, fmt, code_per_byte)
+    return (*_quantize_as(q4, pre, fmt, code_per_byte=code_per_byte), *_quantize_as(k4, 1.0, fmt, code_per_byte=code_per_byte))
 
 
 def quant_mxfp4(q, k, BLKQ=128, BLKK=64, sm_scale=None, tensor_layout="HND", packed=True):

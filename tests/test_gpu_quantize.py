@@ -233,3 +233,44 @@ def test_small_blocks_on_either_side_of_the_step_by_step_conversion(fmt, pre):
     x[..., 5::16] *= 2.0 ** -24
     x = (x * torch.exp2(torch.arange(-126, -62).float())[None, None, :, None]).bfloat16()
     _check(x, pre, fmt)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fmt_a,fmt_b", [(4, 4), (0, 0), (1, 1), (0, 4), (1, 4), (4, 0)])
+@pytest.mark.parametrize("shape_a,shape_b", [((1, 1, 1, 32), (1, 1, 1, 32)), ((2, 3, 129, 64), (2, 1, 77, 64)), ((1, 5, 128, 128), (1, 2, 256, 128)), ((3, 64), (1000, 96)), ((256, 128), (128, 384))])
+def test_two_tensors_in_one_launch_give_the_results_of_two(shape_a, shape_b, fmt_a, fmt_b, dtype):
+    from ours.quant_mxint8 import quantize_pair
+    g = torch.Generator().manual_seed(sum(shape_a))
+    a, b = (torch.randn(*s, generator=g).to(dtype).to(DEV) for s in (shape_a, shape_b))
+    whole = all(s[-1] % 128 == 0 and s[-2] % 128 == 0 for s in (shape_a, shape_b))
+    for per_byte in (False, True):
+        for five in ((False, True) if whole else (False,)):
+            got = quantize_pair(a, b, 0.1275174, 1.0, fmt_a, fmt_b, per_byte, five)
+            want = []
+            for x, pre, fmt in ((a, 0.1275174, fmt_a), (b, 1.0, fmt_b)):
+                from ours.quant_mxint8 import _quantize_as
+                c, s = _quantize_as(x if x.dim() == 4 else x[None, None], pre, fmt, code_per_byte=per_byte, scales_5d=five)
+                want += [c, s] if x.dim() == 4 else [c[0, 0], s[0, 0]]
+            assert all(torch.equal(x, y) and x.shape == y.shape for x, y in zip(got, want))
+    # rows of a wider tensor: strides of their own
+    if len(shape_a) == 4:
+        wide = torch.randn(*shape_a[:-1], shape_a[-1] + 8, generator=g).to(dtype).to(DEV)
+        got = quantize_pair(wide[..., 8:], b, 1.0, 1.0, fmt_a, fmt_b)
+        c, s = quantize_mx(wide[..., 8:].contiguous(), 1.0, fmt_a)
+        assert torch.equal(got[0], c) and torch.equal(got[1], s)
+
+
+def test_codes_of_two_tensors_packed_in_one_launch():
+    from ours.mxfp_attn_kernel import initialize_block_scaled_batched_from_tensor
+    g = torch.Generator().manual_seed(2)
+    for M, N in ((128, 256), (256, 128)):
+        a, b = (torch.randint(0, 16, (1, 2, rows, 128), generator=g, dtype=torch.uint8).to(DEV) for rows in (M, N))
+        sa, sb = (torch.full((1, 2, rows // 128, 1, 32, 4, 4), 127, dtype=torch.uint8, device=DEV) for rows in (M, N))
+        got = initialize_block_scaled_batched_from_tensor(a, b, sa, sb, "mxfp4")
+        for codes, packed in ((a, got[0]), (b, got[2])):
+            assert torch.equal(packed, codes[..., ::2] | codes[..., 1::2] << 4)
+    odd = torch.randint(0, 16, (3, 7), generator=g, dtype=torch.uint8).to(DEV)
+    even = torch.randint(0, 16, (3, 32), generator=g, dtype=torch.uint8).to(DEV)
+    first, second = _lib.host().pack_pair(odd, even, _lib.raw_stream(odd))
+    assert torch.equal(second, even[:, ::2] | even[:, 1::2] << 4)
+    assert torch.equal(first[:, :3], odd[:, :6:2] | odd[:, 1::2] << 4) and torch.equal(first[:, 3], odd[:, 6])
