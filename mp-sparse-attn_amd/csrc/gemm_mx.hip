@@ -251,9 +251,11 @@ bool force_general() {
 
 template <int FMT, int FMTB, typename OutT, bool PAIR>
 void launch_scales(const GemmArgs& g, dim3 grid, hipStream_t st) {
-    if (g.packed)            launch_kernel<FMT, FMTB, OutT, false, true, PAIR, false>(g, grid, st);
-    else if (g.K % 512 == 0) launch_kernel<FMT, FMTB, OutT, true, false, PAIR, false>(g, grid, st);
-    else                     launch_kernel<FMT, FMTB, OutT, false, false, PAIR, false>(g, grid, st);
+    if (g.packed)               launch_kernel<FMT, FMTB, OutT, false, false, true, PAIR, false>(g, grid, st);
+    else if constexpr (PAIR) {
+        if (g.K % 512 == 0)     launch_kernel<FMT, FMTB, OutT, true, false, false, PAIR, false>(g, grid, st);
+        else                    launch_kernel<FMT, FMTB, OutT, true, true, false, PAIR, false>(g, grid, st);
+    }
 }
 
 template <int FMT, int FMTB, typename OutT>
@@ -292,6 +294,7 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
     const bool mixed = fmt_a != MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1;
     const int kind = fmt_a == MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1 ? 0 : mixed ? 1 : 2;
     const bool staged = g.K % 128 == 0 && (fmt_a == fmt_b || mixed) && ((g.M % BM == 0 && g.N % BN == 0) || kind != 0 || g.K % 256 == 0);
+    const bool half = kind == 0 && g.K % 256 == 128 && !g.packed;        // ragged 4-bit products that end in half a unit: not by name
     int tile = 0;
     switch (kernel) {
         case MPSA_GEMM_AUTO: break;
@@ -324,7 +327,7 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
     const Shared& sh = SHARED[kind];
     const double load = tiles(128) / 256.0, slope = sh.base + sh.per_1024 * load;
     const double general = sh.start + sh.tile * load + K / 1024.0 * (slope > sh.least ? slope : sh.least);
-    const double cost16 = gemm_split_cost(g, batches, fmt_a, fmt_b, &tile), cost128 = ring(0, 128), cost256 = staged ? ring(1, 256) : 1e300;
+    const double cost16 = gemm_split_cost(g, batches, fmt_a, fmt_b, &tile), cost128 = ring(0, 128), cost256 = staged || half ? ring(1, 256) : 1e300;
     const double least = fmin(fmin(cost16, cost128), cost256);
     if (general < least) return MPSA_GEMM_GENERAL;
     return cost16 == least ? MPSA_GEMM_SPLIT_TILE(tile / 10, tile % 10) : cost128 == least ? MPSA_GEMM_TILE128 : MPSA_GEMM_TILE256;
@@ -376,7 +379,7 @@ static int gemm_entry(int kernel, const uint8_t* a, const uint8_t* sa, int fmt_a
         gemm_tile_launch(g, batches, fmt_a, fmt_b, c_dtype, st);
     } else if (kernel != MPSA_GEMM_TILE256) {
         gemm_split_launch(g, batches, kernel, fmt_a, fmt_b, c_dtype, st);
-    } else if (M % BM || N % BN) {
+    } else if (M % BM || N % BN || (!packed && fmt_a == MPSA_FMT_E2M1 && K % 256)) {
         gemm_edge_launch(g, batches, fmt_a, fmt_b, c_dtype, st);
     } else {
         const bool mixed = fmt_a != fmt_b;

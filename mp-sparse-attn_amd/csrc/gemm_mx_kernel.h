@@ -20,16 +20,19 @@
 // from each of 8 rows (measured L2 -> LDS: 17 against 31 TB/s chip-wide).  So whenever the number of stages is
 // even (PAIR) the ring is refilled two stages -- one "unit" of 128 bytes per row -- at a time: the unit's LDS image
 // has a 128-byte row pitch, one workgroup barrier per unit, one unit in flight while the other is multiplied.
-// Runs with an odd number of stages (4-bit codes, K % 256 == 128) keep the stage-by-stage ring, three stages in
+// Runs with an odd number of stages (4-bit codes, K % 256 == 128) end in half a unit (HALF; they take the EDGE form, whose loads
+// have their rows apart from the place in a row); with packed scales they keep the stage-by-stage ring, three stages in
 // flight while one is multiplied.  Either way the 16-byte pieces of a row are XOR-swizzled with the row index so
 // that the 128-bit operand reads of 16 consecutive rows hit 16 distinct 4-bank groups, and wave tiles of
 // 128x128 keep LDS reads at 8 operand fragments per 16 matrix instructions.
 //
 // Scale bytes.  A row's scale bytes for one stage are 4 (or 2) bytes in a line of their own, so fetching them
 // stage by stage costs the vector memory path one cache-line access per row per stage - as many accesses as
-// the codes themselves.  When K is a multiple of 512 the kernel instead fetches 16 scale bytes per row at a
+// the codes themselves.  The kernel instead fetches 16 scale bytes per row at a
 // time (a "group" of 4 stages of 4-bit codes, 8 stages of 8-bit codes) into a double-buffered LDS area, one
-// group ahead.  Other K fall back to one 4-byte scale load per row per stage.
+// group ahead: 16 bytes a lane when K is a multiple of 512, else (WORDS) a word a lane, four lanes a row.
+// The step from one 4-byte load per row per stage, which K % 512 != 0 had: 3396 x 15872 x 9856, 8-bit x 4-bit, 579 -> 432 us;
+// 1000 x 14336 x 4224 65.6 -> 50.5; 4096 x 4096 x 4224, 8-bit, 74.7 -> 60.3; 4096 x 4096 x 4352, 4-bit, 47.3 -> 40.7.
 // With the scales in the reference's packed form [rows/128, K/128, 32, 4, 4] (ours/mxfp_attn_kernel.py:56-57) the
 // scale bytes of 128 rows x 128 elements of K are one contiguous 512-byte chunk: a stage's scales are four chunks,
 // one 32-lane load per wave, and a lane reads its scale words for all four row blocks with one 128-bit LDS read.
@@ -77,9 +80,11 @@ __device__ __forceinline__ void load_to_lds(uint32_t lane_off, const uint8_t* wa
 // FMT: element format of A (and of B, unless FMTB says otherwise).  FMTB == E2M1 under an 8-bit FMT is the reference's
 // "mixed" type (ours/block_scaled_matmul.py:318-324): everything follows the 8-bit geometry -- a stage is 64 elements
 // of K, a unit 128 -- except B's codes, which are half as wide: 32 bytes per row and stage, a unit's image 64-byte rows.
-template <int FMT, int FMTB, typename OutT, bool WIDE, bool PK, bool PAIR, bool EDGE>
+template <int FMT, int FMTB, typename OutT, bool WIDE, bool WORDS, bool PK, bool PAIR, bool EDGE, bool HALF>
 __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
-    static_assert(!(WIDE && PK), "packed scales use the per-stage scale area");
+    static_assert(PK ? !WIDE : WIDE && PAIR, "row-major scales come in groups, with units");
+    static_assert(!HALF || (WORDS && EDGE && FMT == MPSA_FMT_E2M1), "half a unit at the end: 4-bit codes, K % 256 == 128");
+    static_assert(!WORDS || (WIDE && PAIR), "words: groups whose rows do not lie on 16 bytes");
     static_assert(NSTAGE == 4, "PAIR: the ring is two units of two stages");
     constexpr bool FP4 = (FMT == MPSA_FMT_E2M1);
     constexpr bool B4 = !FP4 && (FMTB == MPSA_FMT_E2M1);       // 8-bit A against 4-bit B
@@ -190,16 +195,18 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     // Unit u lives in ring half u & 1: [A codes 32 KiB][B codes 32 KiB][scale bytes of its two stages]
     auto unit_base = [&](int u) __attribute__((always_inline)) { return smem + (u & 1) * 2 * STAGE_BYTES; };
     auto issue_unit_part = [&](int u, int part) __attribute__((always_inline)) {
-        const int NU = KT / 2;
+        const int NU = HALF ? (KT + 1) / 2 : KT / 2;
         const int uc = u < NU ? u : NU - 1;               // past the end: re-load the last unit
+        // HALF: the last unit has its first 64 bytes a row, and twice
+        const uint32_t inside = HALF && uc == NU - 1 ? ~64u : ~0u;
         uint8_t* ub = unit_base(u);
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const int c2 = part * 2 + q, x = wave * 8 + c2;
             if constexpr (EDGE) {
                 const uint32_t row = (uint32_t)(x * 8) * (uint32_t)row_bytes + lrow;
-                load_to_lds<16>(min(row, cap_a) + lo[q], a_base + (int64_t)uc * (2 * ROWB), ub + x * 1024);
-                if constexpr (!B4) load_to_lds<16>(min(row, cap_b) + lo[q], b_base + (int64_t)uc * (2 * ROWB), ub + 2 * OP_BYTES + x * 1024);
+                load_to_lds<16>(min(row, cap_a) + (HALF ? lo[q] & inside : lo[q]), a_base + (int64_t)uc * (2 * ROWB), ub + x * 1024);
+                if constexpr (!B4) load_to_lds<16>(min(row, cap_b) + (HALF ? lo[q] & inside : lo[q]), b_base + (int64_t)uc * (2 * ROWB), ub + 2 * OP_BYTES + x * 1024);
             } else {
                 const int64_t go = (int64_t)uc * (2 * ROWB) + (int64_t)x * 8 * row_bytes;
                 load_to_lds<16>(lo[q], a_base + go, ub + x * 1024);
@@ -214,13 +221,6 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
             // codes: one chunk covers the unit, the odd stage takes its scale words from the even stage's registers
             if constexpr (FP4) load_to_lds<16>((uint32_t)lane * 16u, s_pk + (int64_t)uc * 1024, sc + wave * 1024);
             else if (lane < 32) load_to_lds<16>(pko, s_pk + (int64_t)uc * 512, sc + wave * 1024);
-        } else if constexpr (!WIDE) {
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const int sco = FP4 ? (2 * uc + hh) * 4 : uc * 4;
-                load_to_lds<4>(los_a, sa_base + sco, sc + hh * 2 * SC_BYTES + wave * 256);
-                load_to_lds<4>(los_b, sb_base + sco, sc + hh * 2 * SC_BYTES + SC_BYTES + wave * 256);
-            }
         }
     };
     auto issue_part = [&](int kt, int part) __attribute__((always_inline)) {
@@ -236,14 +236,6 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
                 const int64_t kb = FP4 ? kc : (kc >> 1);
                 if (lane < 32) load_to_lds<16>(pko, s_pk + kb * 512, st + 2 * OP_BYTES + wave * 512);
             }
-        } else if constexpr (!WIDE) {
-            if (part == 3) {
-                // four scale bytes per row: the stage's own with 4-bit codes; with 8-bit codes the aligned word
-                // that holds this stage's two bytes (the stage count is even, so the word is inside the row)
-                const int sco = FP4 ? kc * 4 : (kc >> 1) * 4;
-                load_to_lds<4>(los_a, sa_base + sco, st + 2 * OP_BYTES + wave * 256);
-                load_to_lds<4>(los_b, sb_base + sco, st + 2 * OP_BYTES + SC_BYTES + wave * 256);
-            }
         }
     };
     auto issue_stage = [&](int kt) __attribute__((always_inline)) {
@@ -254,13 +246,25 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
 #pragma unroll
         for (int part = 0; part < 4; ++part) issue_unit_part(u, part);
     };
-    // wide path: the 16 scale bytes per row of group grp (two instructions per wave)
+    // wide path: the 16 scale bytes per row of group grp (two instructions per wave).  WORDS (K is no multiple of 512: rows of
+    // scale bytes start on words, and the last group is cut): a word a lane, four neighbouring lanes a row, 16 rows an
+    // instruction; words past the row's end are its last one.
     auto issue_scales = [&](int grp) __attribute__((always_inline)) {
-        const int ng = KT / GROUP;
+        const int ng = (KT + GROUP - 1) / GROUP;
         const int gc = grp < ng ? grp : ng - 1;
         uint8_t* dst = scg + (grp & 1) * 2 * SCG_BYTES + wave * 1024;
-        load_to_lds<16>(los_a, sa_base + gc * 16, dst);
-        load_to_lds<16>(los_b, sb_base + gc * 16, dst + SCG_BYTES);
+        if constexpr (WORDS) {
+            const uint32_t w = (uint32_t)(min(4 * gc + (lane & 3), g.K / 128 - 1) * 4);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int row = wave * 64 + q * 16 + (lane >> 2);
+                load_to_lds<4>((uint32_t)min(row, last_a) * (uint32_t)srow_bytes + w, sa_base, dst + q * 256);
+                load_to_lds<4>((uint32_t)min(row, last_b) * (uint32_t)srow_bytes + w, sb_base, dst + SCG_BYTES + q * 256);
+            }
+        } else {
+            load_to_lds<16>(los_a, sa_base + gc * 16, dst);
+            load_to_lds<16>(los_b, sb_base + gc * 16, dst + SCG_BYTES);
+        }
     };
 
     v16f acc[4][4];
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     // Dword k of a row covers step pair k of the group.  With 8-bit codes the operand sets fill the register file:
     // 32 (or, reading half a group at a time, 16) more registers spill and the kernel gets slower, so that path
     // keeps the 32-bit read per step pair.
-    constexpr bool GREAD = WIDE && FP4;
+    constexpr bool GREAD = WIDE && FP4;                   // (and PAIR)
     v4i w_a[4], w_b[4];
 
     // reads operands of step s of stage kt out of the ring: part 0 the B fragments and their scale bytes,
@@ -322,10 +326,8 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
         const int c0 = PAIR ? 4 * hh : 0;                  // first 16-byte piece of this stage inside the LDS row
         // the row's scale word of this step pair (paths without the per-group read)
         const uint8_t* sc = WIDE ? scg + ((kt / GROUP) & 1) * 2 * SCG_BYTES + 4 * (FP4 ? kt % GROUP : (kt % GROUP) >> 1) + (isb ? SCG_BYTES : 0)
-                          : PAIR ? (PK ? st + 4 * OP_BYTES + hh * 512 + (isb ? 2048 : 0)
-                                       : st + 4 * OP_BYTES + hh * 2 * SC_BYTES + (isb ? SC_BYTES : 0))
+                          : PAIR ? st + 4 * OP_BYTES + hh * 512 + (isb ? 2048 : 0)
                                  : st + 2 * OP_BYTES + (isb ? SC_BYTES : 0);
-        constexpr int sstride = WIDE ? 16 : 4;
         const uint8_t* sg = scg + (grp & 1) * 2 * SCG_BYTES + (isb ? SCG_BYTES : 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
                         for (int q = 0; q < 4; ++q) (isb ? f.rb[q] : f.ra[q]) = (uint32_t)wsc[q];
                     }
                 } else {
-                    (isb ? f.rb[i] : f.ra[i]) = *reinterpret_cast<const uint32_t*>(sc + row * sstride);
+                    (isb ? f.rb[i] : f.ra[i]) = *reinterpret_cast<const uint32_t*>(sc + row * 16);
                 }
             } else {
                 if (isb) f.sb[i] = even.sb[i]; else f.sa[i] = even.sa[i];
@@ -428,7 +430,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     // PAIR: called once per unit, after its second stage has been read: the only loads in flight are the next
     // unit's (and possibly a scale group's), all of which must have landed before that unit is read.
     auto publish = [&]() __attribute__((always_inline)) {
-        constexpr int KEEP = PAIR ? 0 : WIDE ? 2 * CODE_LOADS : PK ? (FP4 ? 2 * (CODE_LOADS + 1) : 2 * CODE_LOADS + 1) : 2 * (CODE_LOADS + 2);
+        constexpr int KEEP = PAIR ? 0 : FP4 ? 2 * (CODE_LOADS + 1) : 2 * CODE_LOADS + 1;
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(wait_imm(KEEP));
         __syncthreads();
@@ -438,9 +440,9 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     Frag f0, f1;
     {
         // stages 1 .. NSTAGE-1 stay in flight (packed 8-bit: only stage 2 of them carries scale loads)
-        // PAIR: unit 1 stays in flight (16 code loads and its scale loads: none, one, or four)
-        constexpr int KEEP = PAIR ? (B4 ? CODE_LOADS + CODE_LOADS / 2 : 2 * CODE_LOADS) + (WIDE ? 0 : PK ? 1 : 4)
-                           : WIDE ? (NSTAGE - 1) * CODE_LOADS : PK ? (FP4 ? (NSTAGE - 1) * (CODE_LOADS + 1) : (NSTAGE - 1) * CODE_LOADS + 1) : (NSTAGE - 1) * (CODE_LOADS + 2);
+        // PAIR: unit 1 stays in flight (16 code loads and its scale loads: none or one)
+        constexpr int KEEP = PAIR ? (B4 ? CODE_LOADS + CODE_LOADS / 2 : 2 * CODE_LOADS) + (WIDE ? 0 : 1)
+                           : FP4 ? (NSTAGE - 1) * (CODE_LOADS + 1) : (NSTAGE - 1) * CODE_LOADS + 1;
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(wait_imm(KEEP));
         __syncthreads();
@@ -461,6 +463,22 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
                 step(f1, f0, kt + 1, 0, (u & 1) != 0, kt + 3, true, 0, u == 1 ? grp + 1 : -1, u == GROUP - 1 ? grp + 1 : -1);
             }
         }
+        if (WORDS && (KT & 2)) {                           // the last group is one unit (and HALF: half a one)
+            const int kt = KT & ~3;
+            step(f0, f1, kt, 1, false, 0, false, 0, -1, -1);
+            step(f1, f0, kt + 1, 0, false, 0, true, 0, -1, -1);
+            step(f0, f1, kt + 1, 1, false, 0, false, 1, -1, -1);
+            if (HALF) publish();
+            step(f1, f0, HALF ? kt + 2 : kt, 0, false, 0, true, 0, -1, -1);
+        }
+        if constexpr (HALF) {
+            if (KT & 2) {                                  // its scale words: the third of the group, or the first
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { w_a[i][0] = w_a[i][2]; w_b[i][0] = w_b[i][2]; }
+            }
+            step(f0, f1, KT - 1, 1, false, 0, false, 0, -1, -1);
+            step(f1, f0, KT - 1, 0, false, 0, true, 0, -1, -1);
+        }
     } else if constexpr (PAIR && FP4) {
         for (int u2 = 0; u2 < KT / 2; ++u2) {
             const int kt = 2 * u2;
@@ -476,20 +494,6 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
             step(f0, f1, kt + 1, 0, false, 0, false, 0, -1, -1);
             publish();
             step(f1, f0, kt + 2, 0, true, kt + 4, true, 0, fetch_at(kt + 1), -1);
-        }
-    } else if constexpr (GREAD) {
-        // one trip = one scale group (4 stages = four step pairs), unrolled so that the dword a pair takes from the
-        // group's scale rows, the refill that fetches the next group's scale bytes and the step that reads them
-        // into registers are all fixed at compile time
-        for (int kt0 = 0; kt0 < KT; kt0 += GROUP) {
-            const int grp = kt0 / GROUP;
-#pragma unroll
-            for (int u = 0; u < GROUP; ++u) {
-                const int kt = kt0 + u;
-                step(f0, f1, kt, 1, false, 0, false, u, -1, -1);
-                publish();
-                step(f1, f0, kt + 1, 0, true, kt + NSTAGE, true, 0, u == 0 ? grp + 1 : -1, u == GROUP - 1 ? grp + 1 : -1);
-            }
         }
     } else if constexpr (FP4) {
         // a stage is two steps: the second step's operands load under the first step's instructions, and the
@@ -534,16 +538,16 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
         }
 }
 
-template <int FMT, int FMTB, typename OutT, bool WIDE, bool PK, bool PAIR, bool EDGE>
+template <int FMT, int FMTB, typename OutT, bool WIDE, bool WORDS, bool PK, bool PAIR, bool EDGE, bool HALF>
 struct GemmLds {
     static inline const bool registered =
-        mpsa_register_lds_kernel(reinterpret_cast<const void*>(gemm_mx_kernel<FMT, FMTB, OutT, WIDE, PK, PAIR, EDGE>), smem_bytes<WIDE>());
+        mpsa_register_lds_kernel(reinterpret_cast<const void*>(gemm_mx_kernel<FMT, FMTB, OutT, WIDE, WORDS, PK, PAIR, EDGE, HALF>), smem_bytes<WIDE>());
 };
 
-template <int FMT, int FMTB, typename OutT, bool WIDE, bool PK, bool PAIR, bool EDGE>
+template <int FMT, int FMTB, typename OutT, bool WIDE, bool WORDS, bool PK, bool PAIR, bool EDGE, bool HALF = false>
 void launch_kernel(const GemmArgs& g, dim3 grid, hipStream_t st) {
-    if (!GemmLds<FMT, FMTB, OutT, WIDE, PK, PAIR, EDGE>::registered) return;
-    hipLaunchKernelGGL((gemm_mx_kernel<FMT, FMTB, OutT, WIDE, PK, PAIR, EDGE>), grid, dim3(256), smem_bytes<WIDE>(), st, g);
+    if (!GemmLds<FMT, FMTB, OutT, WIDE, WORDS, PK, PAIR, EDGE, HALF>::registered) return;
+    hipLaunchKernelGGL((gemm_mx_kernel<FMT, FMTB, OutT, WIDE, WORDS, PK, PAIR, EDGE, HALF>), grid, dim3(256), smem_bytes<WIDE>(), st, g);
 }
 
 
