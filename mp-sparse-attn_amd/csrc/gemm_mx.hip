@@ -283,12 +283,14 @@ void launch_fmt(const GemmArgs& g, int c_dtype, dim3 grid, hipStream_t st) {
 static bool known_fmt(int f) { return f == MPSA_FMT_E2M1 || f == MPSA_FMT_E4M3 || f == MPSA_FMT_E5M2; }
 
 // The kernel of a product: what the caller named (MPSA_GEMM_*), if it takes the shape, or the one with the least estimated time
-// (microseconds, fitted to measurements at 130 shapes and three types from 1 x 1024 x 4096 to 8192^3; the choice costs 1 % over
-// always taking the fastest).  A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started
+// (microseconds, fitted to measurements of every kernel at 820 shapes in three types, M from 1 to 8192, N from 100 to 16384, K from
+// 256 to 14336, weights not all in the cache; the choice costs 1.2 % over always taking the fastest, an earlier fit to 130 shapes
+// cost 4 %, and up to 2.2 times the time where M, N and K are all large: 4140 x 12160 x 10240, 8-bit x 4-bit, 930 us on the general
+// kernel, 424 on 256 x 256 tiles.  4-bit products with K % 256 == 128: 4096 x 4096 x 4224 69 us on 128-wide tiles, 43 on 256-wide).  A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started
 // round of 256 tiles counts whole, at a clock that falls as the chip fills, and every million outputs some.  The general kernel
 // shares a CU between up to three tiles and has no rounds: it is the fastest a few tiles past a whole number of them, and where K
-// is short.  The lines fall near M = 256 (4096-wide layer, K = 4096), where a 128-wide tile takes over from the 16-row blocks,
-// and near 2000 rows, where 256-wide tiles fill the chip.
+// is short; with long K it falls behind, as its tiles pass the L2 by.  The lines fall near M = 256 (4096-wide layer, K = 4096), where
+// a 128-wide tile takes over from the 16-row blocks, and near 2000 rows, where 256-wide tiles fill the chip.
 static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b) {
     const double M = g.M, N = g.N, K = g.K;
     const bool mixed = fmt_a != MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1;
@@ -314,10 +316,10 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
     }
     if (g.K % 128 || force_general()) return MPSA_GEMM_GENERAL;
     struct Ring { double start, round, per_1024, empty, out; };              // empty: share of per_1024 at an empty chip
-    static const Ring RING[2][3] = {{{1.5, 3.8, 3.26, 0.72, 0.26}, {2.5, 3.0, 3.85, 0.79, 0.32}, {1.8, 3.2, 4.65, 0.70, 0.41}},
-                                    {{6.3, 0.0, 4.38, 1.40, 1.44}, {4.0, 6.4, 15.3, 0.59, 0.0}, {2.5, 9.0, 14.9, 0.59, 0.05}}};
-    struct Shared { double start, tile, least, base, per_1024; };            // tile, per_1024: for 256 tiles
-    static const Shared SHARED[3] = {{2.7, 1.6, 7.2, 3.8, 4.2}, {2.2, 2.75, 9.1, 6.7, 3.3}, {2.4, 1.8, 10.0, 4.8, 6.7}};
+    static const Ring RING[2][3] = {{{1.41, 3.49, 3.12, 0.79, 0.226}, {1.89, 3.23, 3.93, 0.724, 0.231}, {1.73, 3.16, 4.59, 0.755, 0.275}},
+                                    {{4.6, 3.19, 8.14, 0.66, 0.249}, {4.16, 4.59, 12.3, 0.618, 0.238}, {4.39, 3.93, 12.9, 0.681, 0.304}}};
+    struct Shared { double start, tile, least, base, per_1024, deep; };      // tile, per_1024: for 256 tiles; deep: more of it at K = 8192
+    static const Shared SHARED[3] = {{2.91, 1.12, 4.98, 3.26, 3.73, 0.122}, {3.13, 1.12, 6.61, 3.35, 4.55, 0.222}, {2.73, 1.49, 7.41, 3.39, 5.52, 0.074}};
     auto tiles = [&](int edge) { return (double)((g.M + edge - 1) / edge) * (double)((g.N + edge - 1) / edge) * (double)batches; };
     auto ring = [&](int which, int edge) {
         const Ring& r = RING[which][kind];
@@ -325,7 +327,7 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
         return r.start + rounds * (r.round + r.per_1024 * clock * K / 1024.0) + r.out * 1e-6 * M * N * (double)batches;
     };
     const Shared& sh = SHARED[kind];
-    const double load = tiles(128) / 256.0, slope = sh.base + sh.per_1024 * load;
+    const double load = tiles(128) / 256.0, slope = sh.base + sh.per_1024 * load * (1.0 + sh.deep * (K < 8192.0 ? K / 8192.0 : 1.0));
     const double general = sh.start + sh.tile * load + K / 1024.0 * (slope > sh.least ? slope : sh.least);
     const double cost16 = gemm_split_cost(g, batches, fmt_a, fmt_b, &tile), cost128 = ring(0, 128), cost256 = staged || half ? ring(1, 256) : 1e300;
     const double least = fmin(fmin(cost16, cost128), cost256);

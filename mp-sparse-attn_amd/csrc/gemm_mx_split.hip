@@ -283,25 +283,51 @@ void launch_b(const GemmArgs& g, int64_t batches, int tile, int fmt_b, int c_dty
 
 }  // namespace
 
-// Estimated microseconds of a product on this kernel with its best tile: 14.5 ns per KiB that a workgroup brings into LDS and
-// a fixed part that grows with the tile (adding up the waves' sums).  Fewer workgroups than CUs gain nothing from a larger
-// tile; beyond that the total falls as tiles grow.
+// Workgroups of a tile that share a CU: its LDS holds so many.
+template <bool A4, bool B4, int MB, int NB>
+constexpr int places_of() {
+    constexpr int c = config(MB, NB, A4, B4);
+    return 163840 / SplitGeom<A4 ? MPSA_FMT_E2M1 : MPSA_FMT_E4M3, B4 ? MPSA_FMT_E2M1 : MPSA_FMT_E4M3, MB, NB, c / 10, c % 10>::SMEM;
+}
+template <bool A4, bool B4>
+int places_of(int tile) {
+    switch (tile) {
+        case 11: return places_of<A4, B4, 1, 1>();
+        case 12: return places_of<A4, B4, 1, 2>();
+        case 14: return places_of<A4, B4, 1, 4>();
+        case 22: return places_of<A4, B4, 2, 2>();
+        case 24: return places_of<A4, B4, 2, 4>();
+        default: return places_of<A4, B4, 4, 4>();
+    }
+}
+
+// Estimated microseconds of a product on this kernel with its best tile, fitted to the measurements that choose() in gemm_mx.hip
+// names.  A workgroup costs by its blocks (adding up the waves' sums), its rows, and its rows times K (what it brings into LDS);
+// workgroups on one CU take longer than one, by less than their number; and where there are more of them than places, whole
+// rounds count for most of it (1.04 of the time of the fastest tile, without the rounds 1.1).
 double gemm_split_cost(const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b, int* tile) {
-    const int tiles[] = {11, 12, 14, 22, 24, 44};
-    double best = 0.0, cost = 0.0;
-    for (int t : tiles) {
+    const bool a4 = fmt_a == MPSA_FMT_E2M1, b4 = fmt_b == MPSA_FMT_E2M1;
+    struct Fit { double start, block, piece, row, power, busy, rounds; };
+    static const Fit FIT[3] = {{2.05, 0.029, 0.194, 0.334, 0.598, 0.79, 0.692}, {2.0, 0.087, 0.177, 0.22, 0.714, 0.569, 0.803}, {2.03, 0.085, 0.175, 0.157, 0.591, 0.69, 0.702}};
+    const Fit& f = FIT[a4 && b4 ? 0 : a4 || b4 ? 1 : 2];
+    double best = 0.0;
+    for (int t : {11, 12, 14, 22, 24, 44}) {
         const int mb = t / 10, nb = t % 10;
-        const double wgs = (double)((g.M + 16 * mb - 1) / (16 * mb)) * ((g.N + 16 * nb - 1) / (16 * nb)) * (double)batches;
-        const double row = mb * (fmt_a == MPSA_FMT_E2M1 ? 0.5 : 1.0) + nb * (fmt_b == MPSA_FMT_E2M1 ? 0.5 : 1.0);
-        const double rank = (0.4 + 0.2 * mb * nb + 0.0145 * 16.0 * row * g.K / 1024.0) * (wgs > 256.0 ? wgs / 256.0 : 1.0);
-        if (best == 0.0 || rank < best) {
-            best = rank;
+        const int places = a4 ? (b4 ? places_of<true, true>(t) : places_of<true, false>(t)) : b4 ? places_of<false, true>(t) : places_of<false, false>(t);
+        const double w = (double)((g.M + 16 * mb - 1) / (16 * mb)) * ((g.N + 16 * nb - 1) / (16 * nb)) * (double)batches / 256.0;      // workgroups per CU
+        const double row = mb * (a4 ? 0.5 : 1.0) + nb * (b4 ? 0.5 : 1.0);
+        double load = w > 1.0 ? pow(w, f.power) : 1.0;
+        if (w > places) {
+            const double full = floor(w / places), rest = w - full * places;
+            load += f.rounds * (full * pow(places, f.power) + (rest <= 0.0 ? 0.0 : rest > 1.0 ? pow(rest, f.power) : 1.0) - load);
+        }
+        const double cost = f.start + (f.block * mb * nb + f.piece * row * g.K / 1024.0 + f.row * row) * load * (1.0 + f.busy * (w < 1.0 ? w : 1.0));
+        if (best == 0.0 || cost < best) {
+            best = cost;
             *tile = t;
-            // against the other kernels: what it takes with the chip's load (within 14 %)
-            cost = 2.0 + (0.05 * mb * nb + 0.06 * row * g.K / 1024.0) * pow(wgs > 256.0 ? wgs / 256.0 : 1.0, 0.95) * (1.0 + 5.3 * (wgs < 256.0 ? wgs / 256.0 : 1.0));
         }
     }
-    return cost;
+    return best;
 }
 
 void gemm_split_launch(const GemmArgs& g, int64_t batches, int tile, int fmt_a, int fmt_b, int c_dtype, hipStream_t st) {
