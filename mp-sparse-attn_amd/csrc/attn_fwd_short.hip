@@ -507,6 +507,7 @@ int launch_fmt(const AttnArgs& a, int splits, hipStream_t st) {
 }  // namespace
 
 int attn_short_launch(const AttnArgs& a, int pv_dtype, int splits, hipStream_t st) {
+    if (splits == 1 && attn_resident_takes(a)) return attn_resident_launch(a, pv_dtype, st);
     if (a.d == 128) return pv_dtype == MPSA_BF16 ? launch_fmt<128, MPSA_BF16>(a, splits, st) : launch_fmt<128, MPSA_F16>(a, splits, st);
     return pv_dtype == MPSA_BF16 ? launch_fmt<64, MPSA_BF16>(a, splits, st) : launch_fmt<64, MPSA_F16>(a, splits, st);
 }

@@ -990,3 +990,24 @@ def test_mean_inside_the_preparation_gives_the_bits_of_the_mean_on_its_own(B, Hk
     want = torch.empty_like(got)
     attention_from_operands(ops, bhnd(want), False, kernel="short1")
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("mode,Nk", [("mxfp8", n) for n in (1, 31, 32, 77, 333, 352, 353)] + [("mixed", n) for n in (33, 300, 447, 448, 449)] + [("mxfp8e5", 100), ("mixed_e5", 64)])
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,dtype,layout,climb", [(2, 16, 16, 4100, torch.bfloat16, "NHD", False), (1, 12, 4, 11001, torch.float16, "HND", True)])
+def test_many_queries_over_the_keys_of_one_head_in_lds(B, Hq, Hkv, Nq, dtype, layout, climb, mode, Nk):
+    """From 4096 blocks of 32 queries on, as many keys as fit, 8-bit Q: the bits of the kernel that streams the keys (which
+    quantized Q takes), with ragged last blocks on both sides and scores that move the running maximum."""
+    from ours.mxfp_attn_kernel import attention_from_operands, mxfp_attn_kernel, prepare_operands
+    g = torch.Generator(device=DEV).manual_seed(Nk)
+    q, k, v = (torch.randn(B, H, N, 128, generator=g, device=DEV, dtype=torch.float32) for H, N in ((Hq, Nq), (Hkv, Nk), (Hkv, Nk)))
+    if climb:                                             # scores that rise along the keys, for some of the queries
+        k += torch.arange(Nk, device=DEV)[:, None] * (8.0 / Nk)
+        q[:, :, ::3] = q[:, :, ::3].abs() * 4.0
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    if layout == "NHD":
+        q, k, v = (t.transpose(1, 2).contiguous() for t in (q, k, v))
+    bhnd = (lambda t: t) if layout == "HND" else (lambda t: t.transpose(1, 2))
+    got = mxfp_attn_kernel(q, k, v, tensor_layout=layout, output_dtype=dtype, block_scale_type=mode, kernel="short1")
+    want = torch.empty_like(got)
+    attention_from_operands(prepare_operands(bhnd(q), bhnd(k), bhnd(v), 128, mode), bhnd(want), False, kernel="short1")
+    assert torch.isfinite(got).all() and torch.equal(got, want)
