@@ -4,6 +4,9 @@
 // 23 us for a 16-row linear layer (a quantization and a product) whose kernels take 7.  Here a call checks the usual case,
 // allocates and launches; it returns None for anything unusual -- another device current, a layout that needs a copy, a shape
 // or type that is an error -- and the caller goes on with its own code, which copies or says what is wrong.
+// (Operand checks here instead of in Python and one layer of calls less: a 160-token prompt 11.3 -> 10.8 us, a 16-row linear layer
+// 14.0 -> 13.5, of which 7 are the two launches.)
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 #include <ATen/ATen.h>
 #include <hip/hip_runtime_api.h>
@@ -14,6 +17,9 @@ namespace py = pybind11;
 using at::Tensor;
 
 namespace {
+
+// Operands come as they are: one that is no tensor is the caller's to refuse.  (No second reference to a tensor is taken either.)
+const Tensor* tensor(py::handle x) { return THPVariable_Check(x.ptr()) ? &THPVariable_Unpack(x.ptr()) : nullptr; }
 
 // on the device that is current
 bool here(const Tensor& t) {
@@ -43,7 +49,10 @@ struct Unlocked {
 
 mpsa_stream_t stream_of(int64_t s) { return reinterpret_cast<mpsa_stream_t>(s); }
 
-py::object quantize(const Tensor& x, double pre, int fmt, int emax, std::optional<int64_t> rows, bool code_per_byte, bool scales_5d, int64_t stream) {
+py::object quantize(py::handle arg, double pre, int fmt, int emax, std::optional<int64_t> rows, bool code_per_byte, bool scales_5d, int64_t stream) {
+    const Tensor* const given = tensor(arg);
+    if (!given) return py::none();
+    const Tensor& x = *given;
     if (x.dim() != 4 || !here(x) || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf)) return py::none();
     const auto s = x.strides();
     if (s[3] != 1 || ((s[0] | s[1] | s[2]) & 7) || !aligned16(x)) return py::none();
@@ -135,8 +144,11 @@ bool operand(const Tensor& t, const Tensor& scale, at::IntArrayRef lead, int64_t
     return scale.size(n) == rows && scale.size(n + 1) == K / 32;
 }
 
-py::object matmul(const Tensor& a, const Tensor& sa, int fmt_a, const Tensor& b, const Tensor& sb, int fmt_b, at::ScalarType dtype,
+py::object matmul(py::handle arg_a, py::handle arg_sa, int fmt_a, py::handle arg_b, py::handle arg_sb, int fmt_b, at::ScalarType dtype,
                   int64_t M, int64_t N, int64_t K, int64_t stream) {
+    const Tensor* const given[4] = {tensor(arg_a), tensor(arg_sa), tensor(arg_b), tensor(arg_sb)};
+    if (!given[0] || !given[1] || !given[2] || !given[3]) return py::none();
+    const Tensor &a = *given[0], &sa = *given[1], &b = *given[2], &sb = *given[3];
     const bool packed = sa.dim() == 5 && sb.dim() == 5;
     if (!here(a) || dtype_id(dtype) < 0 || M <= 0 || N <= 0 || K <= 0 || !operand(a, sa, {}, M, K, fmt_a, packed, a.get_device()) ||
         !operand(b, sb, {}, N, K, fmt_b, packed, a.get_device()))

@@ -43,11 +43,11 @@ def make_configs(block_scale_type="mxfp4", fmt8=None):
 
 def _fmts_of(configs):
     """(fmt_a, fmt_b) of a configs dict."""
-    f8 = _lib.FMT_E4M3 if configs.get("FMT8", "e4m3") == "e4m3" else _lib.FMT_E5M2
-    pick = lambda epb: _lib.FMT_E2M1 if epb == 2 else f8
-    if configs["ELEM_PER_BYTE_A"] not in (1, 2) or configs["ELEM_PER_BYTE_B"] not in (1, 2):
+    epb_a, epb_b = configs["ELEM_PER_BYTE_A"], configs["ELEM_PER_BYTE_B"]
+    if epb_a not in (1, 2) or epb_b not in (1, 2):
         raise ValueError("ELEM_PER_BYTE_A / ELEM_PER_BYTE_B must be 1 or 2")
-    return pick(configs["ELEM_PER_BYTE_A"]), pick(configs["ELEM_PER_BYTE_B"])
+    f8 = _lib.FMT_E4M3 if configs.get("FMT8", "e4m3") == "e4m3" else _lib.FMT_E5M2
+    return _lib.FMT_E2M1 if epb_a == 2 else f8, _lib.FMT_E2M1 if epb_b == 2 else f8
 
 
 def _gemm_kernel_id(kernel):
@@ -95,12 +95,12 @@ def block_scaled_matmul(a, a_scale, b, b_scale, dtype_dst, M, N, K, configs):
     if dtype_dst not in (torch.float32, torch.float16, torch.bfloat16, torch.float8_e5m2):
         raise ValueError(f"Unsupported dtype: {dtype_dst}")
     fmt_a, fmt_b = _fmts_of(configs)
-    _lib.require_device(a, a_scale, b, b_scale)
     kernel = configs.get("KERNEL")
-    if kernel is None:
+    if kernel is None and isinstance(a, torch.Tensor) and a.is_cuda:
         done = _lib.host().matmul(a, a_scale, fmt_a, b, b_scale, fmt_b, dtype_dst, M, N, K, _lib.raw_stream(a))
         if done is not None:
             return done
+    _lib.require_device(a, a_scale, b, b_scale)
     # the reference's packed scale layout goes to the kernel as it is when both operands come that way
     packed = a_scale.dim() == 5 and b_scale.dim() == 5
     if not packed:

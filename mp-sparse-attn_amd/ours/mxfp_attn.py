@@ -14,7 +14,7 @@ block-scaled matmul kernel and compare the scores with the fake-quant product of
 import torch
 
 from . import _lib
-from .mxfp_attn_kernel import mxfp_attn_kernel, initialize_block_scaled_batched_from_tensor, _normalise
+from .mxfp_attn_kernel import _attention, mxfp_attn_kernel, initialize_block_scaled_batched_from_tensor, _normalise
 from .quant_mxint8 import quantize_mx, pre_scale_q, seq_mean, _as_bhnd
 
 
@@ -77,5 +77,5 @@ def mxfp_attn(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False, scale=Non
         _lib.require_device(q, k, v)
         qn, kn, _ = _normalise(q, k, v)
         check_scores_against_reference(_as_bhnd(qn, tensor_layout), _as_bhnd(kn, tensor_layout), block_scale_type, scale, smooth_k)
-    return mxfp_attn_kernel(q, k, v, attn_mask, dropout_p, is_causal, scale, smooth_k, attention_sink, tensor_layout, output_dtype,
-                            return_sparsity, block_scale_type, skip_thresh, BLKQ, route_thresh, kernel)
+    return _attention(q, k, v, attn_mask, dropout_p, is_causal, scale, smooth_k, attention_sink, tensor_layout, output_dtype,
+                      return_sparsity, block_scale_type, skip_thresh, BLKQ, route_thresh, kernel)

@@ -306,6 +306,8 @@ def _normalise(q, k, v):
     """Reference prologue (ours/mxfp_attn_kernel.py:27-31): fp32/fp16 inputs run in fp16, everything else in
     bf16.  V follows Q/K's 16-bit dtype here (the reference always used fp16 for V)."""
     lp = torch.float16 if q.dtype in (torch.float32, torch.float16) else torch.bfloat16
+    if q.dtype is k.dtype is v.dtype is lp:
+        return q, k, v
     return tuple(t if t.dtype is lp else t.to(lp) for t in (q, k, v))
 
 
@@ -395,6 +397,14 @@ def mxfp_attn_kernel(q, k, v, attn_mask=None, dropout_p=0.0,
     whole call; one that does not take the shape raises.  Kernels differ in the order of their sums, and so in the last bits:
     with ``"auto"`` a sequence's result can depend on how many others are in the batch, with ``"sequence"`` (the one that is
     the fastest for a sequence alone) or any other name it does not."""
+    return _attention(q, k, v, attn_mask, dropout_p, is_causal, scale, smooth_k, attention_sink, tensor_layout, output_dtype,
+                      return_sparsity, block_scale_type, skip_thresh, tile, route_thresh, kernel)
+
+
+def _attention(q, k, v, attn_mask, dropout_p, is_causal, scale, smooth_k, attention_sink, tensor_layout, output_dtype, return_sparsity,
+               block_scale_type, skip_thresh, tile, route_thresh, kernel):
+    """:func:`mxfp_attn_kernel` for callers that the graph compiler leaves out already: every layer of that costs a short call most
+    of a microsecond."""
     _lib.require_device(q, k, v)
     _reject_unsupported(attn_mask, dropout_p, attention_sink)
     device = v.device
@@ -408,8 +418,8 @@ def mxfp_attn_kernel(q, k, v, attn_mask=None, dropout_p=0.0,
                  None if skip_thresh is None else float(skip_thresh), tile, None if route_thresh is None else float(route_thresh),
                  kernel)
     if plan is None:                     # some row is not contiguous or not 16-byte aligned
-        return mxfp_attn_kernel(_aligned(q), _aligned(k), _aligned(v), None, 0.0, is_causal, scale, smooth_k, False, tensor_layout,
-                                output_dtype, return_sparsity, block_scale_type, skip_thresh, tile, route_thresh, kernel)
+        return _attention(_aligned(q), _aligned(k), _aligned(v), None, 0.0, is_causal, scale, smooth_k, False, tensor_layout,
+                          output_dtype, return_sparsity, block_scale_type, skip_thresh, tile, route_thresh, kernel)
     desc, nbytes, out_shape, leaves_out, address, named = plan
     if not return_sparsity:
         out = _lib.host().attention(named, address, nbytes, out_shape, output_dtype, q, k, v, _lib.raw_stream(q))

@@ -88,8 +88,7 @@ def _quantize_as(x, pre_scale, fmt, emax_elem=None, out_rows=None, sub=None, cod
     layout (L and D multiples of 128), if asked for: ``mpsa_quantize_mx_as``."""
     if emax_elem is None:
         emax_elem = EMAX_E2M1 if fmt == _lib.FMT_E2M1 else EMAX_8BIT
-    _lib.require_device(x)
-    if sub is None:
+    if sub is None and isinstance(x, torch.Tensor) and x.is_cuda:
         done = _lib.host().quantize(x, pre_scale, fmt, emax_elem, None if out_rows is None else int(out_rows), code_per_byte, scales_5d, _lib.raw_stream(x))
         if done is not None:
             return done
