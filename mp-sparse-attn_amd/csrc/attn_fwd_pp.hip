@@ -191,13 +191,14 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
             }
             if constexpr (WANT8) {
                 odd = fp8_odd(ex, se8);
-                again |= odd;
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     const uint2 y = fp8_convert8<FMT8>(x[c], se8);
                     w8[2 * c] = (int)y.x;
                     w8[2 * c + 1] = (int)y.y;
+                    odd |= fp8_past<FMT8>(y);
                 }
+                again |= odd;
             }
             if (again && !zero) {
 #pragma unroll

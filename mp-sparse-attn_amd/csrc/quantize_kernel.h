@@ -93,8 +93,8 @@ __device__ __forceinline__ float round16(float v) {
 // 128 * 2^-26), and the conversion is the result.  That is one shift-and-add an element and half a minimum; converting
 // the inputs twice, nudged down and up by 2^-17 of themselves, which this replaces, took two products and half a conversion.
 // With the scaled FP8 conversion below (a shift and a clamp an element less) and, in the paired-tile kernel, all of a lane's
-// loads in front: 32/8 heads, 8192 tokens, diag, 336.7 -> 334.5 us a call (kernels alone 359 -> 352); 8 heads of 1024 x 64
-// 15.3 -> 15.1; 2 x 24 heads, 8000 queries over 200 keys 68.4 -> 66.9.
+// loads in front: 32/8 heads, 8192 tokens, diag, 356.2 -> 354.5 us a call; before fp8_past, 8 heads of 1024 x 64 15.3 -> 15.1
+// and 2 x 24 heads, 8000 queries over 200 keys 68.4 -> 66.9.
 // The pattern is that of the E2M1 values and of zero as well; so a lane that finds it converts the nudged inputs, and if
 // they differ (a rounding boundary lies between) it takes the explicit rule.  (2^-17 of a value near a midpoint - the
 // smallest is 0.25 - is at least 1.9e-6.)  Small scales, where x may be subnormal, take the explicit rule as well.
@@ -157,8 +157,9 @@ __device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool
     return w;
 }
 
-// Eight FP8 codes of x[0..7] / 2^se.  The scaled conversion divides and rounds in one instruction a pair; a finite block's
-// values lie below 256 then and never meet the format's maximum.
+// Eight FP8 codes of x[0..7] / 2^se.  The scaled conversion divides and rounds in one instruction a pair.  With the formats' own
+// emax (7) a finite block's values lie below 256 and never meet the format's maximum; what does -- a NaN, or a larger value
+// under another emax -- shows in the codes (fp8_past).
 template <int FMT8>
 __device__ __forceinline__ uint2 fp8_convert8(const float (&x)[8], int se) {
     typedef short v2s __attribute__((ext_vector_type(2)));
@@ -178,7 +179,15 @@ __device__ __forceinline__ uint2 fp8_convert8(const float (&x)[8], int se) {
     return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
 }
 
-// the same one step at a time, with the clamp to the format's maximum: a block with an infinity saturates there
+// Whether a code is the format's NaN or E5M2's infinity: three instructions a word, where clamping first takes one an element.
+template <int FMT8>
+__device__ __forceinline__ bool fp8_past(const uint2& w) {
+    constexpr uint32_t UP = FMT8 == MPSA_FMT_E4M3 ? 0x01010101u : 0x04040404u;       // the first such code to 0x80
+    return ((((w.x & 0x7F7F7F7Fu) + UP) | ((w.y & 0x7F7F7F7Fu) + UP)) & 0x80808080u) != 0u;
+}
+
+// the same one step at a time, with the clamp to the format's maximum: infinities and larger values saturate there, a NaN at
+// its negative
 template <int FMT8, bool SW8>
 __device__ __forceinline__ uint2 fp8_careful8(const float (&x)[8], int se) {
     const float lim = (FMT8 == MPSA_FMT_E4M3) ? 448.0f : 57344.0f;
@@ -188,8 +197,9 @@ __device__ __forceinline__ uint2 fp8_careful8(const float (&x)[8], int se) {
     return make_uint2(fp8_pack4<FMT8, SW8>(y[0], y[1], y[2], y[3]), fp8_pack4<FMT8, SW8>(y[4], y[5], y[6], y[7]));
 }
 
-// whether a block of largest magnitude 2^e or more wants fp8_careful8
-__device__ __forceinline__ bool fp8_odd(int e, int se) { return e >= 128 || se < SMALLEST_SE; }
+// whether a block of largest magnitude 2^e or more wants fp8_careful8 whatever its codes: infinities, and scales that are no
+// normal float32
+__device__ __forceinline__ bool fp8_odd(int e, int se) { return e >= 128 || se < SMALLEST_SE || se > 127; }
 
 // floor(log2(amax)) of a block's largest magnitude, subnormals included; -1 for a block of zeros (whose codes and scale are
 // zero whatever it says)
@@ -232,7 +242,7 @@ __device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exa
             w8 = fp8_convert8<FMT8>(x, se);
             w8.x = zero ? 0u : w8.x;
             w8.y = zero ? 0u : w8.y;
-            again |= fp8_odd(e, se);
+            again |= fp8_odd(e, se) || fp8_past<FMT8>(w8);
         }
         s8 = zero ? 0 : min(max(se + 127, 0), 254);
     }
@@ -247,7 +257,7 @@ __device__ __forceinline__ void quantize_again(const float (&x)[8], int e, int e
         if (rule) w4 = SW8 ? e2m1_pack8_explicit(x, e - emax4) : e2m1_pack8_rule(x, e - emax4);
     }
     if constexpr (DO8) {
-        if (SW8 || fp8_odd(e, e - emax8)) w8 = fp8_careful8<FMT8, SW8>(x, e - emax8);
+        if (SW8 || fp8_odd(e, e - emax8) || fp8_past<FMT8>(w8)) w8 = fp8_careful8<FMT8, SW8>(x, e - emax8);
     }
 }
 

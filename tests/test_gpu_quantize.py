@@ -70,6 +70,31 @@ def test_near_tie_values_follow_the_biased_compare():
     assert mids.numel() == 7
 
 
+@pytest.mark.parametrize("emax", [7, 8, 20, -1])
+@pytest.mark.parametrize("fmt,lim,kind", [(O.FMT_E4M3, 448.0, torch.float8_e4m3fn), (O.FMT_E5M2, 57344.0, torch.float8_e5m2)])
+def test_8bit_codes_of_nan_infinity_and_values_past_the_maximum(fmt, lim, kind, emax):
+    """The clamp to +-maximum in front of the 8-bit rounding, exactly: a NaN leaves it as the negative maximum and counts as zero
+    in its block's largest magnitude, infinities and (under another emax) larger values saturate."""
+    g = torch.Generator().manual_seed(emax + 2)
+    x = torch.randn(1, 2, 96, 128, generator=g) * torch.exp2(torch.randint(-110, 126, (1, 2, 96, 4, 1), generator=g).expand(-1, -1, -1, -1, 32).reshape(1, 2, 96, 128).float())
+    odd = torch.tensor([float("nan"), float("inf"), -float("inf"), -0.0])[torch.randint(0, 4, x.shape, generator=g)]
+    x = torch.where(torch.rand(x.shape, generator=g) < 0.01, odd, x)
+    x[0, 0, :2] = float("nan")
+    x = x.to(torch.bfloat16)
+    pre = 0.1275174
+    y = (x.float() * pre).view(-1, 32)
+    amax = y.nan_to_num(0.0, float("inf"), -float("inf")).abs().amax(1)
+    e = torch.where(amax.isinf(), 128, torch.frexp(amax.nan_to_num(0.0, 1.0))[1] - 1)
+    se = e - emax
+    z = torch.ldexp(y.double(), -se[:, None].double())
+    want = torch.where(z.isnan(), -lim, z.clamp(-lim, lim)).float().to(kind).view(torch.uint8)
+    want[amax == 0] = 0
+    scales = torch.where(amax == 0, 0, (se + 127).clamp(0, 254)).to(torch.uint8)
+    codes, got = quantize_mx(x.to(DEV), pre, fmt, emax_elem=emax)
+    assert torch.equal(got.cpu().view(-1), scales)
+    assert torch.equal(codes.cpu().view(-1, 32), want)
+
+
 def test_dual_equals_single_and_padding_rows_are_zero():
     q, _, _ = make_qkv(1, 4, 4, 200, 128, seed=4)
     pre = O.q_pre_scale(128)
