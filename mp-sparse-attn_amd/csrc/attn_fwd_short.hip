@@ -15,7 +15,7 @@
 // Q may arrive unquantized (a.q_raw): the workgroup quantizes its rows into LDS, eight elements per lane, with the quantizer's
 // own code -- the bits of mpsa_quantize_mx.
 // With 32 heads, 8 KV heads, causal, D = 128 (us of this kernel in a kernel trace; tile kernels): 160 tokens 6.8 (12.8), 1000
-// tokens 17 (25).  2 x 16 heads, 4096 queries over 333 keys: 34 with Q's quantization (47).
+// tokens 17 (25).  Many queries over keys that fit LDS go on to attn_fwd_resident.hip.
 #include "attn_common.h"
 #include "quantize_kernel.h"
 #include "reciprocal.h"

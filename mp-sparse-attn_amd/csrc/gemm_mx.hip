@@ -284,9 +284,9 @@ static bool known_fmt(int f) { return f == MPSA_FMT_E2M1 || f == MPSA_FMT_E4M3 |
 
 // The kernel of a product: what the caller named (MPSA_GEMM_*), if it takes the shape, or the one with the least estimated time
 // (microseconds, fitted to measurements of every kernel at 820 shapes in three types, M from 1 to 8192, N from 100 to 16384, K from
-// 256 to 14336, weights not all in the cache; the choice costs 1.2 % over always taking the fastest, an earlier fit to 130 shapes
-// cost 4 %, and up to 2.2 times the time where M, N and K are all large: 4140 x 12160 x 10240, 8-bit x 4-bit, 930 us on the general
-// kernel, 424 on 256 x 256 tiles.  4-bit products with K % 256 == 128: 4096 x 4096 x 4224 69 us on 128-wide tiles, 43 on 256-wide).  A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started
+// 256 to 14336, weights not all in the cache; the choice costs 1.1 % over always taking the fastest, an earlier fit to 130 shapes
+// cost 4 %, and up to 2.2 times the time where M, N and K are all large: 4140 x 12160 x 10240, 8-bit x 4-bit, 980 us on the general
+// kernel, 427 on 256 x 256 tiles.  4-bit products with K % 256 == 128: 4096 x 4096 x 4224 69 us on 128-wide tiles, 43 on 256-wide).  A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started
 // round of 256 tiles counts whole, at a clock that falls as the chip fills, and every million outputs some.  The general kernel
 // shares a CU between up to three tiles and has no rounds: it is the fastest a few tiles past a whole number of them, and where K
 // is short; with long K it falls behind, as its tiles pass the L2 by.  The lines fall near M = 256 (4096-wide layer, K = 4096), where

@@ -9,8 +9,9 @@
 // at the end, one half of the quarter each.
 // Scale bytes: four words a row at a time (two units of 4-bit codes, four of 8-bit ones), 16 rows per load instruction;
 // fetching a word per row and unit, one lane per line, took longer than the codes.
-// Measured (bf16 output): 1000 x 4096 x 4096 34 -> 18.5 us 4-bit, 43 -> 24 us 8-bit x 4-bit against the general kernel of
-// gemm_mx.hip; 2048^3 18 -> 12 us and 24 -> 14.6 us against 256 x 256 tiles, of which that has 64.  Clock stamps in a copy of this
+// Measured (bf16 output, which leaves through LDS in pieces of 16 bytes): 1000 x 4096 x 4096 16.1 us 4-bit, 20.8 8-bit x 4-bit, 22.9
+// 8-bit (18.5 and 24 the first two when a lane stored its own elements); 2048^3 11.2, 13.1 and 13.9.  Reading the next unit's operands into
+// a second set of registers while one is multiplied takes 1 to 11 % longer.  Clock stamps in a copy of this
 // kernel, 1000 x 4096 x 4096: a unit takes 1390 clocks with 4-bit codes (512 of matrix work), 980 with 8-bit x 4-bit ones and
 // 1060 with 8-bit ones (half a unit's K, 512); prologue and first unit 5000, adding up and storing 5700.
 #include "gemm_mx_args.h"
