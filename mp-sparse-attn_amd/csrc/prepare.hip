@@ -126,12 +126,16 @@ void launch_mode(const PrepArgs& p, bool do4, bool do8, int fmt8, int tile, int 
 // of a call's kernels with the mean on its own, from sums, from rows (pieces in millions): 8 heads, 512 x 128, 16.6 15.4 12.9
 // (1.0); 8 of 1024 x 64 16.9 15.7 14.7 (1.0); 2 x 16 of 333 x 128, 4096 queries, 46.4 44.1 40.6 (1.8); 2 x 32 of 512 x 64 22.5
 // 21.0 20.8 (2.1); 4 x 32 of 512 x 64 27.4 25.2 30.0 (4.2); 2 x 24 of 512 x 128, 4096 queries, 61.4 59.7 61.3 (6.3).  Sums up to
-// 64 chunks (32 heads, 4096 x 64, 86.4 -> 84.8; 8 of 16384 x 64 249.4 -> 249.0), beyond that there is nothing to gain.
+// 64 chunks (32 heads, 4096 x 64, 86.4 -> 84.8) and where the workgroups together read 14 MB of them at most: every one of a head
+// reads them all, which is quadratic in the keys.  A mean of its own against sums, whole calls of 128 queries, us (MB): 8 heads
+// of 4096 x 128 36.6 35.2 (8.4), 6144 44.1 44.1 (19), 16384 88.9 94.9 (134); 40 of 2048 x 128 36.3 36.5 (10), 4096 55.3 57.7 (42),
+// 8656 116 129 (187); 24 of 8192 x 64 53.5 53.6 (25), 16000 92 97 (96).
 MeanSource mpsa_mean_source(int64_t B, int64_t Hkv, int64_t nk, int64_t D) {
     if (mpsa_quantize_sw_encoders()) return MEAN_GIVEN;      // stand-alone kernels
     const double pieces = (double)nk * (double)D / 8.0;
     if (pieces <= 8192.0 && (double)(B * Hkv) * pieces * pieces / 512.0 <= 2.2e6) return MEAN_ROWS_ITSELF;
-    return nk <= 64 * MEAN_ROWS ? MEAN_SUMS : MEAN_GIVEN;
+    const double read = (double)(B * Hkv) * (double)nk * (double)nk * (double)(D * D) / 262144.0;      // bytes of sums, all workgroups
+    return nk <= 64 * MEAN_ROWS && read <= 14e6 ? MEAN_SUMS : MEAN_GIVEN;
 }
 
 // Host side of the preparation: which of the operand sets are made is up to the caller (do4 / do8 of either side; the
