@@ -244,7 +244,8 @@ int mpsa_gemm_mx_batched_packed(const uint8_t* a, const uint8_t* sa5, int fmt_a,
  * The kernels behind the four entry points above.  mpsa_gemm_mx_on is all four in one (packed != 0: scales in the packed form;
  * batch = heads_a = heads_b = 1: the 2-D product) with the kernel named by the caller, for comparisons and measurements;
  * MPSA_GEMM_AUTO is what the others take.  A kernel that does not take the shape gives MPSA_EUNSUPPORTED.
- * mpsa_gemm_kernel says which kernel a call takes (MPSA_GEMM_SPLIT resolved to its tile), or why it would be refused.  (With
+ * mpsa_gemm_kernel says which kernel a call takes (MPSA_GEMM_SPLIT resolved to its tile), in either scale layout, or why it would
+ * be refused; a kernel that it answers can be named.  (With
  * MPSA_GEMM_AUTO a product with K == 128 and 16-bit results in rows that start on 16 bytes runs on a kernel of its own, which
  * gives the bits of MPSA_GEMM_GENERAL.)
  */
@@ -253,7 +254,7 @@ int mpsa_gemm_mx_batched_packed(const uint8_t* a, const uint8_t* sa5, int fmt_a,
 #define MPSA_GEMM_SPLIT 2                                 /* K split between the waves, on the tile estimated to be the fastest: K % 128 == 0 */
 #define MPSA_GEMM_SPLIT_TILE(mb, nb) (10 * (mb) + (nb))   /* the same on tiles of mb x nb 16-row blocks: 1x1 1x2 1x4 2x2 2x4 4x4 */
 #define MPSA_GEMM_TILE128 3                               /* 128 x 128 tiles, ring of four, K split between two waves: K % 128 == 0 */
-#define MPSA_GEMM_TILE256 4                               /* 256 x 256 tiles: one format or 8-bit A with 4-bit B, K % 128 == 0 (256 for ragged 4-bit products) */
+#define MPSA_GEMM_TILE256 4                               /* 256 x 256 tiles: one format or 8-bit A with 4-bit B, K % 128 == 0 (ragged 4-bit products with K % 256 == 128: from 64 tiles on) */
 int mpsa_gemm_mx_on(int kernel, const uint8_t* a, const uint8_t* sa, int fmt_a, const uint8_t* b, const uint8_t* sb, int fmt_b, int packed,
                     int64_t batch, int64_t heads_a, int64_t heads_b, int64_t M, int64_t N, int64_t K,
                     void* c, int c_dtype, int64_t ldc, mpsa_stream_t stream);

@@ -249,25 +249,14 @@ bool force_general() {
     return on;
 }
 
-template <int FMT, int FMTB, typename OutT, bool PAIR>
-void launch_scales(const GemmArgs& g, dim3 grid, hipStream_t st) {
-    if (g.packed)               launch_kernel<FMT, FMTB, OutT, false, false, true, PAIR, false>(g, grid, st);
-    else if constexpr (PAIR) {
-        if (g.K % 512 == 0)     launch_kernel<FMT, FMTB, OutT, true, false, false, PAIR, false>(g, grid, st);
-        else                    launch_kernel<FMT, FMTB, OutT, true, true, false, PAIR, false>(g, grid, st);
-    }
-}
-
 template <int FMT, int FMTB, typename OutT>
 void launch_one(const GemmArgs& g, dim3 grid, hipStream_t st) {
-    // whole cache lines per row (two stages at a time) need an even number of stages: always so with 8-bit codes
-    // (K % 128 == 0), with 4-bit codes when K % 256 == 0
-    if constexpr (FMT != MPSA_FMT_E2M1) {
-        launch_scales<FMT, FMTB, OutT, true>(g, grid, st);
-    } else {
-        if (g.K % 256 == 0) launch_scales<FMT, FMTB, OutT, true>(g, grid, st);
-        else                launch_scales<FMT, FMTB, OutT, false>(g, grid, st);
+    if constexpr (FMT == MPSA_FMT_E2M1) {
+        if (g.K % 256) return launch_kernel<FMT, FMTB, OutT, false, true, false, true>(g, grid, st);      // packed scales
     }
+    if (g.packed)            launch_kernel<FMT, FMTB, OutT, false, true, false>(g, grid, st);
+    else if (g.K % 512 == 0) launch_kernel<FMT, FMTB, OutT, false, false, false>(g, grid, st);
+    else                     launch_kernel<FMT, FMTB, OutT, true, false, false>(g, grid, st);
 }
 
 template <int FMT, int FMTB>
@@ -295,8 +284,10 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
     const double M = g.M, N = g.N, K = g.K;
     const bool mixed = fmt_a != MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1;
     const int kind = fmt_a == MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1 ? 0 : mixed ? 1 : 2;
-    const bool staged = g.K % 128 == 0 && (fmt_a == fmt_b || mixed) && ((g.M % BM == 0 && g.N % BN == 0) || kind != 0 || g.K % 256 == 0);
-    const bool half = kind == 0 && g.K % 256 == 128 && !g.packed;        // ragged 4-bit products that end in half a unit: not by name
+    auto tiles = [&](int edge) { return (double)((g.M + edge - 1) / edge) * (double)((g.N + edge - 1) / edge) * (double)batches; };
+    // ragged 4-bit products that end in half a unit: from a quarter of the chip on (the estimates choose it from 140 tiles on)
+    const bool half = kind == 0 && g.K % 256 && (g.M % BM || g.N % BN);
+    const bool staged = g.K % 128 == 0 && (fmt_a == fmt_b || mixed) && (!half || tiles(256) >= 64.0);
     int tile = 0;
     switch (kernel) {
         case MPSA_GEMM_AUTO: break;
@@ -310,7 +301,7 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
             if (g.K % 128) return mpsa_fail(MPSA_EUNSUPPORTED, "gemm: this kernel needs K %% 128 == 0 (got %d)", g.K);
             return kernel;
         case MPSA_GEMM_TILE256:
-            if (!staged) return mpsa_fail(MPSA_EUNSUPPORTED, "gemm: the 256 x 256 kernel needs one format or 8-bit A with 4-bit B, and K %% 128 == 0 (256 for ragged 4-bit products)");
+            if (!staged) return mpsa_fail(MPSA_EUNSUPPORTED, "gemm: the 256 x 256 kernel needs one format or 8-bit A with 4-bit B, and K %% 128 == 0; ragged 4-bit products with K %% 256 == 128 also 64 tiles");
             return kernel;
         default: return mpsa_fail(MPSA_EINVAL, "gemm: unknown kernel %d", kernel);
     }
@@ -320,7 +311,6 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
                                     {{4.6, 3.19, 8.14, 0.66, 0.249}, {4.16, 4.59, 12.3, 0.618, 0.238}, {4.39, 3.93, 12.9, 0.681, 0.304}}};
     struct Shared { double start, tile, least, base, per_1024, deep; };      // tile, per_1024: for 256 tiles; deep: more of it at K = 8192
     static const Shared SHARED[3] = {{2.91, 1.12, 4.98, 3.26, 3.73, 0.122}, {3.13, 1.12, 6.61, 3.35, 4.55, 0.222}, {2.73, 1.49, 7.41, 3.39, 5.52, 0.074}};
-    auto tiles = [&](int edge) { return (double)((g.M + edge - 1) / edge) * (double)((g.N + edge - 1) / edge) * (double)batches; };
     auto ring = [&](int which, int edge) {
         const Ring& r = RING[which][kind];
         const double rounds = ceil(tiles(edge) / 256.0), clock = r.empty + (1.0 - r.empty) * tiles(edge) / (256.0 * rounds);
@@ -329,7 +319,7 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
     const Shared& sh = SHARED[kind];
     const double load = tiles(128) / 256.0, slope = sh.base + sh.per_1024 * load * (1.0 + sh.deep * (K < 8192.0 ? K / 8192.0 : 1.0));
     const double general = sh.start + sh.tile * load + K / 1024.0 * (slope > sh.least ? slope : sh.least);
-    const double cost16 = gemm_split_cost(g, batches, fmt_a, fmt_b, &tile), cost128 = ring(0, 128), cost256 = staged || half ? ring(1, 256) : 1e300;
+    const double cost16 = gemm_split_cost(g, batches, fmt_a, fmt_b, &tile), cost128 = ring(0, 128), cost256 = staged ? ring(1, 256) : 1e300;
     const double least = fmin(fmin(cost16, cost128), cost256);
     if (general < least) return MPSA_GEMM_GENERAL;
     return cost16 == least ? MPSA_GEMM_SPLIT_TILE(tile / 10, tile % 10) : cost128 == least ? MPSA_GEMM_TILE128 : MPSA_GEMM_TILE256;

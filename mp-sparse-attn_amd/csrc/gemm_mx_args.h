@@ -17,7 +17,8 @@ void gemm_split_launch(const GemmArgs& g, int64_t batches, int tile, int fmt_a, 
 // gemm_mx_tile.hip: 128 x 128 tiles, any M, N and pair of formats, K % 128 == 0
 void gemm_tile_launch(const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b, int c_dtype, hipStream_t st);
 
-// gemm_mx_edge.hip: 256 x 256 tiles with ragged edges; one format or 8-bit A against 4-bit B, K % 256 == 0 (4-bit A) / K % 128 == 0
+// gemm_mx_edge.hip: 256 x 256 tiles with ragged edges, or with 4-bit codes, K % 256 == 128 and row-major scales; one format or 8-bit A
+// against 4-bit B, K % 128 == 0
 void gemm_edge_launch(const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b, int c_dtype, hipStream_t st);
 // gemm_mx_stage.hip: products with one stage of K and 16-bit results
 bool gemm_stage_takes(const GemmArgs& g, int fmt_a, int fmt_b, int c_dtype);

@@ -1,14 +1,16 @@
-// The 256 x 256 kernel's instantiations for ragged M and N (gemm_mx_kernel.h).
+// The 256 x 256 kernel's instantiations for ragged M and N, and for 4-bit products with row-major scales that end in half a unit (gemm_mx_kernel.h).
 #include "gemm_mx_kernel.h"
 
 namespace {
 
 template <int FMT, int FMTB, typename OutT>
 void launch_scales(const GemmArgs& g, dim3 grid, hipStream_t st) {
-    if (g.packed)            launch_kernel<FMT, FMTB, OutT, false, false, true, true, true>(g, grid, st);
-    else if (g.K % 512 == 0) launch_kernel<FMT, FMTB, OutT, true, false, false, true, true>(g, grid, st);
-    else if (FMT != MPSA_FMT_E2M1 || g.K % 256 == 0) launch_kernel<FMT, FMTB, OutT, true, true, false, true, true>(g, grid, st);
-    else if constexpr (FMT == MPSA_FMT_E2M1)         launch_kernel<FMT, FMTB, OutT, true, true, false, true, true, true>(g, grid, st);
+    if constexpr (FMT == MPSA_FMT_E2M1) {
+        if (g.K % 256) return g.packed ? launch_kernel<FMT, FMTB, OutT, false, true, true, true>(g, grid, st) : launch_kernel<FMT, FMTB, OutT, true, false, true, true>(g, grid, st);
+    }
+    if (g.packed)            launch_kernel<FMT, FMTB, OutT, false, true, true>(g, grid, st);
+    else if (g.K % 512 == 0) launch_kernel<FMT, FMTB, OutT, false, false, true>(g, grid, st);
+    else                     launch_kernel<FMT, FMTB, OutT, true, false, true>(g, grid, st);
 }
 
 template <int FMT, int FMTB>

@@ -17,14 +17,15 @@
 // Staging.  Codes go HBM/L2 -> LDS with direct-to-LDS loads (no registers, no LDS-write instructions) into a
 // ring of four stages.  The vector memory path moves cache lines: a wave instruction that takes 64 bytes from each
 // of 16 rows uses half of every 128-byte line it touches and runs at half the rate of one that takes 128 bytes
-// from each of 8 rows (measured L2 -> LDS: 17 against 31 TB/s chip-wide).  So whenever the number of stages is
-// even (PAIR) the ring is refilled two stages -- one "unit" of 128 bytes per row -- at a time: the unit's LDS image
-// has a 128-byte row pitch, one workgroup barrier per unit, one unit in flight while the other is multiplied.
-// Runs with an odd number of stages (4-bit codes, K % 256 == 128) end in half a unit (HALF; they take the EDGE form, whose loads
-// have their rows apart from the place in a row); with packed scales they keep the stage-by-stage ring, three stages in
-// flight while one is multiplied.  Either way the 16-byte pieces of a row are XOR-swizzled with the row index so
-// that the 128-bit operand reads of 16 consecutive rows hit 16 distinct 4-bank groups, and wave tiles of
-// 128x128 keep LDS reads at 8 operand fragments per 16 matrix instructions.
+// from each of 8 rows (measured L2 -> LDS: 17 against 31 TB/s chip-wide).  So the ring is refilled two stages -- one "unit"
+// of 128 bytes per row -- at a time: the unit's LDS image has a 128-byte row pitch, one workgroup barrier per unit, one unit in
+// flight while the other is multiplied.
+// With an odd number of stages (ODD: 4-bit codes, K % 256 == 128) every other row starts in the middle of a line, and whole units
+// gain less.  With row-major scales such runs end in half a unit (HALF; they take the EDGE form, whose loads have their rows apart
+// from the place in a row); with packed ones they keep a stage-by-stage ring (RING), three stages in flight while one is
+// multiplied: 4096 x 4096 x 4224 47.5 us, with units 50.3, 256 x 256 x 4224 27.3 and 29.4.
+// The 16-byte pieces of a row are XOR-swizzled with the row index so that the 128-bit operand reads of 16 consecutive rows hit
+// 16 distinct 4-bank groups, and wave tiles of 128x128 keep LDS reads at 8 operand fragments per 16 matrix instructions.
 //
 // Scale bytes.  A row's scale bytes for one stage are 4 (or 2) bytes in a line of their own, so fetching them
 // stage by stage costs the vector memory path one cache-line access per row per stage - as many accesses as
@@ -47,14 +48,14 @@ namespace {
 
 constexpr int BM = 256, BN = 256;       // workgroup tile
 constexpr int ROWB = 64;                // code bytes per row per stage
-constexpr int NSTAGE = 4;               // LDS ring depth
+constexpr int NSTAGE = 4;               // LDS ring depth: two units of two stages
 constexpr int OP_BYTES = BM * ROWB;     // one operand's codes per stage (16 KiB)
-constexpr int SC_BYTES = BM * 4;        // narrow path: one operand's scale bytes per stage (4 per row)
-constexpr int SCG_BYTES = BM * 16;      // wide path: one operand's scale bytes per group (16 per row)
+constexpr int SC_BYTES = BM * 4;        // packed scales: one operand's scale bytes per stage (4 per row)
+constexpr int SCG_BYTES = BM * 16;      // row-major scales: one operand's scale bytes per group (16 per row)
 constexpr int CODE_LOADS = 2 * (OP_BYTES / 1024 / 4);   // direct-to-LDS code instructions per wave per stage (8)
 
-template <bool WIDE> constexpr int stage_bytes() { return WIDE ? 2 * OP_BYTES : 2 * OP_BYTES + 2 * SC_BYTES; }
-template <bool WIDE> constexpr int smem_bytes() { return NSTAGE * stage_bytes<WIDE>() + (WIDE ? 4 * SCG_BYTES : 0); }
+template <bool PK> constexpr int stage_bytes() { return PK ? 2 * OP_BYTES + 2 * SC_BYTES : 2 * OP_BYTES; }
+template <bool PK> constexpr int smem_bytes() { return NSTAGE * stage_bytes<PK>() + (PK ? 0 : 4 * SCG_BYTES); }
 
 // s_waitcnt immediate: vmcnt(vm), lgkmcnt(0), expcnt untouched
 constexpr int wait_imm(int vm) { return 0x0070 | (vm & 15) | ((vm >> 4) << 14); }
@@ -80,18 +81,17 @@ __device__ __forceinline__ void load_to_lds(uint32_t lane_off, const uint8_t* wa
 // FMT: element format of A (and of B, unless FMTB says otherwise).  FMTB == E2M1 under an 8-bit FMT is the reference's
 // "mixed" type (ours/block_scaled_matmul.py:318-324): everything follows the 8-bit geometry -- a stage is 64 elements
 // of K, a unit 128 -- except B's codes, which are half as wide: 32 bytes per row and stage, a unit's image 64-byte rows.
-template <int FMT, int FMTB, typename OutT, bool WIDE, bool WORDS, bool PK, bool PAIR, bool EDGE, bool HALF>
+template <int FMT, int FMTB, typename OutT, bool WORDS, bool PK, bool EDGE, bool ODD>
 __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
-    static_assert(PK ? !WIDE : WIDE && PAIR, "row-major scales come in groups, with units");
-    static_assert(!HALF || (WORDS && EDGE && FMT == MPSA_FMT_E2M1), "half a unit at the end: 4-bit codes, K % 256 == 128");
-    static_assert(!WORDS || (WIDE && PAIR), "words: groups whose rows do not lie on 16 bytes");
-    static_assert(NSTAGE == 4, "PAIR: the ring is two units of two stages");
+    static_assert(!WORDS || !PK, "words: row-major scales whose rows do not lie on 16 bytes");
+    static_assert(!ODD || FMT == MPSA_FMT_E2M1, "an odd number of stages: 4-bit codes, K % 256 == 128");
+    constexpr bool RING = ODD && PK, HALF = ODD && !PK;
+    static_assert(!HALF || (WORDS && EDGE), "half a unit at the end");
+    static_assert(NSTAGE == 4, "the ring is two units of two stages");
     constexpr bool FP4 = (FMT == MPSA_FMT_E2M1);
     constexpr bool B4 = !FP4 && (FMTB == MPSA_FMT_E2M1);       // 8-bit A against 4-bit B
     static_assert(FMT == FMTB || B4, "the operands share a format, or A is 8-bit and B is E2M1");
-    static_assert(!B4 || PAIR, "mixed formats: K % 128 == 0, so the stage count is even");
-    static_assert(!EDGE || PAIR, "ragged edges: the stage count is even");
-    constexpr int STAGE_BYTES = stage_bytes<WIDE>();
+    constexpr int STAGE_BYTES = stage_bytes<PK>();
     constexpr int GROUP = FP4 ? 4 : 8;                 // stages covered by 16 scale bytes of a row
     const int row_bytes = FP4 ? g.K / 2 : g.K;         // code bytes per matrix row (of A)
     const int row_bytes_b = B4 ? g.K / 2 : row_bytes;  // and of B
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     const int KT = row_bytes / ROWB;
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    uint8_t* const scg = smem + NSTAGE * STAGE_BYTES;  // wide path: [group parity][operand][row][16]
+    uint8_t* const scg = smem + NSTAGE * STAGE_BYTES;  // row-major scales: [group parity][operand][row][16]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // the wave index, known to be uniform
@@ -126,8 +126,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 
-    // ---- direct-to-LDS staging: wave w moves chunks [4w, 4w+4) x 1 KiB of either operand and the scale bytes
-    //      of rows [64w, 64w+64); chunk position p = row*4 + slot holds row's 16-byte piece slot ^ ((row>>2)&3)
+    // ---- direct-to-LDS staging ----
     // batched runs (blockIdx.y): operands of this batch entry; grouped heads share a B operand
     const int bz = blockIdx.y;
     const int bb = bz / g.heads_a, ha = bz - bb * g.heads_a;
@@ -137,7 +136,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     g.b += zb * g.N * row_bytes_b;
     g.sb += zb * g.N * srow_bytes;
     // lane offsets inside a tile's operand (the same for A and B) and inside its scale rows; tile bases are scalar
-    // PAIR: a unit = two consecutive stages = 128 code bytes per row, fetched as whole cache lines: an instruction
+    // a unit = two consecutive stages = 128 code bytes per row, fetched as whole cache lines: an instruction
     // of a wave covers 8 rows x 128 B (half-used lines move at half the rate through the vector memory path).  The
     // unit's LDS image has a 128-byte row pitch; row's 16-byte piece c sits at slot c ^ ((row >> 1) & 7), so that
     // 16 consecutive rows' reads of one piece fall into 16 distinct 4-bank groups.  Instruction x of the unit
@@ -145,32 +144,23 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     // EDGE: the tile's last row inside the matrix, of either operand, and its byte offset
     const int last_a = EDGE ? min(BM - 1, g.M - 1 - m0) : BM - 1, last_b = EDGE ? min(BN - 1, g.N - 1 - n0) : BN - 1;
     const uint32_t cap_a = (uint32_t)last_a * (uint32_t)row_bytes, cap_b = (uint32_t)last_b * (uint32_t)row_bytes_b;
-    uint32_t lo[4];
-    if constexpr (PAIR) {
+    uint32_t lo[2];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int cb = (lane & 7) ^ (4 * e + ((lane >> 4) & 3));
-            lo[e] = (EDGE ? 0u : (uint32_t)(lane >> 3) * (uint32_t)row_bytes) + cb * 16;
-        }
-        lo[2] = lo[3] = 0;
-    } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int p = (wave * 4 + c) * 64 + lane;
-            const int row = p >> 2, slot = p & 3;
-            const int cb = slot ^ ((row >> 2) & 3);
-            lo[c] = (uint32_t)row * (uint32_t)row_bytes + cb * 16;
-        }
+    for (int e = 0; e < 2; ++e) {
+        const int cb = (lane & 7) ^ (4 * e + ((lane >> 4) & 3));
+        lo[e] = (EDGE ? 0u : (uint32_t)(lane >> 3) * (uint32_t)row_bytes) + cb * 16;
     }
-    // mixed formats: a unit of B is 64 bytes per row, fetched like a stage of the stage-by-stage ring (four
-    // instructions per wave, row's piece c at slot c ^ ((row >> 2) & 3))
-    uint32_t lob[4] = {0, 0, 0, 0};
-    if constexpr (B4) {
+    // a unit of a mixed product's B, and a stage of the stage-by-stage ring, is 64 bytes per row: four instructions per wave, 16
+    // rows each, row's piece c at slot c ^ ((row >> 2) & 3)
+    uint32_t lo64a[4] = {0, 0, 0, 0}, lo64b[4] = {0, 0, 0, 0};
+    if constexpr (B4 || RING) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int p = (wave * 4 + c) * 64 + lane;
             const int row = p >> 2, slot = p & 3;
-            lob[c] = (uint32_t)min(row, last_b) * (uint32_t)row_bytes_b + (slot ^ ((row >> 2) & 3)) * 16;
+            const uint32_t piece = (uint32_t)(slot ^ ((row >> 2) & 3)) * 16u;
+            lo64a[c] = (uint32_t)min(row, last_a) * (uint32_t)row_bytes + piece;
+            lo64b[c] = EDGE || B4 ? (uint32_t)min(row, last_b) * (uint32_t)row_bytes_b + piece : lo64a[c];
         }
     }
     const uint32_t los_a = (uint32_t)min(wave * 64 + lane, last_a) * (uint32_t)srow_bytes;
@@ -189,10 +179,9 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     const int chunk = EDGE ? min(wave & 1, (wave < 2 ? last_a : last_b) >> 7) : wave & 1;
     const uint8_t* const s_pk = (wave < 2 ? g.sa + (int64_t)(m0 / 128) * kchunks * 512 : g.sb + (int64_t)(n0 / 128) * kchunks * 512) +
                                 (int64_t)chunk * kchunks * 512;
-    // a stage's loads go out in four parts (two code instructions each, the narrow path's scale words with the
-    // last) so that they can be spread between the matrix instructions of a step
-    // PAIR: part `part` of unit u's loads (four code instructions: two per operand; the scale bytes with the last).
-    // Unit u lives in ring half u & 1: [A codes 32 KiB][B codes 32 KiB][scale bytes of its two stages]
+    // Part `part` of unit u's loads: four code instructions, two per operand (mixed formats: two and one), and the packed scale
+    // bytes with the last.  In four parts so that they can be spread between the matrix instructions of a step.
+    // Unit u lives in ring half u & 1: [A codes 32 KiB][B codes 32 KiB][packed: scale bytes of its two stages]
     auto unit_base = [&](int u) __attribute__((always_inline)) { return smem + (u & 1) * 2 * STAGE_BYTES; };
     auto issue_unit_part = [&](int u, int part) __attribute__((always_inline)) {
         const int NU = HALF ? (KT + 1) / 2 : KT / 2;
@@ -213,7 +202,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
                 if constexpr (!B4) load_to_lds<16>(lo[q], b_base + go, ub + 2 * OP_BYTES + x * 1024);
             }
         }
-        if constexpr (B4) load_to_lds<16>(lob[part], b_base + (int64_t)uc * ROWB, ub + 2 * OP_BYTES + (wave * 4 + part) * 1024);
+        if constexpr (B4) load_to_lds<16>(lo64b[part], b_base + (int64_t)uc * ROWB, ub + 2 * OP_BYTES + (wave * 4 + part) * 1024);
         if (part != 3) return;
         uint8_t* sc = ub + 4 * OP_BYTES;
         if constexpr (PK) {
@@ -223,30 +212,19 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
             else if (lane < 32) load_to_lds<16>(pko, s_pk + (int64_t)uc * 512, sc + wave * 1024);
         }
     };
-    auto issue_part = [&](int kt, int part) __attribute__((always_inline)) {
+    // the same for stage kt of the stage-by-stage ring: one instruction per operand and part
+    auto issue_stage_part = [&](int kt, int part) __attribute__((always_inline)) {
         const int kc = kt < KT ? kt : KT - 1;             // past the end: re-load the last stage (keeps the count uniform)
         uint8_t* st = smem + (kt % NSTAGE) * STAGE_BYTES;
-        load_to_lds<16>(lo[part], a_base + (int64_t)kc * ROWB, st + (wave * 4 + part) * 1024);
-        load_to_lds<16>(lo[part], b_base + (int64_t)kc * ROWB, st + OP_BYTES + (wave * 4 + part) * 1024);
-        if constexpr (PK) {
-            // with 8-bit codes a chunk covers two stages and the odd stage's step takes its scale words from the
-            // even step's registers, so only even stages fetch (any two consecutive stages still issue the same
-            // number of loads, which is what the partial waits count)
-            if (part == 3 && (FP4 || (kt & 1) == 0)) {
-                const int64_t kb = FP4 ? kc : (kc >> 1);
-                if (lane < 32) load_to_lds<16>(pko, s_pk + kb * 512, st + 2 * OP_BYTES + wave * 512);
-            }
-        }
-    };
-    auto issue_stage = [&](int kt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int part = 0; part < 4; ++part) issue_part(kt, part);
+        load_to_lds<16>(lo64a[part], a_base + (int64_t)kc * ROWB, st + (wave * 4 + part) * 1024);
+        load_to_lds<16>(lo64b[part], b_base + (int64_t)kc * ROWB, st + OP_BYTES + (wave * 4 + part) * 1024);
+        if (part == 3 && lane < 32) load_to_lds<16>(pko, s_pk + (int64_t)kc * 512, st + 2 * OP_BYTES + wave * 512);
     };
     auto issue_unit = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
         for (int part = 0; part < 4; ++part) issue_unit_part(u, part);
     };
-    // wide path: the 16 scale bytes per row of group grp (two instructions per wave).  WORDS (K is no multiple of 512: rows of
+    // row-major scales: the 16 scale bytes per row of group grp (two instructions per wave).  WORDS (K is no multiple of 512: rows of
     // scale bytes start on words, and the last group is cut): a word a lane, four neighbouring lanes a row, 16 rows an
     // instruction; words past the row's end are its last one.
     auto issue_scales = [&](int grp) __attribute__((always_inline)) {
@@ -275,30 +253,24 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    if constexpr (WIDE) issue_scales(0);
-    if constexpr (PAIR) {
+    if constexpr (!PK) issue_scales(0);
+    if constexpr (RING) {
+#pragma unroll
+        for (int s = 0; s < NSTAGE; ++s)
+#pragma unroll
+            for (int part = 0; part < 4; ++part) issue_stage_part(s, part);
+    } else {
         issue_unit(0);
         issue_unit(1);
-    } else {
-#pragma unroll
-        for (int s = 0; s < NSTAGE; ++s) issue_stage(s);
     }
 
-    // LDS offsets of this lane's operand rows (row-major 64-byte rows -- PAIR: 128-byte rows --, swizzled chunks)
+    // LDS offsets of this lane's operand rows (128-byte rows; 64-byte ones in the ring and of a mixed product's B; swizzled pieces)
     int offa[4], offb[4], swz_a[4], swz_b[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int ra_ = wm * 128 + i * 32 + r, rb_ = wn * 128 + i * 32 + r;
-        if constexpr (B4) {
-            offa[i] = ra_ * 2 * ROWB; swz_a[i] = (ra_ >> 1) & 7;
-            offb[i] = rb_ * ROWB; swz_b[i] = (rb_ >> 2) & 3;
-        } else if constexpr (PAIR) {
-            offa[i] = ra_ * 2 * ROWB; swz_a[i] = (ra_ >> 1) & 7;
-            offb[i] = rb_ * 2 * ROWB; swz_b[i] = (rb_ >> 1) & 7;
-        } else {
-            offa[i] = ra_ * ROWB; swz_a[i] = (ra_ >> 2) & 3;
-            offb[i] = rb_ * ROWB; swz_b[i] = (rb_ >> 2) & 3;
-        }
+        offa[i] = ra_ * (RING ? ROWB : 2 * ROWB); swz_a[i] = RING ? (ra_ >> 2) & 3 : (ra_ >> 1) & 7;
+        offb[i] = rb_ * (RING || B4 ? ROWB : 2 * ROWB); swz_b[i] = RING || B4 ? (rb_ >> 2) & 3 : (rb_ >> 1) & 7;
     }
 
     // One matrix-instruction step's operands: 4 + 4 fragments and their scale bytes.  Two sets alternate: while
@@ -307,27 +279,27 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     // (bytes h and 2+h of the lane half h).  The word is read once, with the even step's operands, shifted right by
     // 8h when that step starts, and handed on to the odd step's set, whose instructions select byte 2.
     struct Frag { v8i a[4], b[4]; int sa[4], sb[4]; uint32_t ra[4], rb[4]; };
-    // Wide path, 4-bit codes: a row's 16 scale bytes of the current group are read from LDS ONCE per group with one
+    // Row-major scales, 4-bit codes: a row's 16 scale bytes of the current group are read from LDS ONCE per group with one
     // 128-bit read per row (16 consecutive rows x 16 bytes are conflict-free; a 32-bit read per step pair at this
     // 16-byte row pitch is a four-way bank conflict, and those conflicts were 38 % of the kernel's LDS cycles).
     // Dword k of a row covers step pair k of the group.  With 8-bit codes the operand sets fill the register file:
     // 32 (or, reading half a group at a time, 16) more registers spill and the kernel gets slower, so that path
     // keeps the 32-bit read per step pair.
-    constexpr bool GREAD = WIDE && FP4;                   // (and PAIR)
+    constexpr bool GREAD = !PK && FP4;
     v4i w_a[4], w_b[4];
 
     // reads operands of step s of stage kt out of the ring: part 0 the B fragments and their scale bytes,
-    // part 1 the A fragments and theirs.  grp >= 0 (wide path): also this part's scale rows of group grp.
+    // part 1 the A fragments and theirs.  grp >= 0 (GREAD): also this part's scale rows of group grp.
     auto read_part = [&](Frag& f, const Frag& even, int kt, int s, int part, bool fresh, int grp) __attribute__((always_inline)) {
         const bool isb = part == 0;
-        const int hh = kt & 1;                             // PAIR: which stage of its unit
-        const uint8_t* st = PAIR ? unit_base(kt >> 1) : smem + (kt % NSTAGE) * STAGE_BYTES;
-        const uint8_t* lx = PAIR ? (isb ? st + 2 * OP_BYTES : st) : (isb ? st + OP_BYTES : st);
-        const int c0 = PAIR ? 4 * hh : 0;                  // first 16-byte piece of this stage inside the LDS row
+        const int hh = kt & 1;                             // which stage of its unit
+        const uint8_t* st = RING ? smem + (kt % NSTAGE) * STAGE_BYTES : unit_base(kt >> 1);
+        const uint8_t* lx = isb ? st + (RING ? 1 : 2) * OP_BYTES : st;
+        const int c0 = RING ? 0 : 4 * hh;                  // first 16-byte piece of this stage inside the LDS row
         // the row's scale word of this step pair (paths without the per-group read)
-        const uint8_t* sc = WIDE ? scg + ((kt / GROUP) & 1) * 2 * SCG_BYTES + 4 * (FP4 ? kt % GROUP : (kt % GROUP) >> 1) + (isb ? SCG_BYTES : 0)
-                          : PAIR ? st + 4 * OP_BYTES + hh * 512 + (isb ? 2048 : 0)
-                                 : st + 2 * OP_BYTES + (isb ? SC_BYTES : 0);
+        const uint8_t* sc = RING ? st + 2 * OP_BYTES + (isb ? 1024 : 0)
+                          : PK ? st + 4 * OP_BYTES + hh * 512 + (isb ? 2048 : 0)
+                               : scg + ((kt / GROUP) & 1) * 2 * SCG_BYTES + 4 * (FP4 ? kt % GROUP : (kt % GROUP) >> 1) + (isb ? SCG_BYTES : 0);
         const uint8_t* sg = scg + (grp & 1) * 2 * SCG_BYTES + (isb ? SCG_BYTES : 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -343,7 +315,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
                 if constexpr (PK) {
                     // one conflict-free 128-bit read: the scale words of this lane's row in all four row blocks
                     if (i == 0) {
-                        const v4i wsc = *reinterpret_cast<const v4i*>(sc + (isb ? wn : wm) * (PAIR ? 1024 : 512) + r * 16);
+                        const v4i wsc = *reinterpret_cast<const v4i*>(sc + (isb ? wn : wm) * (RING ? 512 : 1024) + r * 16);
 #pragma unroll
                         for (int q = 0; q < 4; ++q) (isb ? f.rb[q] : f.ra[q]) = (uint32_t)wsc[q];
                     }
@@ -379,11 +351,11 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     };
     // One step: the 16 matrix instructions on operand set `cur`, in four rows.  Between them go the LDS reads
     // that fill the other set `nxt` with step ns of stage nkt (rows 0 and 1) and, when `refill` is set, the
-    // loads of stage lkt into the buffer of stage lkt-NSTAGE (two per row; on the wide path the first stage of
-    // a group also brings the next group's scale bytes), so that the matrix pipe keeps running while they issue.
+    // loads of the unit of stage lkt into the buffer of the unit before last (two per operand and row; where a group of scale
+    // bytes is due they follow the last), so that the matrix pipe keeps running while they issue.
     // `odd`: cur is the odd step of its pair (its scale words were handed on by the even step's set)
-    // wide path: `kd` = which dword of the group's scale rows an even step uses; `fetch_grp` >= 0: the refill also
-    // fetches that group's scale bytes; `read_grp` >= 0: the operand reads also bring that group's scale rows into
+    // row-major scales: `fetch_grp` >= 0: the refill also fetches that group's scale bytes.  GREAD: `kd` = which dword of the
+    // group's scale rows an even step uses; `read_grp` >= 0: the operand reads also bring that group's scale rows into
     // registers (the step after the group's last even step, so the registers are free)
     auto step = [&](Frag& cur, Frag& nxt, int nkt, int ns, bool refill, int lkt, bool odd, int kd, int fetch_grp, int read_grp) __attribute__((always_inline)) {
         constexpr int PER = FP4 ? 2 : 3;                   // LDS reads issued behind each matrix instruction
@@ -402,9 +374,9 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             if (refill) {
-                if constexpr (PAIR) issue_unit_part(lkt >> 1, i);     // lkt: first stage of the unit to fetch
-                else issue_part(lkt, i);
-                if constexpr (WIDE) {
+                if constexpr (RING) issue_stage_part(lkt, i);
+                else issue_unit_part(lkt >> 1, i);         // lkt: first stage of the unit to fetch
+                if constexpr (!PK) {
                     if (i == 3 && fetch_grp >= 0) issue_scales(fetch_grp);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -421,28 +393,21 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // Every wave has read stage kt into registers.  Wait until stage kt+1 has landed - everything but the loads
-    // of the two stages issued last - and meet the other waves; after that stage kt's buffer may be refilled.
-    // The next group's scale bytes, fetched with the first stage of a group, land like that stage's codes three
-    // stages later, before the next group's first stage is read.  (The wait leaves 16 loads in flight on the
-    // wide path although the two stages after a scale fetch amount to 18: waiting for two loads more than
-    // needed is harmless and keeps the count a constant.)
-    // PAIR: called once per unit, after its second stage has been read: the only loads in flight are the next
-    // unit's (and possibly a scale group's), all of which must have landed before that unit is read.
+    // Called once per unit, after its second stage has been read into registers: wait for the loads in flight -- the next unit's,
+    // and possibly a scale group's, all of which must have landed before that unit is read -- and meet the other waves; after
+    // that this unit's buffer may be refilled.
+    // Ring: once per stage, after it has been read: wait for the next stage, everything but the loads of the two issued last.
     auto publish = [&]() __attribute__((always_inline)) {
-        constexpr int KEEP = PAIR ? 0 : FP4 ? 2 * (CODE_LOADS + 1) : 2 * CODE_LOADS + 1;
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(wait_imm(KEEP));
+        __builtin_amdgcn_s_waitcnt(wait_imm(RING ? 2 * (CODE_LOADS + 1) : 0));
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
     };
 
     Frag f0, f1;
     {
-        // stages 1 .. NSTAGE-1 stay in flight (packed 8-bit: only stage 2 of them carries scale loads)
-        // PAIR: unit 1 stays in flight (16 code loads and its scale loads: none or one)
-        constexpr int KEEP = PAIR ? (B4 ? CODE_LOADS + CODE_LOADS / 2 : 2 * CODE_LOADS) + (WIDE ? 0 : 1)
-                           : FP4 ? (NSTAGE - 1) * (CODE_LOADS + 1) : (NSTAGE - 1) * CODE_LOADS + 1;
+        // unit 1 stays in flight (its code loads and, packed, its scale load), in the ring the stages after the first
+        constexpr int KEEP = RING ? (NSTAGE - 1) * (CODE_LOADS + 1) : (B4 ? CODE_LOADS + CODE_LOADS / 2 : 2 * CODE_LOADS) + (PK ? 1 : 0);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(wait_imm(KEEP));
         __syncthreads();
@@ -450,10 +415,9 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
     }
     read_part(f0, f0, 0, 0, 0, true, GREAD ? 0 : -1);
     read_part(f0, f0, 0, 0, 1, true, GREAD ? 0 : -1);
-    // wide path without the per-group read: the group whose scale bytes the refill of stage kt also fetches
-    auto fetch_at = [&](int kt) { return (WIDE && kt % GROUP == (PAIR ? 1 : 0)) ? kt / GROUP + 1 : -1; };
-    if constexpr (PAIR && GREAD) {
-        // as below, with the ring refilled unit by unit: barrier and refill after a unit's second stage only
+    if constexpr (GREAD) {
+        // a stage is two steps: the second step's operands load under the first step's instructions, and the next stage's first
+        // operands under the second step's; barrier and refill after a unit's second stage.  One trip = one scale group.
         for (int grp = 0; grp < KT / GROUP; ++grp) {
 #pragma unroll
             for (int u = 0; u < GROUP; ++u) {
@@ -479,37 +443,29 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
             step(f0, f1, KT - 1, 1, false, 0, false, 0, -1, -1);
             step(f1, f0, KT - 1, 0, false, 0, true, 0, -1, -1);
         }
-    } else if constexpr (PAIR && FP4) {
+    } else if constexpr (RING) {
+        for (int kt = 0; kt < KT; ++kt) {
+            step(f0, f1, kt, 1, false, 0, false, 0, -1, -1);
+            publish();
+            step(f1, f0, kt + 1, 0, true, kt + NSTAGE, true, 0, -1, -1);
+        }
+    } else if constexpr (FP4) {
         for (int u2 = 0; u2 < KT / 2; ++u2) {
             const int kt = 2 * u2;
             step(f0, f1, kt, 1, false, 0, false, 0, -1, -1);
             step(f1, f0, kt + 1, 0, false, 0, true, 0, -1, -1);
             step(f0, f1, kt + 1, 1, false, 0, false, 0, -1, -1);
             publish();
-            step(f1, f0, kt + 2, 0, true, kt + 4, true, 0, fetch_at(kt + 1), -1);
+            step(f1, f0, kt + 2, 0, true, kt + 4, true, 0, -1, -1);
         }
-    } else if constexpr (PAIR) {
+    } else {
+        // a stage is one step.  The group whose scale bytes the refill of stage kt also fetches:
+        auto fetch_at = [&](int kt) { return !PK && kt % GROUP == 1 ? kt / GROUP + 1 : -1; };
         for (int u2 = 0; u2 < KT / 2; ++u2) {
             const int kt = 2 * u2;
             step(f0, f1, kt + 1, 0, false, 0, false, 0, -1, -1);
             publish();
             step(f1, f0, kt + 2, 0, true, kt + 4, true, 0, fetch_at(kt + 1), -1);
-        }
-    } else if constexpr (FP4) {
-        // a stage is two steps: the second step's operands load under the first step's instructions, and the
-        // next stage's first operands (after the barrier that publishes it) under the second step's
-        for (int kt = 0; kt < KT; ++kt) {
-            step(f0, f1, kt, 1, false, 0, false, 0, -1, -1);
-            publish();
-            step(f1, f0, kt + 1, 0, true, kt + NSTAGE, true, 0, fetch_at(kt), -1);
-        }
-    } else {
-        // a stage is one step; two stages per trip so that the two operand sets keep their registers
-        for (int kt = 0; kt < KT; kt += 2) {
-            publish();
-            step(f0, f1, kt + 1, 0, true, kt + NSTAGE, false, 0, fetch_at(kt), -1);
-            publish();
-            step(f1, f0, kt + 2, 0, true, kt + 1 + NSTAGE, true, 0, fetch_at(kt + 1), -1);
         }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);                // no direct-to-LDS load may outlive the workgroup
@@ -538,16 +494,16 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
         }
 }
 
-template <int FMT, int FMTB, typename OutT, bool WIDE, bool WORDS, bool PK, bool PAIR, bool EDGE, bool HALF>
+template <int FMT, int FMTB, typename OutT, bool WORDS, bool PK, bool EDGE, bool ODD>
 struct GemmLds {
     static inline const bool registered =
-        mpsa_register_lds_kernel(reinterpret_cast<const void*>(gemm_mx_kernel<FMT, FMTB, OutT, WIDE, WORDS, PK, PAIR, EDGE, HALF>), smem_bytes<WIDE>());
+        mpsa_register_lds_kernel(reinterpret_cast<const void*>(gemm_mx_kernel<FMT, FMTB, OutT, WORDS, PK, EDGE, ODD>), smem_bytes<PK>());
 };
 
-template <int FMT, int FMTB, typename OutT, bool WIDE, bool WORDS, bool PK, bool PAIR, bool EDGE, bool HALF = false>
+template <int FMT, int FMTB, typename OutT, bool WORDS, bool PK, bool EDGE, bool ODD = false>
 void launch_kernel(const GemmArgs& g, dim3 grid, hipStream_t st) {
-    if (!GemmLds<FMT, FMTB, OutT, WIDE, WORDS, PK, PAIR, EDGE, HALF>::registered) return;
-    hipLaunchKernelGGL((gemm_mx_kernel<FMT, FMTB, OutT, WIDE, WORDS, PK, PAIR, EDGE, HALF>), grid, dim3(256), smem_bytes<WIDE>(), st, g);
+    if (!GemmLds<FMT, FMTB, OutT, WORDS, PK, EDGE, ODD>::registered) return;
+    hipLaunchKernelGGL((gemm_mx_kernel<FMT, FMTB, OutT, WORDS, PK, EDGE, ODD>), grid, dim3(256), smem_bytes<PK>(), st, g);
 }
 
 

@@ -147,6 +147,19 @@ def test_kernels_by_name():
     assert L.mpsa_gemm_kernel(13, 4, 4, 1, 1, 256, 256, 256) == -1 and L.mpsa_gemm_kernel(0, 4, 4, 1, 1, 256, 256, 96) == -3
 
 
+@pytest.mark.parametrize("fmt_a,fmt_b", [(4, 4), (0, 0), (1, 1), (0, 4), (4, 0)])
+def test_the_kernel_that_a_product_takes_can_be_named(fmt_a, fmt_b):
+    L, halves = _lib.lib(), 0
+    for M in (1, 16, 100, 256, 1000, 2304, 4224, 8192):
+        for N in (8, 100, 128, 1000, 4096, 4224, 16400):
+            for K in (64, 128, 256, 384, 640, 1152, 4096, 4224):
+                for heads in (1, 8):
+                    kernel = L.mpsa_gemm_kernel(0, fmt_a, fmt_b, 1, heads, M, N, K)
+                    assert kernel > 0 and L.mpsa_gemm_kernel(kernel, fmt_a, fmt_b, 1, heads, M, N, K) == kernel, (M, N, K, heads)
+                    halves += kernel == _lib.GEMM_KERNELS["tile256"] and K % 256 == 128 and M % 256 > 0
+    assert fmt_a != 4 or fmt_b != 4 or halves > 0
+
+
 @pytest.mark.parametrize("name,value", [("MPSA_ATTN_PP", "0"), ("MPSA_GEMM_GENERAL", "1")])
 def test_environment_switches_leave_everything_to_the_general_kernels(name, value):
     code = ("import sys; sys.path.insert(0, %r)\nfrom ours import _lib\nL = _lib.lib()\n"

@@ -659,28 +659,30 @@ def test_products_with_one_stage_of_k(batch, heads, heads_b, M, N, fmt_a, fmt_b)
 
 
 @pytest.mark.parametrize("fmt_a,fmt_b", [(4, 4), (0, 4), (1, 1)])
-@pytest.mark.parametrize("M,N", [(256, 512), (300, 257), (1, 768), (3001, 4099)])
+@pytest.mark.parametrize("M,N", [(256, 512), (300, 257), (1, 768), (3001, 4099), (1, 16392), (2176, 2176)])
 @pytest.mark.parametrize("K", [128, 256, 384, 512, 640, 768, 896, 1024, 1152, 1280, 1664, 3968])
 def test_256_wide_tiles_for_every_remainder_of_k(K, M, N, fmt_a, fmt_b):
-    """Scale bytes come four words a row at a time and codes 256 (4-bit) or 128 elements at a time: every length of the last
-    group and, with 4-bit codes, of the last unit gives the general kernel's bits, in the last row of either matrix too.
-    (Ragged 4-bit products that end in half a unit get there by the choice only, where they are large.)"""
+    """Scale bytes come four words a row at a time (packed ones a chunk) and codes 256 (4-bit) or 128 elements at a time: every
+    length of the last group and, with 4-bit codes, of the last unit gives the general kernel's bits, in the last row of either
+    matrix too, and in 16-bit results, which go through the LDS that the codes came through.  Ragged 4-bit products that end in
+    half a unit are taken from 64 tiles on."""
     L = _lib.lib()
     g = torch.Generator().manual_seed(K + M)
-    half = fmt_a == fmt_b == 4 and K % 256 == 128 and (M % 256 or N % 256)
-    chosen = L.mpsa_gemm_kernel(0, fmt_a, fmt_b, 1, 1, M, N, K) == _lib.GEMM_KERNELS["tile256"]
-    assert chosen or not (half and M > 3000 and K > 1000)
-    if half and not chosen:
+    if fmt_a == fmt_b == 4 and K % 256 == 128 and (M % 256 or N % 256) and ((M + 255) // 256) * ((N + 255) // 256) < 64:
+        assert L.mpsa_gemm_kernel(_lib.GEMM_KERNELS["tile256"], fmt_a, fmt_b, 1, 1, M, N, K) == -3
         return
 
     def codes(rows, fmt):
-        c = torch.randint(0, 256, (rows, K // 2 if fmt == 4 else K), generator=g, dtype=torch.uint8)
+        c = torch.randint(0, 256, (rows, K // 2 if fmt == 4 else K), dtype=torch.uint8, generator=g)
         return (c if fmt == 4 else c & 0xBF).to(DEV)
 
     a, b = codes(M, fmt_a), codes(N, fmt_b)
-    sa, sb = (torch.randint(118, 130, (rows, K // 32), generator=g, dtype=torch.uint8).to(DEV) for rows in (M, N))
-    got, want = (torch.empty(M, N, dtype=torch.float32, device=DEV) for _ in range(2))
-    for out, kernel in ((got, "auto" if half else "tile256"), (want, "general")):
-        _lib.check(L.mpsa_gemm_mx_on(_lib.GEMM_KERNELS[kernel], _lib.ptr(a), _lib.ptr(sa), fmt_a, _lib.ptr(b), _lib.ptr(sb), fmt_b, 0, 1, 1, 1, M, N, K,
-                                     _lib.ptr(out), _lib.F32, N, _lib.stream_ptr(a.device)))
-    assert torch.equal(got, want)
+    sa, sb = (torch.randint(118, 130, (rows, K // 32), dtype=torch.uint8, generator=g).to(DEV) for rows in (M, N))
+    for packed in range(1 + (M % 128 == 0 and N % 128 == 0)):
+        xa, xb = (pack_scale_5d(sa), pack_scale_5d(sb)) if packed else (sa, sb)
+        for dtype in [torch.float32] + [torch.bfloat16] * (N % 8 == 0):
+            got, want = (torch.full((M + 1, N), 7.0, dtype=dtype, device=DEV) for _ in range(2))
+            for out, kernel in ((got, "tile256"), (want, "general")):
+                _lib.check(L.mpsa_gemm_mx_on(_lib.GEMM_KERNELS[kernel], _lib.ptr(a), _lib.ptr(xa), fmt_a, _lib.ptr(b), _lib.ptr(xb), fmt_b, packed, 1, 1, 1, M, N, K,
+                                             _lib.ptr(out), _lib.dtype_id(dtype), N, _lib.stream_ptr(a.device)))
+            assert torch.equal(got, want)
