@@ -246,8 +246,8 @@ int mpsa_gemm_mx_batched_packed(const uint8_t* a, const uint8_t* sa5, int fmt_a,
  * MPSA_GEMM_AUTO is what the others take.  A kernel that does not take the shape gives MPSA_EUNSUPPORTED.
  * mpsa_gemm_kernel says which kernel a call takes (MPSA_GEMM_SPLIT resolved to its tile), in either scale layout, or why it would
  * be refused; a kernel that it answers can be named.  (With
- * MPSA_GEMM_AUTO a product with K == 128 and 16-bit results in rows that start on 16 bytes runs on a kernel of its own, which
- * gives the bits of MPSA_GEMM_GENERAL.)
+ * MPSA_GEMM_AUTO a product with K == 128, 16-bit results in rows that start on 16 bytes and more than 1024 blocks of 16 x 16 results
+ * runs on a kernel of its own, which gives the bits of MPSA_GEMM_GENERAL.)
  */
 #define MPSA_GEMM_AUTO 0
 #define MPSA_GEMM_GENERAL 1                               /* 128 x 128 tiles, two-stage pipeline: every shape */

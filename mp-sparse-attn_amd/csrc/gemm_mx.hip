@@ -272,14 +272,18 @@ void launch_fmt(const GemmArgs& g, int c_dtype, dim3 grid, hipStream_t st) {
 static bool known_fmt(int f) { return f == MPSA_FMT_E2M1 || f == MPSA_FMT_E4M3 || f == MPSA_FMT_E5M2; }
 
 // The kernel of a product: what the caller named (MPSA_GEMM_*), if it takes the shape, or the one with the least estimated time
-// (microseconds, fitted to measurements of every kernel at 820 shapes in three types, M from 1 to 8192, N from 100 to 16384, K from
-// 256 to 14336, weights not all in the cache; the choice costs 1.1 % over always taking the fastest, an earlier fit to 130 shapes
-// cost 4 %, and up to 2.2 times the time where M, N and K are all large: 4140 x 12160 x 10240, 8-bit x 4-bit, 980 us on the general
-// kernel, 427 on 256 x 256 tiles.  4-bit products with K % 256 == 128: 4096 x 4096 x 4224 69 us on 128-wide tiles, 43 on 256-wide).  A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started
+// (microseconds, fitted to measurements of every kernel at 4820 shapes in three types, one product or up to 32, M from 1 to 8192, N
+// from 16 to 16384, K from 128 to 14336, weights not all in the cache; over 2200 others the choice costs 0.8 % over always taking the
+// fastest; at 3 % of them a fit to 130 shapes, which cost 4.6 %, did better by 3 % or more.  A fit to 820 single products with N from
+// 100 cost 1.5 %, most with narrow ones and several at once: 32 x 46 x 128 x 8832 12.7 -> 16.3 us, 2399 x 169 x 6400 8.6 -> 11.6, 4-bit.
+// Where M, N and K are all large: 4140 x 12160 x 10240, 8-bit x 4-bit, 980 us on the general kernel, 427 on 256 x 256 tiles; 4-bit
+// with K % 256 == 128: 4096 x 4096 x 4224 69 us on 128-wide tiles, 43 on 256-wide).  A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started
 // round of 256 tiles counts whole, at a clock that falls as the chip fills, and every million outputs some.  The general kernel
 // shares a CU between up to three tiles and has no rounds: it is the fastest a few tiles past a whole number of them, and where K
 // is short; with long K it falls behind, as its tiles pass the L2 by.  The lines fall near M = 256 (4096-wide layer, K = 4096), where
 // a 128-wide tile takes over from the 16-row blocks, and near 2000 rows, where 256-wide tiles fill the chip.
+static int64_t blocks16(const GemmArgs& g, int64_t batches) { return (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * batches; }
+
 static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b) {
     const double M = g.M, N = g.N, K = g.K;
     const bool mixed = fmt_a != MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1;
@@ -306,11 +310,19 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
         default: return mpsa_fail(MPSA_EINVAL, "gemm: unknown kernel %d", kernel);
     }
     if (g.K % 128 || force_general()) return MPSA_GEMM_GENERAL;
+    if (g.K == 128) {
+        // one stage: a ring gains nothing (the fastest at none of 560 shapes), and the tiles that split K, all of whose waves but one
+        // idle, are the fastest while two workgroups a CU hold them (their time over the general kernel's, 1024 to 2048 blocks: 0.87,
+        // 2048 to 4096: 1.23)
+        if (blocks16(g, batches) > 2048) return MPSA_GEMM_GENERAL;
+        (void)gemm_split_cost(g, batches, fmt_a, fmt_b, &tile);
+        return MPSA_GEMM_SPLIT_TILE(tile / 10, tile % 10);
+    }
     struct Ring { double start, round, per_1024, empty, out; };              // empty: share of per_1024 at an empty chip
-    static const Ring RING[2][3] = {{{1.41, 3.49, 3.12, 0.79, 0.226}, {1.89, 3.23, 3.93, 0.724, 0.231}, {1.73, 3.16, 4.59, 0.755, 0.275}},
-                                    {{4.6, 3.19, 8.14, 0.66, 0.249}, {4.16, 4.59, 12.3, 0.618, 0.238}, {4.39, 3.93, 12.9, 0.681, 0.304}}};
+    static const Ring RING[2][3] = {{{2.063, 3.307, 3.471, 0.639, 0.362}, {1.643, 4.095, 4.156, 0.665, 0.191}, {1.614, 3.847, 5.167, 0.624, 0.202}},
+                                    {{0.452, 8.31, 8.676, 0.609, 0.231}, {1.098, 9.109, 12.72, 0.547, 0.195}, {1.062, 9.889, 14.39, 0.508, 0.094}}};
     struct Shared { double start, tile, least, base, per_1024, deep; };      // tile, per_1024: for 256 tiles; deep: more of it at K = 8192
-    static const Shared SHARED[3] = {{2.91, 1.12, 4.98, 3.26, 3.73, 0.122}, {3.13, 1.12, 6.61, 3.35, 4.55, 0.222}, {2.73, 1.49, 7.41, 3.39, 5.52, 0.074}};
+    static const Shared SHARED[3] = {{3.631, 1.447, 4.908, 2.611, 3.794, 0.53}, {3.691, 1.451, 6.614, 2.13, 4.954, 0.395}, {3.384, 1.997, 7.2, 1.906, 5.484, 0.451}};
     auto ring = [&](int which, int edge) {
         const Ring& r = RING[which][kind];
         const double rounds = ceil(tiles(edge) / 256.0), clock = r.empty + (1.0 - r.empty) * tiles(edge) / (256.0 * rounds);
@@ -354,8 +366,10 @@ static int gemm_entry(int kernel, const uint8_t* a, const uint8_t* sa, int fmt_a
     g.packed = packed ? 1 : 0;
     hipStream_t st = (hipStream_t)stream;
     const int64_t batches = batch * heads_a;
-    const bool stage = kernel == MPSA_GEMM_AUTO && !force_general() && gemm_stage_takes(g, fmt_a, fmt_b, c_dtype);
-    kernel = choose(kernel, g, batches, fmt_a, fmt_b);
+    // From 1024 blocks of 16 x 16 on (the time of the tiles that split K over this kernel's, 768 to 1024 blocks: 0.99, 1024 to 1536:
+    // 1.10; below 256 blocks 0.81: 16 x 4096, 8-bit x 4-bit, 3.2 and 3.9 us, 4096 x 16, 4-bit, 3.2 and 4.2).
+    const bool stage = kernel == MPSA_GEMM_AUTO && !force_general() && gemm_stage_takes(g, fmt_a, fmt_b, c_dtype) && blocks16(g, batches) > 1024;
+    kernel = stage ? MPSA_GEMM_GENERAL : choose(kernel, g, batches, fmt_a, fmt_b);
     if (kernel < 0) return kernel;
     rc = mpsa_ensure_init();
     if (rc != MPSA_OK) return rc;

@@ -302,13 +302,15 @@ int places_of(int tile) {
 }
 
 // Estimated microseconds of a product on this kernel with its best tile, fitted to the measurements that choose() in gemm_mx.hip
-// names.  A workgroup costs by its blocks (adding up the waves' sums), its rows, and its rows times K (what it brings into LDS);
-// workgroups on one CU take longer than one, by less than their number; and where there are more of them than places, whole
-// rounds count for most of it (1.04 of the time of the fastest tile, without the rounds 1.1).
+// names.  A workgroup costs by its blocks (adding up the waves' sums) and rows, and by its rows times K (what it brings into LDS).
+// Workgroups on one CU take longer than one, by less than their number -- the fixed part (`power`) by less than the part that is
+// traffic (`deep`: with one power for both, 8 x 512 x 128 x 9344, 8-bit, took 2 x 2 blocks and 29.8 us, 2 x 4 blocks 21.8) --, and
+// it is the CU with the most of them that counts (`whole`); where there are more than places, whole rounds.
 double gemm_split_cost(const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b, int* tile) {
     const bool a4 = fmt_a == MPSA_FMT_E2M1, b4 = fmt_b == MPSA_FMT_E2M1;
-    struct Fit { double start, block, piece, row, power, busy, rounds; };
-    static const Fit FIT[3] = {{2.05, 0.029, 0.194, 0.334, 0.598, 0.79, 0.692}, {2.0, 0.087, 0.177, 0.22, 0.714, 0.569, 0.803}, {2.03, 0.085, 0.175, 0.157, 0.591, 0.69, 0.702}};
+    struct Fit { double start, block, piece, row, power, busy, rounds, whole, deep; };
+    static const Fit FIT[3] = {{2.488, 0.051, 0.193, 0.246, 0.581, 0.666, 1.098, 0.579, 0.716}, {2.367, 0.084, 0.178, 0.204, 0.715, 0.528, 1.099, 0.717, 0.62},
+                               {2.411, 0.096, 0.163, 0.133, 0.033, 0.667, 1.173, 1.264, 0.79}};
     const Fit& f = FIT[a4 && b4 ? 0 : a4 || b4 ? 1 : 2];
     double best = 0.0;
     for (int t : {11, 12, 14, 22, 24, 44}) {
@@ -316,12 +318,14 @@ double gemm_split_cost(const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b,
         const int places = a4 ? (b4 ? places_of<true, true>(t) : places_of<true, false>(t)) : b4 ? places_of<false, true>(t) : places_of<false, false>(t);
         const double w = (double)((g.M + 16 * mb - 1) / (16 * mb)) * ((g.N + 16 * nb - 1) / (16 * nb)) * (double)batches / 256.0;      // workgroups per CU
         const double row = mb * (a4 ? 0.5 : 1.0) + nb * (b4 ? 0.5 : 1.0);
-        double load = w > 1.0 ? pow(w, f.power) : 1.0;
-        if (w > places) {
+        auto most = [&](double x) { return x > 1.0 ? f.whole * ceil(x) + (1.0 - f.whole) * x : 1.0; };
+        auto load = [&](double power) {
+            const double shared = w > 1.0 ? pow(most(w), power) : 1.0;
+            if (w <= places) return shared;
             const double full = floor(w / places), rest = w - full * places;
-            load += f.rounds * (full * pow(places, f.power) + (rest <= 0.0 ? 0.0 : rest > 1.0 ? pow(rest, f.power) : 1.0) - load);
-        }
-        const double cost = f.start + (f.block * mb * nb + f.piece * row * g.K / 1024.0 + f.row * row) * load * (1.0 + f.busy * (w < 1.0 ? w : 1.0));
+            return shared + f.rounds * (full * pow(places, power) + (rest > 0.0 ? pow(most(rest), power) : 0.0) - shared);
+        };
+        const double cost = f.start + ((f.block * mb * nb + f.row * row) * load(f.power) + f.piece * row * g.K / 1024.0 * load(f.deep)) * (1.0 + f.busy * (w < 1.0 ? w : 1.0));
         if (best == 0.0 || cost < best) {
             best = cost;
             *tile = t;

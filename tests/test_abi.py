@@ -160,6 +160,21 @@ def test_the_kernel_that_a_product_takes_can_be_named(fmt_a, fmt_b):
     assert fmt_a != 4 or fmt_b != 4 or halves > 0
 
 
+def test_the_choice_of_matmul_kernels_at_few_rows_and_narrow_shapes():
+    """Shapes at which the choice was measured to cost 9 to 39 %: one stage of K, several narrow products, and narrow ones with
+    many rows."""
+    L, G = _lib.lib(), _lib.GEMM_KERNELS
+    pick = lambda fa, fb, heads, M, N, K: L.mpsa_gemm_kernel(0, fa, fb, 1, heads, M, N, K)
+    for fa, fb in ((4, 4), (0, 4), (0, 0)):
+        for heads, M, N in ((1, 16, 1024), (1, 16, 4096), (1, 4096, 16), (32, 64, 64), (1, 1, 4096), (8, 10, 256)):
+            assert pick(fa, fb, heads, M, N, 128) in range(11, 45)          # tiles that split K
+        for heads, M, N in ((1, 512, 4096), (1, 256, 16384), (16, 512, 512), (512, 128, 128)):
+            assert pick(fa, fb, heads, M, N, 128) == G["general"]
+    assert pick(4, 4, 1, 2399, 169, 6400) == G["split2x4"] and pick(4, 4, 32, 46, 128, 8832) == G["split2x2"]
+    assert pick(0, 0, 8, 512, 128, 9344) == G["split2x4"] and pick(0, 0, 32, 25, 4608, 11904) == G["split2x4"]
+    assert pick(4, 4, 2, 927, 8586, 1408) == G["general"] and pick(4, 4, 1, 3830, 128, 6016) == G["split2x4"]
+
+
 @pytest.mark.parametrize("name,value", [("MPSA_ATTN_PP", "0"), ("MPSA_GEMM_GENERAL", "1")])
 def test_environment_switches_leave_everything_to_the_general_kernels(name, value):
     code = ("import sys; sys.path.insert(0, %r)\nfrom ours import _lib\nL = _lib.lib()\n"

@@ -658,6 +658,28 @@ def test_products_with_one_stage_of_k(batch, heads, heads_b, M, N, fmt_a, fmt_b)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("fmt_a,fmt_b", [(4, 4), (0, 4), (1, 1), (0, 1)])
+@pytest.mark.parametrize("batch,M,N", [(1, 16, 4096), (1, 256, 1024), (1, 257, 1024), (4, 128, 512), (5, 128, 512), (1, 500, 1000), (1, 512, 1032)])
+def test_products_with_one_stage_of_k_run_on_the_kernel_that_is_said(batch, M, N, fmt_a, fmt_b):
+    """K == 128 with up to 1024 blocks of 16 x 16 results, with more, and with more than 2048: the bits of the kernel that
+    mpsa_gemm_kernel names, or from 1024 blocks on of the general one where 16-bit rows start on 16 bytes."""
+    K, L = 128, _lib.lib()
+    g = torch.Generator().manual_seed(M * N + fmt_a)
+    codes = lambda rows, fmt: (torch.randint(0, 256, (batch, rows, K // 2 if fmt == 4 else K), generator=g, dtype=torch.uint8) & (0xFF if fmt == 4 else 0xBF)).to(DEV)
+    a, b = codes(M, fmt_a), codes(N, fmt_b)
+    sa, sb = (torch.randint(118, 130, (batch, rows, K // 32), generator=g, dtype=torch.uint8).to(DEV) for rows in (M, N))
+    said = L.mpsa_gemm_kernel(0, fmt_a, fmt_b, 1, batch, M, N, K)
+    blocks = (M + 15) // 16 * ((N + 15) // 16) * batch
+    assert (said > 10) == (blocks <= 2048)
+    stage = blocks > 1024 and (fmt_a == fmt_b or fmt_b == 4)
+    for dtype, ldc, kernel in ((torch.bfloat16, N, 1 if stage else said), (torch.bfloat16, N + 1, said), (torch.float32, N, said)):
+        got, want = (torch.full((batch, M, ldc), 3.0, dtype=dtype, device=DEV) for _ in range(2))
+        for out, k in ((got, 0), (want, kernel)):
+            _lib.check(L.mpsa_gemm_mx_on(k, _lib.ptr(a), _lib.ptr(sa), fmt_a, _lib.ptr(b), _lib.ptr(sb), fmt_b, 0, 1, batch, batch, M, N, K,
+                                         _lib.ptr(out), _lib.dtype_id(dtype), ldc, _lib.stream_ptr(a.device)))
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("fmt_a,fmt_b", [(4, 4), (0, 4), (1, 1)])
 @pytest.mark.parametrize("M,N", [(256, 512), (300, 257), (1, 768), (3001, 4099), (1, 16392), (2176, 2176)])
 @pytest.mark.parametrize("K", [128, 256, 384, 512, 640, 768, 896, 1024, 1152, 1280, 1664, 3968])
