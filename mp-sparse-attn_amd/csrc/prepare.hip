@@ -55,7 +55,7 @@ template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D, int SOURCE>
 __device__ __forceinline__ void prepare_block(const PrepArgs& p, uint32_t blk, bool again) {
     if (blk < p.q_total) {
         const uint32_t head = blk / p.bq;
-        quantize_block<XDT, DO4, DO8, FMT8, false>(p.q, blk - head * p.bq, head % p.hq, head / p.hq, p.hq);
+        quantize_block<XDT, DO4, DO8, FMT8, false, true>(p.q, blk - head * p.bq, head % p.hq, head / p.hq, p.hq);
         return;
     }
     blk -= p.q_total;
@@ -68,12 +68,12 @@ __device__ __forceinline__ void prepare_block(const PrepArgs& p, uint32_t blk, b
                 if (again) __syncthreads();      // the other head's mean has been read
                 head_mean<XDT, SOURCE, D>(p, head % p.hkv, head / p.hkv, mean);
             }
-            quantize_block_less<XDT, DO4, DO8, FMT8, false>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv,
+            quantize_block_less<XDT, DO4, DO8, FMT8, false, true>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv,
                                                             [&](int64_t, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
                 less_mean<XDT>(x, *reinterpret_cast<const uint4*>(mean + 8 * col8));
             });
         } else {
-            quantize_block<XDT, DO4, DO8, FMT8, false>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv);
+            quantize_block<XDT, DO4, DO8, FMT8, false, true>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv);
         }
         return;
     }

@@ -828,6 +828,50 @@ def test_q_with_infinities_quantizes_to_the_same_codes_in_the_kernel(bst):
     assert torch.isfinite(a[0, 1, untouched.to(DEV)]).all()      # the other rows of the head do not see the infinity
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bst", ["diag", "mxfp4", "mxfp8", "mixed", "mxfp8e5"])
+def test_odd_values_of_q_quantize_to_the_same_codes_in_every_kernel(bst, dtype):
+    """NaN of either sign, infinities, zeros among other values, subnormal blocks, and values within a few units of a midpoint
+    between two E2M1 codes: the preparation's codes are the stand-alone quantizer's, and the kernels that quantize Q themselves
+    give the bits of prepared Q -- the paired-tile kernel, every number of splits, and the one with a head's keys in LDS."""
+    from ours.mxfp_attn_kernel import prepare_operands, attention_from_operands
+    from ours.quant_mxint8 import quantize_mx
+    nan = float("nan")
+    pre = 1.25 / (1.0 + 5.0 / 128.0)                             # times 1 + 5/128: a midpoint, rounded
+    scale = pre / 1.4426950408889634
+
+    def odd(B, H, N):
+        q = make_qkv(B, H, H, N, 128, seed=N, dtype=torch.float32)[0]
+        g = torch.Generator().manual_seed(N)
+        q[:, :, :64] *= (torch.rand(B, H, 64, 128, generator=g) < 0.5).float()
+        q[0, 0, 100:200] = (1.0 + 5.0 / 128.0) * torch.exp2(torch.randint(-4, 2, (100, 128), generator=g).float())
+        q[0, 1, 80, 40], q[0, 1, 81, 41], q[0, 1, 82, 100], q[0, 2, 17, 3] = nan, -nan, float("inf"), float("-inf")
+        q[0, 1, 90, 32:64], q[0, 2, 91, :32] = nan, 6e-8 if dtype == torch.float16 else 1e-39
+        q[0, 3, 95, 5], q[0, 3, 95, 6] = float("inf"), nan
+        return q.to(dtype).to(DEV)
+
+    def same(a, b):
+        return torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a, nan=0.0), torch.nan_to_num(b, nan=0.0))
+
+    q, (_, k, v) = odd(1, 4, 512), (t.to(DEV) for t in make_qkv(1, 4, 2, 512, 128, seed=78, dtype=dtype))
+    ops = prepare_operands(q, k, v, 128, bst, scale)
+    for codes, scales, fmt in ((ops["q4"], ops["qs4"], _lib.FMT_E2M1), (ops["q8"], ops["qs8"], ops["fmt8"])):
+        if codes is not None:
+            c, s = quantize_mx(q, ops["pre"], fmt)
+            assert torch.equal(codes, c) and torch.equal(scales, s)
+    for kernel in ("paired", "short1", "short2", "short4"):
+        a, b = (torch.empty((1, 4, 512, 128), dtype=torch.float32, device=DEV) for _ in range(2))
+        attention_from_operands(ops, a, True, kernel=kernel)
+        attention_from_operands(prepare_operands(q, k, v, 128, bst, scale, fuse_q=True), b, True, kernel=kernel)
+        assert same(a, b), kernel
+    if bst not in ("diag", "mxfp4"):
+        q, (_, k, v) = odd(2, 16, 4096), (t.to(DEV) for t in make_qkv(2, 16, 16, 333, 128, seed=79, dtype=dtype))
+        a, b = (torch.empty((2, 16, 4096, 128), dtype=torch.float32, device=DEV) for _ in range(2))
+        attention_from_operands(prepare_operands(q, k, v, 128, bst, scale), a, False, kernel="short1")
+        attention_from_operands(prepare_operands(q, k, v, 128, bst, scale, fuse_q=True), b, False, kernel="short1")
+        assert same(a, b)
+
+
 def test_q16_entry_point_rejects_other_shapes():
     L = _lib.lib()
     assert L.mpsa_attn_fwd_q16_supported(1, 32, 8, 8192, 128, 128, 1, _lib.MODE_DIAG) == 1
