@@ -24,6 +24,7 @@ struct AttnArgs {
     const void* q_raw;
     int64_t q_sb, q_sh, q_sn;
     float q_pre;
+    int q_sure;                          // mpsa_e2m1_sure(q_pre, ...): quantize_kernel.h
 };
 
 template <int PVT> struct PV;

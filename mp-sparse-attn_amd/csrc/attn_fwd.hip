@@ -125,11 +125,12 @@ static int attn_entry(int kernel, const RawQ* rq, const uint8_t* q4, const uint8
     a.d = (int)D; a.tile = tile;
     a.skip_thresh = skip_thresh; a.skipped = skipped;
     a.order = order; a.counts = counts;
-    a.q_raw = nullptr; a.q_sb = a.q_sh = a.q_sn = 0; a.q_pre = 1.0f;
+    a.q_raw = nullptr; a.q_sb = a.q_sh = a.q_sn = 0; a.q_pre = 1.0f; a.q_sure = 0;
     if (causal && rows_dealt(B * Hkv, B * Hq * ntq, nt * tile / 64)) a.causal |= ROWS_DEALT;
     hipStream_t st = (hipStream_t)stream;
     if (rq) {
         a.q_raw = rq->q; a.q_sb = rq->strides[0]; a.q_sh = rq->strides[1]; a.q_sn = rq->strides[2]; a.q_pre = rq->pre;
+        a.q_sure = mpsa_e2m1_sure(rq->pre, pv_dtype) ? 1 : 0;
         if (rq->paired_only && !attn_pp_supported(a, pv_dtype))
             return mpsa_fail(MPSA_EUNSUPPORTED, "attn: unquantized q needs the paired-tile kernel's shape (D = 128, tile = 128; "
                                                 "causal: at least two tiles, unmasked: at least six); quantize q with mpsa_attn_prepare and call mpsa_attn_fwd");

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
             if constexpr (WANT4) {
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    w[c] = (int)e2m1_try8(x[c], se, false, rule[c]);
+                    w[c] = (int)e2m1_try8<true>(x[c], se, a.q_sure != 0, rule[c]);
                     again |= rule[c];
                 }
             }

@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 3) void attn_short_kernel(Short
             uint2 w8;
             int s4, s8;
             unpack8<PVT>(G::QR * p + c / (D / 8) < a.nq ? raw[q] : make_uint4(0, 0, 0, 0), x);
-            quantize_most<Q4, Q8, FMT8, false, true>(x, a.q_pre, false, 3, 7, w4, s4, w8, s8, again[q], e[q]);
+            quantize_most<Q4, Q8, FMT8, false, true, true>(x, a.q_pre, a.q_sure != 0, 3, 7, w4, s4, w8, s8, again[q], e[q]);
             any |= again[q];
             put_q(c, w4, s4, w8, s8);
         }

@@ -27,6 +27,7 @@ static inline bool mpsa_aligned16(const void* p) { return (reinterpret_cast<uint
 bool mpsa_register_lds_kernel(const void* kern, int bytes);      // api.hip; always returns true
 int mpsa_ensure_init();                                          // api.hip; MPSA_OK or the failure of mpsa_init()
 int mpsa_seq_mean_static_resolve();                              // quantize.hip; address of the built-in partial-sum array
+bool mpsa_e2m1_sure(float pre, int x_dtype);                     // quantize.hip; whether 16-bit values times pre convert to E2M1 as the rule says, all of them
 // quantize.hip: the float32 sums of chunks of 256 rows that mpsa_seq_mean starts with, without the mean
 int mpsa_seq_mean_partial(const void* x, int x_dtype, int64_t B, int64_t H, int64_t N, int64_t D, const int64_t x_strides[4], float* workspace, hipStream_t st);
 // prepare.hip: how a preparation comes by the mean over K's sequence that it takes off K

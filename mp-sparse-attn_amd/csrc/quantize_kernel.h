@@ -4,6 +4,7 @@
 #pragma once
 #include "mpsa_common.h"
 #include "mx_codec.h"
+#include "midpoints.h"
 
 
 struct QuantArgs {
@@ -13,7 +14,7 @@ struct QuantArgs {
     int n, d;                  // valid rows, row length
     int out_rows;              // rows per (b,h) in the outputs
     float pre;
-    int exact16;               // pre is a power of two: scaled values keep the inputs' 16-bit significands
+    int sure4;                 // mpsa_e2m1_sure(pre, ...)
     int emax4, emax8;
     uint8_t *codes4, *scales4, *codes8, *scales8;
     int spread;                // 4-bit codes one per byte
@@ -91,17 +92,17 @@ __device__ __forceinline__ float round16(float v) {
 // by a power of two leaves the mantissa alone: a value close to one shows in the low 21 bits of x itself.  A value whose bits
 // are 128 units or more away from such a pattern is at least 1.9e-6 away from every midpoint (the smallest, 0.25, from below:
 // 128 * 2^-26), and the conversion is the result.  That is one shift-and-add an element and half a minimum; converting
-// the inputs twice, nudged down and up by 2^-17 of themselves, which this replaces, took two products and half a conversion.
-// With the scaled FP8 conversion below (a shift and a clamp an element less) and, in the paired-tile kernel, all of a lane's
-// loads in front: 32/8 heads, 8192 tokens, diag, 356.2 -> 354.5 us a call; before fp8_past, 8 heads of 1024 x 64 15.3 -> 15.1
-// and 2 x 24 heads, 8000 queries over 200 keys 68.4 -> 66.9.
+// the inputs twice, nudged down and up by 2^-17 of themselves, which this replaces, took two products and half a conversion (32 heads
+// of 8192 x 128 14.9 -> 14.5 us).
 // The pattern is that of the E2M1 values and of zero as well; so a lane that finds it converts the nudged inputs, and if
 // they differ (a rounding boundary lies between) it takes the explicit rule.  (2^-17 of a value near a midpoint - the
 // smallest is 0.25 - is at least 1.9e-6.)  Small scales, where x may be subnormal, take the explicit rule as well.
-// When the pre-scale is a power of two the scaled values are 16-bit inputs times a power of two, at most 11
-// significant bits: such a value is either exactly a midpoint - where the two rules agree (both take the even
-// mantissa) - or at least 2^-12 away from one, so the check is skipped (`exact16`); it would otherwise fire on every
-// exact tie, which 16-bit data hits all the time.
+// Which values have the pattern the host can tell from the pre-scale: a product's mantissa depends on the two mantissas alone, and
+// a 16-bit value has 128 or 1024 of them.  Where none has (63 of 64 pre-scales for bfloat16, seven of eight for float16), or the pre-scale is a
+// power of two -- 16-bit inputs times a power of two, at most 11 significant bits, are either exactly a midpoint, where the two
+// rules agree (both take the even mantissa), or at least 2^-12 away from one --, the check is skipped (`sure`).  It would otherwise
+// fire on every exact tie, and on every zero: with half of the inputs zeros it did, 32 heads of 8192 x 128 16.5 us, with the check
+// on other inputs 14.5, without it 14.0 either way.
 constexpr int SMALLEST_SE = -100;      // x below 2^-126 is less than 2^-26 of a unit then: it rounds to zero in every format
 
 __device__ __forceinline__ uint32_t e2m1_convert8(const float (&x)[8], int se, float f) {
@@ -136,23 +137,25 @@ __device__ __forceinline__ uint32_t e2m1_pack8_rule(const float (&x)[8], int se)
     return e2m1_pack8_explicit(x, se);
 }
 
-// the conversion, and whether e2m1_pack8_rule has to look at it instead
-__device__ __forceinline__ uint32_t e2m1_try8(const float (&x)[8], int se, bool exact16, bool& rule) {
+// the conversion, and whether e2m1_pack8_rule has to look at it instead.  STRAIGHT: the check is made and not used instead of
+// branched around.
+template <bool STRAIGHT = false>
+__device__ __forceinline__ uint32_t e2m1_try8(const float (&x)[8], int se, bool sure, bool& rule) {
     rule = se < SMALLEST_SE;
-    if (!exact16) {
+    if (STRAIGHT || !sure) {
         uint32_t nearest = ~0u;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) nearest = min(nearest, (mpsa_f2u(x[i]) << 11) + (128u << 11));
-        rule |= nearest < (256u << 11);
+        for (int i = 0; i < 8; ++i) nearest = min(nearest, (mpsa_f2u(x[i]) << 11) + MIDPOINT_NEAR);
+        rule |= nearest < 2 * MIDPOINT_NEAR && !sure;
     }
     return e2m1_convert8(x, se, 1.0f);
 }
 
 template <bool HW4>
-__device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool exact16) {
+__device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool sure) {
     if constexpr (!HW4) return e2m1_pack8_explicit(x, se);
     bool rule;
-    uint32_t w = e2m1_try8(x, se, exact16, rule);
+    uint32_t w = e2m1_try8(x, se, sure, rule);
     if (rule) w = e2m1_pack8_rule(x, se);
     return w;
 }
@@ -215,8 +218,8 @@ __device__ __forceinline__ int block_exponent(float amax) {
 // branch.  That is the faster form where other code hangs on the branch -- the preparation (8 heads of 8192 x 128, 8-bit, 13.6 ->
 // 12.4 us; 64 of 1896 x 64 12.4 -> 11.4) and the short-sequence kernel's Q --, not in the stand-alone quantizer (32 heads of 8192 x
 // 128 16.6 -> 16.8, 8 5.5 -> 5.6).
-template <bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8 = false>
-__device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8, bool& again, int& e) {
+template <bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8 = false, bool STRAIGHT4 = false>
+__device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool sure, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8, bool& again, int& e) {
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -235,7 +238,7 @@ __device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exa
     if constexpr (DO4) {
         const int se = e - emax4;
         if constexpr (!SW8) {
-            w4 = e2m1_try8(x, se, exact16, again);
+            w4 = e2m1_try8<STRAIGHT4>(x, se, sure, again);
             w4 = zero ? 0u : w4;
         }
         s4 = zero ? 0 : min(max(se + 127, 0), 254);
@@ -254,10 +257,10 @@ __device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool exa
 }
 
 template <bool DO4, bool DO8, int FMT8, bool SW8>
-__device__ __forceinline__ void quantize_again(const float (&x)[8], int e, int emax4, int emax8, bool exact16, uint32_t& w4, uint2& w8) {
+__device__ __forceinline__ void quantize_again(const float (&x)[8], int e, int emax4, int emax8, bool sure, uint32_t& w4, uint2& w8) {
     if constexpr (DO4) {
         bool rule = true;
-        if constexpr (DO8 && !SW8) (void)e2m1_try8(x, e - emax4, exact16, rule);
+        if constexpr (DO8 && !SW8) (void)e2m1_try8(x, e - emax4, sure, rule);
         if (rule) w4 = SW8 ? e2m1_pack8_explicit(x, e - emax4) : e2m1_pack8_rule(x, e - emax4);
     }
     if constexpr (DO8) {
@@ -266,11 +269,11 @@ __device__ __forceinline__ void quantize_again(const float (&x)[8], int e, int e
 }
 
 template <bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8>
-__device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool exact16, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8) {
+__device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool sure, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8) {
     bool again;
     int e;
-    quantize_most<DO4, DO8, FMT8, SW8, CLAMP8>(x, pre, exact16, emax4, emax8, w4, s4, w8, s8, again, e);
-    if (again) quantize_again<DO4, DO8 && !CLAMP8, FMT8, SW8>(x, e, emax4, emax8, exact16, w4, w8);
+    quantize_most<DO4, DO8, FMT8, SW8, CLAMP8>(x, pre, sure, emax4, emax8, w4, s4, w8, s8, again, e);
+    if (again) quantize_again<DO4, DO8 && !CLAMP8, FMT8, SW8>(x, e, emax4, emax8, sure, w4, w8);
 }
 
 // One workgroup's share: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb (nh heads).
@@ -298,7 +301,7 @@ __device__ __forceinline__ void quantize_block_less(const QuantArgs& a, uint32_t
     uint32_t w4;
     uint2 w8;
     int s4, s8;
-    quantize_chunk<DO4, DO8, FMT8, SW8, CLAMP8>(x, a.pre, a.exact16 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
+    quantize_chunk<DO4, DO8, FMT8, SW8, CLAMP8>(x, a.pre, a.sure4 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
     const int64_t oc = head * chunks + c;                                 // flat output chunk
     int64_t os = oc >> 2;                                                 // and scale
     if (a.scales5d) {
