@@ -99,32 +99,24 @@ __global__ __launch_bounds__(RW * 64, 1) void attn_resident_kernel(ResidentArgs 
         v8i qf[G::SST];
         int qs;
         {
+            // straight through, without a branch, as in the streaming kernel (a check of the codes with a branch behind it: 1.02 of
+            // the time over 820 shapes)
             constexpr int BATCH = 4;
             uint32_t scale = 0;
 #pragma unroll
             for (int q0 = 0; q0 < CHUNKS; q0 += BATCH) {
-                float x[BATCH][8];
-                uint32_t none[BATCH];
-                uint2 w8[BATCH];
-                int no[BATCH], s8[BATCH], e[BATCH];
-                bool again[BATCH], any = false;
 #pragma unroll
                 for (int q = 0; q < BATCH; ++q) {
-                    const int c = (q0 + q) * 64 + lane;
-                    unpack8<PVT>(row_now + c / (D / 8) < a.nq ? raw[q0 + q] : make_uint4(0, 0, 0, 0), x[q]);
-                    quantize_most<false, true, FMT8, false>(x[q], a.q_pre, false, 3, 7, none[q], no[q], w8[q], s8[q], again[q], e[q]);
-                    any |= again[q];
-                }
-                if (any) {
-#pragma unroll
-                    for (int q = 0; q < BATCH; ++q)
-                        if (again[q]) quantize_again<false, true, FMT8, false>(x[q], e[q], 3, 7, false, none[q], w8[q]);
-                }
-#pragma unroll
-                for (int q = 0; q < BATCH; ++q) {
-                    const int c = ((q0 + q) * 64) % (G::QROWS * (D / 8)) + lane;
-                    *reinterpret_cast<uint2*>(ql + c * 8) = w8[q];
-                    if ((lane & 3) == 0) ql[G::QROWS * D + (c >> 2)] = (uint8_t)s8[q];
+                    const int c = (q0 + q) * 64 + lane, at = c % (G::QROWS * (D / 8));
+                    float x[8];
+                    uint32_t none;
+                    uint2 w8;
+                    int no, s8, e;
+                    bool again;
+                    unpack8<PVT>(row_now + c / (D / 8) < a.nq ? raw[q0 + q] : make_uint4(0, 0, 0, 0), x);
+                    quantize_most<false, true, FMT8, false, true>(x, a.q_pre, false, 3, 7, none, no, w8, s8, again, e);
+                    *reinterpret_cast<uint2*>(ql + at * 8) = w8;
+                    if ((lane & 3) == 0) ql[G::QROWS * D + (at >> 2)] = (uint8_t)s8;
                 }
                 // so many rows are there: the lanes that own them take them
                 constexpr int AT_ONCE = G::QROWS * (D / 8) / 64;         // chunks
