@@ -180,9 +180,10 @@ __device__ __forceinline__ void store_output(const AttnArgs& a, int b, int hq, i
 // Short-sequence kernel (attn_fwd_short.hip): every mode but routed, any shape; a.q_raw != nullptr: unquantized Q
 int attn_short_launch(const AttnArgs& a, int pv_dtype, int splits, hipStream_t st);
 
-// The same math where a head's K and V fit one CU's LDS (attn_fwd_resident.hip), for attn_short_launch with one split: same bits
-bool attn_resident_takes(const AttnArgs& a);
-int attn_resident_launch(const AttnArgs& a, int pv_dtype, hipStream_t st);
+// The same math where a head's K and V fit one CU's LDS (attn_fwd_resident.hip), for attn_short_launch with one split: same bits.
+// Workgroups per (batch, KV head), 0: not that kernel's.
+int attn_resident_shares(const AttnArgs& a);
+int attn_resident_launch(const AttnArgs& a, int pv_dtype, int shares, hipStream_t st);
 
 // Tile-skipping variants of the general kernel (modes mxfp4 / mxfp8): attn_fwd_skip.hip
 int attn_skip_launch(const AttnArgs& a, int pv_dtype, hipStream_t st);

@@ -11,12 +11,13 @@
 // instruction, two waves a SIMD), 11 400 for eleven blocks of keys (510 a block of one SIMD: matrix 384, exponentials 256) and 1800
 // for the store.  Whole calls, the streaming kernel -> this one: that shape 42.6 -> 39.9 us; 2 x 8 heads, 10000 over 256, 40.1 ->
 // 36.9; 24 heads, 32000 over 333, mixed, 175 -> 157; 16 heads, 16000 over 352, 64.8 -> 58.3; 24 heads, 30000 over 77, 104 -> 98.
-// Below some 4096 blocks of queries the way into LDS is not paid back (2 x 16 heads, 2048 over 333, 29.0 -> 29.4; 16 heads 20.3 ->
-// 23.5); with 4-bit Q the streaming kernel has three waves a SIMD and wins (2 x 24 heads, 8000 over 200, 66.4 -> 75.8), and with D =
-// 64 four (2 x 24 heads, 3000 over 512, 37.4 -> 39.6).
+// Few blocks of queries a head, few altogether or few keys do not pay the way into LDS back (resident_choice.h); with 4-bit Q the
+// streaming kernel has three waves a SIMD and wins (2 x 24 heads, 8000 over 200, 66.4 -> 75.8), and with D = 64 four (2 x 24 heads,
+// 3000 over 512, 37.4 -> 39.6).
 #include "attn_common.h"
 #include "quantize_kernel.h"
 #include "reciprocal.h"
+#include "resident_choice.h"
 
 namespace {
 
@@ -25,7 +26,7 @@ struct ResidentArgs : AttnArgs {
     int units, group, nqb, tasks, step, nb;               // tasks: blocks of 32 queries of a (batch, KV head); step: waves that share them; nb: blocks of 32 keys
 };
 
-constexpr int D = 128, RW = 8;                            // waves
+constexpr int D = 128, RW = RESIDENT_WAVES;
 
 template <int MODE>
 struct Resident {
@@ -303,13 +304,14 @@ int launch_mode(const ResidentArgs& s, unsigned grid, hipStream_t st) {
 
 }  // namespace
 
-bool attn_resident_takes(const AttnArgs& a) {
-    if (!a.q_raw || a.causal || a.d != D || (a.mode != MPSA_MODE_MXFP8 && a.mode != MPSA_MODE_MIXED)) return false;
-    const int64_t nb = ((int64_t)a.n + 31) / 32, blocks = (int64_t)a.B * a.Hq * ((a.nq + 31) / 32);
-    return nb <= 64 && blocks >= 4096 && (a.mode == MPSA_MODE_MXFP8 ? Resident<MPSA_MODE_MXFP8>::lds((int)nb) : Resident<MPSA_MODE_MIXED>::lds((int)nb)) <= 163840;
+int attn_resident_shares(const AttnArgs& a) {
+    if (!a.q_raw || a.causal || a.d != D || (a.mode != MPSA_MODE_MXFP8 && a.mode != MPSA_MODE_MIXED)) return 0;
+    const int64_t nb = ((int64_t)a.n + 31) / 32;
+    if (nb > 64 || (a.mode == MPSA_MODE_MXFP8 ? Resident<MPSA_MODE_MXFP8>::lds((int)nb) : Resident<MPSA_MODE_MIXED>::lds((int)nb)) > 163840) return 0;
+    return (int)resident_choice(a.B, a.Hq, a.Hkv, a.nq, a.n);
 }
 
-int attn_resident_launch(const AttnArgs& a, int pv_dtype, hipStream_t st) {
+int attn_resident_launch(const AttnArgs& a, int pv_dtype, int shares, hipStream_t st) {
     ResidentArgs s;
     static_cast<AttnArgs&>(s) = a;
     s.units = a.B * a.Hkv;
@@ -317,17 +319,8 @@ int attn_resident_launch(const AttnArgs& a, int pv_dtype, hipStream_t st) {
     s.nqb = (a.nq + 31) / 32;
     s.tasks = s.group * s.nqb;
     s.nb = (a.n + 31) / 32;
-    // workgroups that share a head: the fewest clocks of rounds of 256 of them, each the way into LDS and its waves' blocks
-    int64_t best = INT64_MAX, shares = 1;
-    for (int x = 1; x <= (s.tasks + RW - 1) / RW && x <= 256; ++x) {
-        const int64_t clocks = ((int64_t)s.units * x + 255) / 256 * (13000 + 250 * s.nb + (int64_t)((s.tasks + RW * x - 1) / (RW * x)) * (6800 + 1000 * s.nb));
-        if (clocks < best) {
-            best = clocks;
-            shares = x;
-        }
-    }
-    s.step = (int)shares * RW;
+    s.step = shares * RW;
     s.by_units = reciprocal_of(s.units); s.by_hkv = reciprocal_of(a.Hkv); s.by_nqb = reciprocal_of(s.nqb);
-    const unsigned grid = (unsigned)(s.units * shares);
+    const unsigned grid = (unsigned)((int64_t)s.units * shares);
     return pv_dtype == MPSA_BF16 ? launch_mode<MPSA_BF16>(s, grid, st) : launch_mode<MPSA_F16>(s, grid, st);
 }

@@ -15,7 +15,7 @@
 // Q may arrive unquantized (a.q_raw): the workgroup quantizes its rows into LDS, eight elements per lane, with the quantizer's
 // own code -- the bits of mpsa_quantize_mx.
 // With 32 heads, 8 KV heads, causal, D = 128 (us of this kernel in a kernel trace; tile kernels): 160 tokens 6.8 (12.8), 1000
-// tokens 17 (25).  Many queries over keys that fit LDS go on to attn_fwd_resident.hip.
+// tokens 17 (25).  Many queries over keys that fit LDS may go on to attn_fwd_resident.hip.
 #include "attn_common.h"
 #include "quantize_kernel.h"
 #include "reciprocal.h"
@@ -512,7 +512,7 @@ int launch_fmt(const AttnArgs& a, int splits, hipStream_t st) {
 }  // namespace
 
 int attn_short_launch(const AttnArgs& a, int pv_dtype, int splits, hipStream_t st) {
-    if (splits == 1 && attn_resident_takes(a)) return attn_resident_launch(a, pv_dtype, st);
+    if (const int shares = splits == 1 ? attn_resident_shares(a) : 0) return attn_resident_launch(a, pv_dtype, shares, st);
     if (a.d == 128) return pv_dtype == MPSA_BF16 ? launch_fmt<128, MPSA_BF16>(a, splits, st) : launch_fmt<128, MPSA_F16>(a, splits, st);
     return pv_dtype == MPSA_BF16 ? launch_fmt<64, MPSA_BF16>(a, splits, st) : launch_fmt<64, MPSA_F16>(a, splits, st);
 }

@@ -1037,9 +1037,10 @@ def test_mean_inside_the_preparation_gives_the_bits_of_the_mean_on_its_own(B, Hk
 
 
 @pytest.mark.parametrize("mode,Nk", [("mxfp8", n) for n in (1, 31, 32, 77, 333, 352, 353)] + [("mixed", n) for n in (33, 300, 447, 448, 449)] + [("mxfp8e5", 100), ("mixed_e5", 64)])
-@pytest.mark.parametrize("B,Hq,Hkv,Nq,dtype,layout,climb", [(2, 16, 16, 4100, torch.bfloat16, "NHD", False), (1, 12, 4, 11001, torch.float16, "HND", True)])
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,dtype,layout,climb", [(2, 16, 16, 4100, torch.bfloat16, "NHD", False), (1, 12, 4, 11001, torch.float16, "HND", True),
+                                                             (3, 96, 8, 331, torch.bfloat16, "HND", True), (33, 16, 16, 250, torch.float16, "NHD", False)])
 def test_many_queries_over_the_keys_of_one_head_in_lds(B, Hq, Hkv, Nq, dtype, layout, climb, mode, Nk):
-    """From 4096 blocks of 32 queries on, as many keys as fit, 8-bit Q: the bits of the kernel that streams the keys (which
+    """Many queries over keys that fit LDS, fit just not or are too few, 8-bit Q: the bits of the kernel that streams the keys (which
     quantized Q takes), with ragged last blocks on both sides and scores that move the running maximum."""
     from ours.mxfp_attn_kernel import attention_from_operands, mxfp_attn_kernel, prepare_operands
     g = torch.Generator(device=DEV).manual_seed(Nk)
