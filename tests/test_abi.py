@@ -84,6 +84,35 @@ def test_host_side_argument_validation():
     assert L.mpsa_e2m1_encode(null, 0, null, null) == 0                                            # empty is fine
 
 
+def test_the_two_tensor_entry_points_refuse_what_two_calls_would():
+    """mpsa_quantize_mx_pair and mpsa_e2m1_pack_pair, either operand bad: null jobs and pointers, shapes, formats, strides and
+    alignment; what is empty on both sides is done without a launch."""
+    L = _lib.lib()
+    P = ctypes.pointer
+
+    def job(x=16, B=1, H=2, N=128, D=128, strides=None, fmt=4, codes=16, scales=16, rows=None):
+        return _lib.QuantizeJob(x, B, H, N, D, (ctypes.c_int64 * 4)(*(strides or (H * N * D, N * D, D, 1))), 1.0, fmt, 3 if fmt == 4 else 7, codes, scales, N if rows is None else rows)
+
+    def pair(a, b, dtype=0, per_byte=0, five=0):
+        return L.mpsa_quantize_mx_pair(a and P(a), b and P(b), dtype, per_byte, five, None)
+
+    assert pair(None, job()) == -1 and pair(job(), None) == -1 and b"null job" in L.mpsa_last_error()
+    assert pair(job(), job(), dtype=2) == -1                                                       # f32 inputs
+    for bad, status in ((job(x=None), -1), (job(codes=None), -1), (job(scales=None), -1), (job(fmt=9), -1), (job(fmt=2), -1), (job(D=48), -1), (job(rows=127), -1),
+                        (job(B=-1), -1), (job(strides=(32768, 16384, 128, 2)), -1), (job(x=24), -2), (job(strides=(32768, 16384, 132, 1)), -2), (job(codes=24), -2),
+                        (job(H=65536), -3)):
+        assert pair(bad, job(fmt=0)) == status and pair(job(fmt=1), bad) == status
+    for five in (job(N=127), job(D=96)):                                                           # packed scales: rows and D in multiples of 128
+        assert pair(five, job(), five=1) == -3 and pair(job(), five, five=1) == -3
+    assert pair(job(N=0, x=None, codes=None, scales=None), job(B=0, x=None, codes=None, scales=None)) == 0
+
+    one, null = ctypes.c_void_p(16), ctypes.c_void_p(0)
+    pack = lambda a, na, pa, b, nb, pb: L.mpsa_e2m1_pack_pair(a, 1, na, pa, b, 1, nb, pb, None)
+    assert pack(null, 16, one, one, 16, one) == -1 and pack(one, 16, null, one, 16, one) == -1
+    assert pack(one, -1, one, one, 16, one) == -1 and pack(null, 0, null, null, 16, one) == -1 and pack(null, 0, null, one, -2, one) == -1
+    assert pack(null, 0, null, null, 0, null) == 0
+
+
 def test_python_entry_points_refuse_cpu_tensors_and_bad_arguments():
     from ours.mxfp import MXFP4Tensor, MXScaleTensor
     from ours.mxfp_attn import mxfp_attn
