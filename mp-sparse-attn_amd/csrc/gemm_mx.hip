@@ -272,24 +272,26 @@ void launch_fmt(const GemmArgs& g, int c_dtype, dim3 grid, hipStream_t st) {
 static bool known_fmt(int f) { return f == MPSA_FMT_E2M1 || f == MPSA_FMT_E4M3 || f == MPSA_FMT_E5M2; }
 
 // The kernel of a product: what the caller named (MPSA_GEMM_*), if it takes the shape, or the one with the least estimated time
-// (microseconds, fitted to measurements of every kernel at 4820 shapes in three types, one product or up to 32, M from 1 to 8192, N
-// from 16 to 16384, K from 128 to 14336, weights not all in the cache; over 2200 others the choice costs 0.8 % over always taking the
-// fastest; at 3 % of them a fit to 130 shapes, which cost 4.6 %, did better by 3 % or more.  A fit to 820 single products with N from
-// 100 cost 1.5 %, most with narrow ones and several at once: 32 x 46 x 128 x 8832 12.7 -> 16.3 us, 2399 x 169 x 6400 8.6 -> 11.6, 4-bit.
-// Where M, N and K are all large: 4140 x 12160 x 10240, 8-bit x 4-bit, 980 us on the general kernel, 427 on 256 x 256 tiles; 4-bit
-// with K % 256 == 128: 4096 x 4096 x 4224 69 us on 128-wide tiles, 43 on 256-wide).  A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started
-// round of 256 tiles counts whole, at a clock that falls as the chip fills, and every million outputs some.  The general kernel
-// shares a CU between up to three tiles and has no rounds: it is the fastest a few tiles past a whole number of them, and where K
-// is short; with long K it falls behind, as its tiles pass the L2 by.  The lines fall near M = 256 (4096-wide layer, K = 4096), where
-// a 128-wide tile takes over from the 16-row blocks, and near 2000 rows, where 256-wide tiles fill the chip.
+// (microseconds, from measurements of every kernel at 18 000 shapes in three types, one product or up to 32, M from 1 to 8192, N from
+// 16 to 16384, K from 128 to 14336, weights not all in the cache).  The constants are those with the least time lost by the choice,
+// losses past 5 % and past what an earlier choice lost counted more; over 7500 others it costs 0.5 % over always taking the fastest, and
+// more than 10 % at 1.4 % of them.  Constants with the least error of the estimates cost 0.8 % and 2.5 % (619 x 6784 x 3072, 4-bit,
+// 25.7 -> 34.6 us; 821 x 11136 x 1024, 8-bit, 22.0 -> 28.1), from K = 256 on a fit to 820 single products 1.3 % and 4.5 %, one to 130
+// shapes 5.5 % and 20 %.
+// What is left is luck: with a few workgroups more than CUs, 8-bit tiles of 2 x 2 blocks take 1.8 or 2.4 us per 1024 of K.
+// A ring tile costs a fixed part -- pipeline fill, epilogue -- and one per 1024 of K; a started round of 256 tiles counts whole, at a
+// clock that falls as the chip fills.  The general kernel shares a CU between up to three tiles and has no rounds: it is the
+// fastest a few tiles past a whole number of them, and where K is short; with long K it falls behind, as its tiles pass the L2 by
+// (4140 x 12160 x 10240, 8-bit x 4-bit, 980 us, on 256 x 256 tiles 427).  The lines fall near M = 256 (4096-wide layer, K = 4096),
+// where a 128-wide tile takes over from the 16-row blocks, and near 2000 rows, where 256-wide tiles fill the chip.
 static int64_t blocks16(const GemmArgs& g, int64_t batches) { return (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * batches; }
 
 static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b) {
-    const double M = g.M, N = g.N, K = g.K;
+    const double K = g.K;
     const bool mixed = fmt_a != MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1;
     const int kind = fmt_a == MPSA_FMT_E2M1 && fmt_b == MPSA_FMT_E2M1 ? 0 : mixed ? 1 : 2;
     auto tiles = [&](int edge) { return (double)((g.M + edge - 1) / edge) * (double)((g.N + edge - 1) / edge) * (double)batches; };
-    // ragged 4-bit products that end in half a unit: from a quarter of the chip on (the estimates choose it from 140 tiles on)
+    // ragged 4-bit products that end in half a unit: from a quarter of the chip on (the estimates choose it from 130 tiles on)
     const bool half = kind == 0 && g.K % 256 && (g.M % BM || g.N % BN);
     const bool staged = g.K % 128 == 0 && (fmt_a == fmt_b || mixed) && (!half || tiles(256) >= 64.0);
     int tile = 0;
@@ -318,15 +320,15 @@ static int choose(int kernel, const GemmArgs& g, int64_t batches, int fmt_a, int
         (void)gemm_split_cost(g, batches, fmt_a, fmt_b, &tile);
         return MPSA_GEMM_SPLIT_TILE(tile / 10, tile % 10);
     }
-    struct Ring { double start, round, per_1024, empty, out; };              // empty: share of per_1024 at an empty chip
-    static const Ring RING[2][3] = {{{2.063, 3.307, 3.471, 0.639, 0.362}, {1.643, 4.095, 4.156, 0.665, 0.191}, {1.614, 3.847, 5.167, 0.624, 0.202}},
-                                    {{0.452, 8.31, 8.676, 0.609, 0.231}, {1.098, 9.109, 12.72, 0.547, 0.195}, {1.062, 9.889, 14.39, 0.508, 0.094}}};
+    struct Ring { double start, round, per_1024, empty; };                   // empty: share of per_1024 at an empty chip
+    static const Ring RING[2][3] = {{{0.0, 5.519, 2.87, 1.11}, {2.133, 3.158, 4.755, 0.635}, {0.0, 5.366, 5.753, 0.499}},
+                                    {{2.653, 6.175, 7.599, 0.971}, {2.78, 3.679, 12.764, 0.854}, {0.0, 7.642, 12.526, 1.136}}};
     struct Shared { double start, tile, least, base, per_1024, deep; };      // tile, per_1024: for 256 tiles; deep: more of it at K = 8192
-    static const Shared SHARED[3] = {{3.631, 1.447, 4.908, 2.611, 3.794, 0.53}, {3.691, 1.451, 6.614, 2.13, 4.954, 0.395}, {3.384, 1.997, 7.2, 1.906, 5.484, 0.451}};
+    static const Shared SHARED[3] = {{1.949, 0.002, 7.953, 4.391, 4.181, 0.539}, {2.678, 0.022, 10.204, 2.743, 3.158, 3.752}, {2.015, 1.046, 11.081, 0.008, 5.136, 2.689}};
     auto ring = [&](int which, int edge) {
         const Ring& r = RING[which][kind];
         const double rounds = ceil(tiles(edge) / 256.0), clock = r.empty + (1.0 - r.empty) * tiles(edge) / (256.0 * rounds);
-        return r.start + rounds * (r.round + r.per_1024 * clock * K / 1024.0) + r.out * 1e-6 * M * N * (double)batches;
+        return r.start + rounds * (r.round + r.per_1024 * clock * K / 1024.0);
     };
     const Shared& sh = SHARED[kind];
     const double load = tiles(128) / 256.0, slope = sh.base + sh.per_1024 * load * (1.0 + sh.deep * (K < 8192.0 ? K / 8192.0 : 1.0));

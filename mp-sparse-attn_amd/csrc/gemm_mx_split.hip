@@ -301,31 +301,33 @@ int places_of(int tile) {
     }
 }
 
-// Estimated microseconds of a product on this kernel with its best tile, fitted to the measurements that choose() in gemm_mx.hip
-// names.  A workgroup costs by its blocks (adding up the waves' sums) and rows, and by its rows times K (what it brings into LDS).
-// Workgroups on one CU take longer than one, by less than their number -- the fixed part (`power`) by less than the part that is
-// traffic (`deep`: with one power for both, 8 x 512 x 128 x 9344, 8-bit, took 2 x 2 blocks and 29.8 us, 2 x 4 blocks 21.8) --, and
-// it is the CU with the most of them that counts (`whole`); where there are more than places, whole rounds.
+// Estimated microseconds of a product on this kernel with its best tile, fitted as choose() in gemm_mx.hip says.  A workgroup costs
+// by its blocks (adding up the waves' sums) and rows, and by its rows times K (what it brings into LDS; `tile`: how much more than the
+// others).  Workgroups that share a CU take longer for the traffic alone (with one power for both parts, 8 x 512 x 128 x 9344, 8-bit,
+// took 2 x 2 blocks and 29.8 us, 2 x 4 blocks 21.8), and it is the CU with the most of them that counts (`whole`); where there are
+// more than places, whole rounds.
 double gemm_split_cost(const GemmArgs& g, int64_t batches, int fmt_a, int fmt_b, int* tile) {
     const bool a4 = fmt_a == MPSA_FMT_E2M1, b4 = fmt_b == MPSA_FMT_E2M1;
-    struct Fit { double start, block, piece, row, power, busy, rounds, whole, deep; };
-    static const Fit FIT[3] = {{2.488, 0.051, 0.193, 0.246, 0.581, 0.666, 1.098, 0.579, 0.716}, {2.367, 0.084, 0.178, 0.204, 0.715, 0.528, 1.099, 0.717, 0.62},
-                               {2.411, 0.096, 0.163, 0.133, 0.033, 0.667, 1.173, 1.264, 0.79}};
+    static const int TILES[6] = {11, 12, 14, 22, 24, 44};
+    struct Fit { double start, block, piece, row, rounds, whole, deep, tile[6]; };
+    static const Fit FIT[3] = {{1.984, 0.001, 0.336, 0.714, 1.746, 1.151, 1.058, {-0.151, 0.021, 0.186, -0.228, -0.06, 0.036}},
+                               {1.889, 0.044, 0.26, 0.558, 1.47, 2.106, 0.864, {-0.029, -0.006, 0.16, -0.285, -0.054, -0.024}},
+                               {1.803, 0.124, 0.277, 0.304, 1.513, 1.228, 0.934, {0.072, 0.065, 0.059, -0.049, -0.025, 0.2}}};
     const Fit& f = FIT[a4 && b4 ? 0 : a4 || b4 ? 1 : 2];
     double best = 0.0;
-    for (int t : {11, 12, 14, 22, 24, 44}) {
-        const int mb = t / 10, nb = t % 10;
+    for (int i = 0; i < 6; ++i) {
+        const int t = TILES[i], mb = t / 10, nb = t % 10;
         const int places = a4 ? (b4 ? places_of<true, true>(t) : places_of<true, false>(t)) : b4 ? places_of<false, true>(t) : places_of<false, false>(t);
         const double w = (double)((g.M + 16 * mb - 1) / (16 * mb)) * ((g.N + 16 * nb - 1) / (16 * nb)) * (double)batches / 256.0;      // workgroups per CU
         const double row = mb * (a4 ? 0.5 : 1.0) + nb * (b4 ? 0.5 : 1.0);
-        auto most = [&](double x) { return x > 1.0 ? f.whole * ceil(x) + (1.0 - f.whole) * x : 1.0; };
-        auto load = [&](double power) {
-            const double shared = w > 1.0 ? pow(most(w), power) : 1.0;
-            if (w <= places) return shared;
+        auto shared = [&](double x) { return x > 1.0 ? pow(f.whole * ceil(x) + (1.0 - f.whole) * x, f.deep) : 1.0; };
+        double fixed = 1.0, load = shared(w);
+        if (w > places) {
             const double full = floor(w / places), rest = w - full * places;
-            return shared + f.rounds * (full * pow(places, power) + (rest > 0.0 ? pow(most(rest), power) : 0.0) - shared);
-        };
-        const double cost = f.start + ((f.block * mb * nb + f.row * row) * load(f.power) + f.piece * row * g.K / 1024.0 * load(f.deep)) * (1.0 + f.busy * (w < 1.0 ? w : 1.0));
+            fixed += f.rounds * (ceil(w / places) - 1.0);
+            load += f.rounds * (full * pow(places, f.deep) + (rest > 0.0 ? shared(rest) : 0.0) - load);
+        }
+        const double cost = f.start + (f.block * mb * nb + f.row * row) * fixed + f.piece * (1.0 + f.tile[i]) * row * g.K / 1024.0 * load;
         if (best == 0.0 || cost < best) {
             best = cost;
             *tile = t;

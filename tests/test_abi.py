@@ -202,6 +202,9 @@ def test_the_choice_of_matmul_kernels_at_few_rows_and_narrow_shapes():
     assert pick(4, 4, 1, 2399, 169, 6400) == G["split2x4"] and pick(4, 4, 32, 46, 128, 8832) == G["split2x2"]
     assert pick(0, 0, 8, 512, 128, 9344) == G["split2x4"] and pick(0, 0, 32, 25, 4608, 11904) == G["split2x4"]
     assert pick(4, 4, 2, 927, 8586, 1408) == G["general"] and pick(4, 4, 1, 3830, 128, 6016) == G["split2x4"]
+    # and shapes at which a choice with the least error of its estimates took 26 to 36 % longer
+    assert pick(4, 4, 1, 619, 6784, 3072) == G["tile128"] and pick(0, 0, 1, 821, 11136, 1024) == pick(0, 0, 1, 4925, 4480, 1024) == G["tile256"]
+    assert pick(0, 4, 1, 420, 3072, 12288) == pick(4, 4, 1, 859, 1536, 14080) == G["split4x4"] and pick(4, 4, 23, 1862, 194, 640) == G["general"]
 
 
 @pytest.mark.parametrize("name,value", [("MPSA_ATTN_PP", "0"), ("MPSA_GEMM_GENERAL", "1")])
