@@ -8,7 +8,7 @@
 // operation, and so are its bits: which of the two a call takes can depend on the batch.
 // Clock stamps in a copy of this kernel, 2 x 16 heads, 4096 queries over 333 keys, 8-bit (two blocks of queries a wave): 15 900 until
 // K, V and the first queries are there (16.8 MB of queries from memory in one go), then a block 4600 for Q (8 a lane and
-// instruction, two waves a SIMD), 11 400 for eleven blocks of keys (510 a block of one SIMD: matrix 384, exponentials 256) and 1800
+// instruction, two waves a SIMD; with a branch in it), 11 400 for eleven blocks of keys (510 a block of one SIMD: matrix 384, exponentials 256) and 1800
 // for the store.  Whole calls, the streaming kernel -> this one: that shape 42.6 -> 39.9 us; 2 x 8 heads, 10000 over 256, 40.1 ->
 // 36.9; 24 heads, 32000 over 333, mixed, 175 -> 157; 16 heads, 16000 over 352, 64.8 -> 58.3; 24 heads, 30000 over 77, 104 -> 98.
 // Few blocks of queries a head, few altogether or few keys do not pay the way into LDS back (resident_choice.h); with 4-bit Q the

@@ -1,7 +1,8 @@
 // Block-scaled NT matmul for gfx950: the entry points and the choice between the kernels -- 256 x 256 tiles
 // (gemm_mx_kernel.h, here and in gemm_mx_edge.hip), 128 x 128 tiles (gemm_mx_tile.hip), tiles of a few 16 x 16 blocks with
 // K split between the waves (gemm_mx_split.hip) and the general kernel below, which takes K % 128 == 64 alone and is one of the
-// choices elsewhere: a few tiles past a whole number of 256, and short K (the score product of attention, K = 128).
+// choices elsewhere: a few tiles past a whole number of 256, and short K.  Score products of attention (K = 128) with 16-bit results
+// have a kernel of their own (gemm_mx_stage.hip).
 #include "gemm_mx_kernel.h"
 #include <cmath>
 
@@ -11,7 +12,7 @@ namespace {
 // The reference's kernel tiles 128 x 256 with masked edges (ours/block_scaled_matmul.py:154-267) and takes the two
 // operands' element widths separately (ELEM_PER_BYTE_A / ELEM_PER_BYTE_B, "mixed" = 8-bit A x 4-bit B,
 // ours/block_scaled_matmul.py:318-324).  This kernel takes every shape, also what the others do not (K % 128 == 64, whose scale rows are two-byte aligned only): a workgroup of
-// four waves owns a 128 x 128 tile, a wave 64 x 64 (2 x 2 accumulators), two workgroups share a CU.  K advances
+// four waves owns a 128 x 128 tile, a wave 64 x 64 (2 x 2 accumulators), up to three workgroups share a CU.  K advances
 // 128 elements per stage (two matrix-instruction steps; 64 code bytes per row of a 4-bit operand, 128 of an 8-bit
 // one): the stage's codes travel L2 -> LDS with direct-to-LDS loads into one of two buffers while the other is
 // multiplied, rows XOR-swizzled as in the 256 x 256 kernel; rows past M or N are fetched from the last valid row and
@@ -19,28 +20,6 @@ namespace {
 // ahead (byte by byte when K is not a multiple of 128: the last stage is then half a stage).  Each operand's
 // registers follow its own format's layout (4-bit: the lane half's registers are MX block h of the step; 8-bit:
 // registers 0-3 of both halves are block 0, 4-7 block 1).
-template <int FMT> struct EdgeOp {
-    static constexpr bool FP4 = FMT == MPSA_FMT_E2M1;
-    static constexpr int ROW = FP4 ? 64 : 128;           // code bytes per row per stage
-    static constexpr int CPR = ROW / 16;                 // 16-byte pieces per row
-    static constexpr int BYTES = 128 * ROW;              // the operand's codes of one stage
-    static constexpr int IPW = BYTES / 1024 / 4;         // direct-to-LDS instructions per wave and stage
-    __device__ static __forceinline__ int swz(int row) { return FP4 ? (row >> 2) & 3 : (row >> 1) & 7; }
-    // the fragment of matrix-instruction step k (0 / 1) of the stage, LDS row `row` of the operand's stage image
-    __device__ static __forceinline__ v8i frag(const uint8_t* img, int row, int k, int h) {
-        const uint8_t* p = img + row * ROW;
-        const int f = swz(row);
-        if constexpr (FP4) {
-            const v4i x = *reinterpret_cast<const v4i*>(p + (((2 * k + h) ^ f) * 16));
-            return (v8i){x[0], x[1], x[2], x[3], 0, 0, 0, 0};
-        } else {
-            const v4i x0 = *reinterpret_cast<const v4i*>(p + (((4 * k + h) ^ f) * 16));
-            const v4i x1 = *reinterpret_cast<const v4i*>(p + (((4 * k + h + 2) ^ f) * 16));
-            return (v8i){x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-        }
-    }
-};
-
 // scale byte of row `row`, MX block kb: row-major [rows, K/32] or the packed [rows/128, K/128, 32, 4, 4] form
 __device__ __forceinline__ int load_scale(const uint8_t* s, int row, int kb, int kblocks, bool packed) {
     if (!packed) return s[(int64_t)row * kblocks + kb];

@@ -52,6 +52,29 @@ template <> __device__ __forceinline__ OutE5M2 cvt_out<OutE5M2>(float v) {
     return OutE5M2{(uint8_t)(__builtin_amdgcn_cvt_pk_bf8_f32(v, v, 0, false) & 0xFF)};
 }
 
+// 128 rows of an operand for one stage of 128 elements of K, in LDS: the general kernel and the one for a single stage
+template <int FMT> struct EdgeOp {
+    static constexpr bool FP4 = FMT == MPSA_FMT_E2M1;
+    static constexpr int ROW = FP4 ? 64 : 128;           // code bytes per row per stage
+    static constexpr int CPR = ROW / 16;                 // 16-byte pieces per row
+    static constexpr int BYTES = 128 * ROW;              // the operand's codes of one stage
+    static constexpr int IPW = BYTES / 1024 / 4;         // direct-to-LDS instructions per wave and stage
+    __device__ static __forceinline__ int swz(int row) { return FP4 ? (row >> 2) & 3 : (row >> 1) & 7; }
+    // the fragment of matrix-instruction step k (0 / 1) of the stage, LDS row `row` of the operand's stage image
+    __device__ static __forceinline__ v8i frag(const uint8_t* img, int row, int k, int h) {
+        const uint8_t* p = img + row * ROW;
+        const int f = swz(row);
+        if constexpr (FP4) {
+            const v4i x = *reinterpret_cast<const v4i*>(p + (((2 * k + h) ^ f) * 16));
+            return (v8i){x[0], x[1], x[2], x[3], 0, 0, 0, 0};
+        } else {
+            const v4i x0 = *reinterpret_cast<const v4i*>(p + (((4 * k + h) ^ f) * 16));
+            const v4i x1 = *reinterpret_cast<const v4i*>(p + (((4 * k + h + 2) ^ f) * 16));
+            return (v8i){x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+        }
+    }
+};
+
 // Whether 16-bit results may be stored in pieces of 16 bytes: every row starts on such a piece.
 __device__ __forceinline__ bool rows16_aligned(const GemmArgs& g) { return ((reinterpret_cast<uintptr_t>(g.c) | (uintptr_t)(2 * g.ldc)) & 15) == 0; }
 

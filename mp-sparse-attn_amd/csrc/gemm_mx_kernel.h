@@ -39,8 +39,9 @@
 // one 32-lane load per wave, and a lane reads its scale words for all four row blocks with one 128-bit LDS read.
 //
 // Ragged edges.  EDGE runs take any M and N: rows past the matrix are fetched from its last row (a lane's row offset is
-// capped with one comparison per load) and not stored.  Their own instantiations, so that whole tiles pay nothing: 1000 x
-// 14336 x 4096 takes 37 us 4-bit and 47.5 us 8-bit x 4-bit where 1024 rows take 38 and 52 (the general kernel: 102, 106).
+// capped with one comparison per load) and not stored.  Their own instantiations, so that whole tiles pay nothing; 1000 x
+// 14336 x 4096 and 1024 rows of it take the same, 40.2 and 39.7 us 4-bit, 52.7 and 52.4 8-bit x 4-bit, 58.2 and 59.4 8-bit, a kernel
+// after the other and weights from memory (the general kernel: 102, 106 the first two).
 #pragma once
 #include "gemm_mx_args.h"
 
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(256, 1) void gemm_mx_kernel(GemmArgs g) {
 
     // epilogue: accumulator register e of lane (h, r) is C[8*(e/4) + 4*h + e%4][r] of its 32x32 block
     OutT* c = static_cast<OutT*>(g.c) + (int64_t)bz * g.M * g.ldc;
-    if constexpr (EDGE && sizeof(OutT) == 2) {         // whole tiles gain nothing by it: 8192^3 0.98 to 1.014 of the time
+    if constexpr (EDGE && sizeof(OutT) == 2) {         // whole tiles gain nothing by it: 8192^3 0.98 to 1.014 of the time; in one or two rounds a row less, stored this way, 0.98 to 1.02
         if (rows16_aligned(g)) {
             __syncthreads();                           // the ring is free: everybody has read it, and nothing is on its way into it
 #pragma unroll

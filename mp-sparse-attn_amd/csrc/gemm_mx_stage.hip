@@ -10,33 +10,14 @@
 // results: 16 x 2048 x 2048 25.0 -> 22.7 us 4-bit, 31.2 -> 25.5 8-bit; 32 x 3968 x 3968, 8-bit, 328 -> 202; 16 x 4096 x 4096, 4-bit,
 // 122 -> 104; 4 x 2688 x 2688, 8-bit, 16.3 -> 13.0; 16 x 1024 x 1024, 4-bit, 9.6 -> 8.0; one a workgroup, 8 x 1000 x 1000, 8-bit x
 // 4-bit, 6.8 -> 6.3.  Two and eight tiles are within 5 % of four on most of these and up to 30 % slower on one each.  5.9 TB/s of
-// results at 2048; a fill reaches 7.4.  Stores that pass the L2 by gain 5 to 15 % on some of these shapes and lose 20 to 30 %
+// results at 2048; a fill reaches 7.4.  Fewer than 1024 blocks of 16 x 16 results are for tiles that split K (gemm_mx.hip).  Stores that pass the L2 by gain 5 to 15 % on some of these shapes and lose 20 to 30 %
 // where rows are 4 KiB apart.
 #include "gemm_mx_args.h"
 
 namespace {
 
-template <int FMT> struct StageOp {
-    static constexpr bool FP4 = FMT == MPSA_FMT_E2M1;
-    static constexpr int ROW = FP4 ? 64 : 128;           // code bytes per row
-    static constexpr int CPR = ROW / 16, BYTES = 128 * ROW, IPW = BYTES / 1024 / 4;
-    __device__ static __forceinline__ int swz(int row) { return FP4 ? (row >> 2) & 3 : (row >> 1) & 7; }
-    __device__ static __forceinline__ v8i frag(const uint8_t* img, int row, int k, int h) {
-        const uint8_t* p = img + row * ROW;
-        const int f = swz(row);
-        if constexpr (FP4) {
-            const v4i x = *reinterpret_cast<const v4i*>(p + (((2 * k + h) ^ f) * 16));
-            return (v8i){x[0], x[1], x[2], x[3], 0, 0, 0, 0};
-        } else {
-            const v4i x0 = *reinterpret_cast<const v4i*>(p + (((4 * k + h) ^ f) * 16));
-            const v4i x1 = *reinterpret_cast<const v4i*>(p + (((4 * k + h + 2) ^ f) * 16));
-            return (v8i){x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-        }
-    }
-};
-
 template <int FA, int FB> struct StageLds {
-    static constexpr int A = 0, B = StageOp<FA>::BYTES, SA = B + 2 * StageOp<FB>::BYTES, SB = SA + 512, OUT = SB + 2 * 512, SMEM = OUT + 4 * rows16_bytes<2>();
+    static constexpr int A = 0, B = EdgeOp<FA>::BYTES, SA = B + 2 * EdgeOp<FB>::BYTES, SB = SA + 512, OUT = SB + 2 * 512, SMEM = OUT + 4 * rows16_bytes<2>();
 };
 
 struct StageArgs : GemmArgs {
@@ -45,8 +26,8 @@ struct StageArgs : GemmArgs {
 
 template <int FA, int FB, typename OutT>
 __global__ __launch_bounds__(256, 2) void gemm_mx_stage_kernel(StageArgs g) {
-    typedef StageOp<FA> OA;
-    typedef StageOp<FB> OB;
+    typedef EdgeOp<FA> OA;
+    typedef EdgeOp<FB> OB;
     typedef StageLds<FA, FB> L;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

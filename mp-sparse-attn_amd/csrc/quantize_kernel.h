@@ -216,8 +216,8 @@ __device__ __forceinline__ int block_exponent(float amax) {
 // true, the caller has quantize_again finish the chunk: several chunks in a row share one branch that way, and run interleaved.
 // CLAMP8: the 8-bit codes are the careful ones at once, and never a reason for `again`: three instructions an element more, and no
 // branch.  That is the faster form where other code hangs on the branch -- the preparation (8 heads of 8192 x 128, 8-bit, 13.6 ->
-// 12.4 us; 64 of 1896 x 64 12.4 -> 11.4) and the short-sequence kernel's Q --, not in the stand-alone quantizer (32 heads of 8192 x
-// 128 16.6 -> 16.8, 8 5.5 -> 5.6).
+// 12.4 us; 64 of 1896 x 64 12.4 -> 11.4), and Q in the short-sequence kernel and the one that keeps K and V in LDS --, not in the
+// stand-alone quantizer (32 heads of 8192 x 128 16.6 -> 16.8, 8 5.5 -> 5.6).
 template <bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8 = false, bool STRAIGHT4 = false>
 __device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool sure, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8, bool& again, int& e) {
     float amax = 0.0f;
