@@ -20,6 +20,8 @@ namespace {
 // ahead (byte by byte when K is not a multiple of 128: the last stage is then half a stage).  Each operand's
 // registers follow its own format's layout (4-bit: the lane half's registers are MX block h of the step; 8-bit:
 // registers 0-3 of both halves are block 0, 4-7 block 1).
+// (EdgeOp: gemm_mx_args.h)
+
 // scale byte of row `row`, MX block kb: row-major [rows, K/32] or the packed [rows/128, K/128, 32, 4, 4] form
 __device__ __forceinline__ int load_scale(const uint8_t* s, int row, int kb, int kblocks, bool packed) {
     if (!packed) return s[(int64_t)row * kblocks + kb];
