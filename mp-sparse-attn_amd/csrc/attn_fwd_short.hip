@@ -365,8 +365,9 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 3) void attn_short_kernel(Short
     // once, and a row sum that shows a score far above it sends the wave back to do the block with the maximum first, as does
     // a mask: no reduction and no branch between the scores and the exponentials.
     // Alone on its SIMD a wave feels where its instructions lie: in steps of a word the loop's place moves 8 heads of 128 queries over
-    // 16384 keys, 4-bit, between 56.7 and 59.4 us, with a period of 32 bytes (59.0 where the code in front of it had left it).
-    if constexpr (KS == 4 && D == 128 && MODE == MPSA_MODE_MXFP4) asm volatile(".p2align 5\n\t.fill 2, 4, 0xBF800000");      // s_nop 0
+    // 16384 keys, 4-bit, between 56.7 and 59.4 us, with a period of 32 bytes (59.0 where the code in front of it had left it), and 8
+    // heads of 1024 x 64, causal, diag, between 7.14 and 7.31 (7.27).  The other modes gain less than 1 % or lose.
+    if constexpr (KS == 4 && (D == 128 ? MODE == MPSA_MODE_MXFP4 : DIAG)) asm volatile(".p2align 5\n\t.fill 2, 4, 0xBF800000");      // s_nop 0
 #pragma unroll 1
     for (int j = 1; j < blocks; ++j) {
         turn(j);
