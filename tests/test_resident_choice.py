@@ -13,10 +13,12 @@ from conftest import PKG
 def choice(tmp_path_factory):
     d = tmp_path_factory.mktemp("resident")
     (d / "t.cpp").write_text('#include "%s"\nextern "C" int64_t choice(int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk) { return resident_choice(B, Hq, Hkv, nq, nk); }\n'
-                             % os.path.join(PKG, "csrc", "resident_choice.h"))
+                             'extern "C" int64_t shares(int64_t units, int64_t tasks, int64_t nb) { return resident_shares(units, tasks, nb); }\n' % os.path.join(PKG, "csrc", "resident_choice.h"))
     subprocess.run([os.environ.get("CXX", "g++"), "-O2", "-shared", "-fPIC", "-o", str(d / "t.so"), str(d / "t.cpp")], check=True)
     lib = ctypes.CDLL(str(d / "t.so"))
     lib.choice.argtypes, lib.choice.restype = [ctypes.c_int64] * 5, ctypes.c_int64
+    lib.shares.argtypes, lib.shares.restype = [ctypes.c_int64] * 3, ctypes.c_int64
+    lib.choice.shares = lib.shares
     return lib.choice
 
 
@@ -41,3 +43,11 @@ def test_workgroups_fit_a_launch(choice):
             seen += shares > 0
             assert 0 <= shares <= (tasks + 7) // 8 and B * Hkv * shares * 512 < 1 << 32
     assert seen > 3
+
+
+def test_the_numbers_passed_over_are_no_better(choice):
+    for units in (1, 3, 16, 32, 100, 255, 256, 257, 5000):
+        for tasks in (1, 7, 8, 9, 64, 100, 128, 500, 1000, 2047, 2048, 2049, 8000, 100000):
+            for nb in (1, 3, 11):
+                clocks = lambda x: -(-units * x // 256) * (13000 + 250 * nb + -(-tasks // (8 * x)) * (6800 + 1000 * nb))
+                assert choice.shares(units, tasks, nb) == min(range(1, min(256, -(-tasks // 8)) + 1), key=clocks)
