@@ -4,8 +4,8 @@
 // 23 us for a 16-row linear layer (a quantization and a product) whose kernels take 7.  Here a call checks the usual case,
 // allocates and launches; it returns None for anything unusual -- another device current, a layout that needs a copy, a shape
 // or type that is an error -- and the caller goes on with its own code, which copies or says what is wrong.
-// (Operand checks here instead of in Python and one layer of calls less: a 160-token prompt 11.3 -> 10.8 us, a 16-row linear layer
-// 14.0 -> 13.5, of which 7 are the two launches.)
+// (Operand checks here instead of in Python and one layer of calls less: a 160-token prompt 11.1 -> 10.8 us, a 16-row linear layer
+// 13.9 -> 13.4, of which 7 are the two launches; two processes of one build differ by as much and more.)
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 #include <ATen/ATen.h>
