@@ -341,22 +341,22 @@ int mpsa_attn_fwd_q16_supported(int64_t B, int64_t Hq, int64_t Hkv, int64_t n, i
  * The kernels behind the attention entry points, and those entry points with the kernel named by the caller, for comparisons and
  * measurements.  MPSA_ATTN_AUTO is what the others take: the kernel estimated to finish first.  A kernel that does not take the
  * shape gives MPSA_EUNSUPPORTED.  mpsa_attn_kernel says which kernel a call takes (visiting lists and tile skipping: the general
- * one), or why it would be refused.
+ * one's answer), or why it would be refused.
  *   The kernels split and order the sums over the keys differently and move the running maximum at different places, so that
  * their results differ in the last bits (P is rounded to 16 bits against another maximum).  On one kernel a sequence's result
  * does not depend on the others of the batch; MPSA_ATTN_AUTO looks at B, so that there it can, between batch sizes that take
  * different kernels.  MPSA_ATTN_SEQUENCE makes the choice for one sequence alone: the same bits in any batch, at the price of a
  * choice that is not made for the batch (32 heads, causal: 200 tokens in batches of 8 41 us a call instead of 21).
- *   mpsa_attn_fwd_q16_on takes unquantized Q for the paired-tile kernel and the short-sequence
- * one, any shape of theirs, and nq queries over nk keys.
+ *   mpsa_attn_fwd_q16_on takes unquantized Q for every kernel but the general one, any shape of theirs, and nq queries over nk keys.
  */
 #define MPSA_ATTN_AUTO 0
-#define MPSA_ATTN_GENERAL 1      /* one query tile a workgroup (csrc/attn_fwd_kernel.h): every shape and mode */
+#define MPSA_ATTN_GENERAL 1      /* one query tile a workgroup (csrc/attn_fwd_kernel.h, csrc/attn_fwd_tile.hip): every shape and mode */
 #define MPSA_ATTN_PAIRED 2       /* two query tiles a workgroup (csrc/attn_fwd_pp.hip): the shapes of mpsa_attn_fwd_q16_supported() */
 #define MPSA_ATTN_SHORT1 3       /* 32 queries a wave, a head's keys in one part (csrc/attn_fwd_short.hip), no visiting lists */
 #define MPSA_ATTN_SHORT2 4       /* the same, the keys split between two waves */
 #define MPSA_ATTN_SHORT4 5       /* the same, the keys split between four waves */
 #define MPSA_ATTN_SEQUENCE 6     /* what MPSA_ATTN_AUTO takes for B = 1 */
+#define MPSA_ATTN_TILE 7         /* one query tile a workgroup, softmax inside the P.V product (csrc/attn_fwd_tile.hip): D = 128, tile = 128 */
 int mpsa_attn_kernel(int kernel, int64_t B, int64_t Hq, int64_t Hkv, int64_t nq, int64_t nk, int64_t D, int tile, int causal, int mode);
 int mpsa_attn_fwd_on(int kernel, const uint8_t* q4, const uint8_t* qs4, const uint8_t* q8, const uint8_t* qs8,
                      const uint8_t* k4, const uint8_t* ks4, const uint8_t* k8, const uint8_t* ks8, int fmt8,

@@ -8,7 +8,7 @@
 // key/value head hq / (Hq/Hkv) (ours/online_routing.py:160-171).  Q already carries sm_scale*log2(e)
 // (folded in by the quantizer, ours/quant_mxint8.py:494), so scores are in log2 units.
 //
-// Mapping.  A workgroup owns one TILE-query tile; each of its TILE/32 waves owns 32 queries and walks all
+// Mapping of the kernel in attn_fwd_kernel.h, which takes what D = 128 with tile = 128 (attn_fwd_tile.hip) leaves.  A workgroup owns one TILE-query tile; each of its TILE/32 waves owns 32 queries and walks all
 // keys of every tile.  Both products are computed transposed so that a lane always owns ONE query:
 //   S^T = K Q^T   on v_mfma_scale_f32_32x32x64_f8f6f4: lane (h = lane/32, r = lane%32) of the K operand
 //                 supplies 32 elements of key row r and the E8M0 byte of MX block h of the 64-wide step
@@ -135,7 +135,7 @@ static int attn_entry(int kernel, const RawQ* rq, const uint8_t* q4, const uint8
             return mpsa_fail(MPSA_EUNSUPPORTED, "attn: unquantized q needs the paired-tile kernel's shape (D = 128, tile = 128; "
                                                 "causal: at least two tiles, unmasked: at least six); quantize q with mpsa_attn_prepare and call mpsa_attn_fwd");
     }
-    if (routed) return attn_routed_launch(a, pv_dtype, st);
+    if (routed) return attn_tile_supported(D, tile) ? attn_tile_launch(a, pv_dtype, st) : attn_routed_launch(a, pv_dtype, st);
     if (skip) {
         if (!(skip_thresh == skip_thresh)) return mpsa_fail(MPSA_EINVAL, "attn: skip_thresh is NaN");
         if (skipped && (reinterpret_cast<uintptr_t>(skipped) & 3)) return mpsa_fail(MPSA_EALIGN, "attn: skipped must be 4-byte aligned");
@@ -147,8 +147,9 @@ static int attn_entry(int kernel, const RawQ* rq, const uint8_t* q4, const uint8
     if (kernel == MPSA_ATTN_SHORT2) return attn_short_launch(a, pv_dtype, 2, st);
     if (kernel == MPSA_ATTN_SHORT4) return attn_short_launch(a, pv_dtype, 4, st);
     if (kernel == MPSA_ATTN_PAIRED) return attn_pp_launch(a, pv_dtype, st);
+    if (kernel == MPSA_ATTN_TILE) return attn_tile_launch(a, pv_dtype, st);
     if (rq) return mpsa_fail(MPSA_EUNSUPPORTED, "attn: the general kernel takes quantized q only; quantize it with mpsa_attn_prepare and call mpsa_attn_fwd");
-    if (D == 128 && tile == 128) return launch_dt<128, 128>(a, pv_dtype, st);
+    if (attn_tile_supported(D, tile)) return attn_tile_launch(a, pv_dtype, st);
     if (D == 64 && tile == 64)   return launch_dt<64, 64>(a, pv_dtype, st);
     if (D == 128 && tile == 64)  return launch_dt<128, 64>(a, pv_dtype, st);
     return launch_dt<64, 128>(a, pv_dtype, st);
@@ -222,15 +223,24 @@ extern "C" int mpsa_attn_fwd_q16_supported(int64_t B, int64_t Hq, int64_t Hkv, i
 
 static constexpr double SHORT_LIMIT = 16777216.0;         // blocks of 32 queries: a launch has fewer than 2^32 threads, a workgroup 256
 
-// Whether the short-sequence kernel (attn_fwd_short.hip) is estimated to finish first, and with how many key splits (0: it is
-// not).  Microseconds of either side, fitted to measurements at 90 shapes (1 - 256 heads, 45 - 8192 keys, D = 64 and 128, masked
-// and not); the choice costs 0.4 % over always taking the fastest.  A workgroup of the short kernel takes a fixed time and so
+// The kernel that is estimated to finish first: the short-sequence kernel (attn_fwd_short.hip) with one, two or four key splits,
+// if there are no more blocks of queries than it takes (`fits`), or one that owns whole query tiles.  Microseconds
+// of either side, fitted to measurements at 90 shapes (1 - 256 heads, 45 - 8192 keys, D = 64 and 128, masked and not).  A workgroup of the short kernel takes a fixed time and so
 // much a stage, `full` with all of a CU's places filled, `alone` at the head of the longest chain; a tile kernel's time is its
 // longest workgroup while there are no more of them than CUs.  With 32 heads and D = 128 four splits go up to 250 tokens, two
-// to 1900, where the paired-tile kernel takes over; one split serves many queries over few keys, however many: 40 heads, 32760
+// to 1900; one split serves many queries over few keys, however many: 40 heads, 32760
 // queries over 512 keys (whole calls) 303 us where the general kernel takes 365; 2 x 24 heads, 29157 over 100, 8-bit, 201
 // and 319; and long sequences of many 64-wide heads, 4 x 32 of 12796 tokens, causal, 8-bit, 2.22 ms and 2.96.
-static int short_splits(int64_t B, int64_t Hq, bool paired, int64_t nq, int64_t nk, int64_t D, int tile, int causal) {
+//   Self-attention with D = 128 and tile = 128 has two kernels that own whole query tiles: one a workgroup and two workgroups a CU (attn_fwd_tile.hip), or
+// two a workgroup of the whole CU (attn_fwd_pp.hip), which reads K and V half as often and is 1 to 7 % faster where either fills
+// the chip evenly.  Half as large workgroups fill it more evenly: without the mask the chip works in rounds of 512 or 256
+// workgroups, and a round that leaves one a CU takes 0.8 of a full one (32 heads of 2560 tokens, diag, 106 us in pairs, 88 in
+// single tiles; 64 of 1500 78, 65; 32 of 4096 178, 180); under the mask 512 workgroups or fewer run in one round, a long row beside
+// a short one (8 heads of 8192, 123 and 105; 32 of 2048 44 and 39); with 384 to 640 workgroups single tiles take 0.95 of the time where
+// they are chosen, with 640 to 768 0.98 to 1.01, with 768 to 1024 1.04 and with more 0.98 to 1.0, so from there on pairs.  The constants are
+// those with the least time lost over 1529 shapes of 700 to 20 000 tokens (all types, 1 - 256 heads); over 830 others the choice
+// costs 1.1 % over always taking the fastest, and without the single tiles 3.2.
+static int fastest_kernel(int64_t B, int64_t Hq, bool paired, bool fits, int64_t nq, int64_t nk, int64_t D, int tile, int causal) {
     const bool d128 = D == 128;
     auto tiles = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
     const double heads = (double)(B * Hq);
@@ -238,8 +248,14 @@ static int short_splits(int64_t B, int64_t Hq, bool paired, int64_t nq, int64_t 
     struct Cost { int splits; double fixed, full, alone, places; };
     static const Cost costs[2][3] = {{{1, 3.6, 0.62, 0.41, 768.0}, {2, 3.6, 0.74, 0.44, 768.0}, {4, 3.4, 0.52, 0.44, 512.0}},
                                      {{1, 5.6, 0.85, 0.49, 512.0}, {2, 5.4, 0.86, 0.42, 512.0}, {4, 4.3, 0.48, 0.51, 256.0}}};
-    double mine = 1e300;
-    int splits = 0;
+    double least = 1e300;
+    int kernel = MPSA_ATTN_GENERAL;
+    auto candidate = [&](int name, double us) {
+        if (us < least) {
+            least = us;
+            kernel = name;
+        }
+    };
     for (const Cost& c : costs[d128]) {
         const double wgs = heads * (double)tiles(qb, 4 / c.splits), stages = (double)tiles(kb, c.splits);
         double load = wgs / c.places;
@@ -247,27 +263,28 @@ static int short_splits(int64_t B, int64_t Hq, bool paired, int64_t nq, int64_t 
         else if (load < 1.0)  load = 1.0;
         const double spread = c.fixed * load + c.full * wgs * (causal ? 0.5 * ((double)kb / c.splits + 1.0) : stages) / c.places;
         const double longest = c.fixed + c.alone * stages, us = spread > longest ? spread : longest;
-        if (us < mine) {
-            mine = us;
-            splits = c.splits;
-        }
+        if (fits) candidate(c.splits == 1 ? MPSA_ATTN_SHORT1 : c.splits == 2 ? MPSA_ATTN_SHORT2 : MPSA_ATTN_SHORT4, us);
     }
 
     const double ntq = (double)tiles(nq, tile), ntk = (double)tiles(nk, tile);
-    double other;
-    if (paired) {                                             // attn_fwd_pp.hip: two query tiles a workgroup, one workgroup a CU
+    if (paired) {
         const double pairs = heads * (double)((int64_t)(ntq + 1.0) / 2), one = 10.4 + 1.61 * ntk;
-        if (!causal)           other = (double)tiles((int64_t)pairs, 256) * one;
-        else if (pairs <= 256.0)  other = one;
-        else                      other = 24.0 + 2.1 * pairs * (ntk + 2.0) / 2.0 / 256.0;
+        if (!causal)           candidate(MPSA_ATTN_PAIRED, (double)tiles((int64_t)pairs, 256) * one);
+        else if (pairs <= 256.0)  candidate(MPSA_ATTN_PAIRED, one);
+        else                      candidate(MPSA_ATTN_PAIRED, 24.0 + 2.1 * pairs * (ntk + 2.0) / 2.0 / 256.0);
+        const double wgs = heads * ntq, rest = wgs - 512.0 * (double)(int64_t)(wgs / 512.0);
+        const double rounds = (wgs - rest) / 512.0 + (rest == 0.0 ? 0.0 : rest <= 256.0 ? 0.8 : 1.0);
+        const double longest = wgs > 256.0 ? 10.1 + 1.3 * ntk : 4.4 + 1.36 * ntk, spread = 12.1 + 0.31 * ntk + 2.1 * wgs * (ntk + 1.0) / 2.0 / 512.0;
+        if (!causal)            candidate(MPSA_ATTN_TILE, rounds * (10.3 + 1.66 * ntk));
+        else if (wgs <= 640.0)  candidate(MPSA_ATTN_TILE, spread > longest ? spread : longest);
     } else {                                                  // attn_fwd_kernel.h, and Q's quantization in front of it
         const bool t128 = tile == 128;
         const double wgs = heads * ntq, steps = wgs * (causal ? (ntk + 1.0) / 2.0 : ntk);
         const double step = t128 ? (d128 ? 1.5 : 1.2) : (d128 ? 0.6 : 0.45), slots = d128 && t128 ? 512.0 : 1024.0;
         const double full = 8.0 * wgs / slots + step * steps / 256.0, one = 8.0 + (t128 ? 1.0 : 0.75) * ntk;
-        other = (full > one ? full : one) + 1.0 + heads * (double)nq * (double)D * 3.5 / 4.5e6;
+        candidate(MPSA_ATTN_GENERAL, (full > one ? full : one) + 1.0 + heads * (double)nq * (double)D * 3.5 / 4.5e6);
     }
-    return mine < other ? splits : 0;
+    return kernel;
 }
 
 // MPSA_ATTN_PP=0 in the environment leaves every call to the general kernel
@@ -290,11 +307,12 @@ extern "C" int mpsa_attn_kernel(int kernel, int64_t B, int64_t Hq, int64_t Hkv, 
     switch (kernel) {
         case MPSA_ATTN_AUTO: case MPSA_ATTN_SEQUENCE: {
             if (listed || general_only()) return MPSA_ATTN_GENERAL;
-            const int splits = short_splits(kernel == MPSA_ATTN_AUTO ? B : 1, Hq, paired, nq, nk, D, tile, causal);
-            if (splits && !fits) return paired ? MPSA_ATTN_PAIRED : MPSA_ATTN_GENERAL;
-            return splits == 4 ? MPSA_ATTN_SHORT4 : splits == 2 ? MPSA_ATTN_SHORT2 : splits == 1 ? MPSA_ATTN_SHORT1 : paired ? MPSA_ATTN_PAIRED : MPSA_ATTN_GENERAL;
+            return fastest_kernel(kernel == MPSA_ATTN_AUTO ? B : 1, Hq, paired, fits, nq, nk, D, tile, causal);
         }
         case MPSA_ATTN_GENERAL: return kernel;
+        case MPSA_ATTN_TILE:
+            if (!listed && attn_tile_supported(D, tile)) return kernel;
+            return mpsa_fail(MPSA_EUNSUPPORTED, "attn: the tile kernel by its own name takes D = 128 and tile = 128, and no visiting lists");
         case MPSA_ATTN_PAIRED:
             if (paired) return kernel;
             return mpsa_fail(MPSA_EUNSUPPORTED, "attn: the paired-tile kernel takes self-attention with D = 128 and tile = 128, causal from two tiles on, unmasked from six, and no visiting lists");

@@ -27,8 +27,7 @@
 // once, in the prologue, into an LDS area of their own (read straight from global memory at the diagonal step their
 // latency sat on the wave's critical path).  The running maximum rides in the score MFMA's C operand.  The "mixed" mode
 // (8-bit Q, 4-bit K) differs in the score instruction's operand formats only; the "mxfp8" mode's K ring holds 8-bit tiles.
-#include "attn_common.h"
-#include "quantize_kernel.h"
+#include "attn_q_raw.h"
 
 namespace {
 
@@ -143,93 +142,17 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(AttnArgs a) {
                                                  // those of the parked 8-bit fragments in bytes 1 and 3)
     v4i kf4[KB][SST];
     int ksc[KB];
-    // Both precisions from one pass over the lane's query row: lane half h owns MX blocks h and 2 + h of the row's four
-    // (the 4-bit operand layout), so a block's maximum and shared exponent are lane-local and serve both formats (the
-    // element exponent limits differ: 3 and 7).  The 8-bit operand wants 16 bytes of EVERY block in each lane half
-    // (registers 0-3: block 2s, 4-7: block 2s + 1), so the two lanes of a query trade halves of their blocks afterwards:
-    // one v_permlane32_swap per register pair.  q8f receives the 8-bit fragments when WANT8 is set.
+    // Both precisions from one pass over the lane's query row.  q8f receives the 8-bit fragments when WANT8 is set.
     auto load_q_raw = [&](auto want8_c, v8i (&q8f)[SST]) __attribute__((always_inline)) {
-#pragma clang fp contract(off)        // the quantizer's arithmetic, operation by operation
         constexpr bool WANT8 = decltype(want8_c)::value;
         constexpr bool WANT4 = MODE != MPSA_MODE_MIXED && MODE != MPSA_MODE_MXFP8;   // those two multiply 8-bit Q everywhere
         // rows beyond the sequence (ragged last tile) read the last row instead and are zeroed below
         const bool row_ok = i * TILE + q_local < a.nq;
         const int64_t row_idx = row_ok ? (int64_t)i * TILE + q_local : (int64_t)a.nq - 1;
-        const char* row = static_cast<const char*>(a.q_raw) +
-                          2 * ((int64_t)b * a.q_sb + (int64_t)hq * a.q_sh + row_idx * a.q_sn);
-        uint32_t sbytes = 0, sbytes8 = 0;
         uint4 raw[SST][4];
-#pragma unroll
-        for (int s = 0; s < SST; ++s)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) raw[s][c] = *reinterpret_cast<const uint4*>(row + 2 * (32 * (2 * s + h) + 8 * c));
-#pragma unroll
-        for (int s = 0; s < SST; ++s) {
-            float x[4][8];
-            float amax = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                unpack8<PVT>(raw[s][c], x[c]);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    x[c][e] = x[c][e] * a.q_pre;
-                    amax = __builtin_fmaxf(amax, __builtin_fabsf(x[c][e]));
-                }
-            }
-            const bool zero = mpsa_f2u(amax) == 0u;
-            const int ex = block_exponent(amax);
-            const int se = ex - 3, se8 = ex - 7;             // emax of E2M1: ours/quant_mxint8.py:303; of the 8-bit formats: :191
-            int w[4];
-            int w8[8];
-            bool rule[4], odd = false, again = false;        // chunks, and the block, that the conversions may not be right for
-            if constexpr (WANT4) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    w[c] = (int)e2m1_try8<true>(x[c], se, a.q_sure != 0, rule[c]);
-                    again |= rule[c];
-                }
-            }
-            if constexpr (WANT8) {
-                odd = fp8_odd(ex, se8);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const uint2 y = fp8_convert8<FMT8>(x[c], se8);
-                    w8[2 * c] = (int)y.x;
-                    w8[2 * c + 1] = (int)y.y;
-                    odd |= fp8_past<FMT8>(y);
-                }
-                again |= odd;
-            }
-            if (again && !zero) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    if (WANT4 && rule[c]) w[c] = (int)e2m1_pack8_rule(x[c], se);
-                    if (WANT8 && odd) {
-                        const uint2 y = fp8_careful8<FMT8, false>(x[c], se8);
-                        w8[2 * c] = (int)y.x;
-                        w8[2 * c + 1] = (int)y.y;
-                    }
-                }
-            }
-            if constexpr (WANT4) {
-                qf[s] = (v8i){zero ? 0 : w[0], zero ? 0 : w[1], zero ? 0 : w[2], zero ? 0 : w[3], 0, 0, 0, 0};
-                sbytes |= (uint32_t)(zero ? 0 : min(max(se + 127, 0), 254)) << (16 * s);
-            }
-            if constexpr (WANT8) {
-#pragma unroll
-                for (int c = 0; c < 8; ++c) w8[c] = zero ? 0 : w8[c];
-                // w8[0..3] = bytes 0-15, w8[4..7] = bytes 16-31 of block 2s + h.  Lane half 0 keeps its low half in
-                // registers 0-3 and takes block 2s + 1's low half from its partner into 4-7; lane half 1 keeps its high
-                // half in 4-7 and takes block 2s's high half into 0-3: swap (lanes 32-63 of register i) with (lanes 0-31 of
-                // register 4 + i).
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(w8[q]), "+v"(w8[4 + q]));
-                q8f[s] = (v8i){w8[0], w8[1], w8[2], w8[3], w8[4], w8[5], w8[6], w8[7]};
-                // lane half h hands the matrix core the scale byte of block 2s + h: its own
-                sbytes8 |= (uint32_t)(zero ? 0 : min(max(se8 + 127, 0), 254)) << (16 * s);
-            }
-        }
+        load_query(static_cast<const char*>(a.q_raw) + 2 * ((int64_t)b * a.q_sb + (int64_t)hq * a.q_sh + row_idx * a.q_sn), h, raw);
+        uint32_t sbytes, sbytes8;
+        quantize_query<PVT, FMT8, WANT4, WANT8>(raw, a.q_pre, a.q_sure != 0, qf, sbytes, q8f, sbytes8);
         if constexpr (WANT4) {
             qsc = (int)(sbytes | (sbytes8 << 8));
         } else {

@@ -1,4 +1,4 @@
-// Routed variants of the general fused attention kernel: every (query tile, key tile) pair runs at the precision the
+// Routed variants of the general fused attention kernel (D = 64 or tiles of 64; the others: attn_fwd_tile.hip): every (query tile, key tile) pair runs at the precision the
 // visiting list names (see attn_fwd_kernel.h and route.hip); pairs that are not on the list are skipped.
 #include "attn_fwd_kernel.h"
 
@@ -16,7 +16,6 @@ int launch_dt(const AttnArgs& a, int pv_dtype, hipStream_t st) {
 }  // namespace
 
 int attn_routed_launch(const AttnArgs& a, int pv_dtype, hipStream_t st) {
-    if (a.d == 128 && a.tile == 128) return launch_dt<128, 128>(a, pv_dtype, st);
     if (a.d == 64 && a.tile == 64)   return launch_dt<64, 64>(a, pv_dtype, st);
     if (a.d == 128 && a.tile == 64)  return launch_dt<128, 64>(a, pv_dtype, st);
     return launch_dt<64, 128>(a, pv_dtype, st);

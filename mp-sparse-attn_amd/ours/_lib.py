@@ -16,7 +16,7 @@ FMT_E4M3, FMT_E5M2, FMT_E2M1 = 0, 1, 4
 MODE_MXFP4, MODE_MXFP8, MODE_DIAG, MODE_ROUTED, MODE_MIXED = 0, 1, 2, 3, 4
 
 # names of the MPSA_ATTN_* and MPSA_GEMM_* kernels
-ATTN_KERNELS = {"auto": 0, "general": 1, "paired": 2, "short1": 3, "short2": 4, "short4": 5, "sequence": 6}
+ATTN_KERNELS = {"auto": 0, "general": 1, "paired": 2, "short1": 3, "short2": 4, "short4": 5, "sequence": 6, "tile": 7}
 GEMM_KERNELS = {"auto": 0, "general": 1, "split": 2, "tile128": 3, "tile256": 4,
                 "split1x1": 11, "split1x2": 12, "split1x4": 14, "split2x2": 22, "split2x4": 24, "split4x4": 44}
 

@@ -694,6 +694,26 @@ def test_paired_tile_kernel_causal_with_ragged_and_odd_tile_counts(bst, N, dtype
 
 
 @pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("bst", ["diag_e5", "mxfp4", "mixed", "mxfp8"])
+@pytest.mark.parametrize("N,Nk", [(1, 1), (127, 127), (129, 129), (256, 256), (257, 257), (400, 400), (650, 650), (300, 77), (130, 513)])
+def test_tile_kernel_at_its_edges(N, Nk, bst, causal):
+    """One to six steps, with and without a masked last one, the 8-bit tile first, second or later; Q quantized inside the kernel
+    gives the bits of the prepared route."""
+    from ours.mxfp_attn_kernel import prepare_operands, attention_from_operands
+    if N != Nk and (causal or bst == "diag_e5"):
+        pytest.skip("as many queries as keys")
+    q, _, _ = make_qkv(1, 4, 2, N, 128, seed=2300 + N, dtype=torch.float16, outliers=True)
+    _, k, v = make_qkv(1, 4, 2, Nk, 128, seed=2301 + N, dtype=torch.float16)
+    want = O.attn_mx(q, k, v, tile=128, causal=causal, mode=bst.replace("_e5", ""), fmt8=O.FMT_E5M2 if bst.endswith("e5") else O.FMT_E4M3, out_dtype=torch.float32)
+    _check(q, k, v, want, f"tile, {bst} {N}x{Nk}", out16=torch.float16, is_causal=causal, block_scale_type=bst, tile=128, kernel="tile")
+    q, k, v = q.to(DEV), k.to(DEV), v.to(DEV)
+    prepared = torch.full((1, 4, N, 128), float("nan"), dtype=torch.float32, device=DEV)
+    attention_from_operands(prepare_operands(q, k, v, 128, bst), prepared, causal, kernel="general")
+    inside = mxfp_attn_kernel(q, k, v, is_causal=causal, block_scale_type=bst, tile=128, output_dtype=torch.float32, kernel="tile")
+    assert torch.equal(prepared, inside)
+
+
+@pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("bst", ["diag", "mxfp8"])
 def test_coinciding_outlier_channels_and_the_8bit_matrix_instruction(bst, causal):
     """The one kind of input on which the kernels and the float32 oracle differ by more than the contract's bar, and why.
