@@ -100,24 +100,41 @@ __global__ __launch_bounds__(RW * 64, 1) void attn_resident_kernel(ResidentArgs 
         v8i qf[G::SST];
         int qs;
         {
-            // straight through, without a branch, as in the streaming kernel (a check of the codes with a branch behind it: 1.02 of
-            // the time over 820 shapes)
             constexpr int BATCH = 4;
             uint32_t scale = 0;
 #pragma unroll
             for (int q0 = 0; q0 < CHUNKS; q0 += BATCH) {
+                // straight through; a wave with a rare chunk does the batch again (rows past the last are zeros, as in the streaming kernel)
+                auto inside = [&](int q) { return row_now + ((q0 + q) * 64 + lane) / (D / 8) < a.nq; };
+                auto put = [&](int q, const uint2& w8, int s8) __attribute__((always_inline)) {
+                    const int at = ((q0 + q) * 64 + lane) % (G::QROWS * (D / 8));
+                    *reinterpret_cast<uint2*>(ql + at * 8) = w8;
+                    ql[G::QROWS * D + (at >> 2)] = (uint8_t)s8;
+                };
+                uint32_t none;
+                uint2 w8;
+                int no, s8;
+                bool rare = false;
 #pragma unroll
                 for (int q = 0; q < BATCH; ++q) {
-                    const int c = (q0 + q) * 64 + lane, at = c % (G::QROWS * (D / 8));
                     float x[8];
-                    uint32_t none;
-                    uint2 w8;
-                    int no, s8, e;
-                    bool again;
-                    unpack8<PVT>(row_now + c / (D / 8) < a.nq ? raw[q0 + q] : make_uint4(0, 0, 0, 0), x);
-                    quantize_most<false, true, FMT8, false, true>(x, a.q_pre, false, 3, 7, none, no, w8, s8, again, e);
-                    *reinterpret_cast<uint2*>(ql + at * 8) = w8;
-                    if ((lane & 3) == 0) ql[G::QROWS * D + (at >> 2)] = (uint8_t)s8;
+                    bool r1;
+                    unpack8<PVT>(raw[q0 + q], x);
+                    const float pre = inside(q) ? a.q_pre : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) x[i] *= pre;
+                    quantize_straight<false, true, FMT8>(x, none, no, w8, s8, r1);
+                    rare |= r1;
+                    put(q, w8, s8);
+                }
+                if (__ballot(rare) != 0) {
+#pragma unroll
+                    for (int q = 0; q < BATCH; ++q) {
+                        float x[8];
+                        unpack8<PVT>(inside(q) ? only_here(raw[q0 + q]) : make_uint4(0, 0, 0, 0), x);
+                        quantize_chunk<false, true, FMT8, false, true>(x, a.q_pre, false, 3, 7, none, no, w8, s8);
+                        put(q, w8, s8);
+                    }
                 }
                 // so many rows are there: the lanes that own them take them
                 constexpr int AT_ONCE = G::QROWS * (D / 8) / 64;         // chunks

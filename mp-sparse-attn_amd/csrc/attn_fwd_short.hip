@@ -153,42 +153,51 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 3) void attn_short_kernel(Short
     __builtin_amdgcn_sched_barrier(0);
 
     auto put_q = [&](int c, uint32_t w4, int s4, uint2 w8, int s8) __attribute__((always_inline)) {
+        // (the four lanes of an MX block all write its scale byte: no branch)
         if constexpr (Q4) {
             *reinterpret_cast<uint32_t*>(smem + G::Q4 + c * 4) = w4;
-            if ((tid & 3) == 0) smem[G::QS4 + (c >> 2)] = (uint8_t)s4;
+            smem[G::QS4 + (c >> 2)] = (uint8_t)s4;
         }
         if constexpr (Q8) {
             *reinterpret_cast<uint2*>(smem + G::Q8 + c * 8) = w8;
-            if ((tid & 3) == 0) smem[G::QS8 + (c >> 2)] = (uint8_t)s8;
+            smem[G::QS8 + (c >> 2)] = (uint8_t)s8;
         }
     };
     if (a.q_raw) {
-        // Straight through, without a branch between the chunks, and with 8-bit codes without any (a check of the codes and a branch
-        // behind it cost 17 x 8 heads, 4601 queries over 18 keys, 8-bit, 75.8 -> 80.6 us); the rare chunk whose 4-bit codes the
-        // rule has to look at again starts from its 16-bit elements.
-        int e[CHUNKS];
-        bool again[CHUNKS], any = false;
-#pragma unroll
-        for (int q = 0; q < CHUNKS; ++q) {
-            const int c = q * 256 + tid;
-            float x[8];
-            uint32_t w4;
-            uint2 w8;
-            int s4, s8;
-            unpack8<PVT>(G::QR * p + c / (D / 8) < a.nq ? raw[q] : make_uint4(0, 0, 0, 0), x);
-            quantize_most<Q4, Q8, FMT8, false, true, true>(x, a.q_pre, a.q_sure != 0, 3, 7, w4, s4, w8, s8, again[q], e[q]);
-            any |= again[q];
-            put_q(c, w4, s4, w8, s8);
-        }
-        if (Q4 && any) {
+        // Straight through, without a branch between the chunks.  A wave with a rare chunk does all of its own again, and so do all
+        // where the 4-bit codes are the rule's to look at.  Rows past the last are zeros: nobody reads their results, but a maximum
+        // that moves moves for the whole wave.
+        bool again = Q4 && a.q_sure == 0;
+        auto inside = [&](int q) { return G::QR * p + (q * 256 + tid) / (D / 8) < a.nq; };
+        if (!again) {
+            bool rare = false;
 #pragma unroll
             for (int q = 0; q < CHUNKS; ++q) {
-                if (!again[q]) continue;
                 float x[8];
+                uint32_t w4 = 0;
+                uint2 w8 = make_uint2(0, 0);
+                int s4 = 0, s8 = 0;
+                bool r1;
                 unpack8<PVT>(raw[q], x);
+                const float pre = inside(q) ? a.q_pre : 0.0f;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] *= a.q_pre;
-                *reinterpret_cast<uint32_t*>(smem + G::Q4 + (q * 256 + tid) * 4) = e2m1_pack8_rule(x, e[q] - 3);
+                for (int i = 0; i < 8; ++i) x[i] *= pre;
+                quantize_straight<Q4, Q8, FMT8>(x, w4, s4, w8, s8, r1);
+                rare |= r1;
+                put_q(q * 256 + tid, w4, s4, w8, s8);
+            }
+            again = __ballot(rare) != 0;
+        }
+        if (again) {
+#pragma unroll
+            for (int q = 0; q < CHUNKS; ++q) {
+                float x[8];
+                uint32_t w4;
+                uint2 w8;
+                int s4, s8;
+                unpack8<PVT>(inside(q) ? only_here(raw[q]) : make_uint4(0, 0, 0, 0), x);
+                quantize_chunk<Q4, Q8, FMT8, false, true>(x, a.q_pre, a.q_sure != 0, 3, 7, w4, s4, w8, s8);
+                put_q(q * 256 + tid, w4, s4, w8, s8);
             }
         }
     } else {

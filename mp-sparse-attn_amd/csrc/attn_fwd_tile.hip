@@ -179,8 +179,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(AttnArgs a) {
         const Kept p = kept();
         uint32_t s4, s8;
         v8i none[SST];
-        if constexpr (IS8) quantize_query<PVT, FMT8, false, true>(raw, p->q_pre, p->q_sure != 0, none, s4, qf, s8);
-        else               quantize_query<PVT, FMT8, true, false>(raw, p->q_pre, p->q_sure != 0, qf, s4, none, s8);
+        if constexpr (IS8) quantize_query_careful<PVT, FMT8, false, true>(raw, p->q_pre, p->q_sure != 0, none, s4, qf, s8);
+        else               quantize_query_careful<PVT, FMT8, true, false>(raw, p->q_pre, p->q_sure != 0, qf, s4, none, s8);
         qsc = (int)(IS8 ? s8 : s4);
         const int nq = p->nq;
         if (i * TILE + 32 * wu + 31 >= nq) {              // a wave of the ragged last tile: its padding rows are zeros, as the quantizer pads them

@@ -214,11 +214,9 @@ __device__ __forceinline__ int block_exponent(float amax) {
 // One lane's eight elements (a quarter of an MX block; the quad's other lanes hold the rest): codes and the block's scale
 // bytes in the formats asked for.  x comes back multiplied by `pre`, e is the block's exponent.  Where `again` comes back
 // true, the caller has quantize_again finish the chunk: several chunks in a row share one branch that way, and run interleaved.
-// CLAMP8: the 8-bit codes are the careful ones at once, and never a reason for `again`: three instructions an element more, and no
-// branch.  That is the faster form where other code hangs on the branch -- the preparation (8 heads of 8192 x 128, 8-bit, 13.6 ->
-// 12.4 us; 64 of 1896 x 64 12.4 -> 11.4), and Q in the short-sequence kernel and the one that keeps K and V in LDS --, not in the
-// stand-alone quantizer (32 heads of 8192 x 128 16.6 -> 16.8, 8 5.5 -> 5.6).
-template <bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8 = false, bool STRAIGHT4 = false>
+// CLAMP8: the 8-bit codes are the careful ones at once, and never a reason for `again`: what quantize_straight's callers take rare
+// blocks to.
+template <bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8 = false>
 __device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool sure, int emax4, int emax8, uint32_t& w4, int& s4, uint2& w8, int& s8, bool& again, int& e) {
     float amax = 0.0f;
 #pragma unroll
@@ -238,7 +236,7 @@ __device__ __forceinline__ void quantize_most(float (&x)[8], float pre, bool sur
     if constexpr (DO4) {
         const int se = e - emax4;
         if constexpr (!SW8) {
-            w4 = e2m1_try8<STRAIGHT4>(x, se, sure, again);
+            w4 = e2m1_try8(x, se, sure, again);
             w4 = zero ? 0u : w4;
         }
         s4 = zero ? 0 : min(max(se + 127, 0), 254);
@@ -276,9 +274,60 @@ __device__ __forceinline__ void quantize_chunk(float (&x)[8], float pre, bool su
     if (again) quantize_again<DO4, DO8 && !CLAMP8, FMT8, SW8>(x, e, emax4, emax8, sure, w4, w8);
 }
 
+// What nearly every block is, without a branch: the shared exponents from the bits of the largest magnitude, by a maximum that NaN goes
+// through.  `rare`: a NaN, an infinity, or a scale so small that elements may be subnormal; nothing else here is to be used then.
+// The scale bytes of the others need no clamp, and their 8-bit codes stay below the format's maximum (emax 7).
+struct BlockScale {
+    static constexpr int EMAX4 = 3, EMAX8 = 7;
+    int biased;
+    bool zero, rare;
+    __device__ __forceinline__ int se4() const { return biased - EMAX4 - 127; }
+    __device__ __forceinline__ int se8() const { return biased - EMAX8 - 127; }
+    __device__ __forceinline__ int s4() const { return zero ? 0 : biased - EMAX4; }
+    __device__ __forceinline__ int s8() const { return zero ? 0 : biased - EMAX8; }
+};
+__device__ __forceinline__ BlockScale block_scale(uint32_t amax_bits) {
+    constexpr uint32_t LOW = (uint32_t)(SMALLEST_SE + 127 + BlockScale::EMAX8) << 23;
+    return {(int)(amax_bits >> 23), amax_bits == 0u, amax_bits != 0u && amax_bits - LOW >= 0x7F800000u - LOW};
+}
+
+// quantize_most that way, with half of its instructions (60 and 115 a chunk in both formats), so that several chunks run interleaved:
+// x holds products with the pre-scale; that none is near a midpoint is the caller's to know (`sure`).  Where `rare` comes back true
+// the caller takes the whole wave's chunks to quantize_chunk.  Whole calls, us: 32 query heads over 8, D = 128, causal, diag, 400 tokens
+// 12.8 -> 12.3, 1500 32.4 -> 31.1; 2 x 16 heads, 4096 queries over 333 keys, 8-bit, 39.1 -> 37.7.
+template <bool DO4, bool DO8, int FMT8>
+__device__ __forceinline__ void quantize_straight(const float (&x)[8], uint32_t& w4, int& s4, uint2& w8, int& s8, bool& rare) {
+    float amax = __builtin_fabsf(x[0]);
+#pragma unroll
+    for (int i = 1; i < 8; ++i) amax = __builtin_elementwise_maximum(amax, __builtin_fabsf(x[i]));
+    uint32_t ab = mpsa_f2u(amax);
+    ab = max(ab, dpp_u32<0xB1>(ab));                      // quad_perm [1,0,3,2]
+    ab = max(ab, dpp_u32<0x4E>(ab));                      // quad_perm [2,3,0,1]
+    const BlockScale b = block_scale(ab);
+    rare = b.rare;
+    if constexpr (DO4) {
+        s4 = b.s4();
+        w4 = e2m1_convert8(x, b.se4(), 1.0f);
+        w4 = b.zero ? 0u : w4;
+    }
+    if constexpr (DO8) {
+        s8 = b.s8();
+        w8 = fp8_convert8<FMT8>(x, b.se8());
+        w8.x = b.zero ? 0u : w8.x;
+        w8.y = b.zero ? 0u : w8.y;
+    }
+}
+
+// x, but nothing that is computed from it can be computed elsewhere: what only a rare path wants stays in it
+__device__ __forceinline__ uint4 only_here(uint4 x) {
+    asm("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
+    return x;
+}
+
 // One workgroup's share: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb (nh heads).
 // subtract(head, col8, x): what is taken off a row's chunk before anything else.
-template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8, typename Subtract>
+// STRAIGHT: the scale of every block by the formats' own emax (quantize_straight), without a branch: the preparation's form.
+template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8, bool STRAIGHT, typename Subtract>
 __device__ __forceinline__ void quantize_block_less(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh, Subtract subtract) {
     const uint32_t cpr = (uint32_t)a.d >> 3;                              // 16-byte chunks per row
     const uint32_t chunks = (uint32_t)a.out_rows * cpr;                   // per (b,h)
@@ -288,20 +337,32 @@ __device__ __forceinline__ void quantize_block_less(const QuantArgs& a, uint32_t
     const uint32_t col8 = c - row * cpr;
     const int64_t head = (int64_t)bb * nh + hh;                           // flat (b,h)
 
-    float x[8];
-    if (row < (uint32_t)a.n) {
-        const char* base = static_cast<const char*>(a.x) +
-                           2 * ((int64_t)bb * a.sb + (int64_t)hh * a.sh + (int64_t)row * a.sn + 8 * (int64_t)col8);
-        load8<XDT>(base, x);
-        subtract(head, col8, x);
-    } else {
+    uint4 raw = make_uint4(0, 0, 0, 0);
+    if (row < (uint32_t)a.n)
+        raw = *reinterpret_cast<const uint4*>(static_cast<const char*>(a.x) + 2 * ((int64_t)bb * a.sb + (int64_t)hh * a.sh + (int64_t)row * a.sn + 8 * (int64_t)col8));
+    uint32_t w4 = 0;
+    uint2 w8 = make_uint2(0, 0);
+    int s4 = 0, s8 = 0;
+    bool again = !STRAIGHT || (DO4 && !a.sure4);
+    auto chunk = [&](const uint4& from, float (&x)[8]) __attribute__((always_inline)) {
+        unpack8<XDT>(from, x);
+        if (row < (uint32_t)a.n) subtract(head, col8, x);
+    };
+    if constexpr (STRAIGHT) {
+        if (!again) {
+            float x[8];
+            chunk(raw, x);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = 0.0f;
+            for (int i = 0; i < 8; ++i) x[i] *= a.pre;
+            quantize_straight<DO4, DO8, FMT8>(x, w4, s4, w8, s8, again);
+            again = __ballot(again) != 0;
+        }
     }
-    uint32_t w4;
-    uint2 w8;
-    int s4, s8;
-    quantize_chunk<DO4, DO8, FMT8, SW8, CLAMP8>(x, a.pre, a.sure4 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
+    if (again) {
+        float x[8];
+        chunk(STRAIGHT ? only_here(raw) : raw, x);
+        quantize_chunk<DO4, DO8, FMT8, SW8, STRAIGHT>(x, a.pre, a.sure4 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
+    }
     const int64_t oc = head * chunks + c;                                 // flat output chunk
     int64_t os = oc >> 2;                                                 // and scale
     if (a.scales5d) {
@@ -330,9 +391,9 @@ __device__ __forceinline__ void less_mean(float (&x)[8], const uint4& mean) {
     for (int i = 0; i < 8; ++i) x[i] = round16<XDT>(x[i] - m[i]);
 }
 
-template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8, bool CLAMP8 = false>
+template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8, bool STRAIGHT = false>
 __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh) {
-    quantize_block_less<XDT, DO4, DO8, FMT8, SW8, CLAMP8>(a, bx, hh, bb, nh, [&](int64_t head, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
+    quantize_block_less<XDT, DO4, DO8, FMT8, SW8, STRAIGHT>(a, bx, hh, bb, nh, [&](int64_t head, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
         if (a.sub) less_mean<XDT>(x, *reinterpret_cast<const uint4*>(static_cast<const char*>(a.sub) + 2 * (head * a.d + 8 * (int64_t)col8)));
     });
 }

@@ -892,6 +892,35 @@ def test_odd_values_of_q_quantize_to_the_same_codes_in_every_kernel(bst, dtype):
         assert same(a, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bst", ["diag", "mxfp4", "mxfp8", "mixed"])
+def test_rare_blocks_of_q_and_k_under_a_scale_that_needs_no_check(bst, dtype):
+    """Blocks that the conversions are not the rule for -- NaN, infinities, scales too small --, blocks of zeros and a ragged last
+    block, with a pre-scale whose products are never near a midpoint (the default one): codes and scale bytes of the preparation are the
+    stand-alone quantizer's, and kernels that quantize Q themselves give the bits of prepared Q."""
+    from ours.mxfp_attn_kernel import prepare_operands, attention_from_operands
+    from ours.quant_mxint8 import quantize_mx
+    N = 845
+    q, k, v = make_qkv(1, 4, 2, N, 128, seed=80, dtype=torch.float32)
+    for x in (q, k):
+        x[0, 1, 80, 40], x[0, 1, 81, 41], x[0, 0, 333, 3], x[0, 1, 844, 127] = float("nan"), float("inf"), float("-inf"), float("nan")
+        x[0, 0, 90, 32:64], x[0, 0, 91] = 0.0, 0.0
+        x[0, 1, 200:204, :32] *= 1e-7 if dtype == torch.float16 else 1e-34
+    q, k, v = (t.to(dtype).to(DEV) for t in (q, k, v))
+    ops = prepare_operands(q, k, v, 128, bst)
+    for x, names in ((q, "q"), (k, "k")):
+        for bits, fmt in (("4", _lib.FMT_E2M1), ("8", ops["fmt8"])):
+            codes, scales = ops[names + bits], ops[names + "s" + bits]
+            if codes is not None:
+                c, s = quantize_mx(x, ops["pre"] if names == "q" else 1.0, fmt)
+                assert torch.equal(codes[:, :, :N], c) and torch.equal(scales[:, :, :N], s) and not codes[:, :, N:].any() and not scales[:, :, N:].any()
+    for kernel in ("paired", "short1", "short2", "short4"):
+        a, b = (torch.empty((1, 4, N, 128), dtype=torch.float32, device=DEV) for _ in range(2))
+        attention_from_operands(ops, a, True, kernel=kernel)
+        attention_from_operands(prepare_operands(q, k, v, 128, bst, fuse_q=True), b, True, kernel=kernel)
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a, nan=0.0), torch.nan_to_num(b, nan=0.0)), kernel
+
+
 def test_q16_entry_point_rejects_other_shapes():
     L = _lib.lib()
     assert L.mpsa_attn_fwd_q16_supported(1, 32, 8, 8192, 128, 128, 1, _lib.MODE_DIAG) == 1
