@@ -1,11 +1,12 @@
 // One-launch operand preparation for the fused attention kernel (gfx950): the MX quantization of Q (with
 // sm_scale*log2(e) folded in) and of K (optionally minus its sequence mean) and the value-tile repack of V run as
 // three groups of workgroups of ONE kernel instead of three launches - at the benchmark shape the three kernels take
-// about 45 us together and the gaps between their launches another 20.  The work per workgroup is exactly that of
-// quantize_kernel / v_tiles_kernel (quantize_kernel.h, v_tiles_kernel.h); this file only routes workgroup ids.
+// about 45 us together and the gaps between their launches another 20.  The quantizer's and the repack's own code
+// (quantize_kernel.h, v_tiles_kernel.h); this file routes workgroup ids.
 // Replaces the prologue of the reference's wrapper, ours/mxfp_attn_kernel.py:27-57 (dtype normalisation, quant_mxfp4 /
 // quant_mxfp8e5 calls, operand packaging).
 #include "seq_mean_kernel.h"
+#include "reciprocal.h"
 #include "v_tiles_kernel.h"
 
 namespace {
@@ -13,9 +14,10 @@ namespace {
 struct PrepArgs {
     QuantArgs q, k;
     VTArgs v;
+    Reciprocal by_bq, by_bk, by_bv, by_hq, by_hkv;
     uint32_t bq, bk, bv;          // workgroups per (batch, head) of each job
     uint32_t hq, hkv;
-    uint32_t q_total, k_total, v_total;    // blocks of the Q job, of the K job, of the V job
+    uint32_t q_total, k_total;    // of the Q job, of the K job
     const float* sums;            // [B,Hkv,nchunk,D]: sums of chunks of K's rows (MEAN_SUMS)
     int nchunk;
     float inv_n;
@@ -51,43 +53,42 @@ __device__ __forceinline__ void head_mean(const PrepArgs& p, uint32_t hh, uint32
     __syncthreads();
 }
 
+// A workgroup takes 512 chunks of one head, two a thread, and asks for both before it does anything else (a padded head has a
+// whole number of 512: 64 rows of 64).  What bounds it for short sequences is the wait for memory, and two blocks of 256 one after the
+// other, as it was, waited twice.  With V's rows read four bytes a lane instead of two, whole calls, us: 32 heads over 8, D = 128, causal,
+// diag: 160 tokens 9.44 -> 8.75, 1000 21.7 -> 20.4, 8192 327.8 -> 323.5; 8 heads of 1024 x 64 with the mean 15.45 -> 14.66; 40 heads of
+// 300 x 128 19.3 -> 17.7.  Four chunks a thread, and four words of V, take 0.98 to 1.03 of that.
 template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D, int SOURCE>
-__device__ __forceinline__ void prepare_block(const PrepArgs& p, uint32_t blk, bool again) {
+__global__ __launch_bounds__(256) void prepare_kernel(PrepArgs p) {
+    uint32_t blk = blockIdx.x;
     if (blk < p.q_total) {
-        const uint32_t head = blk / p.bq;
-        quantize_block<XDT, DO4, DO8, FMT8, false, true>(p.q, blk - head * p.bq, head % p.hq, head / p.hq, p.hq);
+        const uint32_t head = divide_by(blk, p.by_bq), bb = divide_by(head, p.by_hq), hh = head - bb * p.hq, c = (blk - head * p.bq) * 512u + threadIdx.x;
+        QuantChunk q[2] = {QuantChunk(p.q, c), QuantChunk(p.q, c + 256u)};
+        q[0].request(p.q, hh, bb);
+        q[1].request(p.q, hh, bb);
+        quantize_chunks<XDT, DO4, DO8, FMT8>(p.q, q, head, [](int64_t, uint32_t, float (&)[8]) __attribute__((always_inline)) {});
         return;
     }
     blk -= p.q_total;
     if (blk < p.k_total) {
-        const uint32_t head = blk / p.bk;
+        const uint32_t head = divide_by(blk, p.by_bk), bb = divide_by(head, p.by_hkv), hh = head - bb * p.hkv, c = (blk - head * p.bk) * 512u + threadIdx.x;
+        QuantChunk q[2] = {QuantChunk(p.k, c), QuantChunk(p.k, c + 256u)};
+        q[0].request(p.k, hh, bb);
+        q[1].request(p.k, hh, bb);
         if constexpr (SOURCE == MEAN_SUMS || SOURCE == MEAN_ROWS_ITSELF) {
             __shared__ __attribute__((aligned(16))) uint16_t mean[D];
-            // (the second block of a workgroup is mostly of the first one's head)
-            if (!again || blk % p.bk == 0) {
-                if (again) __syncthreads();      // the other head's mean has been read
-                head_mean<XDT, SOURCE, D>(p, head % p.hkv, head / p.hkv, mean);
-            }
-            quantize_block_less<XDT, DO4, DO8, FMT8, false, true>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv,
-                                                            [&](int64_t, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
+            head_mean<XDT, SOURCE, D>(p, hh, bb, mean);
+            quantize_chunks<XDT, DO4, DO8, FMT8>(p.k, q, head, [&](int64_t, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
                 less_mean<XDT>(x, *reinterpret_cast<const uint4*>(mean + 8 * col8));
             });
         } else {
-            quantize_block<XDT, DO4, DO8, FMT8, false, true>(p.k, blk - head * p.bk, head % p.hkv, head / p.hkv, p.hkv);
+            quantize_chunks<XDT, DO4, DO8, FMT8>(p.k, q, head, [&](int64_t hd, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) { less_given<XDT>(p.k, hd, col8, x); });
         }
         return;
     }
     blk -= p.k_total;
-    if (blk >= p.v_total) return;
-    const uint32_t head = blk / p.bv;
-    v_tiles_block<TILE, D>(p.v, blk - head * p.bv, head % p.hkv, head / p.hkv, p.hkv);
-}
-
-// two blocks of work per workgroup (measured on the stand-alone quantizer: 8-13 % more bandwidth than one)
-template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D, int SOURCE>
-__global__ __launch_bounds__(256) void prepare_kernel(PrepArgs p) {
-    prepare_block<XDT, DO4, DO8, FMT8, TILE, D, SOURCE>(p, 2 * blockIdx.x, false);
-    prepare_block<XDT, DO4, DO8, FMT8, TILE, D, SOURCE>(p, 2 * blockIdx.x + 1, true);
+    const uint32_t head = divide_by(blk, p.by_bv), bb = divide_by(head, p.by_hkv);
+    v_tiles_block<TILE, D>(p.v, blk - head * p.bv, head - bb * p.hkv, bb, p.hkv);
 }
 
 template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D>
@@ -173,17 +174,19 @@ int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k
     if (rc != MPSA_OK) return rc;
     rc = mpsa_v_tiles_setup(v, dtype, B, Hkv, Nk, D, v_strides, tile, v_tiles, &p.v, &bv);
     if (rc != MPSA_OK) return rc;
+    bq /= 2;                                     // the set-ups count blocks of 256 chunks
+    bk /= 2;
     const int64_t total = (int64_t)bq * Hq * B + (int64_t)(bk + bv) * Hkv * B;
-    if (total >= (int64_t(1) << 31)) return mpsa_fail(MPSA_EUNSUPPORTED, "prepare: problem too large for one launch");
+    if (total >= (int64_t(1) << 30)) return mpsa_fail(MPSA_EUNSUPPORTED, "prepare: problem too large for one launch");
     p.bq = bq; p.bk = bk; p.bv = bv; p.hq = (uint32_t)Hq; p.hkv = (uint32_t)Hkv;
+    p.by_bq = reciprocal_of(bq ? bq : 1); p.by_bk = reciprocal_of(bk); p.by_bv = reciprocal_of(bv); p.by_hq = reciprocal_of(p.hq); p.by_hkv = reciprocal_of(p.hkv);
     p.q_total = (uint32_t)((int64_t)bq * Hq * B); p.k_total = (uint32_t)((int64_t)bk * Hkv * B);
-    p.v_total = (uint32_t)((int64_t)bv * Hkv * B);
     p.sums = mean == MEAN_SUMS ? static_cast<const float*>(k_sub) : nullptr;
     p.nchunk = (int)((Nk + MEAN_ROWS - 1) / MEAN_ROWS);
     p.inv_n = 1.0f / (float)Nk;
     const bool do4 = q_do4 || k_do4, do8 = q_do8 || k_do8;
-    if (dtype == MPSA_BF16) launch_mode<MPSA_BF16>(p, do4, do8, fmt8, tile, (int)D, mean, (unsigned)((total + 1) / 2), st);
-    else                    launch_mode<MPSA_F16>(p, do4, do8, fmt8, tile, (int)D, mean, (unsigned)((total + 1) / 2), st);
+    if (dtype == MPSA_BF16) launch_mode<MPSA_BF16>(p, do4, do8, fmt8, tile, (int)D, mean, (unsigned)total, st);
+    else                    launch_mode<MPSA_F16>(p, do4, do8, fmt8, tile, (int)D, mean, (unsigned)total, st);
     MPSA_CHECK_LAUNCH("prepare");
     return MPSA_OK;
 }

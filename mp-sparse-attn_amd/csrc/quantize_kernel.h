@@ -324,50 +324,32 @@ __device__ __forceinline__ uint4 only_here(uint4 x) {
     return x;
 }
 
-// One workgroup's share: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb (nh heads).
-// subtract(head, col8, x): what is taken off a row's chunk before anything else.
-// STRAIGHT: the scale of every block by the formats' own emax (quantize_straight), without a branch: the preparation's form.
-template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8, bool STRAIGHT, typename Subtract>
-__device__ __forceinline__ void quantize_block_less(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh, Subtract subtract) {
-    const uint32_t cpr = (uint32_t)a.d >> 3;                              // 16-byte chunks per row
-    const uint32_t chunks = (uint32_t)a.out_rows * cpr;                   // per (b,h)
-    const uint32_t c = bx * 256u + threadIdx.x;
-    if (c >= chunks) return;                                              // whole quads leave together (cpr % 4 == 0)
-    const uint32_t row = c / cpr;
-    const uint32_t col8 = c - row * cpr;
-    const int64_t head = (int64_t)bb * nh + hh;                           // flat (b,h)
+// The chunk of 16 bytes that a thread quantizes: number c of a head's, in the outputs; rows past the last count as zeros.
+struct QuantChunk {
+    uint32_t c, row, col8;
+    uint4 raw;
+    __device__ __forceinline__ QuantChunk(const QuantArgs& a, uint32_t number) : c(number) {
+        const uint32_t cpr = (uint32_t)a.d >> 3;                          // 16-byte chunks per row
+        row = c / cpr;
+        col8 = c - row * cpr;
+    }
+    __device__ __forceinline__ bool inside(const QuantArgs& a) const { return row < (uint32_t)a.n; }
+    __device__ __forceinline__ const uint4* at(const QuantArgs& a, uint32_t r, uint32_t hh, uint32_t bb) const {
+        return reinterpret_cast<const uint4*>(static_cast<const char*>(a.x) + 2 * ((int64_t)bb * a.sb + (int64_t)hh * a.sh + (int64_t)r * a.sn + 8 * (int64_t)col8));
+    }
+    // from a head with a row; what lies past the last one is left to quantize_chunks
+    __device__ __forceinline__ void request(const QuantArgs& a, uint32_t hh, uint32_t bb) { raw = *at(a, min(row, (uint32_t)a.n - 1u), hh, bb); }
+};
 
-    uint4 raw = make_uint4(0, 0, 0, 0);
-    if (row < (uint32_t)a.n)
-        raw = *reinterpret_cast<const uint4*>(static_cast<const char*>(a.x) + 2 * ((int64_t)bb * a.sb + (int64_t)hh * a.sh + (int64_t)row * a.sn + 8 * (int64_t)col8));
-    uint32_t w4 = 0;
-    uint2 w8 = make_uint2(0, 0);
-    int s4 = 0, s8 = 0;
-    bool again = !STRAIGHT || (DO4 && !a.sure4);
-    auto chunk = [&](const uint4& from, float (&x)[8]) __attribute__((always_inline)) {
-        unpack8<XDT>(from, x);
-        if (row < (uint32_t)a.n) subtract(head, col8, x);
-    };
-    if constexpr (STRAIGHT) {
-        if (!again) {
-            float x[8];
-            chunk(raw, x);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] *= a.pre;
-            quantize_straight<DO4, DO8, FMT8>(x, w4, s4, w8, s8, again);
-            again = __ballot(again) != 0;
-        }
-    }
-    if (again) {
-        float x[8];
-        chunk(STRAIGHT ? only_here(raw) : raw, x);
-        quantize_chunk<DO4, DO8, FMT8, SW8, STRAIGHT>(x, a.pre, a.sure4 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
-    }
-    const int64_t oc = head * chunks + c;                                 // flat output chunk
+// head: the flat (batch, head)
+template <bool DO4, bool DO8>
+__device__ __forceinline__ void store_chunk(const QuantArgs& a, const QuantChunk& q, int64_t head, uint32_t w4, int s4, uint2 w8, int s8) {
+    const uint32_t cpr = (uint32_t)a.d >> 3, chunks = (uint32_t)a.out_rows * cpr;
+    const int64_t oc = head * chunks + q.c;                               // flat output chunk
     int64_t os = oc >> 2;                                                 // and scale
     if (a.scales5d) {
-        const uint32_t kc = cpr >> 4, block = col8 >> 2;
-        os = head * (chunks >> 2) + (((int64_t)(row >> 7) * kc + (block >> 2)) << 9) + ((row & 31) << 4) + ((row >> 5 & 3) << 2) + (block & 3);
+        const uint32_t kc = cpr >> 4, block = q.col8 >> 2;
+        os = head * (chunks >> 2) + (((int64_t)(q.row >> 7) * kc + (block >> 2)) << 9) + ((q.row & 31) << 4) + ((q.row >> 5 & 3) << 2) + (block & 3);
     }
     const bool quad_leader = (threadIdx.x & 3u) == 0u;
     // an output set that is not wanted has no pointer (one side of a mixed preparation: 8-bit Q, 4-bit K)
@@ -382,6 +364,46 @@ __device__ __forceinline__ void quantize_block_less(const QuantArgs& a, uint32_t
     }
 }
 
+// Several chunks of a thread, straight through (the formats' own emax): the preparation's form.
+// subtract(head, col8, x): what is taken off a row's chunk before anything else.
+template <int XDT, bool DO4, bool DO8, int FMT8, int N, typename Subtract>
+__device__ __forceinline__ void quantize_chunks(const QuantArgs& a, const QuantChunk (&q)[N], int64_t head, Subtract subtract) {
+    uint32_t w4[N];
+    uint2 w8[N];
+    int s4[N], s8[N];
+    bool again = DO4 && !a.sure4;
+    if (!again) {
+        bool rare = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float x[8];
+            bool r;
+            unpack8<XDT>(q[i].raw, x);
+            subtract(head, q[i].col8, x);
+            const float pre = q[i].inside(a) ? a.pre : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] *= pre;
+            w4[i] = 0; s4[i] = 0; w8[i] = make_uint2(0, 0); s8[i] = 0;
+            quantize_straight<DO4, DO8, FMT8>(x, w4[i], s4[i], w8[i], s8[i], r);
+            rare |= r;
+        }
+        again = __ballot(rare) != 0;
+    }
+    if (again) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float x[8];
+            unpack8<XDT>(only_here(q[i].raw), x);
+            subtract(head, q[i].col8, x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = q[i].inside(a) ? x[e] : 0.0f;
+            quantize_chunk<DO4, DO8, FMT8, false, true>(x, a.pre, a.sure4 != 0, a.emax4, a.emax8, w4[i], s4[i], w8[i], s8[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) store_chunk<DO4, DO8>(a, q[i], head, w4[i], s4[i], w8[i], s8[i]);
+}
+
 // x - m in the inputs' 16-bit type
 template <int XDT>
 __device__ __forceinline__ void less_mean(float (&x)[8], const uint4& mean) {
@@ -391,11 +413,32 @@ __device__ __forceinline__ void less_mean(float (&x)[8], const uint4& mean) {
     for (int i = 0; i < 8; ++i) x[i] = round16<XDT>(x[i] - m[i]);
 }
 
-template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8, bool STRAIGHT = false>
+// takes the mean that the caller has at hand off a chunk (quantize_chunks)
+template <int XDT>
+__device__ __forceinline__ void less_given(const QuantArgs& a, int64_t head, uint32_t col8, float (&x)[8]) {
+    if (a.sub) less_mean<XDT>(x, *reinterpret_cast<const uint4*>(static_cast<const char*>(a.sub) + 2 * (head * a.d + 8 * (int64_t)col8)));
+}
+
+// One workgroup's share in the stand-alone kernels: 256 consecutive 16-byte chunks, starting at chunk 256*bx, of head hh of batch bb
+// (nh heads).
+template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8>
 __device__ __forceinline__ void quantize_block(const QuantArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh) {
-    quantize_block_less<XDT, DO4, DO8, FMT8, SW8, STRAIGHT>(a, bx, hh, bb, nh, [&](int64_t head, uint32_t col8, float (&x)[8]) __attribute__((always_inline)) {
-        if (a.sub) less_mean<XDT>(x, *reinterpret_cast<const uint4*>(static_cast<const char*>(a.sub) + 2 * (head * a.d + 8 * (int64_t)col8)));
-    });
+    QuantChunk q(a, bx * 256u + threadIdx.x);
+    if (q.c >= (uint32_t)a.out_rows * ((uint32_t)a.d >> 3)) return;       // whole quads leave together (d % 32 == 0)
+    const int64_t head = (int64_t)bb * nh + hh;                           // flat (b,h)
+    float x[8];
+    if (q.inside(a)) {
+        unpack8<XDT>(*q.at(a, q.row, hh, bb), x);
+        less_given<XDT>(a, head, q.col8, x);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = 0.0f;
+    }
+    uint32_t w4;
+    uint2 w8;
+    int s4, s8;
+    quantize_chunk<DO4, DO8, FMT8, SW8, false>(x, a.pre, a.sure4 != 0, a.emax4, a.emax8, w4, s4, w8, s8);
+    store_chunk<DO4, DO8>(a, q, head, w4, s4, w8, s8);
 }
 
 template <int XDT, bool DO4, bool DO8, int FMT8, bool SW8>

@@ -32,7 +32,8 @@ int mpsa_v_tiles_setup(const void* v, int v_dtype, int64_t B, int64_t H, int64_t
     a.sb = v_strides[0]; a.sh = v_strides[1]; a.sn = v_strides[2];
     a.n = (int)N; a.nt = (int)nt;
     a.out = static_cast<unsigned short*>(v_tiles);
-    *blocks = (unsigned)((per_head + 255) / 256);
+    a.pairs = (reinterpret_cast<uintptr_t>(v) & 3) == 0 && !((v_strides[0] | v_strides[1] | v_strides[2]) & 1);
+    *blocks = (unsigned)(per_head / 512);          // a whole number: a tile has 512 words or more
     return MPSA_OK;
 }
 

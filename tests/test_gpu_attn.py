@@ -892,6 +892,25 @@ def test_odd_values_of_q_quantize_to_the_same_codes_in_every_kernel(bst, dtype):
         assert same(a, b)
 
 
+@pytest.mark.parametrize("D,tile", [(128, 128), (64, 128), (128, 64), (64, 64)])
+@pytest.mark.parametrize("N", [1, 11, 64, 200, 513])
+@pytest.mark.parametrize("odd_rows", [False, True])
+def test_value_tiles_are_the_matrix_operand_order(D, tile, N, odd_rows):
+    """mpsa_v_tiles against the layout written out: word (tile, 32 keys, 16 keys, 32 channels, lane) holds eight keys of one channel,
+    zeros past the last key.  odd_rows: rows that start at any 2-byte address."""
+    g = torch.Generator().manual_seed(N)
+    base = torch.randn(2, 3, N, D + 1, generator=g).bfloat16().to(DEV)
+    v = base[..., 1:] if odd_rows else base[..., 1:].contiguous()
+    nt = (N + tile - 1) // tile
+    out = torch.empty((2, 3, nt, tile * D), dtype=torch.bfloat16, device=DEV)
+    _lib.check(_lib.lib().mpsa_v_tiles(_lib.ptr(v), _lib.BF16, 2, 3, N, D, _lib.strides4(v), tile, _lib.ptr(out), _lib.stream_ptr()))
+    padded = torch.zeros((2, 3, nt * tile, D), dtype=torch.bfloat16)
+    padded[:, :, :N] = v.cpu()
+    # keys as [tile, 32s, 16s, t / 4, h, t % 4], channels as [32s, r]; words in the order tile, 32s, 16s, channel 32s, h, r, t
+    want = padded.view(2, 3, nt, tile // 32, 2, 2, 2, 4, D // 32, 32).permute(0, 1, 2, 3, 4, 8, 6, 9, 5, 7).reshape(2, 3, nt, tile * D)
+    assert torch.equal(out.cpu(), want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bst", ["diag", "mxfp4", "mxfp8", "mixed"])
 def test_rare_blocks_of_q_and_k_under_a_scale_that_needs_no_check(bst, dtype):
