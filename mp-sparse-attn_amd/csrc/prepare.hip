@@ -23,8 +23,13 @@ struct PrepArgs {
     float inv_n;
 };
 
+// Threads of a workgroup, each with two chunks (and two words of V).  One that adds up its head's rows itself has twice as many: there
+// are half as many to read the whole head, and its rows are asked for in half as many rounds.
+__host__ __device__ constexpr int threads_of(int source) { return source == MEAN_ROWS_ITSELF ? 512 : 256; }
+
 // The mean over the sequence of one head of K, in the inputs' type, into LDS: from the chunks' sums, or from the rows
-// themselves (256 / D chunks at most, all asked for at once).  The additions of mpsa_seq_mean in their order, so its bits.
+// themselves (1024 at most, all asked for at once).  The additions of mpsa_seq_mean in their order, so its bits.
+constexpr int MEAN_CHUNKS = 4;
 template <int XDT, int SOURCE, int D>
 __device__ __forceinline__ void head_mean(const PrepArgs& p, uint32_t hh, uint32_t bb, uint16_t* mean) {
     const int c = threadIdx.x;
@@ -32,21 +37,27 @@ __device__ __forceinline__ void head_mean(const PrepArgs& p, uint32_t hh, uint32
     if constexpr (SOURCE == MEAN_SUMS) {
         if (c < D) s = seq_sum(p.sums + ((int64_t)bb * p.hkv + hh) * p.nchunk * D + c, p.nchunk, D);
     } else {
-        constexpr int CHUNKS = 256 / D;
-        __shared__ float part[CHUNKS][256][9], sums[256];
+        constexpr int GROUPS = threads_of(SOURCE) / 256, SLOTS = MEAN_CHUNKS / GROUPS;      // of 256 threads; chunks of 256 rows each
+        static_assert(MEAN_CHUNKS * D <= threads_of(SOURCE), "a thread a sum");
+        __shared__ float part[MEAN_CHUNKS][256][9], sums[MEAN_CHUNKS * D];
         const char* head = static_cast<const char*>(p.k.x) + 2 * ((int64_t)bb * p.k.sb + (int64_t)hh * p.k.sh);
-        MeanChunk<D> chunk[CHUNKS];
+        const int group = __builtin_amdgcn_readfirstlane(c >> 8);
+        MeanChunk<D> chunk[SLOTS];
 #pragma unroll
-        for (int k = 0; k < CHUNKS; ++k)
-            if (k < p.nchunk) chunk[k].request(head, p.k.sn, k * MEAN_ROWS, p.k.n);
+        for (int y = 0; y < SLOTS; ++y) {
+            const int k = y * GROUPS + group;
+            if (k < p.nchunk) chunk[y].request(head, p.k.sn, k * MEAN_ROWS, p.k.n, c & 255);
+        }
 #pragma unroll
-        for (int k = 0; k < CHUNKS; ++k)
-            if (k < p.nchunk) chunk[k].template add<XDT>(part[k], k * MEAN_ROWS, p.k.n);
+        for (int y = 0; y < SLOTS; ++y) {
+            const int k = y * GROUPS + group;
+            if (k < p.nchunk) chunk[y].template add<XDT>(part[k], k * MEAN_ROWS, p.k.n, c & 255);
+        }
         __syncthreads();
         if (c / D < p.nchunk) sums[c] = MeanChunk<D>::total(part[c / D], c % D);
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < CHUNKS; ++k)
+        for (int k = 0; k < MEAN_CHUNKS; ++k)
             if (k < p.nchunk) s += sums[k * D + c % D];
     }
     if (c < D) mean[c] = mean_bits<XDT>(s * p.inv_n);
@@ -59,11 +70,12 @@ __device__ __forceinline__ void head_mean(const PrepArgs& p, uint32_t hh, uint32
 // diag: 160 tokens 9.44 -> 8.75, 1000 21.7 -> 20.4, 8192 327.8 -> 323.5; 8 heads of 1024 x 64 with the mean 15.45 -> 14.66; 40 heads of
 // 300 x 128 19.3 -> 17.7.  Four chunks a thread, and four words of V, take 0.98 to 1.03 of that.
 template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D, int SOURCE>
-__global__ __launch_bounds__(256) void prepare_kernel(PrepArgs p) {
+__global__ __launch_bounds__(threads_of(SOURCE)) void prepare_kernel(PrepArgs p) {
+    constexpr uint32_t THREADS = threads_of(SOURCE);
     uint32_t blk = blockIdx.x;
     if (blk < p.q_total) {
-        const uint32_t head = divide_by(blk, p.by_bq), bb = divide_by(head, p.by_hq), hh = head - bb * p.hq, c = (blk - head * p.bq) * 512u + threadIdx.x;
-        QuantChunk q[2] = {QuantChunk(p.q, c), QuantChunk(p.q, c + 256u)};
+        const uint32_t head = divide_by(blk, p.by_bq), bb = divide_by(head, p.by_hq), hh = head - bb * p.hq, c = (blk - head * p.bq) * (2 * THREADS) + threadIdx.x;
+        QuantChunk q[2] = {QuantChunk(p.q, c), QuantChunk(p.q, c + THREADS)};
         q[0].request(p.q, hh, bb);
         q[1].request(p.q, hh, bb);
         quantize_chunks<XDT, DO4, DO8, FMT8>(p.q, q, head, [](int64_t, uint32_t, float (&)[8]) __attribute__((always_inline)) {});
@@ -71,8 +83,8 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepArgs p) {
     }
     blk -= p.q_total;
     if (blk < p.k_total) {
-        const uint32_t head = divide_by(blk, p.by_bk), bb = divide_by(head, p.by_hkv), hh = head - bb * p.hkv, c = (blk - head * p.bk) * 512u + threadIdx.x;
-        QuantChunk q[2] = {QuantChunk(p.k, c), QuantChunk(p.k, c + 256u)};
+        const uint32_t head = divide_by(blk, p.by_bk), bb = divide_by(head, p.by_hkv), hh = head - bb * p.hkv, c = (blk - head * p.bk) * (2 * THREADS) + threadIdx.x;
+        QuantChunk q[2] = {QuantChunk(p.k, c), QuantChunk(p.k, c + THREADS)};
         q[0].request(p.k, hh, bb);
         q[1].request(p.k, hh, bb);
         if constexpr (SOURCE == MEAN_SUMS || SOURCE == MEAN_ROWS_ITSELF) {
@@ -88,14 +100,14 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepArgs p) {
     }
     blk -= p.k_total;
     const uint32_t head = divide_by(blk, p.by_bv), bb = divide_by(head, p.by_hkv);
-    v_tiles_block<TILE, D>(p.v, blk - head * p.bv, head - bb * p.hkv, bb, p.hkv);
+    v_tiles_block<TILE, D, THREADS>(p.v, blk - head * p.bv, head - bb * p.hkv, bb, p.hkv);
 }
 
 template <int XDT, bool DO4, bool DO8, int FMT8, int TILE, int D>
 void launch_source(const PrepArgs& p, MeanSource source, unsigned grid, hipStream_t st) {
-    if (source == MEAN_SUMS)             hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_SUMS>), dim3(grid), dim3(256), 0, st, p);
-    else if (source == MEAN_ROWS_ITSELF) hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_ROWS_ITSELF>), dim3(grid), dim3(256), 0, st, p);
-    else                                 hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_GIVEN>), dim3(grid), dim3(256), 0, st, p);
+    if (source == MEAN_SUMS)             hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_SUMS>), dim3(grid), dim3(threads_of(MEAN_SUMS)), 0, st, p);
+    else if (source == MEAN_ROWS_ITSELF) hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_ROWS_ITSELF>), dim3(grid), dim3(threads_of(MEAN_ROWS_ITSELF)), 0, st, p);
+    else                                 hipLaunchKernelGGL((prepare_kernel<XDT, DO4, DO8, FMT8, TILE, D, MEAN_GIVEN>), dim3(grid), dim3(threads_of(MEAN_GIVEN)), 0, st, p);
 }
 
 template <int XDT, bool DO4, bool DO8, int FMT8>
@@ -122,19 +134,20 @@ void launch_mode(const PrepArgs& p, bool do4, bool do8, int fmt8, int tile, int 
 
 // Where the mean over K's sequence comes from.  On its own it takes two launches (sums of chunks of 256 rows; their sum), each
 // of which costs the host as much as the preparation does and the device a round trip to memory.  The preparation's workgroups
-// can add up the chunks' sums themselves, or, where a head is at most 128 KiB, its rows: every workgroup reads the whole head,
-// 512 of whose 16-byte pieces it quantizes, which pays until all of them together read some two million pieces.  Microseconds
-// of a call's kernels with the mean on its own, from sums, from rows (pieces in millions): 8 heads, 512 x 128, 16.6 15.4 12.9
-// (1.0); 8 of 1024 x 64 16.9 15.7 14.7 (1.0); 2 x 16 of 333 x 128, 4096 queries, 46.4 44.1 40.6 (1.8); 2 x 32 of 512 x 64 22.5
-// 21.0 20.8 (2.1); 4 x 32 of 512 x 64 27.4 25.2 30.0 (4.2); 2 x 24 of 512 x 128, 4096 queries, 61.4 59.7 61.3 (6.3).  Sums up to
+// can add up the chunks' sums themselves, or its rows: every workgroup reads the whole head, 1024 of whose 16-byte pieces it
+// quantizes.  That pays while the rows are asked for at once and the workgroups are one or two a CU: of 130 shapes (2 to 64 heads, 80 to 2600
+// keys, both widths) all 89 within these bounds are faster that way, by up to 5 us.  Microseconds of whole calls, from sums,
+// from rows (workgroups): 16 heads of 1018 x 128 24.0 21.1 (256); 32 of 653 x 128 31.6 30.1 (352); 48 of 512 x 128 44.7 44.1 (384);
+// 32 of 779 x 128 25.5 26.6 (416); 48 of 611 x 128 27.1 28.3 (480); 32 of 1018 x 64 19.3 17.7 (256); 64 of 1024 x 64 29.7 32.1 (512); past
+// 1024 rows 8 of 1443 x 128 24.7 22.5, 16 of 1414 x 128 31.2 34.8, 4 of 1146 x 128 17.8 19.0, 8 of 1281 x 64 15.4 16.7.  Sums up to
 // 64 chunks (32 heads, 4096 x 64, 86.4 -> 84.8) and where the workgroups together read 14 MB of them at most: every one of a head
 // reads them all, which is quadratic in the keys.  A mean of its own against sums, whole calls of 128 queries, us (MB): 8 heads
 // of 4096 x 128 36.6 35.2 (8.4), 6144 44.1 44.1 (19), 16384 88.9 94.9 (134); 40 of 2048 x 128 36.3 36.5 (10), 4096 55.3 57.7 (42),
 // 8656 116 129 (187); 24 of 8192 x 64 53.5 53.6 (25), 16000 92 97 (96).
 MeanSource mpsa_mean_source(int64_t B, int64_t Hkv, int64_t nk, int64_t D) {
     if (mpsa_quantize_sw_encoders()) return MEAN_GIVEN;      // stand-alone kernels
-    const double pieces = (double)nk * (double)D / 8.0;
-    if (pieces <= 8192.0 && (double)(B * Hkv) * pieces * pieces / 512.0 <= 2.2e6) return MEAN_ROWS_ITSELF;
+    const double workgroups = (double)(B * Hkv) * (double)((nk * D / 8 + 1023) / 1024);
+    if (nk <= MEAN_CHUNKS * MEAN_ROWS && workgroups <= 384.0) return MEAN_ROWS_ITSELF;
     const double read = (double)(B * Hkv) * (double)nk * (double)nk * (double)(D * D) / 262144.0;      // bytes of sums, all workgroups
     return nk <= 64 * MEAN_ROWS && read <= 14e6 ? MEAN_SUMS : MEAN_GIVEN;
 }
@@ -174,8 +187,11 @@ int mpsa_prepare_operands(const void* q, const int64_t* q_strides, const void* k
     if (rc != MPSA_OK) return rc;
     rc = mpsa_v_tiles_setup(v, dtype, B, Hkv, Nk, D, v_strides, tile, v_tiles, &p.v, &bv);
     if (rc != MPSA_OK) return rc;
-    bq /= 2;                                     // the set-ups count blocks of 256 chunks
-    bk /= 2;
+    // the set-ups count blocks of 256 chunks and of 512 words
+    const unsigned blocks = (unsigned)(threads_of(mean) / 256 * 2);
+    bq = (bq + blocks - 1) / blocks;
+    bk = (bk + blocks - 1) / blocks;
+    bv = (bv + blocks / 2 - 1) / (blocks / 2);
     const int64_t total = (int64_t)bq * Hq * B + (int64_t)(bk + bv) * Hkv * B;
     if (total >= (int64_t(1) << 30)) return mpsa_fail(MPSA_EUNSUPPORTED, "prepare: problem too large for one launch");
     p.bq = bq; p.bk = bk; p.bv = bv; p.hq = (uint32_t)Hq; p.hkv = (uint32_t)Hkv;

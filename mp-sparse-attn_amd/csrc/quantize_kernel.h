@@ -400,8 +400,10 @@ __device__ __forceinline__ void quantize_chunks(const QuantArgs& a, const QuantC
             quantize_chunk<DO4, DO8, FMT8, false, true>(x, a.pre, a.sure4 != 0, a.emax4, a.emax8, w4[i], s4[i], w8[i], s8[i]);
         }
     }
+    const uint32_t chunks = (uint32_t)a.out_rows * ((uint32_t)a.d >> 3);
 #pragma unroll
-    for (int i = 0; i < N; ++i) store_chunk<DO4, DO8>(a, q[i], head, w4[i], s4[i], w8[i], s8[i]);
+    for (int i = 0; i < N; ++i)
+        if (q[i].c < chunks) store_chunk<DO4, DO8>(a, q[i], head, w4[i], s4[i], w8[i], s8[i]);       // (whole waves)
 }
 
 // x - m in the inputs' 16-bit type

@@ -23,7 +23,7 @@ __device__ __forceinline__ float seq_sum(const float* x, int count, int stride) 
     return s;
 }
 
-// 256 threads sum MEAN_ROWS rows of one head: a thread owns 8 channels of every (256*8/D)-th row; the row
+// 256 threads, numbered t, sum MEAN_ROWS rows of one head: a thread owns 8 channels of every (256*8/D)-th row; the row
 // groups are then added in a fixed order through LDS, so the result does not depend on timing.  A thread's rows are
 // requested before the first is added: with one load in flight a short sequence took a memory round trip per row
 // (2 x 16 heads, 333 rows: 8.3 us, this way 7.5).
@@ -32,29 +32,29 @@ template <int D> struct MeanChunk {
     static constexpr int RTHREADS = 256 / CPR, EACH = MEAN_ROWS / RTHREADS;
     uint4 raw[EACH];
     // head: the head's first row; n rows, sn elements apart
-    __device__ __forceinline__ void request(const char* head, int64_t sn, int row0, int n) {
-        const char* base = head + 16 * (threadIdx.x % CPR);
+    __device__ __forceinline__ void request(const char* head, int64_t sn, int row0, int n, uint32_t t = threadIdx.x) {
+        const char* base = head + 16 * (t % CPR);
 #pragma unroll
         for (int i = 0; i < EACH; ++i) {
-            const int row = min(row0 + (int)(threadIdx.x / CPR) + i * RTHREADS, n - 1);
+            const int row = min(row0 + (int)(t / CPR) + i * RTHREADS, n - 1);
             raw[i] = *reinterpret_cast<const uint4*>(base + 2 * (int64_t)row * sn);
         }
     }
     // this thread's sums, into LDS
     template <int XDT>
-    __device__ __forceinline__ void add(float (&part)[256][9], int row0, int n) const {
+    __device__ __forceinline__ void add(float (&part)[256][9], int row0, int n, uint32_t t = threadIdx.x) const {
         const int row1 = min(row0 + MEAN_ROWS, n);
         float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < EACH; ++i) {
-            if (row0 + (int)(threadIdx.x / CPR) + i * RTHREADS >= row1) break;
+            if (row0 + (int)(t / CPR) + i * RTHREADS >= row1) break;
             float x[8];
             unpack8<XDT>(raw[i], x);
 #pragma unroll
             for (int q = 0; q < 8; ++q) acc[q] += x[q];
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) part[threadIdx.x][i] = acc[i];
+        for (int i = 0; i < 8; ++i) part[t][i] = acc[i];
     }
     // channel c's sum
     __device__ static __forceinline__ float total(const float (&part)[256][9], int c) {

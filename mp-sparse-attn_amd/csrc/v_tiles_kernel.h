@@ -18,15 +18,16 @@ int mpsa_v_tiles_setup(const void* v, int v_dtype, int64_t B, int64_t H, int64_t
 namespace {
 
 
-// One workgroup's share: 512 consecutive 16-byte output words, starting at word 512*bx, of head hh of batch bb: two a thread,
+// One workgroup's share: 2 THREADS consecutive 16-byte output words, starting at word 2*THREADS*bx, of head hh of batch bb: two a thread,
 // neighbours, whose elements lie side by side in V's rows.  Eight loads of four bytes, all in flight at once, where two words a
 // thread one after the other took sixteen of two bytes (figures: prepare.hip).
-template <int TILE, int D>
+template <int TILE, int D, int THREADS>
 __device__ __forceinline__ void v_tiles_block(const VTArgs& a, uint32_t bx, uint32_t hh, uint32_t bb, uint32_t nh) {
     constexpr int NDB = D / 32;
     constexpr int KB = TILE / 32;
     const uint32_t per_head = (uint32_t)a.nt * (TILE * D / 8);
-    const uint32_t o = bx * 512u + 2u * threadIdx.x;
+    const uint32_t o = bx * (2u * THREADS) + 2u * threadIdx.x;
+    if (o >= per_head) return;
     const uint32_t lane = o & 63u;
     uint32_t rest = o >> 6;
     const uint32_t db = rest % NDB; rest /= NDB;
@@ -60,7 +61,7 @@ __device__ __forceinline__ void v_tiles_block(const VTArgs& a, uint32_t bx, uint
 
 template <int TILE, int D>
 __global__ __launch_bounds__(256) void v_tiles_kernel(VTArgs a) {
-    v_tiles_block<TILE, D>(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
+    v_tiles_block<TILE, D, 256>(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
 }
 
 }  // namespace

@@ -1104,6 +1104,12 @@ def test_mean_inside_the_preparation_gives_the_bits_of_the_mean_on_its_own(B, Hk
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("B,Hkv,N,D", [(2, 3, 64, 64), (1, 2, 769, 128), (1, 3, 1023, 128), (1, 24, 1024, 128), (1, 25, 1024, 128), (1, 48, 960, 64), (1, 2, 1025, 128)])
+def test_mean_of_up_to_four_chunks_of_rows(B, Hkv, N, D):
+    """Heads of less than a workgroup's 1024 pieces, rows in all four of its chunks, and either side of the bounds on rows and workgroups."""
+    test_mean_inside_the_preparation_gives_the_bits_of_the_mean_on_its_own(B, Hkv, N, D, "NHD", "diag", torch.bfloat16)
+
+
 @pytest.mark.parametrize("mode,Nk", [("mxfp8", n) for n in (1, 31, 32, 77, 333, 352, 353)] + [("mixed", n) for n in (33, 300, 447, 448, 449)] + [("mxfp8e5", 100), ("mixed_e5", 64)])
 @pytest.mark.parametrize("B,Hq,Hkv,Nq,dtype,layout,climb", [(2, 16, 16, 4100, torch.bfloat16, "NHD", False), (1, 12, 4, 11001, torch.float16, "HND", True),
                                                              (3, 96, 8, 331, torch.bfloat16, "HND", True), (33, 16, 16, 250, torch.float16, "NHD", False)])
