@@ -20,7 +20,7 @@ BENCH_SOURCES = ["bench/mfma_stream.hip"]
 # the host side of short calls (csrc/host.cpp): a Python extension over torch's C++ API and libmpsa.so
 HOST_LIB = os.path.join(LIBDIR, "mpsa_host.so")
 
-SOURCES = ["api.hip", "formats.hip", "quantize.hip", "v_tiles.hip", "prepare.hip", "gemm_mx.hip", "gemm_mx_split.hip", "gemm_mx_tile.hip", "gemm_mx_edge.hip", "gemm_mx_stage.hip", "attn_fwd.hip", "attn_fwd_skip.hip", "attn_fwd_routed.hip", "attn_fwd_pp.hip", "attn_fwd_tile.hip", "attn_call.hip", "attn_fwd_short.hip", "attn_fwd_resident.hip", "route.hip", "skip_route.hip"]
+SOURCES = ["api.hip", "formats.hip", "quantize.hip", "v_tiles.hip", "prepare.hip", "gemm_mx.hip", "gemm_mx_split.hip", "gemm_mx_tile.hip", "gemm_mx_edge.hip", "gemm_mx_stage.hip", "attn_fwd.hip", "attn_fwd_skip.hip", "attn_fwd_routed.hip", "attn_fwd_pp.hip", "attn_fwd_tile.hip", "attn_call.hip", "attn_fwd_short.hip", "attn_fwd_prompt.hip", "attn_fwd_resident.hip", "route.hip", "skip_route.hip"]
 
 # packed-fp32 instructions are switched off on purpose (the flag is for the device pass; the host
 # pass warns that it does not know the feature, which is harmless)

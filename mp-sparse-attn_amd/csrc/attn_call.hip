@@ -103,6 +103,7 @@ extern "C" int mpsa_attn_call_on(int kernel, const mpsa_attn_desc* d, const void
     if (rc != MPSA_OK) return rc;
     if (!q || !k || !v || !o || !workspace) return mpsa_fail(MPSA_EINVAL, "attn call: null pointer");
     if (!mpsa_aligned16(workspace)) return mpsa_fail(MPSA_EALIGN, "attn call: the workspace must be 16-byte aligned");
+    if (!skipped_share && attn_prompt_supported(d, l.kernel, q, k, v, o)) return attn_prompt_launch(d, q, k, v, o, (hipStream_t)stream);
     uint8_t* const w = static_cast<uint8_t*>(workspace);
     auto at = [&](int64_t off) { return off < 0 ? nullptr : w + off; };
     uint8_t *q4 = at(l.q4), *qs4 = at(l.qs4), *q8 = at(l.q8), *qs8 = at(l.qs8), *k4 = at(l.k4), *ks4 = at(l.ks4), *k8 = at(l.k8), *ks8 = at(l.ks8);

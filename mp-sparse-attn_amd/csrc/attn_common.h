@@ -185,6 +185,11 @@ int attn_short_launch(const AttnArgs& a, int pv_dtype, int splits, hipStream_t s
 int attn_resident_shares(const AttnArgs& a);
 int attn_resident_launch(const AttnArgs& a, int pv_dtype, int shares, hipStream_t st);
 
+// The four-split kernel's math from unquantized Q, K and V, in one launch (attn_fwd_prompt.hip): the whole of a call that takes that
+// kernel, over few keys; same bits
+bool attn_prompt_supported(const mpsa_attn_desc* d, int kernel, const void* q, const void* k, const void* v, const void* o);
+int attn_prompt_launch(const mpsa_attn_desc* d, const void* q, const void* k, const void* v, void* o, hipStream_t st);
+
 // Tile-skipping variants of the general kernel (modes mxfp4 / mxfp8): attn_fwd_skip.hip
 int attn_skip_launch(const AttnArgs& a, int pv_dtype, hipStream_t st);
 

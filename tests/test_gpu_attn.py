@@ -940,6 +940,39 @@ def test_rare_blocks_of_q_and_k_under_a_scale_that_needs_no_check(bst, dtype):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a, nan=0.0), torch.nan_to_num(b, nan=0.0)), kernel
 
 
+@pytest.mark.parametrize("N,Nk", [(128, 128), (129, 129), (160, 160), (225, 225), (256, 256), (257, 257), (1, 1), (33, 33), (130, 31), (200, 97), (97, 256)])
+@pytest.mark.parametrize("bst", ["diag", "diag_e5", "mxfp4", "mxfp8", "mixed"])
+@pytest.mark.parametrize("causal", [True, False])
+def test_one_launch_over_few_keys_gives_the_staged_route(N, Nk, bst, causal):
+    """Q, K and V quantized and laid out by the attention kernel itself: the oracle's result, and the bits of the preparation followed by the
+    four-split kernel, for both layouts and types, tiles of 64, rows of V at odd elements (which go the long way), NaN, infinities,
+    blocks of zeros and scales too small for the conversions."""
+    from mfma8_model import product_8bit
+    from ours.mxfp_attn_kernel import prepare_operands, attention_from_operands
+    if N != Nk and (causal or bst.startswith("diag")):
+        pytest.skip("as many queries as keys")
+    q, k, v = (make_qkv(2, 4, 2, n, 128, seed=3100 + n, dtype=torch.bfloat16, outliers=True)[i] for i, n in enumerate((N, Nk, Nk)))
+    # (outlier channels of q and k coincide in some heads: scores as the 8-bit matrix instruction adds them)
+    want = O.attn_mx(q, k, v, tile=128, causal=causal, mode=bst.replace("_e5", ""), fmt8=O.FMT_E5M2 if bst.endswith("e5") else O.FMT_E4M3, out_dtype=torch.float32, score8=product_8bit)
+    _check(q, k, v, want, f"one launch, {bst} {N}x{Nk}", is_causal=causal, block_scale_type=bst, tile=128, kernel="short4")
+    for dtype, tile, rare in ((torch.bfloat16, 128, False), (torch.float16, 64, False), (torch.float16, 128, True), (torch.bfloat16, 64, True)):
+        a, b, c = (x.float() for x in (q, k, v))
+        if rare:
+            for x in (a, b):
+                rows = x.shape[2]
+                x[0, 1, rows // 2, 40], x[0, 0, rows - 1, 3], x[1, 0, rows // 3, 127] = float("nan"), float("-inf"), float("inf")
+                x[1, 1, rows // 4, 32:64], x[1, 1, rows // 5, :32] = 0.0, x[1, 1, rows // 5, :32] * (1e-7 if dtype == torch.float16 else 1e-34)
+            c[1, 1, c.shape[2] - 1, 5] = float("inf")
+        a, b, c = (x.to(dtype).to(DEV) for x in (a, b, c))
+        staged = torch.empty((2, 4, N, 128), dtype=torch.float32, device=DEV)
+        attention_from_operands(prepare_operands(a, b, c, tile, bst, fuse_q=True), staged, causal, kernel="short4")
+        odd = torch.empty(2, 2, Nk, 129, dtype=dtype, device=DEV)[..., 1:].copy_(c)
+        by_token = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in (a, b, c)]
+        for x in ((a, b, c), (a, b, odd), by_token):
+            got = mxfp_attn_kernel(*x, is_causal=causal, block_scale_type=bst, tile=tile, output_dtype=torch.float32, kernel="short4")
+            assert torch.equal(torch.isnan(got), torch.isnan(staged)) and torch.equal(torch.nan_to_num(got, nan=0.0), torch.nan_to_num(staged, nan=0.0)), (dtype, tile, rare)
+
+
 def test_q16_entry_point_rejects_other_shapes():
     L = _lib.lib()
     assert L.mpsa_attn_fwd_q16_supported(1, 32, 8, 8192, 128, 128, 1, _lib.MODE_DIAG) == 1
