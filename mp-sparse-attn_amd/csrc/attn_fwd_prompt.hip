@@ -14,7 +14,7 @@
 // 7.8, 4-bit 11.0 -> 7.8, 256 tokens 10.8 -> 8.7; 24 heads, 300 queries over 256 keys, 8-bit, 10.6 -> 8.6; 1000 queries over 77 keys, 8 heads 10.6 -> 7.9.
 // What is left of 7.8 is the host's; the kernel's 7.2 are the wait for memory, 0.25 a block of keys, and the splits' last blocks.
 #include "attn_common.h"
-#include "quantize_kernel.h"
+#include "seq_mean_kernel.h"
 #include "reciprocal.h"
 
 namespace {
@@ -24,6 +24,7 @@ struct PromptArgs : AttnArgs {
     int64_t k_sb, k_sh, k_sn, v_sb, v_sh, v_sn;
     Reciprocal by_units, by_group, by_hkv;
     int units, group, nqb, k_sure;
+    float inv_n;
 };
 
 constexpr int KS = 4, D = 128, UNITS = D / 16 / KS;              // splits; 16-dim units each split finishes
@@ -45,12 +46,13 @@ template <int MODE> struct Prompt {
 __device__ __forceinline__ int at4(int r, int c) { return r * 64 + (((c >> 2) ^ ((r >> 2) & 3)) << 4) + 4 * (c & 3); }
 __device__ __forceinline__ int at8(int r, int c) { return r * 128 + (((c >> 1) ^ ((r >> 1) & 7)) << 4) + 8 * (c & 1); }
 
-template <int PVT, int FMT8, int MODE>
+template <int PVT, int FMT8, int MODE, bool SMOOTH>
 __global__ __launch_bounds__(THREADS, 2) void attn_prompt_kernel(PromptArgs a) {
     typedef PV<PVT> P;
     typedef Prompt<MODE> G;
     __shared__ __attribute__((aligned(16))) uint8_t smem[G::SMEM];
     __shared__ float ml[KS * 64];                                // [split][maximum, sum][query]
+    __shared__ __attribute__((aligned(16))) uint16_t mean[SMOOTH ? D : 8];
     v4f* const parts = reinterpret_cast<v4f*>(smem);
     const int tid = threadIdx.x, lane = tid & 63, split = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, r = lane & 31;
@@ -92,13 +94,31 @@ __global__ __launch_bounds__(THREADS, 2) void attn_prompt_kernel(PromptArgs a) {
     uint32_t v[2][2][8], v_next[2][2][8];
     if (split < KS && split < mine) request_v(split, v);
     if (split < KS && split + KS < mine) request_v(split + KS, v_next);
+    MeanChunk<D> head;
+    if (SMOOTH && tid < 256) head.request(kg, a.k_sn, 0, a.n, tid);
     __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the mean over the head's keys: the additions of mpsa_seq_mean, one chunk of MEAN_ROWS, in their order ----
+    if constexpr (SMOOTH) {
+        static_assert(32 * MAX_BLOCKS <= MEAN_ROWS && sizeof(float[256][9]) <= G::SMEM, "one chunk; its sums lie where the operands will");
+        float (&part)[256][9] = *reinterpret_cast<float (*)[256][9]>(smem);
+        if (tid < 256) head.template add<PVT>(part, 0, a.n, tid);
+        __syncthreads();
+        if (tid < D) mean[tid] = mean_bits<PVT>((0.0f + MeanChunk<D>::total(part, tid)) * a.inv_n);
+        __syncthreads();
+    }
 
     // ---- operands of the score product into LDS: straight through, and where a wave has a rare chunk, or 4-bit codes are the rule's
     //      to look at, again the careful way (quantize_kernel.h).  Rows past the last are zeros, like the quantizer's padding. ----
-    auto put = [&](auto do4, auto do8, const uint4& y, int row0, int n, float pre, bool sure, uint8_t* to4, uint8_t* to8) __attribute__((always_inline)) {
+    auto put = [&](auto do4, auto do8, auto key, const uint4& y, int row0, int n, float pre, bool sure, uint8_t* to4, uint8_t* to8) __attribute__((always_inline)) {
         constexpr bool DO4 = decltype(do4)::value, DO8 = decltype(do8)::value;
-        const uint4 raw = row0 + crow < n ? y : make_uint4(0, 0, 0, 0);
+        const bool inside = row0 + crow < n;
+        auto values = [&](const uint4& raw, float (&x)[8]) __attribute__((always_inline)) {
+            unpack8<PVT>(raw, x);
+            if constexpr (SMOOTH && decltype(key)::value) less_mean<PVT>(x, *reinterpret_cast<const uint4*>(mean + 8 * chunk));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = inside ? x[e] : 0.0f;
+        };
         float x[8];
         uint32_t w4 = 0;
         uint2 w8 = make_uint2(0, 0);
@@ -106,14 +126,14 @@ __global__ __launch_bounds__(THREADS, 2) void attn_prompt_kernel(PromptArgs a) {
         bool again = DO4 && !sure;
         if (!again) {
             bool rare;
-            unpack8<PVT>(raw, x);
+            values(y, x);
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] *= pre;
             quantize_straight<DO4, DO8, FMT8>(x, w4, s4, w8, s8, rare);
             again = __ballot(rare) != 0;
         }
         if (again) {
-            unpack8<PVT>(only_here(raw), x);
+            values(only_here(y), x);
             quantize_chunk<DO4, DO8, FMT8, false, true>(x, pre, sure, 3, 7, w4, s4, w8, s8);
         }
         if constexpr (DO4) {
@@ -125,12 +145,12 @@ __global__ __launch_bounds__(THREADS, 2) void attn_prompt_kernel(PromptArgs a) {
             to8[G::ROWS8 + 4 * crow + (chunk >> 2)] = (uint8_t)s8;
         }
     };
-    put(std::bool_constant<G::Q4>{}, std::bool_constant<G::Q8>{}, q, 32 * qb, a.nq, a.q_pre, a.q_sure != 0, smem, smem + G::Q8AT);
+    put(std::bool_constant<G::Q4>{}, std::bool_constant<G::Q8>{}, std::false_type{}, q, 32 * qb, a.nq, a.q_pre, a.q_sure != 0, smem, smem + G::Q8AT);
 #pragma unroll 1
     for (int kb = 0; kb < mine; ++kb) {
         uint8_t* const to = smem + G::KAT + kb * G::KBLOCK;
-        if (!G::K4 || (G::DIAG && kb >= own_first && kb < own_end)) put(std::false_type{}, std::true_type{}, k[0], 32 * kb, a.n, 1.0f, true, nullptr, to);
-        else if constexpr (G::K4)                                   put(std::true_type{}, std::false_type{}, k[0], 32 * kb, a.n, 1.0f, a.k_sure != 0, to, nullptr);
+        if (!G::K4 || (G::DIAG && kb >= own_first && kb < own_end)) put(std::false_type{}, std::true_type{}, std::true_type{}, k[0], 32 * kb, a.n, 1.0f, true, nullptr, to);
+        else if constexpr (G::K4)                                   put(std::true_type{}, std::false_type{}, std::true_type{}, k[0], 32 * kb, a.n, 1.0f, a.k_sure != 0, to, nullptr);
 #pragma unroll
         for (int x = 0; x < MAX_BLOCKS - 1; ++x) k[x] = k[x + 1];
     }
@@ -338,30 +358,35 @@ __global__ __launch_bounds__(THREADS, 2) void attn_prompt_kernel(PromptArgs a) {
 }
 
 template <int PVT, int FMT8, int MODE>
-void launch(const PromptArgs& a, unsigned grid, hipStream_t st) { hipLaunchKernelGGL((attn_prompt_kernel<PVT, FMT8, MODE>), dim3(grid), dim3(THREADS), 0, st, a); }
+void launch(const PromptArgs& a, bool smooth, unsigned grid, hipStream_t st) {
+    if (smooth) hipLaunchKernelGGL((attn_prompt_kernel<PVT, FMT8, MODE, true>), dim3(grid), dim3(THREADS), 0, st, a);
+    else        hipLaunchKernelGGL((attn_prompt_kernel<PVT, FMT8, MODE, false>), dim3(grid), dim3(THREADS), 0, st, a);
+}
 
 template <int PVT, int FMT8>
-void launch_mode(const PromptArgs& a, unsigned grid, hipStream_t st) {
-    if (a.mode == MPSA_MODE_MIXED)      launch<PVT, FMT8, MPSA_MODE_MIXED>(a, grid, st);
-    else if (a.mode == MPSA_MODE_MXFP8) launch<PVT, FMT8, MPSA_MODE_MXFP8>(a, grid, st);
-    else                                launch<PVT, FMT8, MPSA_MODE_DIAG>(a, grid, st);
+void launch_mode(const PromptArgs& a, bool smooth, unsigned grid, hipStream_t st) {
+    if (a.mode == MPSA_MODE_MIXED)      launch<PVT, FMT8, MPSA_MODE_MIXED>(a, smooth, grid, st);
+    else if (a.mode == MPSA_MODE_MXFP8) launch<PVT, FMT8, MPSA_MODE_MXFP8>(a, smooth, grid, st);
+    else                                launch<PVT, FMT8, MPSA_MODE_DIAG>(a, smooth, grid, st);
 }
 
 template <int PVT>
-void launch_fmt(const PromptArgs& a, unsigned grid, hipStream_t st) {
-    if (a.mode == MPSA_MODE_MXFP4)        launch<PVT, MPSA_FMT_E4M3, MPSA_MODE_MXFP4>(a, grid, st);
-    else if (a.fmt8 == MPSA_FMT_E5M2)     launch_mode<PVT, MPSA_FMT_E5M2>(a, grid, st);
-    else                                  launch_mode<PVT, MPSA_FMT_E4M3>(a, grid, st);
+void launch_fmt(const PromptArgs& a, bool smooth, unsigned grid, hipStream_t st) {
+    if (a.mode == MPSA_MODE_MXFP4)        launch<PVT, MPSA_FMT_E4M3, MPSA_MODE_MXFP4>(a, smooth, grid, st);
+    else if (a.fmt8 == MPSA_FMT_E5M2)     launch_mode<PVT, MPSA_FMT_E5M2>(a, smooth, grid, st);
+    else                                  launch_mode<PVT, MPSA_FMT_E4M3>(a, smooth, grid, st);
 }
 
 }  // namespace
 
-// For calls that are the four-split kernel's, without a mean to take off K (which wants all keys of the head first).  Up to 256 keys:
+// For calls that are the four-split kernel's.  Up to 256 keys:
 // every key block costs each workgroup 0.25 us and every second one of a wave 0.5, and at 256 causal ones the kernels' time alone is that of the two
 // launches (8.3 and 8.9 us; 201 tokens 8.0 and 8.7); whole calls gain more (10.8 -> 8.7), since the host's launch is saved too.  The operands of
-// eight blocks are also what fits the static 64 KB of LDS next to Q's.
+// eight blocks are also what fits the static 64 KB of LDS next to Q's.  With a mean to take off K, every workgroup reads all of the head's keys a
+// second time: 160 tokens, diag, 11.3 -> 9.7 us a call, kernels 10.2 -> 9.3; 201 tokens 11.4 -> 10.6, 10.5 -> 10.3; 256 tokens, 4-bit, 11.2 -> 10.7 but
+// the kernels 10.2 -> 10.6, so up to 224.
 bool attn_prompt_supported(const mpsa_attn_desc* d, int kernel, const void* q, const void* k, const void* v, const void* o) {
-    if (kernel != MPSA_ATTN_SHORT4 || d->D != 128 || d->smooth_k || d->skip || d->nk > 32 * MAX_BLOCKS) return false;
+    if (kernel != MPSA_ATTN_SHORT4 || d->D != 128 || d->skip || d->nk > (d->smooth_k ? 224 : 32 * MAX_BLOCKS)) return false;
     if (mpsa_quantize_sw_encoders()) return false;
     // rows on 16 bytes (V: elements two at a time), as the kernel reads them; the other path copes with the rest or refuses it
     const int64_t* const qs = d->q_strides; const int64_t* const ks = d->k_strides; const int64_t* const vs = d->v_strides; const int64_t* const os = d->o_strides;
@@ -384,11 +409,12 @@ int attn_prompt_launch(const mpsa_attn_desc* d, const void* q, const void* k, co
     a.k_sure = mpsa_e2m1_sure(1.0f, d->dtype) ? 1 : 0;
     a.B = (int)d->B; a.Hq = (int)d->Hq; a.Hkv = (int)d->Hkv; a.n = (int)d->nk; a.nq = (int)d->nq;
     a.causal = d->causal ? 1 : 0; a.mode = d->mode; a.fmt8 = d->fmt8; a.o_dtype = d->o_dtype; a.tile = d->tile;
+    a.inv_n = 1.0f / (float)d->nk;
     a.units = a.B * a.Hkv; a.group = a.Hq / a.Hkv; a.nqb = (a.nq + 31) / 32;
     a.by_units = reciprocal_of((uint32_t)a.units); a.by_group = reciprocal_of((uint32_t)a.group); a.by_hkv = reciprocal_of((uint32_t)a.Hkv);
     const unsigned grid = (unsigned)(a.units * a.group * a.nqb);
-    if (d->dtype == MPSA_BF16) launch_fmt<MPSA_BF16>(a, grid, st);
-    else                       launch_fmt<MPSA_F16>(a, grid, st);
+    if (d->dtype == MPSA_BF16) launch_fmt<MPSA_BF16>(a, d->smooth_k != 0, grid, st);
+    else                       launch_fmt<MPSA_F16>(a, d->smooth_k != 0, grid, st);
     MPSA_CHECK_LAUNCH("attn (prompt)");
     return MPSA_OK;
 }

@@ -973,6 +973,27 @@ def test_one_launch_over_few_keys_gives_the_staged_route(N, Nk, bst, causal):
             assert torch.equal(torch.isnan(got), torch.isnan(staged)) and torch.equal(torch.nan_to_num(got, nan=0.0), torch.nan_to_num(staged, nan=0.0)), (dtype, tile, rare)
 
 
+@pytest.mark.parametrize("N,Nk", [(128, 128), (161, 161), (224, 224), (225, 225), (1, 1), (40, 40), (150, 31), (130, 223)])
+@pytest.mark.parametrize("bst", ["diag", "mxfp4", "mxfp8", "mixed_e5"])
+@pytest.mark.parametrize("causal", [True, False])
+def test_one_launch_with_the_mean_gives_the_staged_route(N, Nk, bst, causal):
+    """K less its mean over the sequence inside the one launch: the bits of the mean on its own, the preparation and the four-split kernel.
+    One channel block of a head is the same for all keys (zeros without the mean), another has a large common offset."""
+    from ours.mxfp_attn_kernel import prepare_operands, attention_from_operands
+    if N != Nk and (causal or bst == "diag"):
+        pytest.skip("as many queries as keys")
+    q, k, v = (make_qkv(2, 4, 2, n, 128, seed=3200 + n, dtype=torch.float32)[i] for i, n in enumerate((N, Nk, Nk)))
+    k[0, 1, :, 32:64] = 1.5
+    k[1, 0, :, 64:96] += 40.0
+    for dtype, tile in ((torch.bfloat16, 128), (torch.float16, 64)):
+        a, b, c = (x.to(dtype).to(DEV) for x in (q, k, v))
+        staged = torch.empty((2, 4, N, 128), dtype=torch.float32, device=DEV)
+        attention_from_operands(prepare_operands(a, b, c, tile, bst, smooth_k=True, fuse_q=True), staged, causal, kernel="short4")
+        for x in ((a, b, c), [x.transpose(1, 2).contiguous().transpose(1, 2) for x in (a, b, c)]):
+            got = mxfp_attn_kernel(*x, is_causal=causal, smooth_k=True, block_scale_type=bst, tile=tile, output_dtype=torch.float32, kernel="short4")
+            assert torch.equal(got, staged), (dtype, tile)
+
+
 def test_q16_entry_point_rejects_other_shapes():
     L = _lib.lib()
     assert L.mpsa_attn_fwd_q16_supported(1, 32, 8, 8192, 128, 128, 1, _lib.MODE_DIAG) == 1
