@@ -384,7 +384,9 @@ void launch_fmt(const PromptArgs& a, bool smooth, unsigned grid, hipStream_t st)
 // launches (8.3 and 8.9 us; 201 tokens 8.0 and 8.7); whole calls gain more (10.8 -> 8.7), since the host's launch is saved too.  The operands of
 // eight blocks are also what fits the static 64 KB of LDS next to Q's.  With a mean to take off K, every workgroup reads all of the head's keys a
 // second time: 160 tokens, diag, 11.3 -> 9.7 us a call, kernels 10.2 -> 9.3; 201 tokens 11.4 -> 10.6, 10.5 -> 10.3; 256 tokens, 4-bit, 11.2 -> 10.7 but
-// the kernels 10.2 -> 10.6, so up to 224.
+// the kernels 10.2 -> 10.6, so up to 224.  And up to 256 workgroups, one a CU: a second round quantizes everything again, and the choice has gone
+// over to two splits by then.  By name, two launches -> one, us (workgroups): 160 tokens, diag, 10.8 -> 7.8 (160), 13.6 -> 9.9 (320), 18.7 -> 15.6 (640); 31
+// keys 26.4 -> 25.0 (1512); 340 queries over 256 keys 14.9 -> 14.7 (264), over 224 with a mean 15.7 -> 18.0 (264); 31 with a mean 27.3 -> 29.9 (1512).
 bool attn_prompt_supported(const mpsa_attn_desc* d, int kernel, const void* q, const void* k, const void* v, const void* o) {
     if (kernel != MPSA_ATTN_SHORT4 || d->D != 128 || d->skip || d->nk > (d->smooth_k ? 224 : 32 * MAX_BLOCKS)) return false;
     if (mpsa_quantize_sw_encoders()) return false;
@@ -395,7 +397,7 @@ bool attn_prompt_supported(const mpsa_attn_desc* d, int kernel, const void* q, c
     if ((d->dtype != MPSA_BF16 && d->dtype != MPSA_F16) || (d->o_dtype != MPSA_BF16 && d->o_dtype != MPSA_F16 && d->o_dtype != MPSA_F32)) return false;
     if (d->mode == MPSA_MODE_ROUTED || (d->mode != MPSA_MODE_MXFP4 && d->fmt8 != MPSA_FMT_E4M3 && d->fmt8 != MPSA_FMT_E5M2)) return false;
     if (d->nq != d->nk && (d->causal || d->mode == MPSA_MODE_DIAG)) return false;
-    return d->B <= 65535 && d->Hkv <= 65535 && d->nq < (int64_t(1) << 30) && d->B * d->Hq * ((d->nq + 31) / 32) < (int64_t(1) << 24);
+    return d->B <= 256 && d->Hq <= 256 && d->nq <= 256 * 32 && d->B * d->Hq * ((d->nq + 31) / 32) <= 256;
 }
 
 int attn_prompt_launch(const mpsa_attn_desc* d, const void* q, const void* k, const void* v, void* o, hipStream_t st) {

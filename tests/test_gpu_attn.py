@@ -940,7 +940,7 @@ def test_rare_blocks_of_q_and_k_under_a_scale_that_needs_no_check(bst, dtype):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a, nan=0.0), torch.nan_to_num(b, nan=0.0)), kernel
 
 
-@pytest.mark.parametrize("N,Nk", [(128, 128), (129, 129), (160, 160), (225, 225), (256, 256), (257, 257), (1, 1), (33, 33), (130, 31), (200, 97), (97, 256)])
+@pytest.mark.parametrize("N,Nk", [(128, 128), (129, 129), (160, 160), (225, 225), (256, 256), (257, 257), (1, 1), (33, 33), (130, 31), (200, 97), (97, 256), (1024, 64), (1025, 64)])
 @pytest.mark.parametrize("bst", ["diag", "diag_e5", "mxfp4", "mxfp8", "mixed"])
 @pytest.mark.parametrize("causal", [True, False])
 def test_one_launch_over_few_keys_gives_the_staged_route(N, Nk, bst, causal):
@@ -973,7 +973,7 @@ def test_one_launch_over_few_keys_gives_the_staged_route(N, Nk, bst, causal):
             assert torch.equal(torch.isnan(got), torch.isnan(staged)) and torch.equal(torch.nan_to_num(got, nan=0.0), torch.nan_to_num(staged, nan=0.0)), (dtype, tile, rare)
 
 
-@pytest.mark.parametrize("N,Nk", [(128, 128), (161, 161), (224, 224), (225, 225), (1, 1), (40, 40), (150, 31), (130, 223)])
+@pytest.mark.parametrize("N,Nk", [(128, 128), (161, 161), (224, 224), (225, 225), (1, 1), (40, 40), (150, 31), (130, 223), (1024, 40), (1025, 40)])
 @pytest.mark.parametrize("bst", ["diag", "mxfp4", "mxfp8", "mixed_e5"])
 @pytest.mark.parametrize("causal", [True, False])
 def test_one_launch_with_the_mean_gives_the_staged_route(N, Nk, bst, causal):
