@@ -12,7 +12,8 @@
 // 8.6): 7.2; quantized by four waves 8.9; by every wave for itself, in registers, 9.2 (16 bytes of every 64 a lane are
 // read, and one wave has two blocks to do where three have one).  Whole calls, two launches -> one: 160 tokens, 32 heads over 8, diag 10.8 ->
 // 7.8, 4-bit 11.0 -> 7.8, 256 tokens 10.8 -> 8.7; 24 heads, 300 queries over 256 keys, 8-bit, 10.6 -> 8.6; 1000 queries over 77 keys, 8 heads 10.6 -> 7.9.
-// What is left of 7.8 is the host's; the kernel's 7.2 are the wait for memory, 0.25 a block of keys, and the splits' last blocks.
+// What bounds the 7.8 is the kernel again (a call that allocates no workspace takes as long): its 7.2 are the wait for memory, 0.25 a block of
+// keys, two blocks of scores one after the other in the first wave, and the merge.
 #include "attn_common.h"
 #include "seq_mean_kernel.h"
 #include "reciprocal.h"
