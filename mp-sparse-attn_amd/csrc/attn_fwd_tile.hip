@@ -14,7 +14,7 @@
 // 80 KiB hold two V tiles and two 4-bit K tiles.  A K tile's fragments are in registers a step before its scores, so its
 // buffer takes the tile two steps on; the tile that has to be done again is read from memory.  An 8-bit tile takes both K
 // buffers: its fragments are read at its scores, and a second barrier says that everybody has them.
-// No register is to spare: 242 to 256 without spills.  A spilled register in a long loop costs more than its reload: the wait for
+// No register is to spare: 241 to 256 without spills.  A spilled register in a long loop costs more than its reload: the wait for
 // it waits for the tiles that are on their way as well (40 heads of 32760 tokens, diag, 12.7 ms with three of them, 11.7 without).
 #include "attn_q_raw.h"
 
@@ -315,16 +315,23 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(AttnArgs a) {
     };
     auto softmax = [&](bool first, int limit) __attribute__((always_inline)) {
         if (__any(limit < TILE)) {
-            const int past = limit - 4 * (lane_now() >> 5);
+            int past = limit - 4 * (lane_now() >> 5);
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    // as assembly each comparison's mask is used at once: the compiler makes 64 of them first, more than there
-                    // are scalar registers
-                    float x = st[kb][e];
-                    asm("v_cmp_ge_i32 vcc, %1, %2\n\tv_cndmask_b32 %0, %0, %3, vcc" : "+v"(x) : "s"(32 * kb + 8 * (e >> 2) + (e & 3)), "v"(past), "v"(-__builtin_inff()) : "vcc");
-                    st[kb][e] = x;
+                for (int e = 0; e < 16; e += 2) {
+                    // Two comparisons, then their two selections: left alone the compiler makes all 64 masks first, more than there
+                    // are scalar registers, and four at a time spill one of the diag mode's.  The statements hold no instruction, so the
+                    // waits between matrix instructions, comparisons and selections are the compiler's.
+                    const int key = 32 * kb + 8 * (e >> 2) + (e & 3);
+                    asm volatile("" : "+v"(past));
+                    uint64_t live0 = __builtin_amdgcn_ballot_w64(key < past), live1 = __builtin_amdgcn_ballot_w64(key + 1 < past);
+                    asm volatile("" : "+s"(live0), "+s"(live1));
+                    float x0 = __builtin_amdgcn_inverse_ballot_w64(live0) ? st[kb][e] : -__builtin_inff();
+                    float x1 = __builtin_amdgcn_inverse_ballot_w64(live1) ? st[kb][e + 1] : -__builtin_inff();
+                    asm volatile("" : "+v"(x0), "+v"(x1));
+                    st[kb][e] = x0;
+                    st[kb][e + 1] = x1;
                 }
         }
         const float mx = row_max();
