@@ -294,6 +294,9 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 3) void attn_short_kernel(Short
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < G::SST; ++s) st = score_mfma8<FMT8>(kf[s], q8f[DIAG ? s : 0], st, s, ks, qs8);
+            // 20 wait states lie between an 8-bit product and the use of its result, 12 behind a 4-bit one; where the two paths meet
+            // the compiler counted 12 for both
+            asm volatile("s_nop 7" : "+v"(st));
         } else {
             const uint32_t ks_word = *reinterpret_cast<const uint32_t*>(smem + G::KSC + now * 1024 + w * 256 + lane * 4) >> (D == 128 ? 0 : 16 * (r & 1));
             const int ks = (int)(ks_word >> (8 * h)), f = (r >> G::SH) & (G::CPR - 1);
