@@ -175,8 +175,11 @@ __global__ __launch_bounds__(TILE * 2, 2) void attn_fwd_kernel(AttnArgs a) {
         if constexpr (ROUTED || SKIP || MODE == MPSA_MODE_MXFP8) asm volatile("" : "+v"(ln));
         return ln;
     };
+    // A tile's number, in a scalar register before the addresses are computed: computed by vector instructions and broadcast, an address
+    // would have to lie there five instructions before the load, and the compiler does not count those of an assembly statement.
+    auto uniform = [](int j) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(j); };
     auto issue_k4 = [&](int t, int j) __attribute__((always_inline)) {    // 4-bit K tile j (step t) -> kbuf[t & 1], swizzled rows
-        const uint8_t* src = a.k4 + (khead_row + (int64_t)j * TILE) * G::ROW4;
+        const uint8_t* src = a.k4 + (khead_row + (int64_t)uniform(j) * TILE) * G::ROW4;
         uint8_t* dst = kbuf0 + (t & 1) * G::K_BYTES;
         const int ln = opaque_lane();
 #pragma unroll
@@ -188,7 +191,7 @@ __global__ __launch_bounds__(TILE * 2, 2) void attn_fwd_kernel(AttnArgs a) {
         }
     };
     auto issue_k8 = [&](int j) __attribute__((always_inline)) {           // 8-bit K tile j -> the K area (one buffer), swizzled rows
-        const uint8_t* src = a.k8 + (khead_row + (int64_t)j * TILE) * G::ROW8;
+        const uint8_t* src = a.k8 + (khead_row + (int64_t)uniform(j) * TILE) * G::ROW8;
         const int ln = opaque_lane();
 #pragma unroll
         for (int c = 0; c < (PRE8 ? G::KI8 : 0); ++c) {
@@ -199,7 +202,7 @@ __global__ __launch_bounds__(TILE * 2, 2) void attn_fwd_kernel(AttnArgs a) {
         }
     };
     auto issue_v = [&](int t, int j) __attribute__((always_inline)) {     // V tile j (step t) -> vbuf[t & 1], flat
-        const uint8_t* src = static_cast<const uint8_t*>(a.v) + (khead_row + (int64_t)j * TILE) * (D * 2);
+        const uint8_t* src = static_cast<const uint8_t*>(a.v) + (khead_row + (int64_t)uniform(j) * TILE) * (D * 2);
         uint8_t* dst = vbuf0 + (t & 1) * G::V_BYTES;
         const uint32_t lo = (uint32_t)opaque_lane() * 16u;
 #pragma unroll

@@ -3,6 +3,7 @@ them, but puts none inside an inline assembly statement, and counts no instructi
 uses its result, counted in instructions issued between (s_nop n counts n + 1):
 
 - mask: a vector instruction that writes a mask or another scalar register, to a vector instruction that reads it: 2
+- address: the same, to a memory instruction: 5
 - transcendental: such an instruction, to a vector instruction of another kind that reads its result: 1
 - matrix: a matrix instruction, to a vector instruction or a store that reads its result: its passes and 4.  The compiler takes some
   branches out again that it has counted, so 2 fewer are let pass here.
@@ -68,7 +69,9 @@ def too_close(text):
             read = {r for o in operands[0 if "swap" in op else results:] for r in registers(o)}
             for r in read & last.keys():
                 at, rule, states, by = last[r]
-                wanted = {"mask": 2 if vector else 0, "transcendental": 1 if vector and not op.startswith(TRANS) else 0,
+                if rule == "mask" and not vector:
+                    rule = "address"
+                wanted = {"mask": 2, "address": 5, "transcendental": 1 if vector and not op.startswith(TRANS) else 0,
                           "matrix": 0 if matrix or not (vector or "store" in op) else states}[rule]
                 if now - at - 1 < wanted:
                     bad.append((rule, kernel, by, line, now - at - 1))
@@ -121,7 +124,7 @@ def library(tmp_path_factory):
     return [b for _, found in done for b in found]
 
 
-@pytest.mark.parametrize("rule", ["mask", "transcendental", "matrix"])
+@pytest.mark.parametrize("rule", ["mask", "address", "transcendental", "matrix"])
 def test_no_result_is_used_too_early(library, rule):
     bad = [b[1:] for b in library if b[0] == rule]
     assert not bad, (len(bad), bad[:4])
@@ -131,6 +134,12 @@ def test_no_result_is_used_too_early(library, rule):
 def test_masks_in_a_listing(between, states):
     found = too_close("0000000000001900 <kernel>:\n\tv_cmp_ge_i32_e32 vcc, s3, v66\n" + between + "\tv_cndmask_b32_e32 v51, v51, v67, vcc\n")
     assert [b[4] for b in found] == ([states] if states < 2 else [])
+
+
+@pytest.mark.parametrize("states", [0, 4, 5])
+def test_addresses_in_a_listing(states):
+    found = too_close("0000000000001900 <kernel>:\n\tv_readfirstlane_b32 s7, v5\n" + "\ts_nop 0\n" * states + "\tglobal_load_lds_dwordx4 v8, s[6:7]\n")
+    assert [(b[0], b[4]) for b in found] == ([("address", states)] if states < 5 else [])
 
 
 @pytest.mark.parametrize("op, formats, states", [("v_mfma_f32_32x32x16_bf16", "", 12), ("v_mfma_scale_f32_32x32x64_f8f6f4", " cbsz:4 blgp:4", 12),
