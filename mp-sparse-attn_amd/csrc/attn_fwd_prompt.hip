@@ -380,6 +380,16 @@ void launch_fmt(const PromptArgs& a, bool smooth, unsigned grid, hipStream_t st)
 
 }  // namespace
 
+// The bytes from a [B,H,N,128] tensor's first element to its last
+struct Extent { uintptr_t first, end; };
+static Extent extent_of(const void* p, int64_t B, int64_t H, int64_t N, const int64_t* strides, int64_t bytes) {
+    int64_t lo = 0, hi = 128;
+    const int64_t steps[3] = {(B - 1) * strides[0], (H - 1) * strides[1], (N - 1) * strides[2]};
+    for (int64_t step : steps) (step < 0 ? lo : hi) += step;
+    return {reinterpret_cast<uintptr_t>(p) + (uintptr_t)(lo * bytes), reinterpret_cast<uintptr_t>(p) + (uintptr_t)(hi * bytes)};
+}
+static bool apart(const Extent& x, const Extent& y) { return x.end <= y.first || y.end <= x.first; }
+
 // For calls that are the four-split kernel's.  Up to 256 keys:
 // every key block costs each workgroup 0.25 us and every second one of a wave 0.5, and at 256 causal ones the kernels' time alone is that of the two
 // launches (8.3 and 8.9 us; 201 tokens 8.0 and 8.7); whole calls gain more (10.8 -> 8.7), since the host's launch is saved too.  The operands of
@@ -398,7 +408,11 @@ bool attn_prompt_supported(const mpsa_attn_desc* d, int kernel, const void* q, c
     if ((d->dtype != MPSA_BF16 && d->dtype != MPSA_F16) || (d->o_dtype != MPSA_BF16 && d->o_dtype != MPSA_F16 && d->o_dtype != MPSA_F32)) return false;
     if (d->mode == MPSA_MODE_ROUTED || (d->mode != MPSA_MODE_MXFP4 && d->fmt8 != MPSA_FMT_E4M3 && d->fmt8 != MPSA_FMT_E5M2)) return false;
     if (d->nq != d->nk && (d->causal || d->mode == MPSA_MODE_DIAG)) return false;
-    return d->B <= 256 && d->Hq <= 256 && d->nq <= 256 * 32 && d->B * d->Hq * ((d->nq + 31) / 32) <= 256;
+    if (d->B > 256 || d->Hq > 256 || d->nq > 256 * 32 || d->B * d->Hq * ((d->nq + 31) / 32) > 256) return false;
+    // an output over K's or V's memory: there one workgroup would store what another has yet to read, where the preparation reads all of
+    // both before the attention kernel stores anything
+    const Extent to = extent_of(o, d->B, d->Hq, d->nq, os, d->o_dtype == MPSA_F32 ? 4 : 2);
+    return apart(to, extent_of(k, d->B, d->Hkv, d->nk, ks, 2)) && apart(to, extent_of(v, d->B, d->Hkv, d->nk, vs, 2));
 }
 
 int attn_prompt_launch(const mpsa_attn_desc* d, const void* q, const void* k, const void* v, void* o, hipStream_t st) {
