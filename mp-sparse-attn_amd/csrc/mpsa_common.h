@@ -12,7 +12,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef unsigned short v8us __attribute__((ext_vector_type(8)));
 
 // thread-local error text, filled by mpsa_fail()
 int mpsa_fail(int code, const char* fmt, ...);

@@ -70,9 +70,6 @@ __device__ __forceinline__ void unpack8(const uint4& raw, float (&x)[8]) {
     }
 }
 
-template <int XDT>
-__device__ __forceinline__ void load8(const void* p, float (&x)[8]) { unpack8<XDT>(*reinterpret_cast<const uint4*>(p), x); }
-
 // round a float32 to the 16-bit dtype XDT (nearest even) and back
 template <int XDT>
 __device__ __forceinline__ float round16(float v) {
@@ -149,15 +146,6 @@ __device__ __forceinline__ uint32_t e2m1_try8(const float (&x)[8], int se, bool 
         rule |= nearest < 2 * MIDPOINT_NEAR && !sure;
     }
     return e2m1_convert8(x, se, 1.0f);
-}
-
-template <bool HW4>
-__device__ __forceinline__ uint32_t e2m1_pack8(const float (&x)[8], int se, bool sure) {
-    if constexpr (!HW4) return e2m1_pack8_explicit(x, se);
-    bool rule;
-    uint32_t w = e2m1_try8(x, se, sure, rule);
-    if (rule) w = e2m1_pack8_rule(x, se);
-    return w;
 }
 
 // Eight FP8 codes of x[0..7] / 2^se.  The scaled conversion divides and rounds in one instruction a pair.  With the formats' own
