@@ -445,9 +445,9 @@ int mpsa_skip_route(const uint8_t* q4, const uint8_t* qs4, const uint8_t* q8, co
  * Both operand sets are needed unless the lists name tiles of one precision only: then the other set (q and k codes and
  * scales of that width) may be NULL.  Key tiles not on a query tile's list contribute nothing; a query tile with an
  * empty list returns zeros.  Out-of-range list entries and run lengths are clamped, never followed.
- * It is the general kernel's loop: lists that name one precision throughout (or, without the mask, tile i in 8 bits and the rest
- * in 4) give the bits of the fixed-precision run on MPSA_ATTN_GENERAL; the kernel that run takes by itself may add up in
- * another order.
+ * It is the loop that MPSA_ATTN_GENERAL runs at these shapes (csrc/attn_fwd_tile.hip with D = 128 and tile = 128, csrc/attn_fwd_kernel.h
+ * otherwise): lists that name one precision throughout (or, without the mask, tile i in 8 bits and the rest in 4) give the bits of
+ * the fixed-precision run by that name; the kernel that a run takes by itself may add up in another order.
  */
 int mpsa_attn_fwd_routed(const uint8_t* q4, const uint8_t* qs4, const uint8_t* q8, const uint8_t* qs8,
                          const uint8_t* k4, const uint8_t* ks4, const uint8_t* k8, const uint8_t* ks8, int fmt8,
@@ -458,7 +458,8 @@ int mpsa_attn_fwd_routed(const uint8_t* q4, const uint8_t* qs4, const uint8_t* q
 /*
  * A whole attention call -- smooth-K mean, operand preparation, routing or tile skipping, attention -- on one block of
  * caller-owned memory: the body of the reference's wrapper (ours/mxfp_attn_kernel.py:19-100) behind one entry point, for
- * callers whose short calls are bound by the host.  The same kernels with the same results as the separate entry points.
+ * callers whose short calls are bound by the host.  The same results as the separate entry points give: all of K and V is read
+ * before anything is stored, so that the output may lie over their memory; over Q's only where every query row becomes its own output row.
  * A description holds no pointers and can be kept and shared between threads; one that is not valid gives the error of
  * the entry point that refuses it.
  */

@@ -8,7 +8,8 @@
 // key/value head hq / (Hq/Hkv) (ours/online_routing.py:160-171).  Q already carries sm_scale*log2(e)
 // (folded in by the quantizer, ours/quant_mxint8.py:494), so scores are in log2 units.
 //
-// Mapping of the kernel in attn_fwd_kernel.h, which takes what D = 128 with tile = 128 (attn_fwd_tile.hip) leaves.  A workgroup owns one TILE-query tile; each of its TILE/32 waves owns 32 queries and walks all
+// Mapping of the kernel in attn_fwd_kernel.h, which takes what D = 128 with tile = 128 (attn_fwd_tile.hip) leaves, and there skipping
+// inside the kernel.  A workgroup owns one TILE-query tile; each of its TILE/32 waves owns 32 queries and walks all
 // keys of every tile.  Both products are computed transposed so that a lane always owns ONE query:
 //   S^T = K Q^T   on v_mfma_scale_f32_32x32x64_f8f6f4: lane (h = lane/32, r = lane%32) of the K operand
 //                 supplies 32 elements of key row r and the E8M0 byte of MX block h of the 64-wide step
@@ -234,12 +235,14 @@ static constexpr double SHORT_LIMIT = 16777216.0;         // blocks of 32 querie
 //   Self-attention with D = 128 and tile = 128 has two kernels that own whole query tiles: one a workgroup and two workgroups a CU (attn_fwd_tile.hip), or
 // two a workgroup of the whole CU (attn_fwd_pp.hip), which reads K and V half as often and is 1 to 7 % faster where either fills
 // the chip evenly.  Half as large workgroups fill it more evenly: without the mask the chip works in rounds of 512 or 256
-// workgroups, and a round that leaves one a CU takes 0.8 of a full one (32 heads of 2560 tokens, diag, 106 us in pairs, 88 in
-// single tiles; 64 of 1500 78, 65; 32 of 4096 178, 180); under the mask 512 workgroups or fewer run in one round, a long row beside
-// a short one (8 heads of 8192, 123 and 105; 32 of 2048 44 and 39); with 384 to 640 workgroups single tiles take 0.95 of the time where
+// workgroups, and a round that leaves one a CU takes 0.8 of a full one (32 heads of 2560 tokens, diag, 106 us in pairs, 86 in
+// single tiles; 64 of 1500 76, 61; 32 of 4096 174, 172); under the mask 512 workgroups or fewer run in one round, a long row beside
+// a short one (8 heads of 8192, 126 and 108; 32 of 2048 45 and 38); with 384 to 640 workgroups single tiles take 0.95 of the time where
 // they are chosen, with 640 to 768 0.98 to 1.01, with 768 to 1024 1.04 and with more 0.98 to 1.0, so from there on pairs.  The constants are
-// those with the least time lost over 1529 shapes of 700 to 20 000 tokens (all types, 1 - 256 heads); over 830 others the choice
-// costs 1.1 % over always taking the fastest, and without the single tiles 3.2.
+// those with the least time lost over 1529 shapes of 700 to 20 000 tokens (all types, 1 - 256 heads); over 830 others (whole calls) the choice
+// takes 1.4 % longer than the fastest kernel, which is what the fastest one besides the single tiles takes, too.  Where lengths differ, and
+// unmasked below six tiles, the single-tile kernel is not among the candidates, and MPSA_ATTN_GENERAL, which is it there behind a
+// quantization of Q, is priced as the kernel of attn_fwd_kernel.h: its constants are too high for D = 128 and tile = 128.
 static int fastest_kernel(int64_t B, int64_t Hq, bool paired, bool fits, int64_t nq, int64_t nk, int64_t D, int tile, int causal) {
     const bool d128 = D == 128;
     auto tiles = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
@@ -277,7 +280,7 @@ static int fastest_kernel(int64_t B, int64_t Hq, bool paired, bool fits, int64_t
         const double longest = wgs > 256.0 ? 10.1 + 1.3 * ntk : 4.4 + 1.36 * ntk, spread = 12.1 + 0.31 * ntk + 2.1 * wgs * (ntk + 1.0) / 2.0 / 512.0;
         if (!causal)            candidate(MPSA_ATTN_TILE, rounds * (10.3 + 1.66 * ntk));
         else if (wgs <= 640.0)  candidate(MPSA_ATTN_TILE, spread > longest ? spread : longest);
-    } else {                                                  // attn_fwd_kernel.h, and Q's quantization in front of it
+    } else {                                                  // attn_fwd_kernel.h (fitted before attn_fwd_tile.hip was), and Q's quantization in front of it
         const bool t128 = tile == 128;
         const double wgs = heads * ntq, steps = wgs * (causal ? (ntk + 1.0) / 2.0 : ntk);
         const double step = t128 ? (d128 ? 1.5 : 1.2) : (d128 ? 0.6 : 0.45), slots = d128 && t128 ? 512.0 : 1024.0;

@@ -12,8 +12,10 @@
 // 8.6): 7.2; quantized by four waves 8.9; by every wave for itself, in registers, 9.2 (16 bytes of every 64 a lane are
 // read, and one wave has two blocks to do where three have one).  Whole calls, two launches -> one: 160 tokens, 32 heads over 8, diag 10.8 ->
 // 7.8, 4-bit 11.0 -> 7.8, 256 tokens 10.8 -> 8.7; 24 heads, 300 queries over 256 keys, 8-bit, 10.6 -> 8.6; 1000 queries over 77 keys, 8 heads 10.6 -> 7.9.
-// What bounds the 7.8 is the kernel again (a call that allocates no workspace takes as long): its 7.2 are the wait for memory, 0.25 a block of
-// keys, two blocks of scores one after the other in the first wave, and the merge.
+// These are calls repeated on the same tensors, one queued behind the other; a call that is waited for, with its inputs in memory instead
+// of the caches, 18.1 -> 15.1 (4-bit, 160 tokens).  What bounds the 7.8 is the kernel again (a call that allocates no workspace takes as long).  Its
+// longest wave takes 14 200 clocks: 2 100 until all loads are asked for, 650 for its queries, 3 000 for five blocks of keys, 1 100 to the first
+// scores, 2 300 for two blocks of scores, one after the other, and 2 800 for the merge; with inputs in memory 16 500.
 #include "attn_common.h"
 #include "seq_mean_kernel.h"
 #include "reciprocal.h"
@@ -392,12 +394,13 @@ static bool apart(const Extent& x, const Extent& y) { return x.end <= y.first ||
 
 // For calls that are the four-split kernel's.  Up to 256 keys:
 // every key block costs each workgroup 0.25 us and every second one of a wave 0.5, and at 256 causal ones the kernels' time alone is that of the two
-// launches (8.3 and 8.9 us; 201 tokens 8.0 and 8.7); whole calls gain more (10.8 -> 8.7), since the host's launch is saved too.  The operands of
-// eight blocks are also what fits the static 64 KB of LDS next to Q's.  With a mean to take off K, every workgroup reads all of the head's keys a
+// launches (8.3 and 8.9 us; 201 tokens 8.0 and 8.7); whole calls gain more (10.8 -> 8.7), since the host's launch is saved too.  More than
+// eight blocks would not fit the registers that hold every block's chunk from the start, nor the two blocks of V a wave.  With a mean to take off K, every workgroup reads all of the head's keys a
 // second time: 160 tokens, diag, 11.3 -> 9.7 us a call, kernels 10.2 -> 9.3; 201 tokens 11.4 -> 10.6, 10.5 -> 10.3; 256 tokens, 4-bit, 11.2 -> 10.7 but
-// the kernels 10.2 -> 10.6, so up to 224.  And up to 256 workgroups, one a CU: a second round quantizes everything again, and the choice has gone
-// over to two splits by then.  By name, two launches -> one, us (workgroups): 160 tokens, diag, 10.8 -> 7.8 (160), 13.6 -> 9.9 (320), 18.7 -> 15.6 (640); 31
-// keys 26.4 -> 25.0 (1512); 340 queries over 256 keys 14.9 -> 14.7 (264), over 224 with a mean 15.7 -> 18.0 (264); 31 with a mean 27.3 -> 29.9 (1512).
+// the kernels 10.2 -> 10.6, so up to 224.  And up to 256 workgroups, one a CU, which is as far as the choice takes four splits at all.  Past that,
+// for callers that name the kernel, a second round quantizes everything again: with a mean that loses, 340 queries over 224 keys 15.7 -> 18.0 us (264
+// workgroups), 31 keys 27.3 -> 29.9 (1512); without one it still gains, less and less, 160 tokens, diag, 13.6 -> 9.9 (320), 18.7 -> 15.6 (640), 31 keys
+// 26.4 -> 25.0 (1512), 256 keys 14.9 -> 14.7 (264), and is left to the two launches with the rest.
 bool attn_prompt_supported(const mpsa_attn_desc* d, int kernel, const void* q, const void* k, const void* v, const void* o) {
     if (kernel != MPSA_ATTN_SHORT4 || d->D != 128 || d->skip || d->nk > (d->smooth_k ? 224 : 32 * MAX_BLOCKS)) return false;
     if (mpsa_quantize_sw_encoders()) return false;
